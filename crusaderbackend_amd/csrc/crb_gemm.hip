@@ -1,7 +1,7 @@
 // C-ABI entry points of the GEMM and dense-layer families (fp32, row-major) on the MFMA engine.
 #include "gemm_internal.h"
 #include "gemm_tiny.h"
-#include "igemm_dma.h"
+#include "igemm_split.h"
 #include "operands.h"
 
 namespace crb {
@@ -111,86 +111,93 @@ static int run_tiles(const AOp &a, const BOp &b, const E &e, u32 M, u32 N, u32 K
     }
 }
 
-// ---- products of plain dense matrices on the direct-to-LDS kernel (igemm_dma.h) ---------------------------------------------
-// Taken when the contraction is a multiple of 32, the operands are 16-byte friendly and the tile grid fills the chip in
-// whole rounds; everything else stays on the register-staged engine. Returns 0: not taken; 1: 128 x 128 tiles; 2: 64 x 64.
-struct DmaChoice {
-    int tile;    // 0: not taken; 1: 128 x 128 tiles; 2: 64 x 64; 3: 64 x 64 as eight waves
-    u32 splits;  // > 1: the contraction is cut into this many slices (dense, unbatched results only)
+// ---- products of plain matrices on the split engine (igemm_split.h) -----------------------------------------------------------
+// Eight-wave workgroups, one to a CU, so the time goes by rounds of 256 tiles; a round costs its contraction times the tile's
+// rate plus what every launch pays. Measured (NN; us per round and k, us besides): 256 x 256 tiles 0.150 and 16 (4096^3 631 us,
+// 4096 x 4096 x 256 56), 128 x 128 0.044 and 4 (2048^3 97 us, 4096^3 707), 64 x 64 0.017 and 3.5 (1024^3 20.8, 256 x 4096 x 4096
+// 73, 2048^3 138). Per result the large tile is the cheapest (2.3 : 2.7 : 4.1), the small ones waste less of a last round. The
+// 64 x 64 tile as a four-wave workgroup runs two to a CU: 0.031 per round of 512 when both places are taken (1003 x 1505 x 777,
+// 384 tiles: 30 us against 34 in two rounds of the eight-wave form).
+// With fewer tiles than CUs the contraction may be cut: partial results are written and read back once (about 5 TB/s out of the
+// memory-side cache) by one more launch (3.5 us). The choice is the smallest of these sums.
+typedef SplitCfg<256, 256, 16, 2, 4, 1, 1> SplitLarge;
+typedef SplitCfg<128, 128, 32, 2, 2, 2, 1, true> SplitMid;
+typedef SplitCfg<64, 64, 64, 1, 2, 4, 1, true> SplitSmall;
+typedef SplitCfg<64, 64, 32, 1, 2, 2, 2, true> SplitSmall2;
+struct SplitChoice {
+    int tile;  // 0 large, 1 mid, 2 small, 3 small, two to a CU
+    u32 splits, k_per_z;
 };
-static DmaChoice choose_dma(u32 M, u32 N, u32 K, u32 zdim) {
-    if (K % 32 || K < 256) return {0, 1};  // whole 32-deep slabs; a short contraction is mostly prologue and epilogue
-    const uint64_t tiles_l = uint64_t(ceil_div(M, 128)) * ceil_div(N, 128) * zdim;
-    const uint64_t tiles_s = uint64_t(ceil_div(M, 64)) * ceil_div(N, 64) * zdim;
-    // One 128 x 128 tile per CU already runs close to the MFMA rate, so the time goes by whole rounds of 256 tiles: taken
-    // when the last round is (nearly) full. Measured against the register-staged engine, NN / NT / TN alike:
-    // 2048^3 138 vs 150 us, 4096 x 4096 x 256 76 vs 83, 4096^3 1025 vs 1070; 3072^3 (2.25 rounds) 583 vs 494.
-    if (M >= 128 && N >= 128 && tiles_l >= 256 && tiles_l * 10 >= ceil_div(tiles_l, 256) * 256 * 9) return {1, 1};
-    // 64 x 64 tiles, two per CU: rounds of 512 (512 x 4096 x 1024 40.3 vs 42.8 us, 32768 x 64 x 576 25.3 vs 26.4;
-    // 1024^3 the same as the engine, 1536^3 and 1280 x 1024 x 1024 slower)
-    if (M >= 64 && N >= 64 && K >= 512 && tiles_s >= 512 && tiles_s * 20 >= ceil_div(tiles_s, 512) * 512 * 19) return {2, 1};
-    // At most one 64 x 64 tile per CU: the same tile as an eight-wave workgroup, two waves per SIMD (1024^3 24.0-24.8 us
-    // against the engine's eight-wave tiles at 24.1-25.9, 1024 x 1024 x 2048 44.6-46.1 against 45.6-47.5, 896^3 21.4-21.8
-    // against 21.4-22.8); longer contractions are better cut (below)
-    if (M >= 64 && N >= 64 && K >= 512 && K <= 2048 && tiles_s >= 160 && tiles_s <= 256) return {3, 1};
-    // Few tiles and a long contraction: K is cut so that tiles x slices make one round (partial results to scratch, summed
-    // in fixed order by the split reduction). Measured against the engine's own split plans, M x N x K: 256 x 4096 x 4096
-    // 78 vs 85 us, 512 x 512 x 4096 26.4 vs 29.5, 128 x 2048 x 2048 15.6 vs 17.4, 256 x 1024 x 8192 43.9 vs 50.9; with fewer
-    // than 16 tiles the engine's deeper cuts win (128 x 128 x 8192: 10.5 vs 15.8).
-    if (zdim == 1 && K >= 1024) {
-        if (M >= 128 && N >= 128 && tiles_l >= 64 && tiles_l <= 128 && K / u32(256 / tiles_l) >= 1024) return {1, u32(256 / tiles_l)};
-        if (M >= 64 && N >= 64 && tiles_s >= 16 && tiles_s <= 128) {
-            u32 splits = u32(512 / tiles_s);
-            if (splits > 16) splits = 16;
-            if (K / splits >= 256) return {2, splits};
+static SplitChoice choose_split(u32 M, u32 N, u32 K, u32 zdim) {
+    static constexpr u32 kEdge[4] = {256, 128, 64, 64}, kStep[4] = {16, 32, 64, 32};
+    static constexpr float kPerK[4] = {0.150f, 0.044f, 0.017f, 0.031f}, kFixed[4] = {16.f, 4.f, 3.5f, 3.5f};
+    SplitChoice best{2, 1, K};
+    float best_us = 3e38f;
+    for (int t = 0; t < 4; ++t) {
+        const uint64_t tiles = uint64_t(ceil_div(M, kEdge[t])) * ceil_div(N, kEdge[t]) * zdim;
+        const u32 most = zdim == 1 && tiles < 256 ? (K / 256 < 32 ? K / 256 : 32) : 1;  // a slice keeps 256 k at least
+        for (u32 want = 1; want <= (most > 1 ? most : 1); ++want) {
+            const u32 kz = ceil_div(ceil_div(K, want), kStep[t]) * kStep[t], splits = ceil_div(K, kz);
+            if (splits != want) continue;
+            const uint64_t wgs = tiles * splits;
+            const float k = float(splits > 1 ? kz : K);
+            float us;
+            if (t < 3) {
+                us = float((wgs + 255) / 256) * (k * kPerK[t] + kFixed[t]);
+            } else {  // a last round of at most 256 workgroups has a CU each to itself
+                const u32 rest = u32(wgs % 512);
+                us = float(wgs / 512 + (rest > 256)) * (k * kPerK[t] + kFixed[t]);
+                if (rest && rest <= 256) us += k * 0.0185f + kFixed[t];
+            }
+            if (splits > 1) us += 3.5f + float(2 * splits + 1) * M * N * 4e-6f / 5.f;
+            if (us < best_us) best_us = us, best = SplitChoice{t, splits, kz};
         }
     }
-    return {0, 1};
+    return best;
 }
 
-// Runs the product through the direct-to-LDS kernel when the operands allow it and the shape is one it wins on. Returns
-// false when it did not take the problem (the caller goes on to the engine); `status` is the launch status otherwise.
-template <bool AKF, bool BKF, class E>
-static bool try_dma(const DmaOperand &a, const DmaOperand &b, const E &e, u32 M, u32 N, u32 K, u32 zdim, hipStream_t s, const char *what,
-                    int &status, bool *rowsum_done = nullptr) {
-    if (K % 32 || !dma_operand_ok(a, AKF) || !dma_operand_ok(b, BKF)) return false;
-    const DmaChoice c = choose_dma(M, N, K, zdim);
-    if (!c.tile) return false;
-    if (c.splits > 1) {
-        if (zdim != 1 || e.ld != N || a.cat_k || b.cat_k) return false;
-        const u32 k_per_z = ceil_div(ceil_div(K, c.splits), 32u) * 32u, splits = ceil_div(K, k_per_z);
-        float *ws = nullptr;
-        if ((status = scratch_get(size_t(splits) * M * N * sizeof(float), s, what, &ws))) return true;
-        RowMajorEpi pe{ws, nullptr, N, M * N, 0u};
-        status = c.tile == 1   ? launch_igemm_dma<DmaLarge, AKF, BKF>(a, b, pe, M, N, K, splits, k_per_z, s, what)
-                 : c.tile == 2 ? launch_igemm_dma<DmaSmall, AKF, BKF>(a, b, pe, M, N, K, splits, k_per_z, s, what)
-                               : launch_igemm_dma<DmaSmall8, AKF, BKF>(a, b, pe, M, N, K, splits, k_per_z, s, what);
-        if (status) return true;
-        status = e.row_bias ? launch_splitk_reduce(ws, e.C, M * N, splits, ReduceEpi{e.row_bias, N, M, e.flags}, s, what)
-                            : launch_splitk_reduce(ws, e.C, M * N, splits, ReduceEpi{e.col_bias, 1u << e.col_bias_shift, N >> e.col_bias_shift, e.flags}, s, what);
-        return true;
-    }
-    E e1 = e;
+// Under 2^28 multiply-adds a call is mostly what every launch pays, and the fp32 engine's shorter prologue and smaller code are
+// ahead (fp32 / split, us: 700 x 600 x 100 7.8 / 10.8, 64 x 64 x 4096 8.6 / 10.4, 8 products of 16 x 528 x 41 5.5 / 6.1; above:
+// 528 x 2068 x 137 12.5 / 11.8, 768^3 19.4 / 15.6, 2000 x 2000 x 300 32.9 / 26.0).
+static bool split_pays(u32 M, u32 N, u32 K, u32 zdim) { return uint64_t(M) * N * K * zdim >= (uint64_t(1) << 28); }
+
+template <class Cfg, class AOp, class BOp, class E>
+static int run_split_cfg(const AOp &a, const BOp &b, const E &e, u32 M, u32 N, u32 K, u32 zdim, const SplitChoice &c, hipStream_t s,
+                         const char *what) {
+    if (c.splits == 1) return launch_split<Cfg>(a, b, e, M, N, K, zdim, 0, s, what);
+    float *ws = nullptr;
+    if (int st = scratch_get(size_t(c.splits) * M * N * sizeof(float), s, what, &ws)) return st;
+    RowMajorEpi pe{ws, nullptr, N, M * N, 0u};
+    if (int st = launch_split<Cfg>(a, b, pe, M, N, K, c.splits, c.k_per_z, s, what)) return st;
+    const ReduceEpi re = e.row_bias ? ReduceEpi{e.row_bias, N, M, e.flags} : ReduceEpi{e.col_bias, 1, N, e.flags};
+    return launch_splitk_reduce(ws, e.C, M * N, c.splits, re, s, what);
+}
+// C (M x N, dense rows) = A * B with the epilogue `e`. rowsum_done: whether e's row sums of A were formed along the way.
+template <class AOp, class BOp, class E>
+static int run_split(const AOp &a, const BOp &b, const E &e, u32 M, u32 N, u32 K, u32 zdim, hipStream_t s, const char *what,
+                     bool *rowsum_done = nullptr) {
+    const SplitChoice c = choose_split(M, N, K, zdim);
     if constexpr (E::kRowSum) {
-        if (zdim != 1 || AKF) e1.a_rowsum = nullptr;  // the row sums ride along with one unbatched launch on a row-fast A only
-        if (rowsum_done) *rowsum_done = e1.a_rowsum != nullptr;
+        if (rowsum_done) *rowsum_done = e.a_rowsum != nullptr && c.splits == 1 && zdim == 1;
     }
-    status = c.tile == 1   ? launch_igemm_dma<DmaLarge, AKF, BKF>(a, b, e1, M, N, K, zdim, 0, s, what)
-             : c.tile == 2 ? launch_igemm_dma<DmaSmall, AKF, BKF>(a, b, e1, M, N, K, zdim, 0, s, what)
-                           : launch_igemm_dma<DmaSmall8, AKF, BKF>(a, b, e1, M, N, K, zdim, 0, s, what);
-    return true;
+    switch (c.tile) {
+        case 0: return run_split_cfg<SplitLarge>(a, b, e, M, N, K, zdim, c, s, what);
+        case 1: return run_split_cfg<SplitMid>(a, b, e, M, N, K, zdim, c, s, what);
+        case 2: return run_split_cfg<SplitSmall>(a, b, e, M, N, K, zdim, c, s, what);
+        default: return run_split_cfg<SplitSmall2>(a, b, e, M, N, K, zdim, c, s, what);
+    }
 }
 
-// Scratch bytes run_tiles asks for on a dense M x N result with contraction length K (0: the contraction is not cut).
+// Scratch bytes a product asks for on a dense M x N result with contraction length K (0: the contraction is not cut).
 size_t gemm_scratch_bytes(u32 M, u32 N, u32 K, u32 zdim, bool one_launch_form) {
-    if (one_launch_form && tiny_gemm_fits(M, N, K, zdim)) return 0;  // one launch, no partial results
-    // the direct-to-LDS kernel needs friendly operands, which a size query cannot see: the larger of its need and the engine's
-    size_t dma_need = 0;
-    if (one_launch_form) {  // (callers that name the tiled engine directly never take the direct-to-LDS kernel)
-        const DmaChoice dc = choose_dma(M, N, K, zdim);
-        if (dc.tile && dc.splits > 1) {
-            const u32 k_per_z = ceil_div(ceil_div(K, dc.splits), 32u) * 32u;
-            dma_need = size_t(ceil_div(K, k_per_z)) * M * N * sizeof(float);
+    size_t need = 0;
+    if (one_launch_form) {
+        if (tiny_gemm_fits(M, N, K, zdim)) return 0;  // one launch, no partial results
+        if (split_pays(M, N, K, zdim)) {
+            const SplitChoice c = choose_split(M, N, K, zdim);
+            need = c.splits > 1 ? size_t(c.splits) * M * N * sizeof(float) : 0;
+            if (zdim != 1) return need;
+            // (a K-concatenated batch whose entries are no multiple of 8 long stays on the fp32 engine, which the query cannot see)
         }
     }
     const GemmChoice c = choose_tiles(M, N, K, zdim, true);
@@ -203,7 +210,7 @@ size_t gemm_scratch_bytes(u32 M, u32 N, u32 K, u32 zdim, bool one_launch_form) {
         default: sp = split_for<CfgSmall>(M, N, K, zdim, c.want_splits, true); break;
     }
     const size_t eng = sp.splits > 1 ? size_t(sp.splits) * M * N * sizeof(float) : 0;
-    return eng > dma_need ? eng : dma_need;
+    return need > eng ? need : eng;
 }
 
 static int check_dims(const char *what, u32 M, u32 N, u32 K, u32 batch) {
@@ -250,16 +257,10 @@ static int gemm_nn(const float *A, const float *B, float *C, u32 M, u32 N, u32 K
         return launch_tiny_gemm(TinyGemmArgs{A, B, C, col_bias, row_bias, M, N, K, K, 1, N, 1, N, flags}, K, 0, 0, s, what);
     RowMajorEpi e{C, col_bias, N, M * N, flags};
     e.row_bias = row_bias;
-    if (K % 4 == 0 && N % 4 == 0 && aligned16(A) && aligned16(B)) {
-        int st = CRB_OK;
-        if (try_dma<true, false>(DmaOperand{A, M, K, 0, 0, 0}, DmaOperand{B, N, N, K * N, 0, 0}, e, M, N, K, batch, s, what, st)) return st;
-        MatK<true> a{A, M, K, 0};
-        MatR<true> b{B, N, N, K * N};
-        return run_tiles(a, b, e, M, N, K, batch, s, what);
-    }
-    MatK<false> a{A, M, K, 0};
-    MatR<false> b{B, N, N, K * N};
-    return run_tiles(a, b, e, M, N, K, batch, s, what);
+    if (split_pays(M, N, K, batch)) return run_split(SMatK<>{A, M, K, 0}, SMatR{B, N, N, K * N}, e, M, N, K, batch, s, what);
+    if (K % 4 == 0 && N % 4 == 0 && aligned16(A) && aligned16(B))
+        return run_tiles(MatK<true>{A, M, K, 0}, MatR<true>{B, N, N, K * N}, e, M, N, K, batch, s, what);
+    return run_tiles(MatK<false>{A, M, K, 0}, MatR<false>{B, N, N, K * N}, e, M, N, K, batch, s, what);
 }
 
 static int gemm_tn(const float *A, const float *B, float *C, u32 M, u32 N, u32 K, u32 batch, u32 flags,
@@ -272,24 +273,20 @@ static int gemm_tn(const float *A, const float *B, float *C, u32 M, u32 N, u32 K
         return launch_tiny_gemm(t, K, 0, 0, s, what);
     }
     RowMajorEpi e{C, nullptr, N, M * N, flags};
+    RowMajorAccEpi ea;  // the dense layers' weight gradient
+    static_cast<RowMajorEpi &>(ea) = e;
+    ea.a_rowsum = a_rowsum;
+    if (split_pays(M, N, K, batch)) {
+        const SMatR a{A, M, M, 0}, b{B, N, N, K * N};
+        if (flags & EPI_ACCUM) return run_split(a, b, ea, M, N, K, batch, s, what, rowsum_done);
+        return run_split(a, b, e, M, N, K, batch, s, what);
+    }
     if (M % 4 == 0 && N % 4 == 0 && aligned16(A) && aligned16(B)) {
-        MatR<true> a{A, M, M, 0};
-        MatR<true> b{B, N, N, K * N};
-        int st = CRB_OK;
-        const DmaOperand da{A, M, M, 0, 0, 0}, db{B, N, N, K * N, 0, 0};
-        if (flags & EPI_ACCUM) {  // the dense layers' weight gradient
-            RowMajorAccEpi ea;
-            static_cast<RowMajorEpi &>(ea) = e;
-            ea.a_rowsum = a_rowsum;
-            if (try_dma<false, false>(da, db, ea, M, N, K, batch, s, what, st, rowsum_done)) return st;
-            return run_tiles(a, b, ea, M, N, K, batch, s, what, rowsum_done);
-        }
-        if (try_dma<false, false>(da, db, e, M, N, K, batch, s, what, st)) return st;
+        const MatR<true> a{A, M, M, 0}, b{B, N, N, K * N};
+        if (flags & EPI_ACCUM) return run_tiles(a, b, ea, M, N, K, batch, s, what, rowsum_done);
         return run_tiles(a, b, e, M, N, K, batch, s, what);
     }
-    MatR<false> a{A, M, M, 0};
-    MatR<false> b{B, N, N, K * N};
-    return run_tiles(a, b, e, M, N, K, batch, s, what);
+    return run_tiles(MatR<false>{A, M, M, 0}, MatR<false>{B, N, N, K * N}, e, M, N, K, batch, s, what);
 }
 
 static int gemm_nt(const float *A, const float *B, float *C, u32 M, u32 N, u32 K, const float *col_bias, u32 flags,
@@ -297,16 +294,9 @@ static int gemm_nt(const float *A, const float *B, float *C, u32 M, u32 N, u32 K
     if (tiny_gemm_fits(M, N, K, 1, true))  // A (M x K) row-major, B stored N x K
         return launch_tiny_gemm(TinyGemmArgs{A, B, C, col_bias, nullptr, M, N, K, K, 1, 1, K, N, flags}, K, 0, 0, s, what);
     RowMajorEpi e{C, col_bias, N, 0, flags};
-    if (K % 4 == 0 && aligned16(A) && aligned16(B)) {
-        int st = CRB_OK;
-        if (try_dma<true, true>(DmaOperand{A, M, K, 0, 0, 0}, DmaOperand{B, N, K, 0, 0, 0}, e, M, N, K, 1, s, what, st)) return st;
-        MatK<true> a{A, M, K, 0};
-        MatK<true> b{B, N, K, 0};
-        return run_tiles(a, b, e, M, N, K, 1, s, what);
-    }
-    MatK<false> a{A, M, K, 0};
-    MatK<false> b{B, N, K, 0};
-    return run_tiles(a, b, e, M, N, K, 1, s, what);
+    if (split_pays(M, N, K, 1)) return run_split(SMatK<>{A, M, K, 0}, SMatK<>{B, N, K, 0}, e, M, N, K, 1, s, what);
+    if (K % 4 == 0 && aligned16(A) && aligned16(B)) return run_tiles(MatK<true>{A, M, K, 0}, MatK<true>{B, N, K, 0}, e, M, N, K, 1, s, what);
+    return run_tiles(MatK<false>{A, M, K, 0}, MatK<false>{B, N, K, 0}, e, M, N, K, 1, s, what);
 }
 
 // ---- 3x3 / pad 1 / stride 1 convolution of 2x2 images as dense products over (channel, pixel) pairs -------------------
@@ -417,12 +407,12 @@ int crb_sgemm_nta(const float *A, const float *B, float *C, uint32_t M, uint32_t
     hipStream_t s = hipStream_t(stream);
     if (tiny_gemm_fits(M, N, KK, 1))  // the batch concatenated along the contraction
         return launch_tiny_gemm(TinyGemmArgs{A, B, C, nullptr, nullptr, M, N, KK, K, 1, 1, K, N, EPI_ACCUM}, K, M * K, N * K, s, "crb_sgemm_nta");
+    if (K % 8 == 0 && split_pays(M, N, KK, 1)) {  // octets of the contraction stay inside a batch entry
+        const SMatK<true> a{A, M, K, 0, M * K, FastDiv(K)}, b{B, N, K, 0, N * K, FastDiv(K)};
+        return run_split(a, b, e, M, N, KK, 1, s, "crb_sgemm_nta");
+    }
     if (K % 4 == 0 && aligned16(A) && aligned16(B)) {
-        int st = CRB_OK;
-        if (K % 32 == 0 && try_dma<true, true>(DmaOperand{A, M, K, 0, K, M * K}, DmaOperand{B, N, K, 0, K, N * K}, e, M, N, KK, 1, s, "crb_sgemm_nta", st))
-            return st;
-        MatKCat<true> a{A, M, K, M * K, FastDiv(K)};
-        MatKCat<true> b{B, N, K, N * K, FastDiv(K)};
+        const MatKCat<true> a{A, M, K, M * K, FastDiv(K)}, b{B, N, K, N * K, FastDiv(K)};
         return run_tiles(a, b, e, M, N, KK, 1, s, "crb_sgemm_nta");
     }
     MatKCat<false> a{A, M, K, M * K, FastDiv(K)};

@@ -1,0 +1,53 @@
+// fp32 contractions on the bf16 matrix pipe, with nothing lost from the fp32 operands.
+//
+// gfx950 multiplies bf16 sixteen times as fast as fp32 (v_mfma_f32_32x32x16_bf16: 32 clocks for sixteen k of a 32 x 32 block;
+// v_mfma_f32_32x32x2_f32: 64 clocks for two). A float has 24 significant bits, a bf16 has 8, and
+//   x = hi + mid + lo,  hi = bf16(x), mid = bf16(x - hi), lo = x - hi - mid
+// is exact: rounding to nearest leaves |x - hi| <= 2^-8 of x's leading bit in at most 16 bits, of which mid takes 8 and leaves
+// at most 6. A product of two such sums is nine bf16 products, each exact in fp32. Six of them are formed; the three left out
+// (mid*lo, lo*mid, lo*lo) are together at most 2^-24 of the product, the unit roundoff of one fp32 multiplication. All sums are
+// fp32, in the accumulators of the MFMA. Six sixteenths of the fp32 time per product remain: at the rates the pipes sustain on
+// this part (1.82 PFLOP/s bf16, 155 TFLOP/s fp32, dense random operands) 303 against 155 TFLOP/s of fp32 work.
+// Measured distance from float64 (2-norm, N(0,1) operands; fp32 MFMA / six products / all nine): K = 144 2.15e-7 / 1.74e-7 /
+// 1.74e-7, 576 4.31e-7 / 3.61e-7 / 3.61e-7, 4608 1.22e-6 / 1.07e-6 / 1.07e-6 - sixteen k's share one rounding of the sum, so
+// the results are closer to the exact ones than those of the fp32 pipe, and the three left out are not seen at all.
+// What differs: an operand that is infinite (or rounds to infinity as a bf16, from 3.39e38 up) gives NaN where the fp32 pipe
+// gives an infinity or NaN.
+#pragma once
+#include "crb_common.h"
+
+namespace crb {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef u32 u32x2 __attribute__((ext_vector_type(2)));
+typedef u32 u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kSplit = 3;  // bf16 parts of a float
+
+// The three parts of two floats, packed (x0 in the low half).
+__device__ __forceinline__ void split_pair(float x0, float x1, u32 &hi, u32 &mid, u32 &lo) {
+    const u32 h = __builtin_bit_cast(u32, __builtin_convertvector(f32x2{x0, x1}, bf16x2));
+    const float r0 = x0 - __builtin_bit_cast(float, h << 16), r1 = x1 - __builtin_bit_cast(float, h & 0xffff0000u);
+    const u32 m = __builtin_bit_cast(u32, __builtin_convertvector(f32x2{r0, r1}, bf16x2));
+    const float s0 = r0 - __builtin_bit_cast(float, m << 16), s1 = r1 - __builtin_bit_cast(float, m & 0xffff0000u);
+    hi = h, mid = m, lo = __builtin_bit_cast(u32, __builtin_convertvector(f32x2{s0, s1}, bf16x2));
+}
+
+// The three parts of eight floats, each a 16-byte MFMA fragment (element i in 16-bit slot i).
+__device__ __forceinline__ void split8(const float *x, u32x4 (&part)[kSplit]) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        u32 h, m, l;
+        split_pair(x[2 * p], x[2 * p + 1], h, m, l);
+        part[0][p] = h, part[1][p] = m, part[2][p] = l;
+    }
+}
+
+// The products that are formed: (part of A, part of B), in an order that needs the leading parts first.
+constexpr int kTerms = 6;
+constexpr int kTermA[kTerms] = {0, 0, 1, 1, 0, 2};
+constexpr int kTermB[kTerms] = {0, 1, 0, 1, 2, 0};
+
+}  // namespace crb

@@ -1,0 +1,81 @@
+"""Products on the split engine (three bf16 parts per float, csrc/igemm_split.h) where its tiles and slabs end: remainders of
+every tile edge and of the K slabs, operands off the 16-byte grid, cut contractions, accumulation, row sums; and the
+claim that nothing of the operands' 24 bits is lost."""
+import numpy as np
+import pytest
+
+from oracle import seblas_oracle as orc
+from tests.util import assert_close, to_dev, to_np, uniform
+
+pytestmark = pytest.mark.gpu
+
+# (M, N, K), at least 2^28 multiply-adds: one past / one short of the 256, 128 and 64 tiles, K one past / one short of slabs of
+# 16, 32 and 64, a contraction of a single ragged slab, tall and flat results, few tiles under a long (cut) contraction
+SIZES = [(1025, 1023, 257), (4097, 4095, 17), (129, 2047, 1025), (65, 4097, 1031), (8191, 63, 543), (256, 1024, 1025), (97, 101, 27409),
+         (515, 514, 1033), (2048, 2049, 64)]
+
+
+def product(capi, form, A, B, C, M, N, K):
+    getattr(capi, "sgemm_" + form)(A, B, C, M, N, K)
+
+
+@pytest.mark.parametrize("form", ["nn", "nt", "tn", "nta"])
+@pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
+def test_split_product_edges(dev, form, size):
+    import torch
+    from crusaderbackend_amd import capi
+
+    M, N, K = size
+    A, B = uniform(M + K, M, K), uniform(N + K, K, N)
+    ref = orc.sgemm(A, B)
+    a = np.ascontiguousarray(A.T) if form == "tn" else A
+    b = np.ascontiguousarray(B.T) if form in ("nt", "nta") else B
+
+    def off_grid(x):  # 4 bytes past a 16-byte boundary
+        buf = torch.empty(x.size + 1, device=dev)
+        buf[1:].copy_(torch.from_numpy(x.reshape(-1)))
+        return buf[1:]
+
+    C0 = uniform(7, M, N) if form == "nta" else np.zeros((M, N), np.float32)  # nta accumulates
+    C = to_dev(C0, dev)
+    product(capi, form, off_grid(a), off_grid(b), C, M, N, K)
+    torch.cuda.synchronize()
+    assert_close(to_np(C), ref + C0, K, f"{form} {size}")
+
+
+@pytest.mark.parametrize("batch,IN,OUT", [(257, 1025, 1031), (1031, 513, 519)])
+def test_split_dense_layer_gradients(dev, batch, IN, OUT):
+    import torch
+    from crusaderbackend_amd import capi
+
+    dY, X = uniform(1, batch, OUT), uniform(2, batch, IN)
+    dW0, dB0 = uniform(3, OUT, IN), uniform(4, OUT)
+    dW, dB = to_dev(dW0, dev), to_dev(dB0, dev)
+    capi.linear_wgrad(to_dev(dY, dev), to_dev(X, dev), dW, dB, batch, IN, OUT)
+    torch.cuda.synchronize()
+    assert_close(to_np(dW), dW0 + dY.astype(np.float64).T @ X, batch, "dW")
+    assert_close(to_np(dB), dB0 + dY.astype(np.float64).sum(0), batch, "dB")
+
+
+def test_split_product_loses_nothing_of_its_operands(dev):
+    """Exact results where fp32 has them: operands of 24 significant bits times powers of two, one product per result (a
+    permutation), come back bit for bit; and the distance of a long sum from float64 stays under that of a sum whose every
+    product and addition rounds once to fp32, sqrt(K) * 2^-24 in the 2-norm for operands of one scale."""
+    import torch
+    from crusaderbackend_amd import capi
+
+    n = 1024
+    A = uniform(5, n, n)
+    perm = np.random.RandomState(6).permutation(n)
+    B = np.zeros((n, n), np.float32)
+    B[perm, np.arange(n)] = np.ldexp(1.0, np.arange(n) % 9 - 4).astype(np.float32)
+    C = torch.empty(n, n, device=dev)
+    capi.sgemm_nn(to_dev(A, dev), to_dev(B, dev), C, n, n, n)
+    torch.cuda.synchronize()
+    assert np.array_equal(to_np(C), A[:, perm] * B[perm, np.arange(n)])
+
+    B = uniform(8, n, n)
+    capi.sgemm_nn(to_dev(A, dev), to_dev(B, dev), C, n, n, n)
+    torch.cuda.synchronize()
+    exact = A.astype(np.float64) @ B
+    assert np.linalg.norm(to_np(C) - exact) <= np.sqrt(n) * 2.0**-24 * np.linalg.norm(exact)
