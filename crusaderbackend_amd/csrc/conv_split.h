@@ -1,0 +1,393 @@
+// Convolution forward (stride S) and, at stride 1, data gradient on split bf16 operands (split_bf16.h), any image extent and any
+// padding: Y[n][oc][y][x] = sum over (ic, fh, fw) of W[oc][ic][fh][fw] * X[n][ic][S*y + fh - pad][S*x + fw - pad]; the data
+// gradient is the same with dY as X, the filters' channel roles swapped and their taps mirrored.
+//
+// Pixels are taken flat: images are cut into `strips` column strips of equal width (one where the image is narrow enough), and a
+// workgroup owns PXT consecutive pixels of the (image, strip, row, column) sequence and OCT output channels, so hardly any image
+// extent wastes a tile. What the taps of those pixels touch is a run of rows of the padded strips (S*(H-1)+F rows and
+// S*(SW-1)+F columns each, halo included): CI = 16*KG channels of it at a time are staged in LDS as MFMA fragments, [part]
+// [channel octet][position] units of 16 bytes, double-buffered. A tap is then a constant shift of a lane's position, whatever
+// the width, and a B fragment (32 pixels, 16 channels) is one 16-byte read at lane base + shift.
+// Filters are split by a kernel of their own into fragments in the order the waves consume them (conv_split_filters_kernel) and
+// go from L2 straight into registers, two taps ahead: a filter element is used once per workgroup tile, so LDS would only add
+// a copy, and without them a barrier stands only every F*F taps.
+// KG wave groups take 16 channels each of every staged chunk and exchange their accumulators through LDS at the end.
+//
+// What bounds it: per tap a wave issues 6*TM*TN MFMAs (32 clocks each) against 3*TM KB of filters from L2 and 3*TN KB from LDS:
+// with 2 x 2 blocks per wave and two waves on a SIMD half of the vector memory path's and a quarter of LDS' time, so the MFMAs.
+#pragma once
+#include "igemm_engine.h"
+#include "split_bf16.h"
+
+namespace crb {
+
+template <int F_, int S_, int TM_, int TN_, int WM_, int WN_, int KG_, int MAXPX_, int AHEAD_ = 2, int BSET_ = 2>
+struct ConvSplitCfg {
+    static constexpr int F = F_, S = S_, TM = TM_, TN = TN_, WM = WM_, WN = WN_, KG = KG_, MAXPX = MAXPX_;
+    static constexpr int NT = F * F, CI = 16 * KG, KO = CI / 8, NTH = 64 * WM * WN * KG;
+    static constexpr int OCT = 32 * TM * WM, PXT = 32 * TN * WN;
+    static constexpr int PART = KO * MAXPX * 16, STAGE = kSplit * PART;  // bytes
+    static constexpr int NP = KO * MAXPX / NTH;
+    static_assert(KO * MAXPX % NTH == 0, "whole staging items per thread");
+    static constexpr int AHEAD = AHEAD_;  // taps the filter fragments run ahead
+    static constexpr int BSET = BSET_;    // 2: pixel fragments are read a tap ahead
+};
+
+struct ConvSplitArgs {
+    const float *X;
+    const unsigned char *Wf;  // split filters
+    float *Y;
+    const float *bias;
+    u32 C_IN, C_OUT, chunks;
+    u32 H, W;        // extent of X
+    u32 HW, OHW;     // pixels of an image of X, of Y
+    u32 OW, SW, strips;  // width of Y, of a strip
+    u32 npix;        // pixels of all strips (those past the image's last column are computed and dropped)
+    u32 prow, pitch; // padded rows of a strip, positions of a padded row
+    int pad_y, pad_x;
+    u32 px_tiles, oc_tiles, relu;
+    u32 chunks_z;    // chunks a slice (blockIdx.z) of the contraction takes; slices write partial results `zstride` floats apart
+    size_t zstride;
+    FastDiv ohw, ow, pitch_d, prow_d, strip_d;  // pixels of a strip, its width, ...
+};
+
+// Filters -> fragments: [output block of 32][K group][chunk][tap][part] of 1 KB (lane l: output channel l % 32 of the block,
+// channels 8 * (l / 32) + 0..7 of the group's 16), zero beyond the channel counts. A thread takes one channel octet of one
+// output channel and tap: eight loads in flight, and enough threads to cover the chip (all taps per thread: 147 K filter
+// elements took 14 us, a chain of 72 loads on 8 workgroups).
+template <bool DGRAD>
+__global__ void __launch_bounds__(256) conv_split_filters_kernel(const float *__restrict__ W, unsigned char *__restrict__ Wf, u32 C_IN, u32 C_OUT,
+                                                                 u32 NT, u32 chunks, u32 KG, u32 total) {
+    const u32 t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= total) return;
+    const u32 lane = t & 63, frag = t >> 6;  // fragments in memory order
+    const u32 tap = frag % NT, rest = frag / NT;
+    const u32 ch = rest % chunks, g = (rest / chunks) % KG, ob = rest / (chunks * KG);
+    const u32 oc = ob * 32 + (lane & 31), ic0 = (ch * KG + g) * 16 + 8 * (lane >> 5);
+    float w[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const u32 ic = ic0 + j;
+        const bool ok = oc < C_OUT && ic < C_IN;
+        // forward: W[oc][ic][tap]; data gradient: the filters are stored [C_IN (dY channels)][C_OUT][tap] and mirrored
+        const float v = W[ok ? (DGRAD ? (size_t(ic) * C_OUT + oc) * NT + NT - 1 - tap : (size_t(oc) * C_IN + ic) * NT + tap) : 0];
+        w[j] = ok ? v : 0.f;
+    }
+    u32x4 part[kSplit];
+    split8(w, part);
+    unsigned char *dst = Wf + size_t(frag) * (kSplit * 1024) + lane * 16;
+#pragma unroll
+    for (int p = 0; p < kSplit; ++p) *reinterpret_cast<u32x4 *>(dst + p * 1024) = part[p];
+}
+
+template <class C>
+__global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) {
+    constexpr int TM = C::TM, TN = C::TN, KG = C::KG, NT = C::NT, F = C::F, S = C::S, MAXPX = C::MAXPX, NSET = C::AHEAD + 1;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[2 * C::STAGE];
+    // an XCD gets a contiguous run of tiles, the output-channel tiles of a pixel tile behind one another: they share X in its L2
+    const u32 ntile = a.px_tiles * a.oc_tiles, q8 = ntile / kXcds, r8 = ntile % kXcds, xcd = blockIdx.x % kXcds;
+    const u32 tile = xcd * q8 + (xcd < r8 ? xcd : r8) + blockIdx.x / kXcds;
+    const u32 pt = tile / a.oc_tiles, ot = tile % a.oc_tiles;
+
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = wv % (C::WM * C::WN), kgroup = wv / (C::WM * C::WN);
+    const int wave_m = wave / C::WN, wave_n = wave % C::WN, i32 = lane & 31, h = lane >> 5;
+
+    // ---- the pixels and the staged run of padded rows --------------------------------------------------------------------
+    const u32 p0 = pt * C::PXT, p1 = (p0 + C::PXT < a.npix ? p0 + C::PXT : a.npix) - 1;
+    u32 n0, r0, y0, n1, r1, y1;
+    a.ohw.divmod(p0, n0, r0);
+    y0 = a.ow.div(r0);
+    a.ohw.divmod(p1, n1, r1);
+    y1 = a.ow.div(r1);
+    const u32 R0 = n0 * a.prow + S * y0, wpx = (n1 * a.prow + S * y1 + F - R0) * a.pitch;
+    u32 b_lane[TN];  // LDS byte of the pixel's first tap, this lane's channel half
+#pragma unroll
+    for (int ni = 0; ni < TN; ++ni) {
+        u32 p = p0 + wave_n * (32 * TN) + ni * 32 + i32;
+        p = p < a.npix ? p : a.npix - 1;
+        u32 n, r, y, x;
+        a.ohw.divmod(p, n, r);
+        a.ow.divmod(r, y, x);
+        b_lane[ni] = ((n * a.prow + S * y - R0) * a.pitch + S * x) * 16 + (2 * kgroup + h) * (MAXPX * 16);
+    }
+    // staging: item i of a thread is the channel octet o of position s
+    const u32 img0 = a.strip_d.div(n0);  // (n0, n: strips of all images, counted through)
+    const float *const xbase = a.X + size_t(img0) * a.C_IN * a.HW;
+    u32 off[C::NP];  // bytes from the chunk's first channel of image img0 (the host checks that they fit)
+    u32 valid = 0;
+#pragma unroll
+    for (int i = 0; i < C::NP; ++i) {
+        const u32 u = threadIdx.x + i * C::NTH, o = u / MAXPX, s = u % MAXPX;
+        u32 pr, pc, n, r;
+        a.pitch_d.divmod(s, pr, pc);
+        a.prow_d.divmod(R0 + pr, n, r);
+        u32 img, strip;
+        a.strip_d.divmod(n, img, strip);
+        const int iy = int(r) - a.pad_y, ix = int(pc + S * strip * a.SW) - a.pad_x;
+        const bool in = s < wpx && u32(iy) < a.H && u32(ix) < a.W;
+        valid |= in ? 1u << i : 0u;
+        off[i] = in ? ((img - img0) * a.C_IN * a.HW + 8 * o * a.HW + u32(iy) * a.W + u32(ix)) * 4u : 0u;
+    }
+    float reg[C::NP][8];
+    const bool ragged = a.C_IN % C::CI != 0;
+    const u32 chunk0 = blockIdx.z * a.chunks_z, chunk1 = chunk0 + a.chunks_z < a.chunks ? chunk0 + a.chunks_z : a.chunks;
+    auto at = [](const float *uniform, u32 bytes) { return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(uniform) + bytes); };
+    auto fetch = [&](u32 chunk) {
+        const float *base = xbase + size_t(chunk) * C::CI * a.HW;
+        if (ragged && chunk + 1 == a.chunks) {
+#pragma unroll
+            for (int i = 0; i < C::NP; ++i) {
+                const u32 c0 = chunk * C::CI + 8 * ((threadIdx.x + i * C::NTH) / MAXPX);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const bool ok = c0 + j < a.C_IN;
+                    const float v = at(ok ? base + j * a.HW : xbase, ok ? off[i] : 0u);
+                    reg[i][j] = ok ? v : 0.f;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < C::NP; ++i)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) reg[i][j] = at(base + j * a.HW, off[i]);
+        }
+    };
+    auto commit = [&](unsigned char *sm) {  // (positions behind the run are written too; nothing reads them)
+#pragma unroll
+        for (int i = 0; i < C::NP; ++i) {
+            const u32 u = threadIdx.x + i * C::NTH, o = u / MAXPX, s = u % MAXPX;
+            const bool in = (valid >> i) & 1u;
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = in ? reg[i][j] : 0.f;
+            u32x4 part[kSplit];
+            split8(v, part);
+#pragma unroll
+            for (int p = 0; p < kSplit; ++p) *reinterpret_cast<u32x4 *>(sm + p * C::PART + o * (MAXPX * 16) + s * 16) = part[p];
+        }
+    };
+
+    // ---- filters: this wave's blocks, one 3 KB step (tap) after the other ---------------------------------------------------
+    const u32 steps = a.chunks * NT;
+    const unsigned char *wp[TM];
+#pragma unroll
+    for (int mi = 0; mi < TM; ++mi)
+        wp[mi] = a.Wf + ((size_t(ot * (TM * C::WM) + wave_m * TM + mi) * KG + kgroup) * steps + chunk0 * NT) * (kSplit * 1024);
+    bf16x8 fa[NSET][kSplit][TM];
+    auto load_filters = [&](int set) {  // the next step's fragments
+#pragma unroll
+        for (int mi = 0; mi < TM; ++mi) {
+#pragma unroll
+            for (int p = 0; p < kSplit; ++p) fa[set][p][mi] = *reinterpret_cast<const bf16x8 *>(wp[mi] + p * 1024 + u32(lane) * 16u);
+            wp[mi] += kSplit * 1024;
+        }
+    };
+
+    v16f acc[TM][TN];
+#pragma unroll
+    for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.0f;
+
+    bf16x8 fb[C::BSET][kSplit][TN];
+    auto read_pixels = [&](int set, u32 shift) {
+#pragma unroll
+        for (int p = 0; p < kSplit; ++p)
+#pragma unroll
+            for (int ni = 0; ni < TN; ++ni) fb[set][p][ni] = *reinterpret_cast<const bf16x8 *>(smem + b_lane[ni] + shift + p * C::PART);
+    };
+
+    fetch(chunk0);
+#pragma unroll
+    for (int d = 0; d < C::AHEAD; ++d) load_filters(d);
+    commit(smem);
+    lds_barrier();
+    u32 buf = 0;
+    for (u32 chunk = chunk0; chunk < chunk1; ++chunk, buf = C::STAGE - buf) {
+        if (chunk + 1 < chunk1) fetch(chunk + 1);
+        if (C::BSET == 2) read_pixels(0, buf);
+        // The scheduler is fenced tap by tap: left alone it sinks the requests made for later taps to where they are used.
+#pragma unroll
+        for (int tap = 0; tap < NT; ++tap) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_filters((tap + C::AHEAD) % NSET);  // (behind the last step: padding at the end of the filter buffer)
+            constexpr int BS = C::BSET;
+            if (BS == 1) read_pixels(0, buf + (tap / F * a.pitch + tap % F) * 16);
+            else if (tap + 1 < NT) read_pixels((tap + 1) % BS, buf + ((tap + 1) / F * a.pitch + (tap + 1) % F) * 16);
+            // the next chunk: split and stored in the shadow of the last taps' MFMAs (once more behind the last chunk, for nobody)
+            if (tap == (NT > 1 ? NT - 2 : 0)) commit(smem + (C::STAGE - buf));
+#pragma unroll
+            for (int t = 0; t < kTerms; ++t)
+#pragma unroll
+                for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+                    for (int ni = 0; ni < TN; ++ni)
+                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[tap % NSET][kTermA[t]][mi], fb[tap % BS][kTermB[t]][ni], acc[mi][ni], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < TM * TN * kTerms; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                if (tap == (NT > 1 ? NT - 2 : 0)) {
+                    __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (NT % NSET != 0) {  // the next chunk's first step is in set NT % NSET
+            bf16x8 tmp[NSET][kSplit][TM];
+#pragma unroll
+            for (int s = 0; s < NSET; ++s)
+#pragma unroll
+                for (int p = 0; p < kSplit; ++p)
+#pragma unroll
+                    for (int mi = 0; mi < TM; ++mi) tmp[s][p][mi] = fa[(s + NT) % NSET][p][mi];
+#pragma unroll
+            for (int s = 0; s < NSET; ++s)
+#pragma unroll
+                for (int p = 0; p < kSplit; ++p)
+#pragma unroll
+                    for (int mi = 0; mi < TM; ++mi) fa[s][p][mi] = tmp[s][p][mi];
+        }
+        lds_barrier();
+    }
+
+    // ---- epilogue: 32 lanes store 32 consecutive pixels of a channel --------------------------------------------------------
+    auto store_part = [&](int mi, int ni, int r0, auto nr_c, const float *res) {
+        constexpr int NR = decltype(nr_c)::value;
+        const u32 p = p0 + wave_n * (32 * TN) + ni * 32 + i32;
+        const u32 oc0 = ot * C::OCT + wave_m * (32 * TM) + mi * 32 + 4 * h + 2 * r0;
+        float b[NR];
+#pragma unroll
+        for (int r = 0; r < NR; ++r) b[r] = 0.f;
+        if (a.bias) {
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                const u32 oc = oc0 + 8 * (r / 4) + (r % 4);
+                b[r] = a.bias[oc < a.C_OUT ? oc : a.C_OUT - 1];
+            }
+        }
+        u32 v, rem, img, strip, yy, xx;
+        a.ohw.divmod(p, v, rem);
+        a.ow.divmod(rem, yy, xx);
+        a.strip_d.divmod(v, img, strip);
+        xx += strip * a.SW;
+        if (p >= a.npix || xx >= a.OW) return;
+        float *y = a.Y + blockIdx.z * a.zstride + size_t(img) * a.C_OUT * a.OHW + yy * a.OW + xx;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const u32 oc = oc0 + 8 * (r / 4) + (r % 4);
+            float o = res[r] + b[r];
+            if (a.relu) o = o > 0.f ? o : 0.f;
+            if (oc < a.C_OUT) y[size_t(oc) * a.OHW] = o;
+        }
+    };
+    if constexpr (KG == 1) {
+#pragma unroll
+        for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < TN; ++ni) {
+                float v[16];
+#pragma unroll
+                for (int r = 0; r < 16; ++r) v[r] = acc[mi][ni][r];
+                store_part(mi, ni, 0, std::integral_constant<int, 16>(), v);
+            }
+    } else {
+        // the K groups exchange their accumulators, BR blocks of every wave at a time; each sums (in group order) and stores a share
+        constexpr int NB = TM * TN, BR = NB < KG ? NB : KG, NR = BR * 16 / KG;
+        static_assert(NB % BR == 0 && NR % 4 == 0 && BR * 4096 * C::WM * C::WN * KG <= 2 * C::STAGE, "exchange space");
+        float *x = reinterpret_cast<float *>(smem);
+#pragma unroll
+        for (int q = 0; q < NB / BR; ++q) {
+            if (q) lds_barrier();
+            float *dst = x + (kgroup * C::WM * C::WN + wave) * BR * 1024 + lane;
+#pragma unroll
+            for (int f = 0; f < BR * 16; ++f) dst[f * 64] = acc[(q * BR + f / 16) / TN][(q * BR + f / 16) % TN][f % 16];
+            lds_barrier();
+            const int f0 = kgroup * NR;
+            float v[NR];
+            const float *src = x + wave * BR * 1024 + f0 * 64 + lane;
+#pragma unroll
+            for (int r = 0; r < NR; ++r) v[r] = src[r * 64];
+#pragma unroll
+            for (int g = 1; g < KG; ++g)
+#pragma unroll
+                for (int r = 0; r < NR; ++r) v[r] += src[g * C::WM * C::WN * BR * 1024 + r * 64];
+            const int b = q * BR + f0 / 16;
+            store_part(b / TN, b % TN, f0 % 16, std::integral_constant<int, NR>(), v);
+        }
+    }
+}
+
+// Positions of the longest run of padded rows that a tile of PXT consecutive pixels touches. Tiles start at multiples of PXT, so
+// their places inside an image repeat; where that takes long, the bound for any start.
+inline u32 conv_split_window(u32 pxt, u32 OH, u32 OW, u32 F, u32 S) {
+    const u32 ohw = OH * OW, prow = S * (OH - 1) + F, pitch = S * (OW - 1) + F;
+    u32 g = pxt, r = ohw;
+    while (r) {
+        const u32 t = g % r;
+        g = r, r = t;
+    }
+    const u32 period = ohw / g;
+    if (period > 64) {
+        const u32 rows = (pxt - 2) / OW + 2, crossings = (pxt - 2) / ohw + 1;
+        const int gap = int(prow) - int(S * OH);  // padded rows that an image boundary adds
+        return (S * (rows - 1) + F + (gap > 0 ? u32(gap) * crossings : 0u)) * pitch;
+    }
+    u32 most = 0;
+    for (u32 k = 0; k < period; ++k) {
+        const u32 b = k * pxt % ohw, e = b + pxt - 1;  // first and last pixel, counted from the first one's image
+        const u32 rows = e / ohw * prow + S * (e % ohw / OW) + F - S * (b / OW);
+        most = rows > most ? rows : most;
+    }
+    return most * pitch;
+}
+
+// Column strips of an output of extent OH x OW for a configuration: the fewest whose run fits its LDS; 0: none does.
+template <class C>
+inline u32 conv_split_strips(u32 OH, u32 OW) {
+    for (u32 ns = ceil_div(OW, 64u); ns <= OW && ns <= 16; ++ns)
+        if (conv_split_window(C::PXT, OH, ceil_div(OW, ns), C::F, C::S) <= u32(C::MAXPX)) return ns;
+    return 0;
+}
+
+template <class C>
+inline size_t conv_split_filter_bytes(u32 C_IN, u32 C_OUT) {
+    const size_t chunks = ceil_div(C_IN, u32(C::CI)), blocks = ceil_div(C_OUT, u32(C::OCT)) * (C::OCT / 32);
+    return (blocks * C::KG * chunks * C::NT + C::AHEAD) * kSplit * 1024;
+}
+
+// Wf: conv_split_filter_bytes of scratch. (OH, OW): extent of the result, (H, W): of X; window origin (-pad_y, -pad_x); strips:
+// conv_split_strips. slices > 1: the contraction is cut; partial results go to `part` (slices x the result) and are summed in
+// fixed order by one more launch, which applies bias and ReLU.
+template <class C, bool DGRAD>
+inline int launch_conv_split(const float *Wt, const float *X, float *Y, const float *bias, unsigned char *Wf, u32 N, u32 C_IN, u32 C_OUT, u32 H,
+                             u32 W, u32 OH, u32 OW, u32 strips, u32 slices, float *part, int pad_y, int pad_x, u32 relu, hipStream_t s,
+                             const char *what) {
+    ConvSplitArgs a;
+    a.X = X, a.Wf = Wf, a.Y = slices > 1 ? part : Y, a.bias = slices > 1 ? nullptr : bias;
+    a.C_IN = C_IN, a.C_OUT = C_OUT, a.chunks = ceil_div(C_IN, u32(C::CI));
+    a.strips = strips, a.SW = ceil_div(OW, strips);
+    a.H = H, a.W = W, a.HW = H * W, a.OHW = OH * OW, a.OW = OW, a.npix = N * strips * OH * a.SW;
+    a.prow = C::S * (OH - 1) + C::F, a.pitch = C::S * (a.SW - 1) + C::F;
+    a.pad_y = pad_y, a.pad_x = pad_x;
+    a.px_tiles = ceil_div(a.npix, u32(C::PXT)), a.oc_tiles = ceil_div(C_OUT, u32(C::OCT)), a.relu = slices > 1 ? 0 : relu;
+    const u32 count = N * C_OUT * OH * OW;
+    a.chunks_z = ceil_div(a.chunks, slices), a.zstride = count;
+    a.ohw.init(OH * a.SW), a.ow.init(a.SW), a.pitch_d.init(a.pitch), a.prow_d.init(a.prow), a.strip_d.init(strips);
+    const uint64_t tiles = uint64_t(a.px_tiles) * a.oc_tiles;
+    if (tiles > 0x7fffffffull) return fail(CRB_EINVAL_SHAPE, "%s: launch grid too large", what);
+    const u32 total = a.oc_tiles * (C::OCT / 32) * C::KG * a.chunks * C::NT * 64;
+    hipLaunchKernelGGL(conv_split_filters_kernel<DGRAD>, dim3(ceil_div(total, 256u)), dim3(256), 0, s, Wt, Wf, C_IN, C_OUT, u32(C::NT), a.chunks,
+                       u32(C::KG), total);
+    if (int st = check_launch(what)) return st;
+    hipLaunchKernelGGL((conv_split_kernel<C>), dim3(u32(tiles), 1, slices), dim3(C::NTH), 0, s, a);
+    int st = check_launch(what);
+    if (st == CRB_OK && slices > 1) st = launch_splitk_reduce(part, Y, count, slices, ReduceEpi{bias, OH * OW, C_OUT, relu ? u32(EPI_RELU) : 0u}, s, what);
+    return st;
+}
+
+}  // namespace crb

@@ -5,6 +5,7 @@
 #include "conv3x3_tiled_wgrad.h"
 #include "conv3x3_wgrad.h"
 #include "conv3x3_wgrad_image.h"
+#include "conv_split.h"
 #include "conv1x1_s2.h"
 #include "conv1x1_wgrad.h"
 #include "conv1x1_stream.h"
@@ -324,6 +325,132 @@ static int launch_tiled_any(const float *Wt, const float *X, float *Y, const flo
 #undef CRB_TILED
 }
 
+// ---- forward and stride-1 data gradient on split bf16 operands (conv_split.h) -------------------------------------------------
+// Configurations <F, S, TM, TN, WM, WN, KG, MAXPX, AHEAD, BSET>: output channels x pixels of a workgroup tile and K groups.
+//   0: 64 x 128, four waves, two workgroups per CU      1: 128 x 64, four waves, two per CU
+//   2: 128 x 64 in two K groups, one per CU             3: 64 x 64 in four K groups, one per CU
+// The choice is the smallest estimate: 6 us for the filters' launch and the workgroups' first and last phases, plus rounds x steps
+// (16 channels of one tap) x a step's rate. Measured at batch 128, 64 -> 64 @32, 128 -> 128 @16, 256 -> 256 @8, 512 -> 512 @4: 0.64 us
+// where a CU holds two of the first two's workgroups, 0.35 where all hold one, 0.34 and 0.19 for the others; on a few dozen CUs
+// (64 -> 64 @20 batch 8, 128 -> 128 @14 batch 8, 256 -> 256 @7 batch 4) 0.17 for the first two. A contraction may be cut into slices
+// on grids that leave CUs idle: one more launch, and the partial results written and read once.
+struct ConvSplitPlan {
+    int cfg = -1;
+    u32 strips = 0, slices = 1;
+    size_t filter_bytes = 0, bytes = 0;  // split filters; with the partial results behind them
+};
+template <int F, int S>
+struct ConvSplitSet {
+    static constexpr int PX = S == 2 ? 384 : 256;
+    typedef ConvSplitCfg<F, S, 1, 2, 2, S == 2 ? 1 : 2, 1, PX, 4, 2> C0;
+    typedef ConvSplitCfg<F, S, 1, 2, 4, 1, 1, PX, 2, 2> C1;
+    typedef ConvSplitCfg<F, S, 1, 2, 4, 1, 2, S == 2 ? 384 : 256, 2, 1> C2;
+    typedef ConvSplitCfg<F, S, 1, 2, 2, 1, 4, 192, 2, 1> C3;
+};
+template <int F, int S>
+static ConvSplitPlan conv_split_plan_for(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 W, u32 OH, u32 OW, float &best_us) {
+    typedef ConvSplitSet<F, S> Set;
+    ConvSplitPlan best;
+    best_us = 3e38f;
+    const float count = float(N) * C_OUT * OH * OW;
+    auto consider = [&](int id, auto cfg, float rate, u32 per_cu) {
+        typedef decltype(cfg) C;
+        const u32 strips = conv_split_strips<C>(OH, OW);
+        // offsets inside the images a tile touches are 32-bit byte offsets
+        if (!strips || (uint64_t(C::PXT) / (uint64_t(OH) * ceil_div(OW, strips)) + 3) * C_IN * H * W * 4 > 0xffffffffull) return;
+        const uint64_t tiles = uint64_t(ceil_div(N * strips * OH * ceil_div(OW, strips), u32(C::PXT))) * ceil_div(C_OUT, u32(C::OCT));
+        const u32 chunks = ceil_div(C_IN, u32(C::CI)), per_round = 256 * per_cu;
+        for (u32 z = 1; z <= chunks && z <= 16; ++z) {
+            const u32 cz = ceil_div(chunks, z);
+            if (ceil_div(chunks, cz) != z || (z > 1 && tiles * z > per_round)) continue;
+            const uint64_t wgs = tiles * z;
+            const u32 rest = u32(wgs % per_round);
+            const float alone = per_cu == 1 ? rate : 0.17f + 0.18f * float(rest) / 256.f;
+            float us = 6.f + float(cz * C::NT) * (float(wgs / per_round) * rate + (rest == 0 ? 0.f : rest <= 256 ? alone : rate));
+            us = us < 12.f ? 12.f : us;
+            if (z > 1) us += 3.5f + float(2 * z + 1) * count * 4e-6f / 5.f;
+            if (us < best_us) {
+                best_us = us;
+                best.cfg = id, best.strips = strips, best.slices = z, best.filter_bytes = conv_split_filter_bytes<C>(C_IN, C_OUT);
+                best.filter_bytes = (best.filter_bytes + 255) & ~size_t(255);
+                best.bytes = best.filter_bytes + (z > 1 ? size_t(z) * N * C_OUT * OH * OW * sizeof(float) : 0);
+            }
+        }
+    };
+    consider(0, typename Set::C0(), S == 2 ? 0.32f : 0.64f, 2);
+    consider(1, typename Set::C1(), 0.64f, 2);
+    consider(2, typename Set::C2(), 0.68f, 1);  // (per step of 32 channels)
+    consider(3, typename Set::C3(), 0.77f, 1);  // (per step of 64 channels)
+    return best;
+}
+// (OH, OW): the pass's result, (H, W): what it reads; direct: a width-specialised kernel takes the pass otherwise
+static ConvSplitPlan conv_split_plan(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 W, u32 OH, u32 OW, u32 F, u32 S, bool direct) {
+    const float mflop = 2e-6f * N * OH * OW * C_IN * C_OUT * F * F;
+    if (C_IN < 16 || C_OUT < 24 || mflop < (direct ? 2000.f : 100.f)) return ConvSplitPlan();
+    ConvSplitPlan p;
+    float us = 0.f;
+    if (F == 3 && S == 1) p = conv_split_plan_for<3, 1>(N, C_IN, C_OUT, H, W, OH, OW, us);
+    if (F == 5 && S == 1) p = conv_split_plan_for<5, 1>(N, C_IN, C_OUT, H, W, OH, OW, us);
+    if (F == 3 && S == 2) p = conv_split_plan_for<3, 2>(N, C_IN, C_OUT, H, W, OH, OW, us);
+    // against the fp32 kernels: the tiled one's throughput or, on few workgroups, the length of a workgroup's contraction; the
+    // engine's throughput
+    const float k = float(C_IN * F * F);
+    const float fp32_us = tiled_pays(N, C_IN, C_OUT, OH, OW, F * F) ? 3.f + std::max(mflop / 75.f, 0.03f * k) : 10.f + mflop / 45.f;
+    if (p.cfg >= 0 && !direct && us > fp32_us) p.cfg = -1;
+    return p;
+}
+// 3x3, pad 1, stride 1 (output = input extent) or stride 2 with even input extents (output = half)
+static bool direct_shape(const crb_conv_geom *g, u32 stride) {
+    return g->FH == 3 && g->FW == 3 && g->sH == stride && g->sW == stride && g->pH == 1 && g->pW == 1 &&
+           g->IH == stride * g->OH && g->IW == stride * g->OW;
+}
+// The plan of a layer's forward pass / data gradient (cfg < 0: not taken): square filters, one stride, any padding up to F - 1.
+static ConvSplitPlan conv_split_fwd_plan(const crb_conv_geom *g, bool aligned) {
+    if (g->FH != g->FW || g->sH != g->sW || g->pH >= g->FH || g->pW >= g->FW) return ConvSplitPlan();
+    bool direct = false;
+    if (aligned && direct_shape(g, 1))
+        try_direct<false, 1>(nullptr, nullptr, nullptr, nullptr, g->N, g->IC, g->OC, g->OH, g->OW, g->IH, 0, nullptr, "", direct, true);
+    else if (aligned && direct_shape(g, 2))
+        try_direct<false, 2>(nullptr, nullptr, nullptr, nullptr, g->N, g->IC, g->OC, g->OH, g->OW, g->IH, 0, nullptr, "", direct, true);
+    return conv_split_plan(g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, g->FH, g->sH, direct);
+}
+static ConvSplitPlan conv_split_dgrad_plan(const crb_conv_geom *g, bool aligned) {
+    if (g->FH != g->FW || g->sH != 1 || g->sW != 1 || g->pH >= g->FH || g->pW >= g->FW) return ConvSplitPlan();
+    bool direct = false;
+    if (aligned && direct_shape(g, 1))
+        try_direct<true, 1>(nullptr, nullptr, nullptr, nullptr, g->N, g->OC, g->IC, g->OH, g->OW, g->OH, 0, nullptr, "", direct, true);
+    return conv_split_plan(g->N, g->OC, g->IC, g->OH, g->OW, g->IH, g->IW, g->FH, 1, direct);
+}
+template <int F, int S, bool DG>
+static int run_conv_split_set(const ConvSplitPlan &p, const float *Wt, const float *X, float *Y, const float *bias, unsigned char *wf, u32 N, u32 C_IN,
+                              u32 C_OUT, u32 H, u32 W, u32 OH, u32 OW, int pad_y, int pad_x, u32 relu, hipStream_t s, const char *what) {
+    typedef ConvSplitSet<F, S> Set;
+    float *part = reinterpret_cast<float *>(wf + p.filter_bytes);
+    switch (p.cfg) {
+        case 0: return launch_conv_split<typename Set::C0, DG>(Wt, X, Y, bias, wf, N, C_IN, C_OUT, H, W, OH, OW, p.strips, p.slices, part, pad_y, pad_x, relu, s, what);
+        case 1: return launch_conv_split<typename Set::C1, DG>(Wt, X, Y, bias, wf, N, C_IN, C_OUT, H, W, OH, OW, p.strips, p.slices, part, pad_y, pad_x, relu, s, what);
+        case 2: return launch_conv_split<typename Set::C2, DG>(Wt, X, Y, bias, wf, N, C_IN, C_OUT, H, W, OH, OW, p.strips, p.slices, part, pad_y, pad_x, relu, s, what);
+        default: return launch_conv_split<typename Set::C3, DG>(Wt, X, Y, bias, wf, N, C_IN, C_OUT, H, W, OH, OW, p.strips, p.slices, part, pad_y, pad_x, relu, s, what);
+    }
+}
+static int run_conv_split_fwd(const ConvSplitPlan &p, const float *W, const float *X, float *Y, const float *bias, const crb_conv_geom *g, u32 relu,
+                              hipStream_t s, const char *what) {
+    unsigned char *wf = nullptr;
+    if (int st = scratch_get(p.bytes, s, what, &wf)) return st;
+    const int py = int(g->pH), px = int(g->pW);
+    if (g->sH == 2) return run_conv_split_set<3, 2, false>(p, W, X, Y, bias, wf, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, py, px, relu, s, what);
+    if (g->FH == 5) return run_conv_split_set<5, 1, false>(p, W, X, Y, bias, wf, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, py, px, relu, s, what);
+    return run_conv_split_set<3, 1, false>(p, W, X, Y, bias, wf, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, py, px, relu, s, what);
+}
+static int run_conv_split_dgrad(const ConvSplitPlan &p, const float *W, const float *dY, float *dX, const crb_conv_geom *g, hipStream_t s,
+                                const char *what) {
+    unsigned char *wf = nullptr;
+    if (int st = scratch_get(p.bytes, s, what, &wf)) return st;
+    const int py = int(g->FH) - 1 - int(g->pH), px = int(g->FW) - 1 - int(g->pW);
+    if (g->FH == 5) return run_conv_split_set<5, 1, true>(p, W, dY, dX, nullptr, wf, g->N, g->OC, g->IC, g->OH, g->OW, g->IH, g->IW, py, px, 0, s, what);
+    return run_conv_split_set<3, 1, true>(p, W, dY, dX, nullptr, wf, g->N, g->OC, g->IC, g->OH, g->OW, g->IH, g->IW, py, px, 0, s, what);
+}
+
 // Direct kernel configurations for 1x1 / stride 1 / no padding layers <W, ROWS, CI, OCT, PBW, OBW, DGRAD, OCC, NBUF, S, FS=1>.
 // The output-channel tile is the widest of 64 / 48 / 32 / 16 that wastes at most a quarter of its channels and still
 // yields enough workgroups for the chip; if none does, the batched GEMM forms run instead.
@@ -402,12 +529,6 @@ static int try_pointwise(const float *Wt, const float *X, float *Y, const float 
 // batched forms of the GEMM family (forward NN with a per-row bias, data gradient TN, weight gradient accumulate-NT).
 static bool pointwise_shape(const crb_conv_geom *g) {
     return g->FH == 1 && g->FW == 1 && g->sH == 1 && g->sW == 1 && g->pH == 0 && g->pW == 0;
-}
-
-// 3x3, pad 1, stride 1 (output = input extent) or stride 2 with even input extents (output = half)
-static bool direct_shape(const crb_conv_geom *g, u32 stride) {
-    return g->FH == 3 && g->FW == 3 && g->sH == stride && g->sW == stride && g->pH == 1 && g->pW == 1 &&
-           g->IH == stride * g->OH && g->IW == stride * g->OW;
 }
 
 // 3x3 / pad 1 / stride 2 on any extent whose images the tiled kernel can address
@@ -705,6 +826,7 @@ static bool bwd_pair(const crb_conv_geom *g, bool run, const float *Wt, const fl
 // results are identical to crb_conv_dgrad followed by crb_conv_wgrad.
 static bool bwd_fused(const crb_conv_geom *g, bool run, const float *Wt, const float *dY, const float *X, float *dX, float *dW,
                       float *ws, hipStream_t s, WgradDirectPlan &plan, int &status) {
+    if (conv_split_dgrad_plan(g, true).cfg >= 0) return false;  // the data gradient has a faster kernel of its own
 #define CRB_PAIR(...) bwd_pair<__VA_ARGS__>(g, run, Wt, dY, X, dX, dW, ws, s, plan, status)
     typedef DirectCfg<32, 8, 16, 16, 4, 1, true, 2, 1, 1, 3, 4> D32a;
     typedef DirectCfg<16, 8, 16, 32, 2, 2, true, 2, 2, 1> D16a;             // chunks of 16 channels
@@ -886,6 +1008,8 @@ int crb_conv_fwd(const float *W, const float *X, float *Y, const float *bias_or_
     if (pointwise_shape(g))
         return gemm_nn_rowbias(W, X, Y, g->OC, g->IH * g->IW, g->IC, g->N, bias_or_null,
                                (flags & CRB_FLAG_RELU) ? u32(EPI_RELU) : 0u, s, "crb_conv_fwd");
+    if (const ConvSplitPlan p = conv_split_fwd_plan(g, aligned16(X) && aligned16(Y)); p.cfg >= 0 && !tiny2x2_shape(g))
+        return run_conv_split_fwd(p, W, X, Y, bias_or_null, g, flags & CRB_FLAG_RELU, s, "crb_conv_fwd");
     if (tiny2x2_shape(g) && aligned16(X) && aligned16(Y))
         return conv2x2_fwd(W, X, Y, bias_or_null, g->N, g->IC, g->OC, (flags & CRB_FLAG_RELU) ? u32(EPI_RELU) : 0u, s, "crb_conv_fwd");
     if (aligned16(X) && aligned16(Y) && (direct_shape(g, 1) || direct_shape(g, 2))) {
@@ -925,6 +1049,8 @@ int crb_conv_dgrad(const float *W, const float *dY, float *dX, const crb_conv_ge
     }
     if (pointwise_shape(g))
         return gemm_tn_batched(W, dY, dX, g->IC, g->IH * g->IW, g->OC, g->N, hipStream_t(stream), "crb_conv_dgrad");
+    if (const ConvSplitPlan p = conv_split_dgrad_plan(g, aligned16(dY) && aligned16(dX)); p.cfg >= 0 && !tiny2x2_shape(g))
+        return run_conv_split_dgrad(p, W, dY, dX, g, hipStream_t(stream), "crb_conv_dgrad");
     if (tiny2x2_shape(g) && aligned16(dY) && aligned16(dX))
         return conv2x2_dgrad(W, dY, dX, g->N, g->IC, g->OC, hipStream_t(stream), "crb_conv_dgrad");
     if (aligned16(dY) && aligned16(dX) && (direct_shape(g, 1) || direct_shape(g, 2))) {
@@ -1114,6 +1240,7 @@ size_t crb_conv_fwd_workspace_bytes(const crb_conv_geom *g, int operands_aligned
         if (done) return 0;
     }
     if (pointwise_shape(g)) return gemm_scratch_bytes(g->OC, g->IH * g->IW, g->IC, g->N);
+    if (const ConvSplitPlan p = conv_split_fwd_plan(g, operands_aligned16 != 0); p.cfg >= 0 && !tiny2x2_shape(g)) return p.bytes;
     if (tiny2x2_shape(g) && operands_aligned16) return gemm_scratch_bytes(g->N, g->OC * 4, g->IC * 4, 1, false);
     if (operands_aligned16 && (direct_shape(g, 1) || direct_shape(g, 2))) {
         if (g->sH == 1)
@@ -1135,6 +1262,7 @@ size_t crb_conv_dgrad_workspace_bytes(const crb_conv_geom *g, int operands_align
         if (done) return 0;
     }
     if (pointwise_shape(g)) return gemm_scratch_bytes(g->IC, g->IH * g->IW, g->OC, g->N);
+    if (const ConvSplitPlan p = conv_split_dgrad_plan(g, operands_aligned16 != 0); p.cfg >= 0 && !tiny2x2_shape(g)) return p.bytes;
     if (tiny2x2_shape(g) && operands_aligned16) return gemm_scratch_bytes(g->N, g->IC * 4, g->OC * 4, 1, false);
     if (operands_aligned16 && (direct_shape(g, 1) || direct_shape(g, 2))) {
         if (g->sH == 1)
