@@ -39,7 +39,7 @@ struct ConvSplitArgs {
     float *Y;
     const float *bias;
     u32 C_IN, C_OUT, chunks;
-    u32 H, W;        // extent of X
+    u32 images, H, W;  // of X
     u32 HW, OHW;     // pixels of an image of X, of Y
     u32 OW, SW, strips;  // width of Y, of a strip
     u32 npix;        // pixels of all strips (those past the image's last column are computed and dropped)
@@ -112,9 +112,8 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
     }
     // staging: item i of a thread is the channel octet o of position s
     const u32 img0 = a.strip_d.div(n0);  // (n0, n: strips of all images, counted through)
-    const float *const xbase = a.X + size_t(img0) * a.C_IN * a.HW;
+    const BufferRange xrange = buffer_range(a.X + size_t(img0) * a.C_IN * a.HW, (size_t(a.images) - img0) * a.C_IN * a.HW);
     u32 off[C::NP];  // bytes from the chunk's first channel of image img0 (the host checks that they fit)
-    u32 valid = 0;
 #pragma unroll
     for (int i = 0; i < C::NP; ++i) {
         const u32 u = threadIdx.x + i * C::NTH, o = u / MAXPX, s = u % MAXPX;
@@ -125,43 +124,34 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
         a.strip_d.divmod(n, img, strip);
         const int iy = int(r) - a.pad_y, ix = int(pc + S * strip * a.SW) - a.pad_x;
         const bool in = s < wpx && u32(iy) < a.H && u32(ix) < a.W;
-        valid |= in ? 1u << i : 0u;
-        off[i] = in ? ((img - img0) * a.C_IN * a.HW + 8 * o * a.HW + u32(iy) * a.W + u32(ix)) * 4u : 0u;
+        const u32 bytes = ((img - img0) * a.C_IN * a.HW + 8 * o * a.HW + u32(iy) * a.W + u32(ix)) * 4u;
+        off[i] = in ? bytes : kOutside;
     }
     float reg[C::NP][8];
     const bool ragged = a.C_IN % C::CI != 0;
     const u32 chunk0 = blockIdx.z * a.chunks_z, chunk1 = chunk0 + a.chunks_z < a.chunks ? chunk0 + a.chunks_z : a.chunks;
-    auto at = [](const float *uniform, u32 bytes) { return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(uniform) + bytes); };
     auto fetch = [&](u32 chunk) {
-        const float *base = xbase + size_t(chunk) * C::CI * a.HW;
+        const u32 c0 = chunk * C::CI;
         if (ragged && chunk + 1 == a.chunks) {
 #pragma unroll
             for (int i = 0; i < C::NP; ++i) {
-                const u32 c0 = chunk * C::CI + 8 * ((threadIdx.x + i * C::NTH) / MAXPX);
+                const u32 o = (threadIdx.x + i * C::NTH) / MAXPX;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const bool ok = c0 + j < a.C_IN;
-                    const float v = at(ok ? base + j * a.HW : xbase, ok ? off[i] : 0u);
-                    reg[i][j] = ok ? v : 0.f;
-                }
+                for (int j = 0; j < 8; ++j) reg[i][j] = buffer_load(xrange, c0 + 8 * o + j < a.C_IN ? off[i] : kOutside, (c0 + j) * a.HW * 4u);
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < C::NP; ++i)
+            for (int j = 0; j < 8; ++j)
 #pragma unroll
-                for (int j = 0; j < 8; ++j) reg[i][j] = at(base + j * a.HW, off[i]);
+                for (int i = 0; i < C::NP; ++i) reg[i][j] = buffer_load(xrange, off[i], (c0 + j) * a.HW * 4u);
         }
     };
     auto commit = [&](unsigned char *sm) {  // (positions behind the run are written too; nothing reads them)
 #pragma unroll
         for (int i = 0; i < C::NP; ++i) {
             const u32 u = threadIdx.x + i * C::NTH, o = u / MAXPX, s = u % MAXPX;
-            const bool in = (valid >> i) & 1u;
-            float v[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = in ? reg[i][j] : 0.f;
             u32x4 part[kSplit];
-            split8(v, part);
+            split8(reg[i], part);
 #pragma unroll
             for (int p = 0; p < kSplit; ++p) *reinterpret_cast<u32x4 *>(sm + p * C::PART + o * (MAXPX * 16) + s * 16) = part[p];
         }
@@ -371,7 +361,7 @@ inline int launch_conv_split(const float *Wt, const float *X, float *Y, const fl
     a.X = X, a.Wf = Wf, a.Y = slices > 1 ? part : Y, a.bias = slices > 1 ? nullptr : bias;
     a.C_IN = C_IN, a.C_OUT = C_OUT, a.chunks = ceil_div(C_IN, u32(C::CI));
     a.strips = strips, a.SW = ceil_div(OW, strips);
-    a.H = H, a.W = W, a.HW = H * W, a.OHW = OH * OW, a.OW = OW, a.npix = N * strips * OH * a.SW;
+    a.images = N, a.H = H, a.W = W, a.HW = H * W, a.OHW = OH * OW, a.OW = OW, a.npix = N * strips * OH * a.SW;
     a.prow = C::S * (OH - 1) + C::F, a.pitch = C::S * (a.SW - 1) + C::F;
     a.pad_y = pad_y, a.pad_x = pad_x;
     a.px_tiles = ceil_div(a.npix, u32(C::PXT)), a.oc_tiles = ceil_div(C_OUT, u32(C::OCT)), a.relu = slices > 1 ? 0 : relu;

@@ -6,6 +6,7 @@
 #include "conv3x3_wgrad.h"
 #include "conv3x3_wgrad_image.h"
 #include "conv_split.h"
+#include "conv_split_wgrad.h"
 #include "conv1x1_s2.h"
 #include "conv1x1_wgrad.h"
 #include "conv1x1_stream.h"
@@ -329,6 +330,7 @@ static int launch_tiled_any(const float *Wt, const float *X, float *Y, const flo
 // Configurations <F, S, TM, TN, WM, WN, KG, MAXPX, AHEAD, BSET>: output channels x pixels of a workgroup tile and K groups.
 //   0: 64 x 128, four waves, two workgroups per CU      1: 128 x 64, four waves, two per CU
 //   2: 128 x 64 in two K groups, one per CU             3: 64 x 64 in four K groups, one per CU
+//   4: 32 x 256, four waves, two per CU
 // The choice is the smallest estimate: 6 us for the filters' launch and the workgroups' first and last phases, plus rounds x steps
 // (16 channels of one tap) x a step's rate. Measured at batch 128, 64 -> 64 @32, 128 -> 128 @16, 256 -> 256 @8, 512 -> 512 @4: 0.64 us
 // where a CU holds two of the first two's workgroups, 0.35 where all hold one, 0.34 and 0.19 for the others; on a few dozen CUs
@@ -341,11 +343,12 @@ struct ConvSplitPlan {
 };
 template <int F, int S>
 struct ConvSplitSet {
-    static constexpr int PX = S == 2 ? 384 : 256;
+    static constexpr int PX = S == 2 || F == 5 ? 384 : 256;
     typedef ConvSplitCfg<F, S, 1, 2, 2, S == 2 ? 1 : 2, 1, PX, 4, 2> C0;
     typedef ConvSplitCfg<F, S, 1, 2, 4, 1, 1, PX, 2, 2> C1;
-    typedef ConvSplitCfg<F, S, 1, 2, 4, 1, 2, S == 2 ? 384 : 256, 2, 1> C2;
+    typedef ConvSplitCfg<F, S, 1, 2, 4, 1, 2, PX, 2, 1> C2;
     typedef ConvSplitCfg<F, S, 1, 2, 2, 1, 4, 192, 2, 1> C3;
+    typedef ConvSplitCfg<F, S, 1, 2, 1, S == 2 ? 2 : 4, 1, 384, 4, 2> C4;
 };
 template <int F, int S>
 static ConvSplitPlan conv_split_plan_for(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 W, u32 OH, u32 OW, float &best_us) {
@@ -356,8 +359,8 @@ static ConvSplitPlan conv_split_plan_for(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 
     auto consider = [&](int id, auto cfg, float rate, u32 per_cu) {
         typedef decltype(cfg) C;
         const u32 strips = conv_split_strips<C>(OH, OW);
-        // offsets inside the images a tile touches are 32-bit byte offsets
-        if (!strips || (uint64_t(C::PXT) / (uint64_t(OH) * ceil_div(OW, strips)) + 3) * C_IN * H * W * 4 > 0xffffffffull) return;
+        // the images a tile touches lie within 2 GiB (buffer loads)
+        if (!strips || (uint64_t(C::PXT) / (uint64_t(OH) * ceil_div(OW, strips)) + 3) * C_IN * H * W * 4 > 0x7fffffffull) return;
         const uint64_t tiles = uint64_t(ceil_div(N * strips * OH * ceil_div(OW, strips), u32(C::PXT))) * ceil_div(C_OUT, u32(C::OCT));
         const u32 chunks = ceil_div(C_IN, u32(C::CI)), per_round = 256 * per_cu;
         for (u32 z = 1; z <= chunks && z <= 16; ++z) {
@@ -381,6 +384,7 @@ static ConvSplitPlan conv_split_plan_for(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 
     consider(1, typename Set::C1(), 0.64f, 2);
     consider(2, typename Set::C2(), 0.68f, 1);  // (per step of 32 channels)
     consider(3, typename Set::C3(), 0.77f, 1);  // (per step of 64 channels)
+    consider(4, typename Set::C4(), S == 2 ? 0.32f : 0.66f, 2);
     return best;
 }
 // (OH, OW): the pass's result, (H, W): what it reads; direct: a width-specialised kernel takes the pass otherwise
@@ -430,6 +434,7 @@ static int run_conv_split_set(const ConvSplitPlan &p, const float *Wt, const flo
         case 0: return launch_conv_split<typename Set::C0, DG>(Wt, X, Y, bias, wf, N, C_IN, C_OUT, H, W, OH, OW, p.strips, p.slices, part, pad_y, pad_x, relu, s, what);
         case 1: return launch_conv_split<typename Set::C1, DG>(Wt, X, Y, bias, wf, N, C_IN, C_OUT, H, W, OH, OW, p.strips, p.slices, part, pad_y, pad_x, relu, s, what);
         case 2: return launch_conv_split<typename Set::C2, DG>(Wt, X, Y, bias, wf, N, C_IN, C_OUT, H, W, OH, OW, p.strips, p.slices, part, pad_y, pad_x, relu, s, what);
+        case 4: return launch_conv_split<typename Set::C4, DG>(Wt, X, Y, bias, wf, N, C_IN, C_OUT, H, W, OH, OW, p.strips, p.slices, part, pad_y, pad_x, relu, s, what);
         default: return launch_conv_split<typename Set::C3, DG>(Wt, X, Y, bias, wf, N, C_IN, C_OUT, H, W, OH, OW, p.strips, p.slices, part, pad_y, pad_x, relu, s, what);
     }
 }
@@ -768,6 +773,76 @@ static bool wgrad_direct(const crb_conv_geom *g, bool run, const float *dY, cons
     return false;
 }
 
+// ---- weight gradient on split bf16 operands (conv_split_wgrad.h) -----------------------------------------------------------------
+// Configurations <F, S, WM, WN, KG, MAXPX>: 32 x 32 channels and 128 pixels a tile, or 64 x 32 and 64 (wide images in fewer strips,
+// and 4 x 4 images, whose eight padded images do not fit the first's LDS); stride 2: 128 x 32 and 32. A tile of either of the first
+// two keeps a CU busy for 3.3 us (128 -> 128 @16 batch 128: 16 tiles a CU, 57 us); the slices, 37 KB or 74 KB per workgroup, are
+// written and read once. The choice is the smaller sum.
+struct SplitWgradChoice {
+    int cfg = -1;
+    SplitWgradPlan plan;
+};
+template <int F, int S>
+struct SplitWgradSet {
+    typedef SplitWgradCfg<F, S, 1, 1, 8, 256> C0;
+    typedef SplitWgradCfg<F, S, 2, 1, 4, 256> C1;
+};
+template <>
+struct SplitWgradSet<3, 2> {
+    typedef SplitWgradCfg<3, 2, 4, 1, 2, 256> C0;
+    typedef C0 C1;
+};
+template <int F, int S>
+static SplitWgradChoice split_wgrad_choice_for(const crb_conv_geom *g, float &best_us) {
+    typedef SplitWgradSet<F, S> Set;
+    SplitWgradChoice best;
+    best_us = 3e38f;
+    auto consider = [&](int id, auto cfg) {
+        typedef decltype(cfg) C;
+        const SplitWgradPlan p = split_wgrad_plan<C>(g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW);
+        if (!p.strips || (p.splits > 1 && uint64_t(p.splits) * g->OC * g->IC * F * F > 0x7fffffffull)) return;
+        const u32 rows = F / C::ROWS, rounds = ceil_div(p.pairs * p.splits * rows, 256u);
+        float us = 5.f + float(rounds * p.tiles_z) * 3.3f * C::NTW / 9.f;
+        if (p.splits > 1) us += 3.f + 2.f * float(p.workspace_bytes) / 5e6f;
+        if (us < best_us) best_us = us, best.cfg = id, best.plan = p;
+    };
+    consider(0, typename Set::C0());
+    if constexpr (S == 1) consider(1, typename Set::C1());
+    return best;
+}
+// cfg < 0: not taken.
+static SplitWgradChoice split_wgrad_choice(const crb_conv_geom *g) {
+    const SplitWgradChoice none;
+    if (g->FH != g->FW || g->sH != g->sW || g->pH >= g->FH || g->pW >= g->FW || g->IC < 16 || g->OC < 16 || tiny2x2_shape(g)) return none;
+    WgradDirectPlan dp;
+    int st = 0;
+    const bool direct = wgrad_direct(g, false, nullptr, nullptr, nullptr, nullptr, nullptr, dp, st);
+    const float mflop = 2e-6f * g->N * g->OH * g->OW * g->IC * g->OC * g->FH * g->FW;
+    if (mflop < (direct ? 2000.f : 100.f)) return none;
+    float us = 0.f;
+    SplitWgradChoice c;
+    if (g->FH == 3 && g->sH == 1) c = split_wgrad_choice_for<3, 1>(g, us);
+    if (g->FH == 5 && g->sH == 1) c = split_wgrad_choice_for<5, 1>(g, us);
+    // (the stride-2 tile is 128 output channels wide: 32 -> 32 @56 batch 32 28 -> 31 us, 64 -> 128 @56 64 -> 51)
+    if (g->FH == 3 && g->sH == 2 && g->OC >= 64) c = split_wgrad_choice_for<3, 2>(g, us);
+    return c;
+}
+template <int F, int S>
+static int run_split_wgrad_set(const SplitWgradChoice &c, const float *dY, const float *X, float *dW, float *ws, const crb_conv_geom *g, hipStream_t s,
+                               const char *what) {
+    typedef SplitWgradSet<F, S> Set;
+    const int py = int(g->pH), px = int(g->pW);
+    if (c.cfg == 0) return launch_split_wgrad<typename Set::C0>(c.plan, dY, X, dW, ws, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, py, px, s, what);
+    return launch_split_wgrad<typename Set::C1>(c.plan, dY, X, dW, ws, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, py, px, s, what);
+}
+// dW == nullptr: the slices stay in ws, unsummed
+static int run_split_wgrad(const SplitWgradChoice &c, const float *dY, const float *X, float *dW, float *ws, const crb_conv_geom *g, hipStream_t s,
+                           const char *what) {
+    if (g->sH == 2) return run_split_wgrad_set<3, 2>(c, dY, X, dW, ws, g, s, what);
+    if (g->FH == 5) return run_split_wgrad_set<5, 1>(c, dY, X, dW, ws, g, s, what);
+    return run_split_wgrad_set<3, 1>(c, dY, X, dW, ws, g, s, what);
+}
+
 // ---- data gradient and weight gradient of one layer in one launch ------------------------------------------------------
 // The two gradients of a layer are independent (dX = f(W, dY), dW += f(dY, X)), and each of their kernels alone leaves the
 // chip idle while it ramps up, loads its first tiles and drains. Launched as one grid — the longer-running kind of workgroup
@@ -826,7 +901,7 @@ static bool bwd_pair(const crb_conv_geom *g, bool run, const float *Wt, const fl
 // results are identical to crb_conv_dgrad followed by crb_conv_wgrad.
 static bool bwd_fused(const crb_conv_geom *g, bool run, const float *Wt, const float *dY, const float *X, float *dX, float *dW,
                       float *ws, hipStream_t s, WgradDirectPlan &plan, int &status) {
-    if (conv_split_dgrad_plan(g, true).cfg >= 0) return false;  // the data gradient has a faster kernel of its own
+    if (conv_split_dgrad_plan(g, true).cfg >= 0 || split_wgrad_choice(g).cfg >= 0) return false;  // a gradient has a faster kernel of its own
 #define CRB_PAIR(...) bwd_pair<__VA_ARGS__>(g, run, Wt, dY, X, dX, dW, ws, s, plan, status)
     typedef DirectCfg<32, 8, 16, 16, 4, 1, true, 2, 1, 1, 3, 4> D32a;
     typedef DirectCfg<16, 8, 16, 32, 2, 2, true, 2, 2, 1> D16a;             // chunks of 16 channels
@@ -1102,6 +1177,7 @@ size_t crb_conv_wgrad_workspace_bytes(const crb_conv_geom *g) {
     }
     if (tiny2x2_shape(g)) return size_t(g->OC) * g->IC * 16 * sizeof(float);  // (oc, p) x (ic, p') product before the tap fold
     if (shortcut_shape(g)) return sc_wgrad_plan(g->N, g->IC, g->OC, g->OH, g->OW).workspace_bytes;
+    if (const SplitWgradChoice c = split_wgrad_choice(g); c.cfg >= 0) return c.plan.workspace_bytes;
     {
         WgradDirectPlan dp;
         TiledWgradPlan tp;
@@ -1158,6 +1234,18 @@ int crb_conv_wgrad(const float *dY, const float *X, float *dW, const crb_conv_ge
             return st;
         }
         return launch_sc_wgrad(dY, X, dW, part, sp, g->N, g->IC, g->OC, g->OH, g->OW, s, "crb_conv_wgrad");
+    }
+    if (const SplitWgradChoice c = split_wgrad_choice(g); c.cfg >= 0) {
+        float *sws = static_cast<float *>(workspace);
+        if (c.plan.workspace_bytes) {
+            if (sws) {
+                if (workspace_bytes < c.plan.workspace_bytes)
+                    return fail(CRB_EWORKSPACE, "crb_conv_wgrad: workspace %zu bytes < required %zu", workspace_bytes, c.plan.workspace_bytes);
+            } else if (int sg = scratch_get(c.plan.workspace_bytes, s, "crb_conv_wgrad", &sws)) {
+                return sg;
+            }
+        }
+        return run_split_wgrad(c, dY, X, dW, sws, g, s, "crb_conv_wgrad");
     }
     if (aligned16(dY) && aligned16(X)) {
         WgradDirectPlan dp;
@@ -1319,7 +1407,9 @@ uint32_t crb_conv_bwd_slices(const crb_conv_geom *g) {
         const u32 n = sc_wgrad_plan(g->N, g->IC, g->OC, g->OH, g->OW).splits;
         return n > 1 ? n : 0;
     }
+    // (layers without a width-specialised kernel have no sliced form)
     if (!wgrad_direct(g, false, nullptr, nullptr, nullptr, nullptr, nullptr, dp, st)) return 0;
+    if (const SplitWgradChoice c = split_wgrad_choice(g); c.cfg >= 0) return c.plan.splits > 1 ? c.plan.splits : 0;
     return dp.splits > 1 ? dp.splits : 0;
 }
 
@@ -1352,6 +1442,12 @@ int crb_conv_bwd_sliced(const float *W, const float *dY, const float *X, float *
             return fail(CRB_EWORKSPACE, "crb_conv_bwd_sliced: workspace %zu bytes < required %zu", workspace_bytes, dp.workspace_bytes);
         bwd_fused(g, true, W, dY, X, dX, nullptr, ws, s, dp, st);
         return st;
+    }
+    if (const SplitWgradChoice c = split_wgrad_choice(g); c.cfg >= 0) {
+        if (workspace_bytes < c.plan.workspace_bytes)
+            return fail(CRB_EWORKSPACE, "crb_conv_bwd_sliced: workspace %zu bytes < required %zu", workspace_bytes, c.plan.workspace_bytes);
+        if (int sd = crb_conv_dgrad(W, dY, dX, g, stream)) return sd;
+        return run_split_wgrad(c, dY, X, nullptr, ws, g, s, "crb_conv_bwd_sliced");
     }
     wgrad_direct(g, false, nullptr, nullptr, nullptr, nullptr, nullptr, dp, st);
     if (workspace_bytes < dp.workspace_bytes)

@@ -45,6 +45,19 @@ __device__ __forceinline__ void split8(const float *x, u32x4 (&part)[kSplit]) {
     }
 }
 
+// A float at `voffset + soffset` bytes behind a uniform base, by a buffer load: the address needs no vector arithmetic beyond
+// voffset, and an element that is to read as zero (halo, channels past the tensor) is named by kOutside, which the resource's
+// range check turns into 0. Ranges are under 2 GiB.
+constexpr u32 kOutside = 0x80000000u;
+typedef __amdgpu_buffer_rsrc_t BufferRange;
+__device__ __forceinline__ BufferRange buffer_range(const float *base, size_t floats) {
+    const size_t bytes = floats * 4;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base), 0, int(bytes < 0x7fffffffu ? bytes : 0x7fffffffu), 0x00020000);
+}
+__device__ __forceinline__ float buffer_load(BufferRange r, u32 voffset, u32 soffset) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, int(voffset), int(soffset), 0));
+}
+
 // The products that are formed: (part of A, part of B), in an order that needs the leading parts first.
 constexpr int kTerms = 6;
 constexpr int kTermA[kTerms] = {0, 0, 1, 1, 0, 2};

@@ -1,0 +1,40 @@
+"""Convolutions on the split engine (csrc/conv_split.h, conv_split_wgrad.h) where their tiles, strips, channel chunks and slices
+end, against the CPU oracle."""
+import numpy as np
+import pytest
+
+from oracle import seblas_oracle as orc
+from tests.util import assert_close, he_normal, normal, to_dev, to_np
+
+pytestmark = pytest.mark.gpu
+
+# (N, IC, H, W, OC, F, stride, pad): a last pixel tile of a few pixels, images narrower than a filter's reach and wider than a
+# strip (uneven strips, a strip of padding columns), several images per tile, channels one past / one short of 16, 32 and 64,
+# a contraction cut into slices, every padding, 5x5 with its rows in separate workgroups, stride 2 with odd extents
+SHAPES = [(3, 64, 31, 33, 65, 3, 1, 1), (2, 33, 67, 61, 63, 3, 1, 1), (1, 47, 29, 131, 49, 3, 1, 1), (33, 96, 7, 5, 97, 3, 1, 1), (5, 129, 13, 14, 127, 3, 1, 0),
+          (3, 80, 15, 17, 48, 3, 1, 2), (2, 300, 9, 11, 70, 3, 1, 1), (7, 31, 21, 19, 33, 5, 1, 2), (3, 40, 18, 23, 65, 5, 1, 0), (2, 36, 12, 50, 40, 5, 1, 4),
+          (4, 65, 33, 27, 97, 3, 2, 1), (3, 48, 30, 31, 66, 3, 2, 0), (70, 512, 4, 4, 96, 3, 1, 1), (64, 64, 32, 32, 64, 3, 1, 1), (9, 72, 20, 3, 80, 3, 1, 1)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_split_convolution_edges(dev, shape):
+    import torch
+    from crusaderbackend_amd import capi
+
+    N, IC, H, W, OC, F, s, p = shape
+    g = capi.ConvGeom.make(N, IC, H, W, OC, F, F, s, s, p, p)
+    X, Wt, dY, b = normal(1, N, IC, H, W), he_normal(2, OC, IC, F, F), normal(3, N, OC, g.OH, g.OW), normal(4, OC)
+    dW0 = he_normal(5, OC, IC, F, F)
+    Xd, Wd, dYd, bd, dW = (to_dev(a, dev) for a in (X, Wt, dY, b, dW0))
+    Y, dX = torch.empty(N, OC, g.OH, g.OW, device=dev), torch.empty(N, IC, H, W, device=dev)
+    capi.conv_fwd(Wd, Xd, Y, bd, g, capi.CRB_FLAG_RELU)
+    capi.conv_dgrad(Wd, dYd, dX, g)
+    capi.conv_wgrad(dYd, Xd, dW, g)
+    torch.cuda.synchronize()
+    assert_close(to_np(Y), np.maximum(orc.conv(Wt, X, b, s, s, p, p), 0), IC * F * F, f"forward {shape}")
+    assert_close(to_np(dX), orc.convDerive(Wt, dY, (H, W), s, s, p, p), OC * F * F, f"data gradient {shape}")
+    assert_close(to_np(dW), orc.convError(dY, X, dW0, s, s, p, p), N * g.OH * g.OW, f"weight gradient {shape}")
+    dX2, dW2 = torch.empty_like(dX), to_dev(dW0, dev)
+    capi.conv_bwd(Wd, dYd, Xd, dX2, dW2, g)
+    torch.cuda.synchronize()
+    assert torch.equal(dX, dX2) and torch.equal(dW, dW2)  # one call for both gradients: the same bits
