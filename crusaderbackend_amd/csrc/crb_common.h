@@ -29,6 +29,9 @@ inline int scratch_get(size_t bytes, hipStream_t stream, const char *what, T **o
     *out = static_cast<T *>(p);
     return st;
 }
+// Whether scratch_get would serve such a request (taking that its hipMalloc succeeds): a kernel that wants scratch yields to one
+// that needs less where a scope or bound workspace is too small for it, or a capture forbids growth.
+bool scratch_available(size_t bytes, hipStream_t stream);
 int scratch_bind(void *ptr, size_t bytes, hipStream_t stream);
 void arena_release();
 // While alive, every scratch_get of this thread is served from [ptr, ptr + bytes) or refused; nothing is allocated.

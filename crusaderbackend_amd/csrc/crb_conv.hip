@@ -1064,6 +1064,27 @@ static int static_scratch_ptr(const char *what, void **out) {
     return CRB_OK;
 }
 
+// Scratch of crb_conv_wgrad; split: where the kernel on split operands may be taken.
+static size_t wgrad_scratch_bytes(const crb_conv_geom *g, bool split) {
+    if (pointwise_shape(g)) {  // pixel-contraction kernel, or (unaligned / wide layers) the accumulate-NT GEMM form
+        const size_t gemm = uint64_t(g->IH) * g->IW * g->N > 0x7fffffffull ? 0 : gemm_scratch_bytes(g->OC, g->IC, g->IH * g->IW * g->N, 1, split);
+        if (!pw_wgrad_fits(g->IC, g->OC, g->IH * g->IW)) return gemm;
+        return std::max(gemm, pw_wgrad_plan(g->N, g->IC, g->OC, g->IH * g->IW).workspace_bytes);
+    }
+    if (tiny2x2_shape(g)) return size_t(g->OC) * g->IC * 16 * sizeof(float);  // (oc, p) x (ic, p') product before the tap fold
+    if (shortcut_shape(g)) return sc_wgrad_plan(g->N, g->IC, g->OC, g->OH, g->OW).workspace_bytes;
+    if (const SplitWgradChoice c = split_wgrad_choice(g); split && c.cfg >= 0) return c.plan.workspace_bytes;
+    {
+        WgradDirectPlan dp;
+        TiledWgradPlan tp;
+        int st = 0;
+        if (wgrad_direct(g, false, nullptr, nullptr, nullptr, nullptr, nullptr, dp, st)) return dp.workspace_bytes;
+        if (wgrad_tiled(g, false, nullptr, nullptr, nullptr, nullptr, nullptr, tp, st)) return tp.workspace_bytes;
+    }
+    const WgradPlan p = wgrad_plan(g);
+    return p.splits > 1 ? size_t(p.splits) * p.M * p.Ncols * sizeof(float) : 0;
+}
+
 }  // namespace crb
 
 using namespace crb;
@@ -1088,7 +1109,7 @@ int crb_conv_fwd(const float *W, const float *X, float *Y, const float *bias_or_
     if (pointwise_shape(g))
         return gemm_nn_rowbias(W, X, Y, g->OC, g->IH * g->IW, g->IC, g->N, bias_or_null,
                                (flags & CRB_FLAG_RELU) ? u32(EPI_RELU) : 0u, s, "crb_conv_fwd");
-    if (const ConvSplitPlan p = conv_split_fwd_plan(g, aligned16(X) && aligned16(Y)); p.cfg >= 0 && !tiny2x2_shape(g))
+    if (const ConvSplitPlan p = conv_split_fwd_plan(g, aligned16(X) && aligned16(Y)); p.cfg >= 0 && !tiny2x2_shape(g) && scratch_available(p.bytes, s))
         return run_conv_split_fwd(p, W, X, Y, bias_or_null, g, flags & CRB_FLAG_RELU, s, "crb_conv_fwd");
     if (tiny2x2_shape(g) && aligned16(X) && aligned16(Y))
         return conv2x2_fwd(W, X, Y, bias_or_null, g->N, g->IC, g->OC, (flags & CRB_FLAG_RELU) ? u32(EPI_RELU) : 0u, s, "crb_conv_fwd");
@@ -1129,7 +1150,8 @@ int crb_conv_dgrad(const float *W, const float *dY, float *dX, const crb_conv_ge
     }
     if (pointwise_shape(g))
         return gemm_tn_batched(W, dY, dX, g->IC, g->IH * g->IW, g->OC, g->N, hipStream_t(stream), "crb_conv_dgrad");
-    if (const ConvSplitPlan p = conv_split_dgrad_plan(g, aligned16(dY) && aligned16(dX)); p.cfg >= 0 && !tiny2x2_shape(g))
+    if (const ConvSplitPlan p = conv_split_dgrad_plan(g, aligned16(dY) && aligned16(dX));
+        p.cfg >= 0 && !tiny2x2_shape(g) && scratch_available(p.bytes, hipStream_t(stream)))
         return run_conv_split_dgrad(p, W, dY, dX, g, hipStream_t(stream), "crb_conv_dgrad");
     if (tiny2x2_shape(g) && aligned16(dY) && aligned16(dX))
         return conv2x2_dgrad(W, dY, dX, g->N, g->IC, g->OC, hipStream_t(stream), "crb_conv_dgrad");
@@ -1175,23 +1197,7 @@ int crb_conv_dgrad(const float *W, const float *dY, float *dX, const crb_conv_ge
 
 size_t crb_conv_wgrad_workspace_bytes(const crb_conv_geom *g) {
     if (check_geom("crb_conv_wgrad_workspace_bytes", g)) return 0;
-    if (pointwise_shape(g)) {  // pixel-contraction kernel, or (unaligned / wide layers) the accumulate-NT GEMM form
-        const size_t gemm = uint64_t(g->IH) * g->IW * g->N > 0x7fffffffull ? 0 : gemm_scratch_bytes(g->OC, g->IC, g->IH * g->IW * g->N, 1);
-        if (!pw_wgrad_fits(g->IC, g->OC, g->IH * g->IW)) return gemm;
-        return std::max(gemm, pw_wgrad_plan(g->N, g->IC, g->OC, g->IH * g->IW).workspace_bytes);
-    }
-    if (tiny2x2_shape(g)) return size_t(g->OC) * g->IC * 16 * sizeof(float);  // (oc, p) x (ic, p') product before the tap fold
-    if (shortcut_shape(g)) return sc_wgrad_plan(g->N, g->IC, g->OC, g->OH, g->OW).workspace_bytes;
-    if (const SplitWgradChoice c = split_wgrad_choice(g); c.cfg >= 0) return c.plan.workspace_bytes;
-    {
-        WgradDirectPlan dp;
-        TiledWgradPlan tp;
-        int st = 0;
-        if (wgrad_direct(g, false, nullptr, nullptr, nullptr, nullptr, nullptr, dp, st)) return dp.workspace_bytes;
-        if (wgrad_tiled(g, false, nullptr, nullptr, nullptr, nullptr, nullptr, tp, st)) return tp.workspace_bytes;
-    }
-    const WgradPlan p = wgrad_plan(g);
-    return p.splits > 1 ? size_t(p.splits) * p.M * p.Ncols * sizeof(float) : 0;
+    return wgrad_scratch_bytes(g, true);
 }
 
 int crb_conv_wgrad(const float *dY, const float *X, float *dW, const crb_conv_geom *g, void *workspace,
@@ -1240,16 +1246,12 @@ int crb_conv_wgrad(const float *dY, const float *X, float *dW, const crb_conv_ge
         }
         return launch_sc_wgrad(dY, X, dW, part, sp, g->N, g->IC, g->OC, g->OH, g->OW, s, "crb_conv_wgrad");
     }
-    if (const SplitWgradChoice c = split_wgrad_choice(g); c.cfg >= 0) {
+    // (scratch that holds too little for its slices may still be enough for the kernels below)
+    if (const SplitWgradChoice c = split_wgrad_choice(g);
+        c.cfg >= 0 && (workspace ? workspace_bytes >= c.plan.workspace_bytes : scratch_available(c.plan.workspace_bytes, s))) {
         float *sws = static_cast<float *>(workspace);
-        if (c.plan.workspace_bytes) {
-            if (sws) {
-                if (workspace_bytes < c.plan.workspace_bytes)
-                    return fail(CRB_EWORKSPACE, "crb_conv_wgrad: workspace %zu bytes < required %zu", workspace_bytes, c.plan.workspace_bytes);
-            } else if (int sg = scratch_get(c.plan.workspace_bytes, s, "crb_conv_wgrad", &sws)) {
-                return sg;
-            }
-        }
+        if (c.plan.workspace_bytes && !sws)
+            if (int sg = scratch_get(c.plan.workspace_bytes, s, "crb_conv_wgrad", &sws)) return sg;
         return run_split_wgrad(c, dY, X, dW, sws, g, s, "crb_conv_wgrad");
     }
     if (aligned16(dY) && aligned16(X)) {
@@ -1312,7 +1314,8 @@ int crb_conv_wgrad(const float *dY, const float *X, float *dW, const crb_conv_ge
 int crb_conv_wgrad_noalloc(const float *dY, const float *X, float *dW, const crb_conv_geom *g, void *stream) {
     if (!dY || !X || !dW) return fail(CRB_ENULL, "crb_conv_wgrad_noalloc: null operand");
     if (int st = check_geom("crb_conv_wgrad_noalloc", g)) return st;
-    const size_t need = crb_conv_wgrad_workspace_bytes(g);
+    size_t need = wgrad_scratch_bytes(g, true);
+    if (need > kStaticScratchBytes) need = wgrad_scratch_bytes(g, false);  // the kernel behind the split one
     if (need > kStaticScratchBytes)
         return fail(CRB_EWORKSPACE,
                     "crb_conv_wgrad_noalloc: this geometry needs %zu bytes of scratch, the built-in buffer holds %zu; use "

@@ -55,6 +55,30 @@ ScratchScope::ScratchScope(void *ptr, size_t bytes) : prev_ptr(g_scope_ptr), pre
 }
 ScratchScope::~ScratchScope() { g_scope_ptr = prev_ptr, g_scope_bytes = prev_bytes, g_scope_used = prev_used; }
 
+// a capture query that fails (the legacy stream while another stream captures in global mode) counts as capturing
+static bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return cap != hipStreamCaptureStatusNone;
+}
+
+bool scratch_available(size_t bytes, hipStream_t stream) {
+    if (!bytes) return true;
+    if (g_scope_ptr) {
+        const size_t at = (g_scope_used + 255) & ~size_t(255);
+        return at <= g_scope_bytes && bytes <= g_scope_bytes - at;
+    }
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return true;  // (scratch_get reports it)
+    std::lock_guard<std::mutex> lk(g_arena_mu);
+    const auto it = g_arenas.find(std::make_pair(dev, stream));
+    if (it != g_arenas.end() && bytes <= it->second.bytes) return true;
+    return !(it != g_arenas.end() && it->second.bound) && !capturing(stream);
+}
+
 int scratch_get(size_t bytes, hipStream_t stream, const char *what, void **out) {
     *out = nullptr;
     if (g_scope_ptr) {
@@ -81,14 +105,7 @@ int scratch_get(size_t bytes, hipStream_t stream, const char *what, void **out) 
         *out = a.ptr;
         return CRB_OK;
     }
-    // growing means hipMalloc, which a stream capture cannot record
-    // (a capture query that fails — the legacy stream while another stream captures in global mode — counts as capturing)
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
-        (void)hipGetLastError();
-        cap = hipStreamCaptureStatusActive;
-    }
-    if (cap != hipStreamCaptureStatusNone)
+    if (capturing(stream))  // growing means hipMalloc, which a stream capture cannot record
         return fail(CRB_EWORKSPACE,
                     "%s: needs %zu bytes of scratch while the stream is being captured; bind a workspace to the stream "
                     "(crb_bind_workspace) or run the call once before capturing", what, bytes);

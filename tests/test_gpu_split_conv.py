@@ -38,3 +38,28 @@ def test_split_convolution_edges(dev, shape):
     capi.conv_bwd(Wd, dYd, Xd, dX2, dW2, g)
     torch.cuda.synchronize()
     assert torch.equal(dX, dX2) and torch.equal(dW, dW2)  # one call for both gradients: the same bits
+
+
+@pytest.mark.parametrize("shape", [(32, 64, 28, 28, 64, 3, 1, 1), (32, 64, 28, 28, 64, 5, 1, 2)], ids=lambda s: "x".join(map(str, s)))
+def test_layers_run_where_the_split_kernels_have_no_scratch(dev, shape):
+    """A bound workspace too small for the split filters leaves the passes to the kernels that need none."""
+    import torch
+    from crusaderbackend_amd import capi
+
+    N, IC, H, W, OC, F, s, p = shape
+    g = capi.ConvGeom.make(N, IC, H, W, OC, F, F, s, s, p, p)
+    assert capi.conv_fwd_workspace_bytes(g) > 256 and capi.conv_dgrad_workspace_bytes(g) > 256
+    X, Wt, dY = normal(1, N, IC, H, W), he_normal(2, OC, IC, F, F), normal(3, N, OC, g.OH, g.OW)
+    Xd, Wd, dYd = (to_dev(a, dev) for a in (X, Wt, dY))
+    Y, dX = torch.empty(N, OC, g.OH, g.OW, device=dev), torch.empty(N, IC, H, W, device=dev)
+    st, tiny = torch.cuda.Stream(device=dev), torch.empty(64, device=dev)
+    torch.cuda.synchronize()
+    try:
+        capi.bind_workspace(tiny, stream=st)
+        capi.conv_fwd(Wd, Xd, Y, None, g, stream=st)
+        capi.conv_dgrad(Wd, dYd, dX, g, stream=st)
+        st.synchronize()
+    finally:
+        capi.bind_workspace(None, stream=st)
+    assert_close(to_np(Y), orc.conv(Wt, X, None, s, s, p, p), IC * F * F, f"forward {shape}")
+    assert_close(to_np(dX), orc.convDerive(Wt, dY, (H, W), s, s, p, p), OC * F * F, f"data gradient {shape}")
