@@ -36,6 +36,8 @@ struct ConvSplitCfg {
 struct ConvSplitArgs {
     const float *X;
     const unsigned char *Wf;  // split filters
+    const float *Wt;          // the filters: element (output channel, input channel, tap) at oc * w_oc + ic * w_ic + tap (mirrored: NT-1-tap)
+    u32 w_oc, w_ic, mirrored;
     float *Y;
     const float *bias;
     u32 C_IN, C_OUT, chunks;
@@ -274,6 +276,22 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
             if (a.relu) o = o > 0.f ? o : 0.f;
             if (oc < a.C_OUT) y[size_t(oc) * a.OHW] = o;
         }
+        for (u32 redo = not_finite<NR>(res); redo; redo &= redo - 1) {
+            const u32 r = __builtin_ctz(redo), oc = oc0 + 8 * (r / 4) + (r % 4);
+            if (oc >= a.C_OUT) continue;
+            float sum = 0.f;
+            const u32 c1 = chunk1 * C::CI < a.C_IN ? chunk1 * C::CI : a.C_IN;
+            for (u32 ic = chunk0 * C::CI; ic < c1 && !__builtin_isnan(sum); ++ic)
+                for (u32 tap = 0; tap < u32(NT); ++tap) {
+                    const int iy = int(S * yy + tap / F) - a.pad_y, ix = int(S * xx + tap % F) - a.pad_x;
+                    if (u32(iy) >= a.H || u32(ix) >= a.W) continue;
+                    const float w = a.Wt[size_t(oc) * a.w_oc + size_t(ic) * a.w_ic + (a.mirrored ? NT - 1 - tap : tap)];
+                    sum = fmaf(w, a.X[(size_t(img) * a.C_IN + ic) * a.HW + u32(iy) * a.W + u32(ix)], sum);
+                }
+            if (a.bias) sum += a.bias[oc];
+            if (a.relu) sum = sum > 0.f ? sum : 0.f;
+            y[size_t(oc) * a.OHW] = sum;
+        }
     };
     if constexpr (KG == 1) {
 #pragma unroll
@@ -358,6 +376,7 @@ inline int launch_conv_split(const float *Wt, const float *X, float *Y, const fl
                              u32 W, u32 OH, u32 OW, u32 strips, u32 slices, float *part, int pad_y, int pad_x, u32 relu, hipStream_t s,
                              const char *what) {
     ConvSplitArgs a;
+    a.Wt = Wt, a.w_oc = DGRAD ? C::NT : C_IN * C::NT, a.w_ic = DGRAD ? C_OUT * C::NT : C::NT, a.mirrored = DGRAD;
     a.X = X, a.Wf = Wf, a.Y = slices > 1 ? part : Y, a.bias = slices > 1 ? nullptr : bias;
     a.C_IN = C_IN, a.C_OUT = C_OUT, a.chunks = ceil_div(C_IN, u32(C::CI));
     a.strips = strips, a.SW = ceil_div(OW, strips);

@@ -55,7 +55,6 @@ __device__ __forceinline__ u32 small_div(u32 n, u32 m) { return __umul24(n, m) >
 
 __device__ __forceinline__ bf16x8 read_transposed(const unsigned char *lds0, const unsigned char *lds1) {
     typedef short s16x4 __attribute__((ext_vector_type(4)));
-    typedef short s16x8 __attribute__((ext_vector_type(8)));
     typedef __attribute__((address_space(3))) s16x4 *lp;
     const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(lds0)), b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(lds1));
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -269,6 +268,22 @@ __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a
         for (int t = 0; t < NTW; ++t) x[(row * C::ICT + wn * 32 + (lane & 31)) * NTW + t] = own[t][i];
     }
     lds_barrier();
+    // this slice's sum of one filter element from the fp32 operands (split_bf16.h: sums that are not finite)
+    auto plain_sum = [&](u32 oc, u32 ic, u32 fh, u32 fw) {
+        float sum = 0.f;
+        const u32 p1 = t1 * PXT < a.npix ? t1 * PXT : a.npix;
+        for (u32 p = t0 * PXT; p < p1 && !__builtin_isnan(sum); ++p) {
+            u32 v, r, y, xx, img, strip;
+            a.ohw.divmod(p, v, r);
+            a.ow.divmod(r, y, xx);
+            a.strip_d.divmod(v, img, strip);
+            xx += strip * a.SW;
+            const int iy = int(S * y + fh) - a.pad_y, ix = int(S * xx + fw) - a.pad_x;
+            if (xx >= a.OW || u32(iy) >= a.H || u32(ix) >= a.W) continue;
+            sum = fmaf(a.dY[(size_t(img) * a.OC + oc) * a.OHW + y * a.OW + xx], a.X[(size_t(img) * a.IC + ic) * a.HW + u32(iy) * a.W + u32(ix)], sum);
+        }
+        return sum;
+    };
     constexpr u32 ROW = C::ICT * NTW;
     const u32 nic = a.IC - ic0 < u32(C::ICT) ? a.IC - ic0 : u32(C::ICT);
     float *out = a.out + (a.splits > 1 ? size_t(z) * a.OC * a.IC * (F * F) : 0);
@@ -276,7 +291,9 @@ __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a
         const u32 oc = e / ROW, rest = e % ROW, ic = rest / NTW, t = rest % NTW;
         if (oc0 + oc < a.OC && ic < nic) {
             float *dst = out + ((size_t(oc0 + oc) * a.IC + ic0 + ic) * (F * F) + fh0 * F + t);
-            if (a.splits > 1) *dst = x[e]; else *dst += x[e];
+            float v = x[e];
+            if (!__builtin_isfinite(v)) v = plain_sum(oc0 + oc, ic0 + ic, fh0 + t / F, t % F);
+            if (a.splits > 1) *dst = v; else *dst += v;
         }
     }
 }

@@ -26,10 +26,8 @@ typedef float v2fu __attribute__((ext_vector_type(2), aligned(4)));
 
 // How an operand of the split engine is read.
 enum SplitLoad {
-    LOAD_K8,    // k-contiguous: fetch8(row, k, klimit, out[8])
-    LOAD_ROWS,  // row-contiguous: fetch_rows<RV>(row, k, klimit, out[RV])
-    LOAD_ROW1,  // gathers, lanes along rows: prep_row / prep_k / fetch of one element
-    LOAD_KLANE  // gathers, lanes along k: the same, pairs of k exchanged between neighbouring lanes
+    LOAD_K8,   // k-contiguous: a cursor's fetch gives eight k of one row
+    LOAD_ROWS  // row-contiguous: eight k of RV neighbouring rows
 };
 
 // ---- plain matrices, any size and alignment ----------------------------------------------------------------------------
@@ -50,6 +48,11 @@ struct SMatK {
         u32 k;  // offset of the item's octet inside a slab
     };
     __device__ __forceinline__ void bind(u32 z) { base += size_t(z) * zstride; }
+    __device__ __forceinline__ float at(u32 row, u32 k) const {
+        u32 nd = 0, kk = k;
+        if constexpr (CAT) cat_k.divmod(k, nd, kk);
+        return base[size_t(nd) * cat_stride + size_t(row) * ld + kk];
+    }
     __device__ __forceinline__ Cursor cursor(u32 row, u32 k) const { return {base + size_t(row < rows ? row : rows - 1) * ld, k}; }
     template <bool TAIL>
     __device__ __forceinline__ void fetch(const Cursor &c, u32 k0, u32 klimit, float (&out)[8]) const {
@@ -87,6 +90,7 @@ struct SMatR {
         u32 k, left;  // rows from the item's first to the matrix' end (0: none, the item repeats the last row)
     };
     __device__ __forceinline__ void bind(u32 z) { base += size_t(z) * zstride; }
+    __device__ __forceinline__ float at(u32 row, u32 k) const { return base[size_t(k) * ld + row]; }
     __device__ __forceinline__ Cursor cursor(u32 row, u32 k) const {
         return {base + (row < rows ? row : rows - 1), k, row < rows ? rows - row : 0u};
     }
@@ -448,7 +452,14 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
                 rowb[r] = epi.row_bias_at(row < d.M ? row : d.M - 1);
             }
         }
-        if (whole) {
+        const u32 redo = not_finite<NR>(v);
+        if (__builtin_expect(__any(int(redo)), 0)) {
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                const u32 row = rbase + 8 * (r / 4) + (r % 4);
+                if (row < d.M && !(redo >> r & 1)) epi.store(row, cs, v[r], rowb[r]);
+            }
+        } else if (whole) {
             if (accumulates) {
 #pragma unroll
                 for (int r = 0; r < NR; ++r) oldv[r] = *epi.at(rbase + 8 * (r / 4) + (r % 4), col);
@@ -462,8 +473,21 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
                 if (row < d.M) epi.store(row, cs, v[r], rowb[r]);
             }
         }
+        return redo;  // what is not stored yet
+    };
+    // the sums of a part that were not finite, from the fp32 operands (split_bf16.h)
+    auto redo_part = [&](int mi, int ni, int r0, u32 redo) {
+        for (; redo; redo &= redo - 1) {
+            const u32 r = __builtin_ctz(redo), col = col0 + wave_n * Cfg::WTN + ni * 32 + i32;
+            const u32 row = row0 + wave_m * Cfg::WTM + mi * 32 + 4 * h + 2 * r0 + 8 * (r / 4) + (r % 4);
+            if (row >= d.M || col >= d.N) continue;
+            float sum = 0.f;
+            for (u32 k = kbeg; k < kend && !__builtin_isnan(sum); ++k) sum = fmaf(a.at(row, k), b.at(col, k), sum);
+            epi.store(row, epi.prep_col(col, d.N), sum, row_biased ? epi.row_bias_at(row) : 0.f);
+        }
     };
     if constexpr (KG == 1) {
+        u32 redo[TM][TN], any = 0;
 #pragma unroll
         for (int ni = 0; ni < TN; ++ni)
 #pragma unroll
@@ -471,8 +495,16 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
                 float v[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) v[r] = acc[mi][ni][r];
-                store_part(mi, ni, 0, std::integral_constant<int, 16>(), v);
+                any |= redo[mi][ni] = store_part(mi, ni, 0, std::integral_constant<int, 16>(), v);
             }
+        if (__builtin_expect(any != 0, 0)) {
+            for (int blk = 0; blk < TM * TN; ++blk) {
+                u32 m = 0;
+#pragma unroll
+                for (int i = 0; i < TM * TN; ++i) m = i == blk ? redo[i / TN][i % TN] : m;
+                redo_part(blk / TN, blk % TN, 0, m);
+            }
+        }
     } else {
         // The groups exchange their accumulators through the staging space (idle: the last slab's barrier has passed), BR blocks
         // of every wave at a time, and each group sums (in group order) and stores its share of them: all waves store.
@@ -495,8 +527,8 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
             for (int g = 1; g < KG; ++g)
 #pragma unroll
                 for (int r = 0; r < NR; ++r) v[r] += src[g * Cfg::WM * Cfg::WN * BR * 1024 + r * 64];
-            const int b = q * BR + f0 / 16;
-            store_part(b / TN, b % TN, f0 % 16, std::integral_constant<int, NR>(), v);
+            const int blk = q * BR + f0 / 16;
+            redo_part(blk / TN, blk % TN, f0 % 16, store_part(blk / TN, blk % TN, f0 % 16, std::integral_constant<int, NR>(), v));
         }
     }
 }

@@ -11,8 +11,10 @@
 // Measured distance from float64 (2-norm, N(0,1) operands; fp32 MFMA / six products / all nine): K = 144 2.15e-7 / 1.74e-7 /
 // 1.74e-7, 576 4.31e-7 / 3.61e-7 / 3.61e-7, 4608 1.22e-6 / 1.07e-6 / 1.07e-6 - sixteen k's share one rounding of the sum, so
 // the results are closer to the exact ones than those of the fp32 pipe, and the three left out are not seen at all.
-// What differs: an operand that is infinite (or rounds to infinity as a bf16, from 3.39e38 up) gives NaN where the fp32 pipe
-// gives an infinity or NaN.
+// An operand that is infinite, or rounds to infinity as a bf16 (from 3.39e38 up), has NaN among its parts, so it always shows
+// as NaN in the sum. The epilogues form every sum that is not finite once more from the fp32 operands, element by element, and
+// stop at a NaN: such results are those of an fp32 contraction (infinities keep their sign, large finite values stay finite).
+// Operands under 2^-110 have a last part that a bf16 cannot hold whole: an absolute error of 2^-134.
 #pragma once
 #include "crb_common.h"
 
@@ -56,6 +58,15 @@ __device__ __forceinline__ BufferRange buffer_range(const float *base, size_t fl
 }
 __device__ __forceinline__ float buffer_load(BufferRange r, u32 voffset, u32 soffset) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, int(voffset), int(soffset), 0));
+}
+
+// Bit r of the result: sum v[r] is not finite.
+template <int NR>
+__device__ __forceinline__ u32 not_finite(const float *v) {
+    u32 m = 0;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) m |= __builtin_isfinite(v[r]) ? 0u : 1u << r;
+    return m;
 }
 
 // The products that are formed: (part of A, part of B), in an order that needs the leading parts first.

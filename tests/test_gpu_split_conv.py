@@ -63,3 +63,36 @@ def test_layers_run_where_the_split_kernels_have_no_scratch(dev, shape):
         capi.bind_workspace(None, stream=st)
     assert_close(to_np(Y), orc.conv(Wt, X, None, s, s, p, p), IC * F * F, f"forward {shape}")
     assert_close(to_np(dX), orc.convDerive(Wt, dY, (H, W), s, s, p, p), OC * F * F, f"data gradient {shape}")
+
+
+@pytest.mark.parametrize("shape", [(3, 64, 31, 33, 65, 3, 1, 1), (2, 300, 9, 11, 70, 3, 1, 1), (7, 31, 21, 19, 33, 5, 1, 2), (4, 65, 33, 27, 97, 3, 2, 1)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_infinities_and_the_largest_floats(dev, shape):
+    """Infinite operands and ones that round to infinity in 16 bits give what a contraction in fp32 gives: infinities of the
+    right sign, NaN only where infinities meet or a NaN enters, finite results elsewhere."""
+    import torch
+    import torch.nn.functional as F_
+    from crusaderbackend_amd import capi
+
+    N, IC, H, W, OC, F, s, p = shape
+    g = capi.ConvGeom.make(N, IC, H, W, OC, F, F, s, s, p, p)
+    gen = torch.Generator().manual_seed(9)
+
+    def half(*size):  # in [-0.5, 0.5], no zeros
+        t = torch.rand(*size, generator=gen) - 0.5
+        return torch.where(t == 0, torch.full_like(t, 0.25), t)
+
+    X, Wt, dY = half(N, IC, H, W), half(OC, IC, F, F), half(N, OC, g.OH, g.OW)
+    X[0, 3, 4, 5], X[N - 1, IC - 1, 3, 6], X[1, 1, 5, 4] = float("inf"), float("nan"), -3.4e38
+    dY[0, 2, 2, 3], dY[N - 1, OC - 1, 2, 2] = float("-inf"), 3.4e38
+    Xr, Wr = X.double().requires_grad_(), Wt.double().requires_grad_()
+    Yr = F_.conv2d(Xr, Wr, stride=s, padding=p)
+    Yr.backward(dY.double())
+    Y, dX, dW = torch.empty(N, OC, g.OH, g.OW, device=dev), torch.empty(N, IC, H, W, device=dev), torch.zeros(OC, IC, F, F, device=dev)
+    capi.conv_fwd(Wt.to(dev), X.to(dev), Y, None, g)
+    capi.conv_dgrad(Wt.to(dev), dY.to(dev), dX, g)
+    capi.conv_wgrad(dY.to(dev), X.to(dev), dW, g)
+    torch.cuda.synchronize()
+    for what, got, ref, K in (("Y", Y, Yr, IC * F * F), ("dX", dX, Xr.grad, OC * F * F), ("dW", dW, Wr.grad, N * g.OH * g.OW)):
+        # K terms under 1/4, or that and one of 1.7e38, each rounded once or twice
+        np.testing.assert_allclose(to_np(got), ref.detach().float().numpy(), rtol=K * 2.0**-23, atol=K * K * 2.0**-25, equal_nan=True, err_msg=what)

@@ -79,3 +79,46 @@ def test_split_product_loses_nothing_of_its_operands(dev):
     torch.cuda.synchronize()
     exact = A.astype(np.float64) @ B
     assert np.linalg.norm(to_np(C) - exact) <= np.sqrt(n) * 2.0**-24 * np.linalg.norm(exact)
+
+
+# 256 x 256, 128 x 128 and 64 x 64 tiles, a cut contraction
+@pytest.mark.parametrize("size", [(4096, 4095, 32), (2048, 2048, 65), (1024, 1024, 257), (256, 1024, 1025)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("form", ["nn", "nt", "tn", "wgrad"])
+def test_infinities_and_the_largest_floats(dev, form, size):
+    """Infinite operands and ones that round to infinity in 16 bits give what a product in fp32 gives: infinities of the right
+    sign, NaN only where infinities meet or a NaN enters, finite results elsewhere."""
+    import torch
+    from crusaderbackend_amd import capi
+
+    M, N, K = size
+    A, B = uniform(1, M, K) / 2, uniform(2, K, N) / 2
+    A[A == 0], B[B == 0] = 0.25, 0.25
+    A[3, 5], A[M - 1, K - 1], A[40, 7] = np.inf, np.nan, 3.4e38
+    B[2, 9], B[5, N - 1], B[K - 1, 70] = -np.inf, np.inf, -3.4e38
+    A[65, 2], A[66, 2] = 0.5, -0.5
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32)
+    a = np.ascontiguousarray(A.T) if form in ("tn", "wgrad") else A
+    b = np.ascontiguousarray(B.T) if form == "nt" else B
+    if form == "wgrad":  # accumulates, with the row sums of A on the side
+        C, dB = torch.zeros(M, N, device=dev), torch.zeros(M, device=dev)
+        capi.linear_wgrad(to_dev(a, dev), to_dev(b, dev), C, dB, K, N, M)
+    else:
+        C = torch.empty(M, N, device=dev)
+        product(capi, form, to_dev(a, dev), to_dev(b, dev), C, M, N, K)
+    torch.cuda.synchronize()
+    # K terms under 1/4, or that and one of 1.7e38, each rounded once or twice
+    np.testing.assert_allclose(to_np(C), ref, rtol=K * 2.0**-23, atol=K * K * 2.0**-25, equal_nan=True)
+
+
+def test_small_operands_keep_their_bits(dev):
+    """Parts of operands down to 2^-110 are bf16 numbers, subnormal ones among them."""
+    import torch
+    from crusaderbackend_amd import capi
+
+    n = 1024
+    A = np.ldexp(np.float32(1) + np.abs(uniform(5, n, n)), -109).astype(np.float32)
+    C = torch.empty(n, n, device=dev)
+    capi.sgemm_nn(to_dev(A, dev), to_dev(np.eye(n, dtype=np.float32), dev), C, n, n, n)
+    torch.cuda.synchronize()
+    assert np.array_equal(to_np(C), A)
