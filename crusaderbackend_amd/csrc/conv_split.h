@@ -276,7 +276,9 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
             if (a.relu) o = o > 0.f ? o : 0.f;
             if (oc < a.C_OUT) y[size_t(oc) * a.OHW] = o;
         }
-        for (u32 redo = not_finite<NR>(res); redo; redo &= redo - 1) {
+        u32 redo = not_finite<NR>(res);
+        if (__all(redo == (1u << NR) - 1)) return;
+        for (; redo; redo &= redo - 1) {
             const u32 r = __builtin_ctz(redo), oc = oc0 + 8 * (r / 4) + (r % 4);
             if (oc >= a.C_OUT) continue;
             float sum = 0.f;

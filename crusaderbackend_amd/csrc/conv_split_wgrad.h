@@ -267,7 +267,13 @@ __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a
 #pragma unroll
         for (int t = 0; t < NTW; ++t) x[(row * C::ICT + wn * 32 + (lane & 31)) * NTW + t] = own[t][i];
     }
-    lds_barrier();
+    bool bad = false;
+#pragma unroll
+    for (int t = 0; t < NTW; ++t)
+#pragma unroll
+        for (int i = 0; i < NR; ++i) bad |= !__builtin_isfinite(own[t][i]);
+    // (a thread holds all taps of its channel pairs: an eighth of the threads is two output channels, or four input channels)
+    const bool redo = __syncthreads_count(bad) <= C::NTH / 8;
     // this slice's sum of one filter element from the fp32 operands (split_bf16.h: sums that are not finite)
     auto plain_sum = [&](u32 oc, u32 ic, u32 fh, u32 fw) {
         float sum = 0.f;
@@ -292,7 +298,7 @@ __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a
         if (oc0 + oc < a.OC && ic < nic) {
             float *dst = out + ((size_t(oc0 + oc) * a.IC + ic0 + ic) * (F * F) + fh0 * F + t);
             float v = x[e];
-            if (!__builtin_isfinite(v)) v = plain_sum(oc0 + oc, ic0 + ic, fh0 + t / F, t % F);
+            if (redo && !__builtin_isfinite(v)) v = plain_sum(oc0 + oc, ic0 + ic, fh0 + t / F, t % F);
             if (a.splits > 1) *dst = v; else *dst += v;
         }
     }

@@ -12,8 +12,10 @@
 // 1.74e-7, 576 4.31e-7 / 3.61e-7 / 3.61e-7, 4608 1.22e-6 / 1.07e-6 / 1.07e-6 - sixteen k's share one rounding of the sum, so
 // the results are closer to the exact ones than those of the fp32 pipe, and the three left out are not seen at all.
 // An operand that is infinite, or rounds to infinity as a bf16 (from 3.39e38 up), has NaN among its parts, so it always shows
-// as NaN in the sum. The epilogues form every sum that is not finite once more from the fp32 operands, element by element, and
+// as NaN in the sum. The epilogues form sums that are not finite once more from the fp32 operands, element by element, and
 // stop at a NaN: such results are those of an fp32 contraction (infinities keep their sign, large finite values stay finite).
+// A convolution's block without a single finite sum, and a weight gradient's with more than an eighth of them not finite, belong
+// to tensors that have diverged throughout and are left at NaN: summing on made a diverged VGG-16 step 3.0 ms instead of 2.2.
 // Operands under 2^-110 have a last part that a bf16 cannot hold whole: an absolute error of 2^-134.
 #pragma once
 #include "crb_common.h"
