@@ -277,14 +277,14 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
             if (oc < a.C_OUT) y[size_t(oc) * a.OHW] = o;
         }
         u32 redo = not_finite<NR>(res);
-        if (__all(redo == (1u << NR) - 1)) return;
+        if (a.mirrored && __all(redo == (1u << NR) - 1)) return;  // (split_bf16.h)
         for (; redo; redo &= redo - 1) {
             const u32 r = __builtin_ctz(redo), oc = oc0 + 8 * (r / 4) + (r % 4);
             if (oc >= a.C_OUT) continue;
             float sum = 0.f;
             const u32 c1 = chunk1 * C::CI < a.C_IN ? chunk1 * C::CI : a.C_IN;
             for (u32 ic = chunk0 * C::CI; ic < c1 && !__builtin_isnan(sum); ++ic)
-                for (u32 tap = 0; tap < u32(NT); ++tap) {
+                for (u32 tap = 0; tap < u32(NT) && !__builtin_isnan(sum); ++tap) {
                     const int iy = int(S * yy + tap / F) - a.pad_y, ix = int(S * xx + tap % F) - a.pad_x;
                     if (u32(iy) >= a.H || u32(ix) >= a.W) continue;
                     const float w = a.Wt[size_t(oc) * a.w_oc + size_t(ic) * a.w_ic + (a.mirrored ? NT - 1 - tap : tap)];

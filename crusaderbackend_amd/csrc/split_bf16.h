@@ -14,8 +14,9 @@
 // An operand that is infinite, or rounds to infinity as a bf16 (from 3.39e38 up), has NaN among its parts, so it always shows
 // as NaN in the sum. The epilogues form sums that are not finite once more from the fp32 operands, element by element, and
 // stop at a NaN: such results are those of an fp32 contraction (infinities keep their sign, large finite values stay finite).
-// A convolution's block without a single finite sum, and a weight gradient's with more than an eighth of them not finite, belong
-// to tensors that have diverged throughout and are left at NaN: summing on made a diverged VGG-16 step 3.0 ms instead of 2.2.
+// A data gradient's block without a single finite sum, and a weight gradient's with more than an eighth of them not finite, belong
+// to tensors that have diverged throughout and are left at NaN: summing on made a diverged VGG-16 step 3.8 ms (data gradients
+// alone) instead of 2.3. Activations are always formed again: a ReLU would make 0 of the NaN that stands for an infinity.
 // Operands under 2^-110 have a last part that a bf16 cannot hold whole: an absolute error of 2^-134.
 #pragma once
 #include "crb_common.h"

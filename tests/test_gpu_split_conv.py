@@ -96,3 +96,25 @@ def test_infinities_and_the_largest_floats(dev, shape):
     for what, got, ref, K in (("Y", Y, Yr, IC * F * F), ("dX", dX, Xr.grad, OC * F * F), ("dW", dW, Wr.grad, N * g.OH * g.OW)):
         # K terms under 1/4, or that and one of 1.7e38, each rounded once or twice
         np.testing.assert_allclose(to_np(got), ref.detach().float().numpy(), rtol=K * 2.0**-23, atol=K * K * 2.0**-25, equal_nan=True, err_msg=what)
+
+
+@pytest.mark.parametrize("shape", [(3, 64, 31, 33, 65, 3, 1, 1), (2, 300, 9, 11, 70, 3, 1, 1), (7, 31, 21, 19, 33, 5, 1, 2), (4, 65, 33, 27, 97, 3, 2, 1)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_layers_that_overflow_throughout(dev, shape):
+    """Every product of a channel over- or underflows the largest float: infinities of the right sign, and ReLU keeps the positive."""
+    import torch
+    from crusaderbackend_amd import capi
+
+    N, IC, H, W, OC, F, s, p = shape
+    g = capi.ConvGeom.make(N, IC, H, W, OC, F, F, s, s, p, p)
+    gen = torch.Generator().manual_seed(10)
+    X, Wt = torch.rand(N, IC, H, W, generator=gen) + 1, torch.rand(OC, IC, F, F, generator=gen) + 1
+    X, Wt = X * 1e25, Wt * 1e20
+    Wt[OC // 2] *= -1
+    ref = torch.full((N, OC, g.OH, g.OW), float("inf"))
+    ref[:, OC // 2] = float("-inf")
+    Y = torch.empty(N, OC, g.OH, g.OW, device=dev)
+    for flags, want in ((0, ref), (capi.CRB_FLAG_RELU, ref.clamp(min=0))):
+        capi.conv_fwd(Wt.to(dev), X.to(dev), Y, None, g, flags)
+        torch.cuda.synchronize()
+        assert torch.equal(Y.cpu(), want)
