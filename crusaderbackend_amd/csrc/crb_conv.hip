@@ -387,10 +387,11 @@ static ConvSplitPlan conv_split_plan_for(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 
     consider(4, typename Set::C4(), S == 2 ? 0.32f : 0.66f, 2);
     return best;
 }
-// (OH, OW): the pass's result, (H, W): what it reads; direct: a width-specialised kernel takes the pass otherwise
-static ConvSplitPlan conv_split_plan(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 W, u32 OH, u32 OW, u32 F, u32 S, bool direct) {
+// (OH, OW): the pass's result, (H, W): what it reads; direct: a width-specialised kernel takes the pass otherwise; it is worth it
+// from `least` MFLOP
+static ConvSplitPlan conv_split_plan(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 W, u32 OH, u32 OW, u32 F, u32 S, bool direct, float least) {
     const float mflop = 2e-6f * N * OH * OW * C_IN * C_OUT * F * F;
-    if (C_IN < 16 || C_OUT < 24 || mflop < (direct ? 2000.f : 100.f)) return ConvSplitPlan();
+    if (C_IN < 16 || C_OUT < 24 || mflop < least) return ConvSplitPlan();
     ConvSplitPlan p;
     float us = 0.f;
     if (F == 3 && S == 1) p = conv_split_plan_for<3, 1>(N, C_IN, C_OUT, H, W, OH, OW, us);
@@ -420,15 +421,19 @@ static ConvSplitPlan conv_split_fwd_plan(const crb_conv_geom *g, bool aligned) {
     // faster (64 -> 64 @32 batch 128 79 against 57 us, 512 -> 512 @4 84 against 62): new roundings there flip a few ReLU signs and
     // pooling choices, and a VGG-16 training step at a fresh start (its loss grows 5-fold over the first update) carries these
     // into 2 to 5 % of the second step's input gradient. New roundings in the gradients alone leave 0.06 to 0.3 %.
-    if (direct) return ConvSplitPlan();
-    return conv_split_plan(g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, g->FH, g->sH, false);
+    // Under eight images, where calls are inference, that kernel puts one long contraction each on a few dozen CUs and takes as long
+    // for one image as for seven; the split kernel cuts the contraction. One / seven images, us: 64 -> 64 @32 41 -> 16 / 42 -> 13,
+    // 64 -> 128 @16 24 -> 17 / 24 -> 17, 128 -> 128 @16 43 -> 17 / 44 -> 19, 256 -> 256 @8 49 -> 19 / 50 -> 22, 256 -> 512 @4 26 -> 21 /
+    // 27 -> 25, 512 -> 512 @4 49 -> 23 / 49 -> 25. Under K = 512 or 30 MFLOP the filters' and the slices' launches eat the gain.
+    if (direct && (g->N >= 8 || g->sH != 1 || g->IC * 9 < 512)) return ConvSplitPlan();
+    return conv_split_plan(g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, g->FH, g->sH, direct, direct ? 30.f : 100.f);
 }
 static ConvSplitPlan conv_split_dgrad_plan(const crb_conv_geom *g, bool aligned) {
     if (g->FH != g->FW || g->sH != 1 || g->sW != 1 || g->pH >= g->FH || g->pW >= g->FW) return ConvSplitPlan();
     bool direct = false;
     if (aligned && direct_shape(g, 1))
         try_direct<true, 1>(nullptr, nullptr, nullptr, nullptr, g->N, g->OC, g->IC, g->OH, g->OW, g->OH, 0, nullptr, "", direct, true);
-    return conv_split_plan(g->N, g->OC, g->IC, g->OH, g->OW, g->IH, g->IW, g->FH, 1, direct);
+    return conv_split_plan(g->N, g->OC, g->IC, g->OH, g->OW, g->IH, g->IW, g->FH, 1, direct, direct ? 2000.f : 100.f);
 }
 template <int F, int S, bool DG>
 static int run_conv_split_set(const ConvSplitPlan &p, const float *Wt, const float *X, float *Y, const float *bias, unsigned char *wf, u32 N, u32 C_IN,
