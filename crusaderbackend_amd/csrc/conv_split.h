@@ -247,6 +247,85 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
         lds_barrier();
     }
 
+    // ---- sums that are not finite: this wave's blocks once more, on the fp32 MFMA from the fp32 operands (split_bf16.h) ------
+    // Two channels of a tap per MFMA, 16 a step, the next step's operands requested ahead. Taps outside the image take no part
+    // (an infinite filter element would make NaN of the zero read there): a lane's accumulators all belong to its pixel, so
+    // it keeps the old ones. Ends early where every sum is a NaN.
+    if (__builtin_expect(__any(int(any_not_finite(acc))), 0)) {
+        struct Step {
+            float w[8][TM], x[8][TN];
+            bool in[TN];
+        };
+        int py[TN], px[TN];
+        u32 img_off[TN];
+        const float *wrow[TM];
+#pragma unroll
+        for (int ni = 0; ni < TN; ++ni) {
+            u32 p = p0 + wave_n * (32 * TN) + ni * 32 + i32;
+            p = p < a.npix ? p : a.npix - 1;
+            u32 v, r, y, x, img, strip;
+            a.ohw.divmod(p, v, r);
+            a.ow.divmod(r, y, x);
+            a.strip_d.divmod(v, img, strip);
+            py[ni] = int(S * y) - a.pad_y, px[ni] = int(S * (x + strip * a.SW)) - a.pad_x, img_off[ni] = (img - img0) * a.C_IN * a.HW;
+        }
+#pragma unroll
+        for (int mi = 0; mi < TM; ++mi) {
+            const u32 oc = ot * C::OCT + wave_m * (32 * TM) + mi * 32 + i32;
+            wrow[mi] = a.Wt + size_t(oc < a.C_OUT ? oc : a.C_OUT - 1) * a.w_oc;
+        }
+        auto fetch_step = [&](u32 s, Step &f) {
+            const u32 tap = s % NT, c0 = (chunk0 + s / NT) * C::CI + 16 * kgroup;
+#pragma unroll
+            for (int ni = 0; ni < TN; ++ni) {
+                const int iy = py[ni] + int(tap / F), ix = px[ni] + int(tap % F);
+                f.in[ni] = u32(iy) < a.H && u32(ix) < a.W;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const u32 ic = c0 + 2 * j + h, bytes = (img_off[ni] + ic * a.HW + u32(iy) * a.W + u32(ix)) * 4u;
+                    f.x[j][ni] = buffer_load(xrange, f.in[ni] && ic < a.C_IN ? bytes : kOutside, 0);
+                }
+            }
+#pragma unroll
+            for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const u32 ic = c0 + 2 * j + h;
+                    const float w = wrow[mi][ic < a.C_IN ? size_t(ic) * a.w_ic + (a.mirrored ? NT - 1 - tap : tap) : 0];
+                    f.w[j][mi] = ic < a.C_IN ? w : 0.f;
+                }
+        };
+        const u32 count = (chunk1 - chunk0) * NT;
+        Step next;
+        fetch_step(0, next);
+#pragma unroll
+        for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.0f;
+#pragma unroll 1
+        for (u32 s = 0; s < count; ++s) {
+            const Step now = next;
+            if (s + 1 < count) fetch_step(s + 1, next);
+            u32 numbers = 0;
+#pragma unroll
+            for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+                for (int ni = 0; ni < TN; ++ni) {
+                    v16f sum = acc[mi][ni];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(now.w[j][mi], now.x[j][ni], sum, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        acc[mi][ni][r] = now.in[ni] ? sum[r] : acc[mi][ni][r];
+                        numbers |= __builtin_isnan(acc[mi][ni][r]) ? 0u : 1u;
+                    }
+                }
+            if (!__any(int(numbers))) break;
+        }
+    }
+
     // ---- epilogue: 32 lanes store 32 consecutive pixels of a channel --------------------------------------------------------
     auto store_part = [&](int mi, int ni, int r0, auto nr_c, const float *res) {
         constexpr int NR = decltype(nr_c)::value;
@@ -275,24 +354,6 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
             float o = res[r] + b[r];
             if (a.relu) o = o > 0.f ? o : 0.f;
             if (oc < a.C_OUT) y[size_t(oc) * a.OHW] = o;
-        }
-        u32 redo = not_finite<NR>(res);
-        if (a.mirrored && __all(redo == (1u << NR) - 1)) return;  // (split_bf16.h)
-        for (; redo; redo &= redo - 1) {
-            const u32 r = __builtin_ctz(redo), oc = oc0 + 8 * (r / 4) + (r % 4);
-            if (oc >= a.C_OUT) continue;
-            float sum = 0.f;
-            const u32 c1 = chunk1 * C::CI < a.C_IN ? chunk1 * C::CI : a.C_IN;
-            for (u32 ic = chunk0 * C::CI; ic < c1 && !__builtin_isnan(sum); ++ic)
-                for (u32 tap = 0; tap < u32(NT) && !__builtin_isnan(sum); ++tap) {
-                    const int iy = int(S * yy + tap / F) - a.pad_y, ix = int(S * xx + tap % F) - a.pad_x;
-                    if (u32(iy) >= a.H || u32(ix) >= a.W) continue;
-                    const float w = a.Wt[size_t(oc) * a.w_oc + size_t(ic) * a.w_ic + (a.mirrored ? NT - 1 - tap : tap)];
-                    sum = fmaf(w, a.X[(size_t(img) * a.C_IN + ic) * a.HW + u32(iy) * a.W + u32(ix)], sum);
-                }
-            if (a.bias) sum += a.bias[oc];
-            if (a.relu) sum = sum > 0.f ? sum : 0.f;
-            y[size_t(oc) * a.OHW] = sum;
         }
     };
     if constexpr (KG == 1) {

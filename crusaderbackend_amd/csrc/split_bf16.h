@@ -12,11 +12,11 @@
 // 1.74e-7, 576 4.31e-7 / 3.61e-7 / 3.61e-7, 4608 1.22e-6 / 1.07e-6 / 1.07e-6 - sixteen k's share one rounding of the sum, so
 // the results are closer to the exact ones than those of the fp32 pipe, and the three left out are not seen at all.
 // An operand that is infinite, or rounds to infinity as a bf16 (from 3.39e38 up), has NaN among its parts, so it always shows
-// as NaN in the sum. The epilogues form sums that are not finite once more from the fp32 operands, element by element, and
-// stop at a NaN: such results are those of an fp32 contraction (infinities keep their sign, large finite values stay finite).
-// A data gradient's block without a single finite sum, and a weight gradient's with more than an eighth of them not finite, belong
-// to tensors that have diverged throughout and are left at NaN: summing on made a diverged VGG-16 step 3.8 ms (data gradients
-// alone) instead of 2.3. Activations are always formed again: a ReLU would make 0 of the NaN that stands for an infinity.
+// as NaN in the sum. Sums that are not finite are formed once more from the fp32 operands and are those of an fp32 contraction
+// (infinities keep their sign, large finite values stay finite). Convolutions forward and data gradients: a wave does its blocks
+// again on the fp32 MFMA, straight from memory (one infinity in 64 -> 64 @56 batch 32: 68 -> 109 us, a channel of infinities 269;
+// element by element it was 3.2 and 7.2 ms). Products: element by element, up to a NaN; weight gradients as well, but for
+// blocks with more than an eighth of their sums not finite, which are left at NaN.
 // Operands under 2^-110 have a last part that a bf16 cannot hold whole: an absolute error of 2^-134.
 #pragma once
 #include "crb_common.h"
@@ -61,6 +61,19 @@ __device__ __forceinline__ BufferRange buffer_range(const float *base, size_t fl
 }
 __device__ __forceinline__ float buffer_load(BufferRange r, u32 voffset, u32 soffset) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, int(voffset), int(soffset), 0));
+}
+
+// Whether one of a lane's accumulators is not finite.
+template <class V, int TM, int TN>
+__device__ __forceinline__ bool any_not_finite(const V (&acc)[TM][TN]) {
+    bool bad = false;
+#pragma unroll
+    for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) bad |= !__builtin_isfinite(acc[mi][ni][r]);
+    return bad;
 }
 
 // Bit r of the result: sum v[r] is not finite.

@@ -120,3 +120,41 @@ def test_layers_that_overflow_throughout(dev, shape):
         capi.conv_fwd(Wt.to(dev), X.to(dev), Y, None, g, flags)
         torch.cuda.synchronize()
         assert torch.equal(Y.cpu(), want)
+
+
+def check_against_float64(got, ref, K, what):
+    """ref: float64 sums of K terms of one sign, of which each product and partial sum rounds to fp32 once (infinities: exactly)."""
+    ref = ref.detach()
+    np.testing.assert_allclose(to_np(got).astype(np.float64), np.where(np.abs(ref.numpy()) > 3.4028235e38, np.copysign(np.inf, ref.numpy()), ref.numpy()),
+                               rtol=(K + 1) * 2.0**-23, equal_nan=True, err_msg=what)
+
+
+# the last pixel of (17, 256, 7, 7) stands alone in its block of 32
+LARGE = [(17, 256, 7, 7, 256, 3, 1, 1), (3, 64, 31, 33, 65, 3, 1, 1), (16, 64, 24, 23, 72, 5, 1, 2)]
+
+
+@pytest.mark.parametrize("shape", LARGE, ids=lambda s: "x".join(map(str, s)))
+def test_data_gradients_of_operands_that_round_to_infinity(dev, shape):
+    """Output gradients beyond the largest bf16, one of them or all, with finite sums; and infinite ones throughout."""
+    import torch
+    import torch.nn.functional as F_
+    from crusaderbackend_amd import capi
+
+    N, IC, H, W, OC, F, s, p = shape
+    g = capi.ConvGeom.make(N, IC, H, W, OC, F, F, s, s, p, p)
+    assert capi.conv_dgrad_workspace_bytes(g) > OC * IC * F * F * 6  # the three parts of the filters: on split operands
+    gen = torch.Generator().manual_seed(11)
+    Wt, dY = torch.rand(OC, IC, F, F, generator=gen) * 0.5 + 0.25, torch.rand(N, OC, g.OH, g.OW, generator=gen) + 0.5
+    one = dY.clone()
+    one[N - 1, OC // 3, g.OH - 1, g.OW - 1] = 3.4e38
+    negative = Wt.clone()
+    negative[:, IC // 2] *= -1
+    for what, w, dy in (("one", Wt, one), ("all", Wt * 1e-5, torch.full_like(dY, 3.4e38)), ("infinite", negative, torch.full_like(dY, float("inf")))):
+        dX = torch.empty(N, IC, H, W, device=dev)
+        capi.conv_dgrad(w.to(dev), dy.to(dev), dX, g)
+        torch.cuda.synchronize()
+        if what == "infinite":
+            assert torch.equal(dX.cpu(), torch.where(torch.arange(IC).reshape(1, -1, 1, 1) == IC // 2, float("-inf"), float("inf")).expand_as(dX))
+        else:
+            ref = F_.conv_transpose2d(dy.double(), w.double(), stride=s, padding=p)
+            check_against_float64(dX, ref, OC * F * F, what)
