@@ -335,7 +335,6 @@ inline SplitWgradPlan split_wgrad_plan(u32 N, u32 IC, u32 OC, u32 H, u32 W, u32 
     return p;
 }
 
-// dW == nullptr: the slices stay in ws, unsummed.
 template <class C>
 inline int launch_split_wgrad(const SplitWgradPlan &p, const float *dY, const float *X, float *dW, float *ws, u32 N, u32 IC, u32 OC, u32 H, u32 W,
                               u32 OH, u32 OW, int pad_y, int pad_x, hipStream_t s, const char *what) {
@@ -352,7 +351,7 @@ inline int launch_split_wgrad(const SplitWgradPlan &p, const float *dY, const fl
     if (uint64_t(p.pairs) * p.splits > 0x7fffffffull) return fail(CRB_EINVAL_SHAPE, "%s: launch grid too large", what);
     hipLaunchKernelGGL((split_wgrad_kernel<C>), dim3(p.pairs * p.splits, C::F / C::ROWS), dim3(C::NTH), 0, s, a);
     if (int st = check_launch(what)) return st;
-    if (p.splits > 1 && dW) return launch_splitk_reduce(ws, dW, OC * IC * C::F * C::F, p.splits, ReduceEpi{nullptr, 1, 1, EPI_ACCUM}, s, what);
+    if (p.splits > 1) return launch_splitk_reduce(ws, dW, OC * IC * C::F * C::F, p.splits, ReduceEpi{nullptr, 1, 1, EPI_ACCUM}, s, what);
     return CRB_OK;
 }
 

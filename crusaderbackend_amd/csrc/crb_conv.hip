@@ -417,10 +417,11 @@ static ConvSplitPlan conv_split_fwd_plan(const crb_conv_geom *g, bool aligned) {
         try_direct<false, 1>(nullptr, nullptr, nullptr, nullptr, g->N, g->IC, g->OC, g->OH, g->OW, g->IH, 0, nullptr, "", direct, true);
     else if (aligned && direct_shape(g, 2))
         try_direct<false, 2>(nullptr, nullptr, nullptr, nullptr, g->N, g->IC, g->OC, g->OH, g->OW, g->IH, 0, nullptr, "", direct, true);
-    // A width-specialised layer's forward pass keeps its kernel, and so the bits of its activations, though the split one is the
-    // faster (64 -> 64 @32 batch 128 79 against 57 us, 512 -> 512 @4 84 against 62): new roundings there flip a few ReLU signs and
-    // pooling choices, and a VGG-16 training step at a fresh start (its loss grows 5-fold over the first update) carries these
-    // into 2 to 5 % of the second step's input gradient. New roundings in the gradients alone leave 0.06 to 0.3 %.
+    // A width-specialised layer keeps its kernels in training, and so the bits of its activations and gradients, though the split
+    // ones are the faster (64 -> 64 @32 batch 128 79 against 57 us, 512 -> 512 @4 84 against 62; a VGG-16 step 2.69 against 2.29 ms
+    // with the gradients alone): new roundings flip a few ReLU signs and pooling choices, and a VGG-16 training run at a fresh
+    // start (its loss grows 5-fold over the first update) carries these into 2 to 5 % of the second step's input gradient, or
+    // with the forward pass kept 0.06 to 0.3 %.
     // Under eight images, where calls are inference, that kernel puts one long contraction each on a few dozen CUs and takes as long
     // for one image as for seven; the split kernel cuts the contraction. One / seven images, us: 64 -> 64 @32 41 -> 16 / 42 -> 13,
     // 64 -> 128 @16 24 -> 17 / 24 -> 17, 128 -> 128 @16 43 -> 17 / 44 -> 19, 256 -> 256 @8 49 -> 19 / 50 -> 22, 256 -> 512 @4 26 -> 21 /
@@ -433,7 +434,8 @@ static ConvSplitPlan conv_split_dgrad_plan(const crb_conv_geom *g, bool aligned)
     bool direct = false;
     if (aligned && direct_shape(g, 1))
         try_direct<true, 1>(nullptr, nullptr, nullptr, nullptr, g->N, g->OC, g->IC, g->OH, g->OW, g->OH, 0, nullptr, "", direct, true);
-    return conv_split_plan(g->N, g->OC, g->IC, g->OH, g->OW, g->IH, g->IW, g->FH, 1, direct, direct ? 2000.f : 100.f);
+    if (direct) return ConvSplitPlan();  // (as the forward pass: the gradients enter the weights of the same training run)
+    return conv_split_plan(g->N, g->OC, g->IC, g->OH, g->OW, g->IH, g->IW, g->FH, 1, false, 100.f);
 }
 template <int F, int S, bool DG>
 static int run_conv_split_set(const ConvSplitPlan &p, const float *Wt, const float *X, float *Y, const float *bias, unsigned char *wf, u32 N, u32 C_IN,
@@ -828,7 +830,7 @@ static SplitWgradChoice split_wgrad_choice(const crb_conv_geom *g) {
     int st = 0;
     const bool direct = wgrad_direct(g, false, nullptr, nullptr, nullptr, nullptr, nullptr, dp, st);
     const float mflop = 2e-6f * g->N * g->OH * g->OW * g->IC * g->OC * g->FH * g->FW;
-    if (mflop < (direct ? 2000.f : 100.f)) return none;
+    if (direct || mflop < 100.f) return none;  // (width-specialised layers: conv_split_fwd_plan)
     float us = 0.f;
     SplitWgradChoice c;
     if (g->FH == 3 && g->sH == 1) c = split_wgrad_choice_for<3, 1>(g, us);
@@ -845,7 +847,6 @@ static int run_split_wgrad_set(const SplitWgradChoice &c, const float *dY, const
     if (c.cfg == 0) return launch_split_wgrad<typename Set::C0>(c.plan, dY, X, dW, ws, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, py, px, s, what);
     return launch_split_wgrad<typename Set::C1>(c.plan, dY, X, dW, ws, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, py, px, s, what);
 }
-// dW == nullptr: the slices stay in ws, unsummed
 static int run_split_wgrad(const SplitWgradChoice &c, const float *dY, const float *X, float *dW, float *ws, const crb_conv_geom *g, hipStream_t s,
                            const char *what) {
     if (g->sH == 2) return run_split_wgrad_set<3, 2>(c, dY, X, dW, ws, g, s, what);
@@ -911,7 +912,6 @@ static bool bwd_pair(const crb_conv_geom *g, bool run, const float *Wt, const fl
 // results are identical to crb_conv_dgrad followed by crb_conv_wgrad.
 static bool bwd_fused(const crb_conv_geom *g, bool run, const float *Wt, const float *dY, const float *X, float *dX, float *dW,
                       float *ws, hipStream_t s, WgradDirectPlan &plan, int &status) {
-    if (conv_split_dgrad_plan(g, true).cfg >= 0 || split_wgrad_choice(g).cfg >= 0) return false;  // a gradient has a faster kernel of its own
 #define CRB_PAIR(...) bwd_pair<__VA_ARGS__>(g, run, Wt, dY, X, dX, dW, ws, s, plan, status)
     typedef DirectCfg<32, 8, 16, 16, 4, 1, true, 2, 1, 1, 3, 4> D32a;
     typedef DirectCfg<16, 8, 16, 32, 2, 2, true, 2, 2, 1> D16a;             // chunks of 16 channels
@@ -1420,9 +1420,7 @@ uint32_t crb_conv_bwd_slices(const crb_conv_geom *g) {
         const u32 n = sc_wgrad_plan(g->N, g->IC, g->OC, g->OH, g->OW).splits;
         return n > 1 ? n : 0;
     }
-    // (layers without a width-specialised kernel have no sliced form)
     if (!wgrad_direct(g, false, nullptr, nullptr, nullptr, nullptr, nullptr, dp, st)) return 0;
-    if (const SplitWgradChoice c = split_wgrad_choice(g); c.cfg >= 0) return c.plan.splits > 1 ? c.plan.splits : 0;
     return dp.splits > 1 ? dp.splits : 0;
 }
 
@@ -1455,12 +1453,6 @@ int crb_conv_bwd_sliced(const float *W, const float *dY, const float *X, float *
             return fail(CRB_EWORKSPACE, "crb_conv_bwd_sliced: workspace %zu bytes < required %zu", workspace_bytes, dp.workspace_bytes);
         bwd_fused(g, true, W, dY, X, dX, nullptr, ws, s, dp, st);
         return st;
-    }
-    if (const SplitWgradChoice c = split_wgrad_choice(g); c.cfg >= 0) {
-        if (workspace_bytes < c.plan.workspace_bytes)
-            return fail(CRB_EWORKSPACE, "crb_conv_bwd_sliced: workspace %zu bytes < required %zu", workspace_bytes, c.plan.workspace_bytes);
-        if (int sd = crb_conv_dgrad(W, dY, dX, g, stream)) return sd;
-        return run_split_wgrad(c, dY, X, nullptr, ws, g, s, "crb_conv_bwd_sliced");
     }
     wgrad_direct(g, false, nullptr, nullptr, nullptr, nullptr, nullptr, dp, st);
     if (workspace_bytes < dp.workspace_bytes)

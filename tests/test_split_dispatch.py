@@ -1,0 +1,19 @@
+"""Which calls the kernels on split operands take, seen from what the size queries say (no GPU is touched)."""
+import pytest
+
+from crusaderbackend_amd import capi
+
+
+def queries(N, IC, H, W, OC, F, s, p):
+    g = capi.ConvGeom.make(N, IC, H, W, OC, F, F, s, s, p, p)
+    return capi.conv_fwd_workspace_bytes(g), capi.conv_dgrad_workspace_bytes(g), capi.conv_wgrad_workspace_bytes(g)
+
+
+# the 3x3 layers of VGG-16 on CIFAR images, with the slices their fp32 weight gradients are cut into
+@pytest.mark.parametrize("layer", [(64, 32, 64, 32), (64, 16, 128, 16), (128, 16, 128, 8), (128, 8, 256, 4), (256, 8, 256, 2), (256, 4, 512, 1),
+                                   (512, 4, 512, 1)], ids=lambda s: "x".join(map(str, s)))
+def test_width_grid_layers_train_on_the_fp32_kernels(layer):
+    """A training step of these layers keeps its bits: none of its three passes runs on split operands (no room for split
+    filters, slices of the fp32 weight gradient)."""
+    IC, H, OC, slices = layer
+    assert queries(128, IC, H, H, OC, 3, 1, 1) == (0, 0, slices * OC * IC * 36 if slices > 1 else 0)
