@@ -2,7 +2,7 @@
 //   dW[oc][ic][fh][fw] += sum over pixels (n, y, x) of dY[n][oc][y][x] * X[n][ic][S*y + fh - pad][S*x + fw - pad].
 //
 // For every tap a product (oc x ic) whose contraction index is the pixel. Pixels are taken flat over column strips of the images,
-// as in conv_split.h: a tile is PXT consecutive pixels, of which each K group of the workgroup's waves takes STEPS times sixteen -
+// as in conv_split.h: a tile is PXT consecutive pixels, of which each K group of the workgroup's waves takes sixteen -
 // one MFMA step for each of its taps. Both operands are staged channel-fastest, [part][channel octet][position] units of 16 bytes (the
 // split happens on the way), X with the halo its taps need; the fragments, which want eight consecutive pixels of one channel, are
 // read with the transposing LDS read (ds_read_b64_tr_b16: sixteen lanes name four positions x sixteen channels and receive four
@@ -22,11 +22,11 @@
 
 namespace crb {
 
-template <int F_, int S_, int WM_, int WN_, int KG_, int MAXPX_, int STEPS_ = 1>
+template <int F_, int S_, int WM_, int WN_, int KG_, int MAXPX_>
 struct SplitWgradCfg {
-    static constexpr int F = F_, S = S_, WM = WM_, WN = WN_, KG = KG_, MAXPX = MAXPX_, STEPS = STEPS_;
+    static constexpr int F = F_, S = S_, WM = WM_, WN = WN_, KG = KG_, MAXPX = MAXPX_;
     static constexpr int ROWS = F <= 3 ? F : 1, NTW = ROWS * F;  // filter rows, taps of a workgroup (5x5: one row, blockIdx.y)
-    static constexpr int NTH = 64 * WM * WN * KG, PXT = 16 * KG * STEPS, OCT = 32 * WM, ICT = 32 * WN;
+    static constexpr int NTH = 64 * WM * WN * KG, PXT = 16 * KG, OCT = 32 * WM, ICT = 32 * WN;
     static constexpr int XO = ICT / 8, DO = OCT / 8;             // channel octets
     // 64 bytes behind each octet: the four octets a transposing read touches then start 64 bytes apart in a 256-byte bank row
     static constexpr int XOCT = MAXPX * 16 + 64, DOCT = PXT * 16 + 64, XPART = XO * XOCT, DPART = DO * DOCT;
@@ -62,7 +62,7 @@ __device__ __forceinline__ bf16x8 read_transposed(const unsigned char *lds0, con
 
 template <class C>
 __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a) {
-    constexpr int F = C::F, S = C::S, KG = C::KG, NTW = C::NTW, MAXPX = C::MAXPX, PXT = C::PXT, STEPS = C::STEPS;
+    constexpr int F = C::F, S = C::S, KG = C::KG, NTW = C::NTW, MAXPX = C::MAXPX, PXT = C::PXT;
     __shared__ __attribute__((aligned(256))) unsigned char smem[C::LDS];
     // slice z of all channel blocks has ids equal mod `splits`: with a multiple of 8 of them they share an XCD's L2
     const u32 z = blockIdx.x % a.splits, pair = blockIdx.x / a.splits, ot = pair / a.ic_tiles, it = pair % a.ic_tiles;
@@ -170,18 +170,16 @@ __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[t][r] = 0.0f;
 
-    // LDS positions of this lane's two pixels of every step (the second four positions on)
-    u32 xs[STEPS][2];
+    // LDS positions of this lane's two pixels (the second four positions on)
+    u32 xs[2];
     auto positions = [&](const First &f) {
 #pragma unroll
-        for (int st = 0; st < STEPS; ++st)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                u32 k = kpos + st * (16 * KG) + 4 * i, dv, y, x;
-                k = f.p + k < a.npix ? k : 0;  // (dY is zero there)
-                pixel(f, k, dv, y, x);
-                xs[st][i] = ((dv * a.prow + S * (y - f.y) + fh0) * a.pitch + S * x) * 16 + x_lane;
-            }
+        for (int i = 0; i < 2; ++i) {
+            u32 k = kpos + 4 * i, dv, y, x;
+            k = f.p + k < a.npix ? k : 0;  // (dY is zero there)
+            pixel(f, k, dv, y, x);
+            xs[i] = ((dv * a.prow + S * (y - f.y) + fh0) * a.pitch + S * x) * 16 + x_lane;
+        }
     };
     auto main_loop = [&](auto ragged_c) {
         First cur = first_pixel((t0 < t1 ? t0 : 0u) * PXT);
@@ -196,33 +194,29 @@ __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a
         for (u32 tile = t0; tile < t1; ++tile, buf = C::STAGE - buf) {
             if (tile + 1 < t1) cur = following(cur);  // (behind the last tile: that tile once more, for nobody)
             bf16x8 fa[kSplit], fb[2][kSplit];
-            auto read_x = [&](int set, int st, int tap) {
+            auto read_x = [&](int set, int tap) {
                 const u32 shift = ((tap / F) * a.pitch + tap % F) * 16 + buf;
 #pragma unroll
-                for (int p = 0; p < kSplit; ++p) fb[set][p] = read_transposed(smem + xs[st][0] + shift + p * C::XPART, smem + xs[st][1] + shift + p * C::XPART);
+                for (int p = 0; p < kSplit; ++p) fb[set][p] = read_transposed(smem + xs[0] + shift + p * C::XPART, smem + xs[1] + shift + p * C::XPART);
             };
-            auto read_d = [&](int st) {
-                const unsigned char *dsm = smem + buf + kSplit * C::XPART + d_lane + st * (256 * KG);
+            const unsigned char *dsm = smem + buf + kSplit * C::XPART + d_lane;
 #pragma unroll
-                for (int p = 0; p < kSplit; ++p) fa[p] = read_transposed(dsm + p * C::DPART, dsm + p * C::DPART + 64);
-            };
-            // Steps and taps in one sequence of NM = STEPS * NTW blocks of six MFMAs; X's fragments are read a block ahead. The next
-            // tile is requested beside the first blocks, split and stored beside the last ones, one item each; the positions of its
-            // pixels follow. Each of these regions is fenced, and inside it the other work is spread between the MFMAs.
-            constexpr int NM = STEPS * NTW, HEAD = NM >= 9 ? 3 : 1;
-            read_d(0);
-            read_x(0, 0, 0);
+            for (int p = 0; p < kSplit; ++p) fa[p] = read_transposed(dsm + p * C::DPART, dsm + p * C::DPART + 64);
+            // A block of six MFMAs per tap; X's fragments are read a block ahead. The next tile is requested beside the first blocks,
+            // split and stored beside the last ones, one item each; the positions of its pixels follow. Each of these regions is
+            // fenced, and inside it the other work is spread between the MFMAs.
+            constexpr int HEAD = NTW >= 9 ? 3 : 1;
+            read_x(0, 0);
 #pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                const int st = m / NTW, tap = m % NTW, item = m - (NM - ITEMS);
+            for (int m = 0; m < NTW; ++m) {
+                const int item = m - (NTW - ITEMS);
                 if (m == 0 || m >= HEAD) __builtin_amdgcn_sched_barrier(0);
                 if (m == 0) fetch(cur, ragged_c);
-                if (m + 1 < NM) read_x((m + 1) & 1, (m + 1) / NTW, (m + 1) % NTW);
+                if (m + 1 < NTW) read_x((m + 1) & 1, m + 1);
                 if (item >= 0) commit_item(smem + (C::STAGE - buf), item);
 #pragma unroll
-                for (int t = 0; t < kTerms; ++t) acc[tap] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kTermA[t]], fb[m & 1][kTermB[t]], acc[tap], 0, 0, 0);
-                if (tap == NTW - 1 && st + 1 < STEPS) read_d(st + 1);
-                if (m == NM - 1) positions(cur);
+                for (int t = 0; t < kTerms; ++t) acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kTermA[t]], fb[m & 1][kTermB[t]], acc[m], 0, 0, 0);
+                if (m == NTW - 1) positions(cur);
 #pragma unroll
                 for (int t = 0; t < kTerms; ++t) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
