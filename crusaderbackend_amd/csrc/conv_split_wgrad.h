@@ -266,24 +266,60 @@ __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a
     for (int t = 0; t < NTW; ++t)
 #pragma unroll
         for (int i = 0; i < NR; ++i) bad |= !__builtin_isfinite(own[t][i]);
-    // (a thread holds all taps of its channel pairs: an eighth of the threads is two output channels, or four input channels)
-    const bool redo = __syncthreads_count(bad) <= C::NTH / 8;
-    // this slice's sum of one filter element from the fp32 operands (split_bf16.h: sums that are not finite)
-    auto plain_sum = [&](u32 oc, u32 ic, u32 fh, u32 fw) {
-        float sum = 0.f;
-        const u32 p1 = t1 * PXT < a.npix ? t1 * PXT : a.npix;
-        for (u32 p = t0 * PXT; p < p1 && !__builtin_isnan(sum); ++p) {
-            u32 v, r, y, xx, img, strip;
-            a.ohw.divmod(p, v, r);
-            a.ow.divmod(r, y, xx);
-            a.strip_d.divmod(v, img, strip);
-            xx += strip * a.SW;
-            const int iy = int(S * y + fh) - a.pad_y, ix = int(S * xx + fw) - a.pad_x;
-            if (xx >= a.OW || u32(iy) >= a.H || u32(ix) >= a.W) continue;
-            sum = fmaf(a.dY[(size_t(img) * a.OC + oc) * a.OHW + y * a.OW + xx], a.X[(size_t(img) * a.IC + ic) * a.HW + u32(iy) * a.W + u32(ix)], sum);
+    // ---- sums that are not finite: formed again on the fp32 MFMA from the fp32 operands (split_bf16.h) ------------------------
+    // The waves take the 32 x 32 channels of one tap in turn, over all pixels of the slice: two per MFMA, eight a step, the next
+    // step's operands requested ahead. Where the tap of a pixel lies outside the image both operands are zero (an infinite
+    // gradient would make NaN of the zero read there). Ends early where every sum is a NaN.
+    if (__builtin_expect(__syncthreads_or(bad), 0)) {
+        for (int unit = wv; unit < NW * NTW; unit += NW * KG) {
+            const int tap = unit % NTW, um = unit / NTW / C::WN, un = unit / NTW % C::WN, i32 = lane & 31, h = lane >> 5;
+            float *const res = x + ((um * 32 + 4 * h) * C::ICT + un * 32 + i32) * NTW + tap;  // register r: row 8 * (r / 4) + r % 4
+            bool again = false;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) again |= !__builtin_isfinite(res[(8 * (r / 4) + r % 4) * C::ICT * NTW]);
+            if (!__any(int(again))) continue;
+            struct Step {
+                float d[4], x[4];
+            };
+            const u32 oc = oc0 + um * 32 + i32, ic = ic0 + un * 32 + i32;
+            const float *drow = a.dY + size_t(oc < a.OC ? oc : a.OC - 1) * a.OHW, *xrow = a.X + size_t(ic < a.IC ? ic : a.IC - 1) * a.HW;
+            auto fetch_step = [&](u32 p0, Step &f) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const u32 p = p0 + 2 * q + h;
+                    u32 v, rem, py, px, img, strip;
+                    a.ohw.divmod(p < a.npix ? p : a.npix - 1, v, rem);
+                    a.ow.divmod(rem, py, px);
+                    a.strip_d.divmod(v, img, strip);
+                    px += strip * a.SW;
+                    const int iy = int(S * py) + fh0 + tap / F - a.pad_y, ix = int(S * px) + tap % F - a.pad_x;
+                    const bool in = p < a.npix && px < a.OW && u32(iy) < a.H && u32(ix) < a.W;
+                    const float d = drow[in ? size_t(img) * a.OC * a.OHW + py * a.OW + px : 0];
+                    const float e = xrow[in ? size_t(img) * a.IC * a.HW + u32(iy) * a.W + u32(ix) : 0];
+                    f.d[q] = in && oc < a.OC ? d : 0.f, f.x[q] = in && ic < a.IC ? e : 0.f;
+                }
+            };
+            v16f sum;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sum[r] = 0.0f;
+            Step next;
+            fetch_step(t0 * PXT, next);
+#pragma unroll 1
+            for (u32 p = t0 * PXT; p < t1 * PXT; p += 8) {
+                const Step now = next;
+                fetch_step(p + 8, next);  // (behind the slice's last pixel: for nobody)
+                u32 numbers = 0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(now.d[q], now.x[q], sum, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) numbers |= __builtin_isnan(sum[r]) ? 0u : 1u;
+                if (!__any(int(numbers))) break;
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) res[(8 * (r / 4) + r % 4) * C::ICT * NTW] = sum[r];
         }
-        return sum;
-    };
+        lds_barrier();
+    }
     constexpr u32 ROW = C::ICT * NTW;
     const u32 nic = a.IC - ic0 < u32(C::ICT) ? a.IC - ic0 : u32(C::ICT);
     float *out = a.out + (a.splits > 1 ? size_t(z) * a.OC * a.IC * (F * F) : 0);
@@ -291,9 +327,7 @@ __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a
         const u32 oc = e / ROW, rest = e % ROW, ic = rest / NTW, t = rest % NTW;
         if (oc0 + oc < a.OC && ic < nic) {
             float *dst = out + ((size_t(oc0 + oc) * a.IC + ic0 + ic) * (F * F) + fh0 * F + t);
-            float v = x[e];
-            if (redo && !__builtin_isfinite(v)) v = plain_sum(oc0 + oc, ic0 + ic, fh0 + t / F, t % F);
-            if (a.splits > 1) *dst = v; else *dst += v;
+            if (a.splits > 1) *dst = x[e]; else *dst += x[e];
         }
     }
 }

@@ -13,10 +13,9 @@
 // the results are closer to the exact ones than those of the fp32 pipe, and the three left out are not seen at all.
 // An operand that is infinite, or rounds to infinity as a bf16 (from 3.39e38 up), has NaN among its parts, so it always shows
 // as NaN in the sum. Sums that are not finite are formed once more from the fp32 operands and are those of an fp32 contraction
-// (infinities keep their sign, large finite values stay finite). Convolutions forward and data gradients: a wave does its blocks
-// again on the fp32 MFMA, straight from memory (one infinity in 64 -> 64 @56 batch 32: 68 -> 109 us, a channel of infinities 269;
-// element by element it was 3.2 and 7.2 ms). Products: element by element, up to a NaN; weight gradients as well, but for
-// blocks with more than an eighth of their sums not finite, which are left at NaN.
+// (infinities keep their sign, large finite values stay finite). Convolutions: on the fp32 MFMA, straight from memory, by waves
+// for their blocks (one infinity in 64 -> 64 @56 batch 32: 68 -> 109 us, a channel of infinities 269, its weight gradient 66 ->
+// 709 and 757; element by element the forward pass took 3.2 and 7.2 ms). Products: element by element, up to a NaN.
 // Operands under 2^-110 have a last part that a bf16 cannot hold whole: an absolute error of 2^-134.
 #pragma once
 #include "crb_common.h"

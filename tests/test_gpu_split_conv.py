@@ -158,3 +158,32 @@ def test_data_gradients_of_operands_that_round_to_infinity(dev, shape):
         else:
             ref = F_.conv_transpose2d(dy.double(), w.double(), stride=s, padding=p)
             check_against_float64(dX, ref, OC * F * F, what)
+
+
+# 64 x 32 channels and 64 pixels a tile in one strip; 32 x 32 and 128; 5x5, whose filter rows are separate workgroups; stride 2
+LARGE_W = [(17, 96, 13, 13, 64, 3, 1, 1), (3, 64, 31, 33, 65, 3, 1, 1), (16, 64, 24, 23, 72, 5, 1, 2), (4, 65, 33, 27, 97, 3, 2, 1)]
+
+
+@pytest.mark.parametrize("shape", LARGE_W, ids=lambda s: "x".join(map(str, s)))
+def test_weight_gradients_of_operands_that_round_to_infinity(dev, shape):
+    """Inputs beyond the largest bf16 in five of a tile's 32 channels, or everywhere, with finite sums; and infinite gradients."""
+    import torch
+    from crusaderbackend_amd import capi
+
+    N, IC, H, W, OC, F, s, p = shape
+    g = capi.ConvGeom.make(N, IC, H, W, OC, F, F, s, s, p, p)
+    gen = torch.Generator().manual_seed(12)
+    X, dY = torch.rand(N, IC, H, W, generator=gen) + 0.5, torch.rand(N, OC, g.OH, g.OW, generator=gen) * 0.5 + 0.25
+    few = X.clone()
+    few[N - 1, 3:8, H // 2, W // 2] = 3.4e38
+    infinite = dY.clone()
+    infinite[:, OC // 2] = float("-inf")
+    K = N * g.OH * g.OW
+    for what, x, dy in (("few", few, dY), ("all", torch.full_like(X, 3.4e38), dY * (1 / K)), ("infinite", X, infinite)):
+        dW = torch.zeros(OC, IC, F, F, device=dev)
+        capi.conv_wgrad(dy.to(dev), x.to(dev), dW, g)
+        torch.cuda.synchronize()
+        ref = torch.nn.grad.conv2d_weight(torch.where(x.isinf(), 1.0, x).double(), (OC, IC, F, F), dy.double().nan_to_num(0, 0, 0), stride=s, padding=p)
+        if what == "infinite":
+            ref[OC // 2] = float("-inf")
+        check_against_float64(dW, ref, K, what)
