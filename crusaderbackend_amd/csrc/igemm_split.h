@@ -48,11 +48,6 @@ struct SMatK {
         u32 k;  // offset of the item's octet inside a slab
     };
     __device__ __forceinline__ void bind(u32 z) { base += size_t(z) * zstride; }
-    __device__ __forceinline__ float at(u32 row, u32 k) const {
-        u32 nd = 0, kk = k;
-        if constexpr (CAT) cat_k.divmod(k, nd, kk);
-        return base[size_t(nd) * cat_stride + size_t(row) * ld + kk];
-    }
     __device__ __forceinline__ Cursor cursor(u32 row, u32 k) const { return {base + size_t(row < rows ? row : rows - 1) * ld, k}; }
     template <bool TAIL>
     __device__ __forceinline__ void fetch(const Cursor &c, u32 k0, u32 klimit, float (&out)[8]) const {
@@ -90,7 +85,6 @@ struct SMatR {
         u32 k, left;  // rows from the item's first to the matrix' end (0: none, the item repeats the last row)
     };
     __device__ __forceinline__ void bind(u32 z) { base += size_t(z) * zstride; }
-    __device__ __forceinline__ float at(u32 row, u32 k) const { return base[size_t(k) * ld + row]; }
     __device__ __forceinline__ Cursor cursor(u32 row, u32 k) const {
         return {base + (row < rows ? row : rows - 1), k, row < rows ? rows - row : 0u};
     }
@@ -432,6 +426,35 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
             __syncthreads();
         }
     }
+    // ---- sums that are not finite: the block (mi, ni) once more, on the fp32 MFMA from the fp32 operands (split_bf16.h) ------
+    // A lane's eight k of a row per step, as the panels are read; two k per MFMA. Ends early where every sum is a NaN.
+    auto fp32_block = [&](int mi, int ni) {
+        const typename AOp::Cursor ca = a.cursor(row0 + wave_m * Cfg::WTM + mi * 32 + i32, 8 * h);
+        const typename BOp::Cursor cb = b.cursor(col0 + wave_n * Cfg::WTN + ni * 32 + i32, 8 * h);
+        auto octet = [&](const auto &op, const auto &cur, u32 k0, float (&out)[1][8]) {
+            if constexpr (std::decay_t<decltype(op)>::kLoad == LOAD_K8)
+                op.template fetch<true>(cur, k0, kend, out[0]);
+            else
+                op.template fetch<1, true, false>(cur, k0, kend, out);
+        };
+        v16f sum;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum[r] = 0.0f;
+#pragma unroll 1
+        for (u32 k0 = kbeg; k0 < kend; k0 += 16) {
+            float av[1][8], bv[1][8];
+            octet(a, ca, k0, av);
+            octet(b, cb, k0, bv);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(av[0][j], bv[0][j], sum, 0, 0, 0);
+            u32 numbers = 0;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) numbers |= __builtin_isnan(sum[r]) ? 0u : 1u;
+            if (!__any(int(numbers))) break;
+        }
+        return sum;
+    };
+
     // ---- epilogue: 32 lanes store 32 consecutive columns of a row ---------------------------------------------------------
     const bool whole = row0 + BM <= d.M && col0 + BN <= d.N;
     const bool accumulates = epi.accumulates(), row_biased = epi.has_row_bias();
@@ -452,14 +475,10 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
                 rowb[r] = epi.row_bias_at(row < d.M ? row : d.M - 1);
             }
         }
-        const u32 redo = not_finite<NR>(v);
-        if (__builtin_expect(__any(int(redo)), 0)) {
-#pragma unroll
-            for (int r = 0; r < NR; ++r) {
-                const u32 row = rbase + 8 * (r / 4) + (r % 4);
-                if (row < d.M && !(redo >> r & 1)) epi.store(row, cs, v[r], rowb[r]);
-            }
-        } else if (whole) {
+        // (nothing is on its way past this point on either path to it: without the wait here the compiler puts one for every
+        // load that may have been made, on whichever path, in front of each store: 1003 x 1505 x 777 28.0 -> 29.3 us)
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+        if (whole) {
             if (accumulates) {
 #pragma unroll
                 for (int r = 0; r < NR; ++r) oldv[r] = *epi.at(rbase + 8 * (r / 4) + (r % 4), col);
@@ -473,21 +492,15 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
                 if (row < d.M) epi.store(row, cs, v[r], rowb[r]);
             }
         }
-        return redo;  // what is not stored yet
     };
-    // the sums of a part that were not finite, from the fp32 operands (split_bf16.h)
-    auto redo_part = [&](int mi, int ni, int r0, u32 redo) {
-        for (; redo; redo &= redo - 1) {
-            const u32 r = __builtin_ctz(redo), col = col0 + wave_n * Cfg::WTN + ni * 32 + i32;
-            const u32 row = row0 + wave_m * Cfg::WTM + mi * 32 + 4 * h + 2 * r0 + 8 * (r / 4) + (r % 4);
-            if (row >= d.M || col >= d.N) continue;
-            float sum = 0.f;
-            for (u32 k = kbeg; k < kend && !__builtin_isnan(sum); ++k) sum = fmaf(a.at(row, k), b.at(col, k), sum);
-            epi.store(row, epi.prep_col(col, d.N), sum, row_biased ? epi.row_bias_at(row) : 0.f);
-        }
+    auto not_finite = [](const float *v, int n) {
+        bool bad = false;
+        for (int r = 0; r < n; ++r) bad |= !__builtin_isfinite(v[r]);
+        return __builtin_expect(__any(int(bad)), 0);
     };
     if constexpr (KG == 1) {
-        u32 redo[TM][TN], any = 0;
+        // (blocks that are not finite wait until the accumulators of the others have been stored: both do not fit the registers)
+        u32 again = 0;
 #pragma unroll
         for (int ni = 0; ni < TN; ++ni)
 #pragma unroll
@@ -495,15 +508,17 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
                 float v[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) v[r] = acc[mi][ni][r];
-                any |= redo[mi][ni] = store_part(mi, ni, 0, std::integral_constant<int, 16>(), v);
+                if (not_finite(v, 16)) again |= 1u << (mi * TN + ni);
+                else store_part(mi, ni, 0, std::integral_constant<int, 16>(), v);
             }
-        if (__builtin_expect(any != 0, 0)) {
-            for (int blk = 0; blk < TM * TN; ++blk) {
-                u32 m = 0;
+#pragma unroll 1
+        for (; again; again &= again - 1) {
+            const int blk = __builtin_ctz(again);
+            const v16f sum = fp32_block(blk / TN, blk % TN);
+            float v[16];
 #pragma unroll
-                for (int i = 0; i < TM * TN; ++i) m = i == blk ? redo[i / TN][i % TN] : m;
-                redo_part(blk / TN, blk % TN, 0, m);
-            }
+            for (int r = 0; r < 16; ++r) v[r] = sum[r];
+            store_part(blk / TN, blk % TN, 0, std::integral_constant<int, 16>(), v);
         }
     } else {
         // The groups exchange their accumulators through the staging space (idle: the last slab's barrier has passed), BR blocks
@@ -511,6 +526,7 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
         constexpr int NB = TM * TN, BR = NB < KG ? NB : KG, NR = BR * 16 / KG;
         static_assert(BR >= 1 && NB % BR == 0 && NR % 4 == 0 && NR <= 16 && BR * 4096 * Cfg::WM * Cfg::WN * KG <= 2 * STAGE, "exchange space");
         float *x = reinterpret_cast<float *>(smem);
+        const int f0 = kgroup * NR;  // this group's share of BR blocks' registers
 #pragma unroll
         for (int q = 0; q < NB / BR; ++q) {
             if (q) lds_barrier();
@@ -518,7 +534,6 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
 #pragma unroll
             for (int f = 0; f < BR * 16; ++f) dst[f * 64] = acc[(q * BR + f / 16) / TN][(q * BR + f / 16) % TN][f % 16];
             lds_barrier();
-            const int f0 = kgroup * NR;
             float v[NR];
             const float *src = x + wave * BR * 1024 + f0 * 64 + lane;
 #pragma unroll
@@ -528,7 +543,16 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
 #pragma unroll
                 for (int r = 0; r < NR; ++r) v[r] += src[g * Cfg::WM * Cfg::WN * BR * 1024 + r * 64];
             const int blk = q * BR + f0 / 16;
-            redo_part(blk / TN, blk % TN, f0 % 16, store_part(blk / TN, blk % TN, f0 % 16, std::integral_constant<int, NR>(), v));
+            if (not_finite(v, NR)) {
+                const v16f sum = fp32_block(blk / TN, blk % TN);
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    v[r] = sum[r];
+#pragma unroll
+                    for (int at = NR; at < 16; at += NR) v[r] = f0 % 16 == at ? sum[at + r] : v[r];
+                }
+            }
+            store_part(blk / TN, blk % TN, f0 % 16, std::integral_constant<int, NR>(), v);
         }
     }
 }

@@ -75,15 +75,6 @@ __device__ __forceinline__ bool any_not_finite(const V (&acc)[TM][TN]) {
     return bad;
 }
 
-// Bit r of the result: sum v[r] is not finite.
-template <int NR>
-__device__ __forceinline__ u32 not_finite(const float *v) {
-    u32 m = 0;
-#pragma unroll
-    for (int r = 0; r < NR; ++r) m |= __builtin_isfinite(v[r]) ? 0u : 1u << r;
-    return m;
-}
-
 // The products that are formed: (part of A, part of B), in an order that needs the leading parts first.
 constexpr int kTerms = 6;
 constexpr int kTermA[kTerms] = {0, 0, 1, 1, 0, 2};

@@ -122,3 +122,41 @@ def test_small_operands_keep_their_bits(dev):
     capi.sgemm_nn(to_dev(A, dev), to_dev(np.eye(n, dtype=np.float32), dev), C, n, n, n)
     torch.cuda.synchronize()
     assert np.array_equal(to_np(C), A)
+
+
+# 256 x 256, 128 x 128, 64 x 64 tiles of eight and of four waves, a cut contraction
+@pytest.mark.parametrize("size", [(2304, 2300, 90), (2048, 2048, 65), (1024, 1024, 257), (1003, 1505, 777), (256, 1024, 1025)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("form", ["nn", "nt", "tn", "nta"])
+def test_products_that_overflow_throughout(dev, form, size):
+    """No sum is finite: infinities of the right sign, NaN in one row, in the order of the finite product's time."""
+    import torch
+    from crusaderbackend_amd import capi
+
+    M, N, K = size
+    A, B = torch.rand(M, K, device=dev) + 1, torch.rand(K, N, device=dev) + 1
+    big = A * 1e25
+    big[M // 2] *= -1
+    big[M // 3, K // 2] = float("nan")
+    ref = torch.full((M, N), float("inf"), device=dev)
+    ref[M // 2], ref[M // 3] = float("-inf"), float("nan")
+    C = torch.zeros(M, N, device=dev)
+
+    def lay(x, turn):
+        return x.t().contiguous() if turn else x
+
+    def timed(a, b):
+        a, b = lay(a, form == "tn"), lay(b, form in ("nt", "nta"))
+        t = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        product(capi, form, a, b, C, M, N, K)
+        t[0].record()
+        product(capi, form, a, b, C, M, N, K)
+        t[1].record()
+        torch.cuda.synchronize()
+        return t[0].elapsed_time(t[1])
+
+    finite = timed(A, B)
+    over = timed(big, B * 1e20)
+    assert torch.equal(C.isnan(), ref.isnan()) and torch.equal(C.nan_to_num(0, 1, -1), ref.nan_to_num(0, 1, -1))
+    # fp32 matrix instructions on operands straight from memory; a sum at a time it was 40 to 300 times as long
+    assert over < 25 * max(finite, 0.02), (over, finite)
