@@ -251,7 +251,7 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
     // Two channels of a tap per MFMA, 16 a step, the next step's operands requested ahead. Taps outside the image take no part
     // (an infinite filter element would make NaN of the zero read there): a lane's accumulators all belong to its pixel, so
     // it keeps the old ones. Ends early where every sum is a NaN.
-    if (__builtin_expect(__any(int(any_not_finite(acc))), 0)) {
+    if (__builtin_expect(__any(int(scale_down(acc))), 0)) {
         struct Step {
             float w[8][TM], x[8][TN];
             bool in[TN];

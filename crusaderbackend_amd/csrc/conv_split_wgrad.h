@@ -251,7 +251,7 @@ __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a
                 float v = x[(wave * C::RT + t) * 1024 + (kgroup * NR + i) * 64 + lane];
 #pragma unroll
                 for (int g = 1; g < KG; ++g) v += x[((g * NW + wave) * C::RT + t) * 1024 + (kgroup * NR + i) * 64 + lane];
-                own[q * C::RT + t][i] = v;
+                own[q * C::RT + t][i] = v * kSplitDown;
             }
     }
     lds_barrier();

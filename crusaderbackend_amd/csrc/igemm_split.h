@@ -8,7 +8,7 @@
 // consecutive k (row-contiguous) and the transposition happens in the packing of its registers, for nothing.
 //
 // What bounds it: per K step of 16 a wave issues 6 * TM * TN MFMAs (192 clocks per block) against 3 * (TM + TN) fragment reads
-// of 1 KB and its share of the split (5.5 VALU operations per staged element), so the ratio of all three goes with the tile
+// of 1 KB and its share of the split (6.5 VALU operations per staged element), so the ratio of all three goes with the tile
 // edge; 2 x 2 blocks per wave keep LDS under the MFMA time, smaller tiles do not.
 //
 // MFMA 32x32x16 bf16 operand mapping (wave64, lane l): A = A[i = l%32][k = 8*(l/32) + 0..7], B = B[k = 8*(l/32) + 0..7][j = l%32],
@@ -300,7 +300,7 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
             }
         };
         constexpr int NM = TM * TN * kTerms * (BK / 16 / KG);
-        constexpr int VPM = ((PA::NP * PA::RV + PB::NP * PB::RV) * 48 + NM - 1) / NM;
+        constexpr int VPM = ((PA::NP * PA::RV + PB::NP * PB::RV) * 56 + NM - 1) / NM;
         // between two MFMAs: one fragment read, a share of the split's arithmetic, one store to LDS
         auto interleave = [&]() {
 #pragma unroll
@@ -507,7 +507,7 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
             for (int mi = 0; mi < TM; ++mi) {
                 float v[16];
 #pragma unroll
-                for (int r = 0; r < 16; ++r) v[r] = acc[mi][ni][r];
+                for (int r = 0; r < 16; ++r) v[r] = acc[mi][ni][r] * kSplitDown;
                 if (not_finite(v, 16)) again |= 1u << (mi * TN + ni);
                 else store_part(mi, ni, 0, std::integral_constant<int, 16>(), v);
             }
@@ -542,6 +542,8 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
             for (int g = 1; g < KG; ++g)
 #pragma unroll
                 for (int r = 0; r < NR; ++r) v[r] += src[g * Cfg::WM * Cfg::WN * BR * 1024 + r * 64];
+#pragma unroll
+            for (int r = 0; r < NR; ++r) v[r] *= kSplitDown;
             const int blk = q * BR + f0 / 16;
             if (not_finite(v, NR)) {
                 const v16f sum = fp32_block(blk / TN, blk % TN);

@@ -11,12 +11,11 @@
 // Measured distance from float64 (2-norm, N(0,1) operands; fp32 MFMA / six products / all nine): K = 144 2.15e-7 / 1.74e-7 /
 // 1.74e-7, 576 4.31e-7 / 3.61e-7 / 3.61e-7, 4608 1.22e-6 / 1.07e-6 / 1.07e-6 - sixteen k's share one rounding of the sum, so
 // the results are closer to the exact ones than those of the fp32 pipe, and the three left out are not seen at all.
-// An operand that is infinite, or rounds to infinity as a bf16 (from 3.39e38 up), has NaN among its parts, so it always shows
+// An operand that is infinite, or beyond the range that is split (kSplitUp), has NaN among its parts, so it always shows
 // as NaN in the sum. Sums that are not finite are formed once more from the fp32 operands and are those of an fp32 contraction
 // (infinities keep their sign, large finite values stay finite). Convolutions: on the fp32 MFMA, straight from memory, by waves
 // for their blocks (one infinity in 64 -> 64 @56 batch 32: 68 -> 109 us, a channel of infinities 269, its weight gradient 66 ->
 // 709 and 757; element by element the forward pass took 3.2 and 7.2 ms). Products: element by element, up to a NaN.
-// Operands under 2^-110 have a last part that a bf16 cannot hold whole: an absolute error of 2^-134.
 #pragma once
 #include "crb_common.h"
 
@@ -39,12 +38,17 @@ __device__ __forceinline__ void split_pair(float x0, float x1, u32 &hi, u32 &mid
     hi = h, mid = m, lo = __builtin_bit_cast(u32, __builtin_convertvector(f32x2{s0, s1}, bf16x2));
 }
 
+// Operands are split at 2^16 times their value and the sums taken back by 2^-32 (both exact): the last part of a float under
+// 2^-110 has bits below 2^-133, which a bf16 cannot hold; at 2^16 times the value it has none, down to the smallest float. What
+// the scale moves out of range, operands from 2^112 and sums from 2^96 up, shows as a sum that is not finite and is formed again.
+constexpr float kSplitUp = 65536.f, kSplitDown = 1.f / (65536.f * 65536.f);
+
 // The three parts of eight floats, each a 16-byte MFMA fragment (element i in 16-bit slot i).
 __device__ __forceinline__ void split8(const float *x, u32x4 (&part)[kSplit]) {
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
         u32 h, m, l;
-        split_pair(x[2 * p], x[2 * p + 1], h, m, l);
+        split_pair(x[2 * p] * kSplitUp, x[2 * p + 1] * kSplitUp, h, m, l);
         part[0][p] = h, part[1][p] = m, part[2][p] = l;
     }
 }
@@ -62,16 +66,16 @@ __device__ __forceinline__ float buffer_load(BufferRange r, u32 voffset, u32 sof
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, int(voffset), int(soffset), 0));
 }
 
-// Whether one of a lane's accumulators is not finite.
+// A lane's accumulators at their own scale; whether one of them is not finite.
 template <class V, int TM, int TN>
-__device__ __forceinline__ bool any_not_finite(const V (&acc)[TM][TN]) {
+__device__ __forceinline__ bool scale_down(V (&acc)[TM][TN]) {
     bool bad = false;
 #pragma unroll
     for (int mi = 0; mi < TM; ++mi)
 #pragma unroll
         for (int ni = 0; ni < TN; ++ni)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) bad |= !__builtin_isfinite(acc[mi][ni][r]);
+            for (int r = 0; r < 16; ++r) acc[mi][ni][r] *= kSplitDown, bad |= !__builtin_isfinite(acc[mi][ni][r]);
     return bad;
 }
 

@@ -187,3 +187,33 @@ def test_weight_gradients_of_operands_that_round_to_infinity(dev, shape):
         if what == "infinite":
             ref[OC // 2] = float("-inf")
         check_against_float64(dW, ref, K, what)
+
+
+@pytest.mark.parametrize("shape", LARGE + LARGE_W[:1] + LARGE_W[3:], ids=lambda s: "x".join(map(str, s)))
+def test_operands_down_to_the_smallest_normal_float(dev, shape):
+    """Filters or activations of 2^-126 and a little more against ones of 2^60: as close to float64 as ordinary ones."""
+    import torch
+    import torch.nn.functional as F_
+    from crusaderbackend_amd import capi
+
+    N, IC, H, W, OC, F, s, p = shape
+    g = capi.ConvGeom.make(N, IC, H, W, OC, F, F, s, s, p, p)
+    gen = torch.Generator().manual_seed(13)
+
+    def near(e, *size):
+        t = torch.ldexp(torch.rand(*size, generator=gen) + 1, torch.tensor(e))
+        return torch.where(torch.rand(*size, generator=gen) < 0.3, -t, t)
+
+    for ew, ex in ((-126, 60), (60, -126)):
+        Wt, X, dY = near(ew, OC, IC, F, F), near(ex, N, IC, H, W), near(ex, N, OC, g.OH, g.OW)
+        Xs = near(186 + ex if ex < 0 else -126, N, IC, H, W)  # of the weight gradient: 2^60 against 2^-126 both ways
+        Y, dX, dW = torch.empty(N, OC, g.OH, g.OW, device=dev), torch.empty(N, IC, H, W, device=dev), torch.zeros(OC, IC, F, F, device=dev)
+        capi.conv_fwd(Wt.to(dev), X.to(dev), Y, None, g)
+        capi.conv_dgrad(Wt.to(dev), dY.to(dev), dX, g)
+        capi.conv_wgrad(dY.to(dev), Xs.to(dev), dW, g)
+        torch.cuda.synchronize()
+        Xr, Wr = torch.zeros(N, IC, H, W, dtype=torch.double, requires_grad=True), Wt.double()
+        F_.conv2d(Xr, Wr, stride=s, padding=p).backward(dY.double())
+        for what, got, ref, K in (("Y", Y, F_.conv2d(X.double(), Wr, stride=s, padding=p), IC * F * F), ("dX", dX, Xr.grad, OC * F * F),
+                                  ("dW", dW, torch.nn.grad.conv2d_weight(Xs.double(), Wt.shape, dY.double(), stride=s, padding=p), N * g.OH * g.OW)):
+            assert (got.cpu().double() - ref).norm() <= np.sqrt(K) * 2.0**-24 * ref.norm(), what

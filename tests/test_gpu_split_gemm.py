@@ -160,3 +160,24 @@ def test_products_that_overflow_throughout(dev, form, size):
     assert torch.equal(C.isnan(), ref.isnan()) and torch.equal(C.nan_to_num(0, 1, -1), ref.nan_to_num(0, 1, -1))
     # fp32 matrix instructions on operands straight from memory; a sum at a time it was 40 to 300 times as long
     assert over < 25 * max(finite, 0.02), (over, finite)
+
+
+@pytest.mark.parametrize("form", ["nn", "nt", "tn", "nta"])
+@pytest.mark.parametrize("size", [(2304, 2300, 90), (2048, 2048, 65), (1024, 1024, 257), (1003, 1505, 777)], ids=lambda s: "x".join(map(str, s)))
+def test_operands_down_to_the_smallest_normal_float(dev, form, size):
+    """Operands of 2^-126 and a little more against ones of 2^60 and back: as close to float64 as ordinary ones."""
+    import torch
+    from crusaderbackend_amd import capi
+
+    M, N, K = size
+    for ea, eb in ((-126, 60), (60, -126), (-126, -10)):
+        A, B = (np.ldexp(np.float32(1) + np.abs(uniform(5 + i, *s)), e).astype(np.float32) for i, (s, e) in enumerate((((M, K), ea), ((K, N), eb))))
+        A[::3], B[:, ::3] = -A[::3], -B[:, ::3]
+        exact = A.astype(np.float64) @ B.astype(np.float64)
+        a = np.ascontiguousarray(A.T) if form == "tn" else A
+        b = np.ascontiguousarray(B.T) if form in ("nt", "nta") else B
+        C = torch.zeros(M, N, device=dev)
+        product(capi, form, to_dev(a, dev), to_dev(b, dev), C, M, N, K)
+        torch.cuda.synchronize()
+        # every product and addition rounds once, or (results under 2^-126) to the step of the subnormal numbers
+        assert np.linalg.norm(to_np(C) - exact) <= np.sqrt(K) * 2.0**-24 * np.linalg.norm(exact) + np.sqrt(M * N) * K * 2.0**-150
