@@ -257,11 +257,12 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
     };
     auto read_frags = [&](Frags &f, const unsigned char *sm, int st) {
 #pragma unroll
-        for (int p = 0; p < kSplit; ++p) {
+        for (int i = 0; i < kSplit; ++i) {
+            const int p = kPartOrderA[i], q = kPartOrderB[i];
 #pragma unroll
             for (int mi = 0; mi < TM; ++mi) f.a[p][mi] = *reinterpret_cast<const bf16x8 *>(sm + a_lane + p * PA::PART + 2 * st * KG * PA::OCT + mi * 512);
 #pragma unroll
-            for (int ni = 0; ni < TN; ++ni) f.b[p][ni] = *reinterpret_cast<const bf16x8 *>(sm + b_lane + p * PB::PART + 2 * st * KG * PB::OCT + ni * 512);
+            for (int ni = 0; ni < TN; ++ni) f.b[q][ni] = *reinterpret_cast<const bf16x8 *>(sm + b_lane + q * PB::PART + 2 * st * KG * PB::OCT + ni * 512);
         }
     };
     auto mfmas = [&](const Frags &f) {

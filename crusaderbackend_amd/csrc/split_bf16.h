@@ -8,14 +8,15 @@
 // (mid*lo, lo*mid, lo*lo) are together at most 2^-24 of the product, the unit roundoff of one fp32 multiplication. All sums are
 // fp32, in the accumulators of the MFMA. Six sixteenths of the fp32 time per product remain: at the rates the pipes sustain on
 // this part (1.82 PFLOP/s bf16, 155 TFLOP/s fp32, dense random operands) 303 against 155 TFLOP/s of fp32 work.
-// Measured distance from float64 (2-norm, N(0,1) operands; fp32 MFMA / six products / all nine): K = 144 2.15e-7 / 1.74e-7 /
-// 1.74e-7, 576 4.31e-7 / 3.61e-7 / 3.61e-7, 4608 1.22e-6 / 1.07e-6 / 1.07e-6 - sixteen k's share one rounding of the sum, so
-// the results are closer to the exact ones than those of the fp32 pipe, and the three left out are not seen at all.
+// Measured distance from float64 (2-norm, N(0,1) operands; fp32 MFMA / these products): K = 90 1.70e-7 / 0.97e-7, 257 2.87e-7 /
+// 1.20e-7, 777 4.98e-7 / 2.99e-7 - sixteen k's share one rounding of the sum, so the results are closer to the exact ones than those
+// of the fp32 pipe. (With the leading parts first 1.25e-7, 1.44e-7, 3.10e-7; forming all nine showed no difference to those.)
 // An operand that is infinite, or beyond the range that is split (kSplitUp), has NaN among its parts, so it always shows
 // as NaN in the sum. Sums that are not finite are formed once more from the fp32 operands and are those of an fp32 contraction
 // (infinities keep their sign, large finite values stay finite). Convolutions: on the fp32 MFMA, straight from memory, by waves
 // for their blocks (one infinity in 64 -> 64 @56 batch 32: 68 -> 109 us, a channel of infinities 269, its weight gradient 66 ->
-// 709 and 757; element by element the forward pass took 3.2 and 7.2 ms). Products: element by element, up to a NaN.
+// 709 and 757; element by element the forward pass took 3.2 and 7.2 ms). Products the same, by blocks (4096^3 overflowing
+// throughout 0.65 -> 4.6 ms).
 #pragma once
 #include "crb_common.h"
 
@@ -79,9 +80,12 @@ __device__ __forceinline__ bool scale_down(V (&acc)[TM][TN]) {
     return bad;
 }
 
-// The products that are formed: (part of A, part of B), in an order that needs the leading parts first.
+// The products that are formed: (part of A, part of B), the smallest first: where one term is most of a sum, the roundings before
+// the last are then of its small parts (a sum of one product: off by 1.45 units in the last place at most, rms 0.39; the other way
+// round 3.38 and 0.60; one fp32 multiplication 0.5 and 0.29). kPartOrder: the parts in the order in which they are needed.
 constexpr int kTerms = 6;
-constexpr int kTermA[kTerms] = {0, 0, 1, 1, 0, 2};
-constexpr int kTermB[kTerms] = {0, 1, 0, 1, 2, 0};
+constexpr int kTermA[kTerms] = {2, 0, 1, 1, 0, 0};
+constexpr int kTermB[kTerms] = {0, 2, 1, 0, 1, 0};
+constexpr int kPartOrderA[kSplit] = {2, 0, 1}, kPartOrderB[kSplit] = {0, 2, 1};
 
 }  // namespace crb

@@ -181,3 +181,25 @@ def test_operands_down_to_the_smallest_normal_float(dev, form, size):
         torch.cuda.synchronize()
         # every product and addition rounds once, or (results under 2^-126) to the step of the subnormal numbers
         assert np.linalg.norm(to_np(C) - exact) <= np.sqrt(K) * 2.0**-24 * np.linalg.norm(exact) + np.sqrt(M * N) * K * 2.0**-150
+
+
+@pytest.mark.parametrize("form", ["nn", "nt", "tn", "nta"])
+@pytest.mark.parametrize("size", [(2304, 2300, 90), (2048, 2048, 65), (1024, 1024, 257), (1003, 1505, 777)], ids=lambda s: "x".join(map(str, s)))
+def test_sums_of_one_product(dev, form, size):
+    """Rows of A that hold one nonzero element, operands of 24 significant bits: what is left of a product is at most 2^-24 of it,
+    a unit in the last place of a float in [1, 2) two of that, and its last rounding half a unit: 1.5 units."""
+    import torch
+    from crusaderbackend_amd import capi
+
+    M, N, K = size
+    A, at = np.zeros((M, K), np.float32), np.random.RandomState(3).randint(0, K, M)
+    value, B = 1 + np.abs(uniform(4, M)), 1 + np.abs(uniform(5, K, N))
+    A[np.arange(M), at] = value
+    exact = value.astype(np.float64)[:, None] * B.astype(np.float64)[at]
+    a = np.ascontiguousarray(A.T) if form == "tn" else A
+    b = np.ascontiguousarray(B.T) if form in ("nt", "nta") else B
+    C = torch.zeros(M, N, device=dev)
+    product(capi, form, to_dev(a, dev), to_dev(b, dev), C, M, N, K)
+    torch.cuda.synchronize()
+    ulps = np.abs(to_np(C) - exact) / np.ldexp(1.0, np.floor(np.log2(exact)).astype(int) - 23)
+    assert ulps.max() <= 1.5, (ulps.max(), np.sqrt((ulps**2).mean()))
