@@ -336,8 +336,9 @@ struct SplitWgradPlan {
     u32 strips = 0, pairs = 0, splits = 0, tiles = 0, tiles_z = 0;
     size_t workspace_bytes = 0;
 };
+// most: bytes the slices may take
 template <class C>
-inline SplitWgradPlan split_wgrad_plan(u32 N, u32 IC, u32 OC, u32 H, u32 W, u32 OH, u32 OW) {
+inline SplitWgradPlan split_wgrad_plan(u32 N, u32 IC, u32 OC, u32 H, u32 W, u32 OH, u32 OW, size_t most) {
     SplitWgradPlan p;
     for (u32 ns = ceil_div(OW, 64u); ns <= OW && ns <= 16; ++ns)
         if (conv_split_window(C::PXT, OH, ceil_div(OW, ns), C::F, C::S) <= u32(C::MAXPX)) {
@@ -357,9 +358,11 @@ inline SplitWgradPlan split_wgrad_plan(u32 N, u32 IC, u32 OC, u32 H, u32 W, u32 
     const u32 rows = C::F / C::ROWS;
     u32 splits = p.pairs * rows >= 256 ? 1 : 256 / (p.pairs * rows);  // one workgroup per CU
     if (splits > ceil_div(p.tiles, 4u)) splits = ceil_div(p.tiles, 4u);
+    const size_t slice = size_t(OC) * IC * C::F * C::F * sizeof(float);
+    if (splits > 1 && splits > most / slice) splits = most / slice > 1 ? u32(most / slice) : 1;
     p.tiles_z = ceil_div(p.tiles, splits);
     p.splits = ceil_div(p.tiles, p.tiles_z);
-    p.workspace_bytes = p.splits > 1 ? size_t(p.splits) * OC * IC * C::F * C::F * sizeof(float) : 0;
+    p.workspace_bytes = p.splits > 1 ? p.splits * slice : 0;
     return p;
 }
 

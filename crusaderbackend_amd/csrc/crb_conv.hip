@@ -785,6 +785,8 @@ static bool wgrad_direct(const crb_conv_geom *g, bool run, const float *dY, cons
     return false;
 }
 
+constexpr size_t kStaticScratchBytes = CRB_NOALLOC_SCRATCH_BYTES;  // the buffer built into the library (below)
+
 // ---- weight gradient on split bf16 operands (conv_split_wgrad.h) -----------------------------------------------------------------
 // Configurations <F, S, WM, WN, KG, MAXPX>: 32 x 32 channels and 128 pixels a tile, or 64 x 32 and 64 (wide images in fewer strips,
 // and 4 x 4 images, whose eight padded images do not fit the first's LDS); stride 2: 128 x 32 and 32. A tile of either of the first
@@ -805,13 +807,13 @@ struct SplitWgradSet<3, 2> {
     typedef C0 C1;
 };
 template <int F, int S>
-static SplitWgradChoice split_wgrad_choice_for(const crb_conv_geom *g, float &best_us) {
+static SplitWgradChoice split_wgrad_choice_for(const crb_conv_geom *g, size_t most, float &best_us) {
     typedef SplitWgradSet<F, S> Set;
     SplitWgradChoice best;
     best_us = 3e38f;
     auto consider = [&](int id, auto cfg) {
         typedef decltype(cfg) C;
-        const SplitWgradPlan p = split_wgrad_plan<C>(g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW);
+        const SplitWgradPlan p = split_wgrad_plan<C>(g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, most);
         if (!p.strips || (p.splits > 1 && uint64_t(p.splits) * g->OC * g->IC * F * F > 0x7fffffffull)) return;
         const u32 rows = F / C::ROWS, rounds = ceil_div(p.pairs * p.splits * rows, 256u);
         float us = 5.f + float(rounds * p.tiles_z) * 3.3f * C::NTW / 9.f;
@@ -822,6 +824,7 @@ static SplitWgradChoice split_wgrad_choice_for(const crb_conv_geom *g, float &be
     if constexpr (S == 1) consider(1, typename Set::C1());
     return best;
 }
+static size_t wgrad_scratch_bytes(const crb_conv_geom *g, bool split);
 // cfg < 0: not taken.
 static SplitWgradChoice split_wgrad_choice(const crb_conv_geom *g) {
     const SplitWgradChoice none;
@@ -831,12 +834,23 @@ static SplitWgradChoice split_wgrad_choice(const crb_conv_geom *g) {
     const bool direct = wgrad_direct(g, false, nullptr, nullptr, nullptr, nullptr, nullptr, dp, st);
     const float mflop = 2e-6f * g->N * g->OH * g->OW * g->IC * g->OC * g->FH * g->FW;
     if (direct || mflop < 100.f) return none;  // (width-specialised layers: conv_split_fwd_plan)
-    float us = 0.f;
-    SplitWgradChoice c;
-    if (g->FH == 3 && g->sH == 1) c = split_wgrad_choice_for<3, 1>(g, us);
-    if (g->FH == 5 && g->sH == 1) c = split_wgrad_choice_for<5, 1>(g, us);
-    // (the stride-2 tile is 128 output channels wide: 32 -> 32 @56 batch 32 28 -> 31 us, 64 -> 128 @56 64 -> 51)
-    if (g->FH == 3 && g->sH == 2 && g->OC >= 64) c = split_wgrad_choice_for<3, 2>(g, us);
+    auto choice = [&](size_t most) {
+        float us = 0.f;
+        SplitWgradChoice c;
+        if (g->FH == 3 && g->sH == 1) c = split_wgrad_choice_for<3, 1>(g, most, us);
+        if (g->FH == 5 && g->sH == 1) c = split_wgrad_choice_for<5, 1>(g, most, us);
+        // (the stride-2 tile is 128 output channels wide: 32 -> 32 @56 batch 32 28 -> 31 us, 64 -> 128 @56 64 -> 51)
+        if (g->FH == 3 && g->sH == 2 && g->OC >= 64) c = split_wgrad_choice_for<3, 2>(g, most, us);
+        return c;
+    };
+    SplitWgradChoice c = choice(SIZE_MAX);
+    if (c.cfg >= 0 && c.plan.workspace_bytes) {
+        // Slices take no more than the built-in buffer, or nothing, where those of the fp32 kernel do not: layers whose gradient
+        // can be had without an allocation stay such layers.
+        const size_t fp32 = wgrad_scratch_bytes(g, false);
+        if (!fp32) c = choice(0);
+        else if (c.plan.workspace_bytes > kStaticScratchBytes && fp32 <= kStaticScratchBytes) c = choice(kStaticScratchBytes);
+    }
     return c;
 }
 template <int F, int S>
@@ -1047,7 +1061,6 @@ static BiasGradPlan bias_grad_plan(u32 N, u32 cols, bool vec) {
 // Device memory that exists as long as the code object is loaded: one copy per GPU, at an address of its own on each. In
 // host code the array's name is only a handle for hipGetSymbolAddress; kernels and copies get the address that call
 // returns for the current device.
-constexpr size_t kStaticScratchBytes = CRB_NOALLOC_SCRATCH_BYTES;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 constexpr int kMaxDevices = 64;
 static std::mutex g_static_mu;
@@ -1078,7 +1091,8 @@ static size_t wgrad_scratch_bytes(const crb_conv_geom *g, bool split) {
     }
     if (tiny2x2_shape(g)) return size_t(g->OC) * g->IC * 16 * sizeof(float);  // (oc, p) x (ic, p') product before the tap fold
     if (shortcut_shape(g)) return sc_wgrad_plan(g->N, g->IC, g->OC, g->OH, g->OW).workspace_bytes;
-    if (const SplitWgradChoice c = split_wgrad_choice(g); split && c.cfg >= 0) return c.plan.workspace_bytes;
+    if (split)
+        if (const SplitWgradChoice c = split_wgrad_choice(g); c.cfg >= 0) return c.plan.workspace_bytes;
     {
         WgradDirectPlan dp;
         TiledWgradPlan tp;
@@ -1251,12 +1265,16 @@ int crb_conv_wgrad(const float *dY, const float *X, float *dW, const crb_conv_ge
         }
         return launch_sc_wgrad(dY, X, dW, part, sp, g->N, g->IC, g->OC, g->OH, g->OW, s, "crb_conv_wgrad");
     }
-    // (scratch that holds too little for its slices may still be enough for the kernels below)
-    if (const SplitWgradChoice c = split_wgrad_choice(g);
-        c.cfg >= 0 && (workspace ? workspace_bytes >= c.plan.workspace_bytes : scratch_available(c.plan.workspace_bytes, s))) {
+    if (const SplitWgradChoice c = split_wgrad_choice(g); c.cfg >= 0) {
         float *sws = static_cast<float *>(workspace);
-        if (c.plan.workspace_bytes && !sws)
-            if (int sg = scratch_get(c.plan.workspace_bytes, s, "crb_conv_wgrad", &sws)) return sg;
+        if (c.plan.workspace_bytes) {
+            if (sws) {
+                if (workspace_bytes < c.plan.workspace_bytes)
+                    return fail(CRB_EWORKSPACE, "crb_conv_wgrad: workspace %zu bytes < required %zu", workspace_bytes, c.plan.workspace_bytes);
+            } else if (int sg = scratch_get(c.plan.workspace_bytes, s, "crb_conv_wgrad", &sws)) {
+                return sg;
+            }
+        }
         return run_split_wgrad(c, dY, X, dW, sws, g, s, "crb_conv_wgrad");
     }
     if (aligned16(dY) && aligned16(X)) {
@@ -1319,8 +1337,7 @@ int crb_conv_wgrad(const float *dY, const float *X, float *dW, const crb_conv_ge
 int crb_conv_wgrad_noalloc(const float *dY, const float *X, float *dW, const crb_conv_geom *g, void *stream) {
     if (!dY || !X || !dW) return fail(CRB_ENULL, "crb_conv_wgrad_noalloc: null operand");
     if (int st = check_geom("crb_conv_wgrad_noalloc", g)) return st;
-    size_t need = wgrad_scratch_bytes(g, true);
-    if (need > kStaticScratchBytes) need = wgrad_scratch_bytes(g, false);  // the kernel behind the split one
+    const size_t need = wgrad_scratch_bytes(g, true);
     if (need > kStaticScratchBytes)
         return fail(CRB_EWORKSPACE,
                     "crb_conv_wgrad_noalloc: this geometry needs %zu bytes of scratch, the built-in buffer holds %zu; use "

@@ -217,3 +217,34 @@ def test_operands_down_to_the_smallest_normal_float(dev, shape):
         for what, got, ref, K in (("Y", Y, F_.conv2d(X.double(), Wr, stride=s, padding=p), IC * F * F), ("dX", dX, Xr.grad, OC * F * F),
                                   ("dW", dW, torch.nn.grad.conv2d_weight(Xs.double(), Wt.shape, dY.double(), stride=s, padding=p), N * g.OH * g.OW)):
             assert (got.cpu().double() - ref).norm() <= np.sqrt(K) * 2.0**-24 * ref.norm(), what
+
+
+@pytest.mark.parametrize("shape", [(8, 148, 24, 23, 210, 3, 2, 1), (12, 36, 51, 46, 165, 3, 2, 1), (16, 739, 8, 7, 416, 3, 2, 1), (9, 48, 40, 41, 64, 3, 1, 1)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_the_gradient_that_allocates_nothing_has_the_same_bits(dev, shape):
+    """crb_conv_wgrad on a workspace of the queried size, on the library's arena, on the built-in buffer, and recorded there."""
+    import torch
+    from crusaderbackend_amd import capi
+
+    N, IC, H, W, OC, F, s, p = shape
+    g = capi.ConvGeom.make(N, IC, H, W, OC, F, F, s, s, p, p)
+    X, dY = torch.randn(N, IC, H, W, device=dev), torch.randn(N, OC, g.OH, g.OW, device=dev)
+    need = capi.conv_wgrad_workspace_bytes(g)
+    assert need <= capi.NOALLOC_SCRATCH_BYTES
+    got = [torch.zeros(OC, IC, F, F, device=dev) for _ in range(4)]
+    capi.conv_wgrad(dY, X, got[0], g, workspace=torch.empty(max(need, 4) // 4, device=dev))
+    capi.conv_wgrad(dY, X, got[1], g)
+    capi.conv_wgrad_noalloc(dY, X, got[2], g)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream(device=dev)):
+        capi.conv_wgrad_noalloc(dY, X, got[3], g, stream=torch.cuda.current_stream())
+    for _ in range(3):
+        got[3].zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(got[0], x) for x in got[1:])
+    if need:
+        with pytest.raises(capi.CrbError) as ei:
+            capi.conv_wgrad(dY, X, got[0], g, workspace=torch.empty(need // 8, device=dev))
+        assert ei.value.status == capi.CRB_EWORKSPACE

@@ -17,3 +17,12 @@ def test_width_grid_layers_train_on_the_fp32_kernels(layer):
     filters, slices of the fp32 weight gradient)."""
     IC, H, OC, slices = layer
     assert queries(128, IC, H, H, OC, 3, 1, 1) == (0, 0, slices * OC * IC * 36 if slices > 1 else 0)
+
+
+def test_layers_of_the_built_in_buffer_stay_in_it():
+    """Layers whose fp32 weight gradient takes slices of at most the built-in buffer's size, or none, need no more on split
+    operands: crb_conv_wgrad_noalloc takes them, on the kernel that crb_conv_wgrad takes."""
+    for (N, IC, H, W, OC, F, s, p), fp32 in (((8, 148, 24, 23, 210, 3, 2, 1), 5.34), ((12, 36, 51, 46, 165, 3, 2, 1), 5.92)):
+        assert fp32 < queries(N, IC, H, W, OC, F, s, p)[2] / 2**20 <= 8, "on split operands"
+    for shape in ((16, 739, 8, 7, 416, 3, 2, 1), (1, 544, 28, 27, 443, 3, 2, 1)):
+        assert queries(*shape)[2] == 0
