@@ -833,7 +833,12 @@ static SplitWgradChoice split_wgrad_choice(const crb_conv_geom *g) {
     int st = 0;
     const bool direct = wgrad_direct(g, false, nullptr, nullptr, nullptr, nullptr, nullptr, dp, st);
     const float mflop = 2e-6f * g->N * g->OH * g->OW * g->IC * g->OC * g->FH * g->FW;
-    if (direct || mflop < 100.f) return none;  // (width-specialised layers: conv_split_fwd_plan)
+    if (direct) return none;  // (width-specialised layers: conv_split_fwd_plan)
+    // Against the fp32 kernels behind it on 70 random layers (16 to 512 channels, 5 to 64 wide, 100 MFLOP to 16 GFLOP): 0.91 to 4.5
+    // times as fast, geometric mean 1.6. The ones under 1 were those of under 32 output channels, which leave a part of every block
+    // idle, and 100 to 240 MFLOP (188 -> 28 @27x22 batch 2 22.0 -> 24.1 us, 97 -> 22 @33x31 batch 6 23.8 -> 24.4); from there on even
+    // 18 gain (370 -> 18 @6x11 batch 59, 467 MFLOP, 29.0 -> 24.4).
+    if (mflop < (g->OC < 32 ? 250.f : 100.f)) return none;
     auto choice = [&](size_t most) {
         float us = 0.f;
         SplitWgradChoice c;
