@@ -331,8 +331,10 @@ static int launch_tiled_any(const float *Wt, const float *X, float *Y, const flo
 //   0: 64 x 128, four waves, two workgroups per CU      1: 128 x 64, four waves, two per CU
 //   2: 128 x 64 in two K groups, one per CU             3: 64 x 64 in four K groups, one per CU
 //   4: 32 x 256, four waves, two per CU
-// The choice is the smallest estimate: 6 us for the filters' launch and the workgroups' first and last phases, plus rounds x steps
-// (16 channels of one tap) x a step's rate. Measured at batch 128, 64 -> 64 @32, 128 -> 128 @16, 256 -> 256 @8, 512 -> 512 @4: 0.64 us
+// The choice is the smallest estimate: 6 us for the filters' launch and the workgroups' first and last phases, what splitting the
+// filters and reading the parts back takes (kFilterUs a million elements; by the difference of measured times and the rest of the
+// estimate, 18 layers of 4 to 53 million: 2.9 to 4.2 us for 3x3 filters, 4.2 to 5.2 for 5x5), plus rounds x steps (16 channels of one
+// tap) x a step's rate. Measured at batch 128, 64 -> 64 @32, 128 -> 128 @16, 256 -> 256 @8, 512 -> 512 @4: 0.64 us
 // where a CU holds two of the first two's workgroups, 0.35 where all hold one, 0.34 and 0.19 for the others; on a few dozen CUs
 // (64 -> 64 @20 batch 8, 128 -> 128 @14 batch 8, 256 -> 256 @7 batch 4) 0.17 for the first two. A contraction may be cut into slices
 // on grids that leave CUs idle: one more launch, and the partial results written and read once.
@@ -355,7 +357,7 @@ static ConvSplitPlan conv_split_plan_for(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 
     typedef ConvSplitSet<F, S> Set;
     ConvSplitPlan best;
     best_us = 3e38f;
-    const float count = float(N) * C_OUT * OH * OW;
+    const float count = float(N) * C_OUT * OH * OW, kFilterUs = F == 5 ? 4.8f : 3.4f, wide = kFilterUs * 1e-6f * C_IN * C_OUT * F * F;
     auto consider = [&](int id, auto cfg, float rate, u32 per_cu) {
         typedef decltype(cfg) C;
         const u32 strips = conv_split_strips<C>(OH, OW);
@@ -370,7 +372,7 @@ static ConvSplitPlan conv_split_plan_for(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 
             const u32 rest = u32(wgs % per_round);
             const float alone = per_cu == 1 ? rate : 0.17f + 0.18f * float(rest) / 256.f;
             float us = 6.f + float(cz * C::NT) * (float(wgs / per_round) * rate + (rest == 0 ? 0.f : rest <= 256 ? alone : rate));
-            us = us < 12.f ? 12.f : us;
+            us = (us < 12.f ? 12.f : us) + wide;
             if (z > 1) us += 3.5f + float(2 * z + 1) * count * 4e-6f / 5.f;
             if (us < best_us) {
                 best_us = us;
@@ -392,15 +394,18 @@ static ConvSplitPlan conv_split_plan_for(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 
 static ConvSplitPlan conv_split_plan(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 W, u32 OH, u32 OW, u32 F, u32 S, bool direct, float least) {
     const float mflop = 2e-6f * N * OH * OW * C_IN * C_OUT * F * F;
     if (C_IN < 16 || C_OUT < 24 || mflop < least) return ConvSplitPlan();
+    if (uint64_t(C_IN) * C_OUT * F * F * (2 * kSplit) > (256u << 20)) return ConvSplitPlan();  // (scratch: 256 MiB of split filters)
     ConvSplitPlan p;
     float us = 0.f;
     if (F == 3 && S == 1) p = conv_split_plan_for<3, 1>(N, C_IN, C_OUT, H, W, OH, OW, us);
     if (F == 5 && S == 1) p = conv_split_plan_for<5, 1>(N, C_IN, C_OUT, H, W, OH, OW, us);
     if (F == 3 && S == 2) p = conv_split_plan_for<3, 2>(N, C_IN, C_OUT, H, W, OH, OW, us);
     // against the fp32 kernels: the tiled one's throughput or, on few workgroups, the length of a workgroup's contraction; the
-    // engine's throughput
-    const float k = float(C_IN * F * F);
-    const float fp32_us = tiled_pays(N, C_IN, C_OUT, OH, OW, F * F) ? 3.f + std::max(mflop / 75.f, 0.03f * k) : 10.f + mflop / 45.f;
+    // engine's throughput or, where a few images meet wide filters, the reading of these. There the filters' split does not pay
+    // (fp32 / split, us: 1088 -> 1096 5x5 @4 batch 3 122 / 192, 1122 -> 1874 5x5 @5 batch 4 213 / 348, 1648 -> 2000 @10 batch 1 110 /
+    // 151, 1969 -> 1892 @5 batch 2 142 / 166; but 1143 -> 1163 5x5 @7 batch 6 466 / 317, 869 -> 785 @16 batch 3 274 / 95).
+    const float k = float(C_IN * F * F), engine = std::max(mflop / 60.f, 3.4e-6f * k * C_OUT);
+    const float fp32_us = tiled_pays(N, C_IN, C_OUT, OH, OW, F * F) ? 3.f + std::max(mflop / 68.f, 0.03f * k) : 20.f + engine;
     if (p.cfg >= 0 && !direct && us > fp32_us) p.cfg = -1;
     return p;
 }

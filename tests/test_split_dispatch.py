@@ -33,3 +33,17 @@ def test_short_weight_gradients_of_few_output_channels_stay_on_fp32():
     for shape, slices in (((2, 188, 27, 22, 28, 3, 1, 1), 5), ((51, 113, 7, 7, 26, 3, 1, 1), 10)):
         N, IC, H, W, OC, F, s, p = shape
         assert queries(*shape)[2] == slices * OC * IC * F * F * 4
+
+
+def on_split_operands(query, shape):
+    N, IC, H, W, OC, F, s, p = shape
+    return 6 * OC * IC * F * F <= query < 8 * OC * IC * F * F + (64 << 20)
+
+
+def test_wide_filters_are_split_where_that_pays():
+    """A few small images against wide filters stay on fp32, in the little scratch of those kernels; larger work is split."""
+    for shape in ((3, 1088, 4, 4, 1096, 5, 1, 2), (4, 1122, 5, 5, 1874, 5, 1, 2), (1, 1648, 10, 10, 2000, 3, 1, 1), (1, 1622, 11, 11, 679, 5, 1, 2),
+                  (1, 4096, 7, 7, 4096, 3, 1, 1), (7, 1897, 7, 7, 1166, 3, 2, 1)):
+        assert max(queries(*shape)[:2]) <= 64 << 20, shape
+    for shape in ((6, 1143, 7, 7, 1163, 5, 1, 2), (3, 1335, 15, 15, 429, 3, 1, 1), (3, 869, 16, 17, 785, 3, 1, 1), (5, 1119, 7, 7, 436, 3, 1, 1)):
+        assert all(on_split_operands(q, shape) for q in queries(*shape)[:2]), shape
