@@ -50,6 +50,7 @@ struct ConvSplitArgs {
     u32 px_tiles, oc_tiles, relu;
     u32 chunks_z;    // chunks a slice (blockIdx.z) of the contraction takes; slices write partial results `zstride` floats apart
     size_t zstride;
+    u32 z0, add;     // (PLAIN) the slice that blockIdx.z == 0 takes, and whether it adds to Y
     FastDiv ohw, ow, pitch_d, prow_d, strip_d;  // pixels of a strip, its width, ...
 };
 
@@ -82,7 +83,9 @@ __global__ void __launch_bounds__(256) conv_split_filters_kernel(const float *__
     for (int p = 0; p < kSplit; ++p) *reinterpret_cast<u32x4 *>(dst + p * 1024) = part[p];
 }
 
-template <class C>
+// PLAIN: for calls that no scratch can be had for. The filters are split as they are read, a lane's eight channels of a tap from eight
+// places, and slices of the contraction are launched one after the other, each adding to Y: the same bits, several times the time.
+template <class C, bool PLAIN = false>
 __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) {
     constexpr int TM = C::TM, TN = C::TN, KG = C::KG, NT = C::NT, F = C::F, S = C::S, MAXPX = C::MAXPX, NSET = C::AHEAD + 1;
     __shared__ __attribute__((aligned(16))) unsigned char smem[2 * C::STAGE];
@@ -131,7 +134,7 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
     }
     float reg[C::NP][8];
     const bool ragged = a.C_IN % C::CI != 0;
-    const u32 chunk0 = blockIdx.z * a.chunks_z, chunk1 = chunk0 + a.chunks_z < a.chunks ? chunk0 + a.chunks_z : a.chunks;
+    const u32 chunk0 = (blockIdx.z + (PLAIN ? a.z0 : 0u)) * a.chunks_z, chunk1 = chunk0 + a.chunks_z < a.chunks ? chunk0 + a.chunks_z : a.chunks;
     auto fetch = [&](u32 chunk) {
         const u32 c0 = chunk * C::CI;
         if (ragged && chunk + 1 == a.chunks) {
@@ -166,7 +169,28 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
     for (int mi = 0; mi < TM; ++mi)
         wp[mi] = a.Wf + ((size_t(ot * (TM * C::WM) + wave_m * TM + mi) * KG + kgroup) * steps + chunk0 * NT) * (kSplit * 1024);
     bf16x8 fa[NSET][kSplit][TM];
+    u32 plain_step = chunk0 * NT;
     auto load_filters = [&](int set) {  // the next step's fragments
+        if constexpr (PLAIN) {
+            const u32 tap = plain_step % NT, ic0 = (plain_step / NT) * C::CI + 16 * kgroup + 8 * h;
+#pragma unroll
+            for (int mi = 0; mi < TM; ++mi) {
+                const u32 oc = ot * C::OCT + wave_m * (32 * TM) + mi * 32 + i32;
+                float w[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const bool ok = oc < a.C_OUT && ic0 + j < a.C_IN;
+                    const float v = a.Wt[ok ? size_t(oc) * a.w_oc + size_t(ic0 + j) * a.w_ic + (a.mirrored ? NT - 1 - tap : tap) : 0];
+                    w[j] = ok ? v : 0.f;
+                }
+                u32x4 part[kSplit];
+                split8(w, part);
+#pragma unroll
+                for (int p = 0; p < kSplit; ++p) fa[set][p][mi] = __builtin_bit_cast(bf16x8, part[p]);
+            }
+            ++plain_step;
+            return;
+        }
 #pragma unroll
         for (int mi = 0; mi < TM; ++mi) {
 #pragma unroll
@@ -351,7 +375,11 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
             const u32 oc = oc0 + 8 * (r / 4) + (r % 4);
-            float o = res[r] + b[r];
+            float o = res[r];
+            if constexpr (PLAIN) {
+                if (a.add && oc < a.C_OUT) o = y[size_t(oc) * a.OHW] + o;
+            }
+            o += b[r];
             if (a.relu) o = o > 0.f ? o : 0.f;
             if (oc < a.C_OUT) y[size_t(oc) * a.OHW] = o;
         }
@@ -431,7 +459,7 @@ inline size_t conv_split_filter_bytes(u32 C_IN, u32 C_OUT) {
     return (blocks * C::KG * chunks * C::NT + C::AHEAD) * kSplit * 1024;
 }
 
-// Wf: conv_split_filter_bytes of scratch. (OH, OW): extent of the result, (H, W): of X; window origin (-pad_y, -pad_x); strips:
+// Wf: conv_split_filter_bytes of scratch, or null (PLAIN). (OH, OW): extent of the result, (H, W): of X; window origin (-pad_y, -pad_x); strips:
 // conv_split_strips. slices > 1: the contraction is cut; partial results go to `part` (slices x the result) and are summed in
 // fixed order by one more launch, which applies bias and ReLU.
 template <class C, bool DGRAD>
@@ -453,12 +481,22 @@ inline int launch_conv_split(const float *Wt, const float *X, float *Y, const fl
     const uint64_t tiles = uint64_t(a.px_tiles) * a.oc_tiles;
     if (tiles > 0x7fffffffull) return fail(CRB_EINVAL_SHAPE, "%s: launch grid too large", what);
     const u32 total = a.oc_tiles * (C::OCT / 32) * C::KG * a.chunks * C::NT * 64;
+    if (!Wf) {
+        a.Y = Y, a.zstride = 0;
+        for (u32 z = 0; z < slices; ++z) {
+            a.z0 = z, a.add = z > 0;
+            if (z + 1 == slices) a.bias = bias, a.relu = relu;
+            hipLaunchKernelGGL((conv_split_kernel<C, true>), dim3(u32(tiles)), dim3(C::NTH), 0, s, a);
+            if (int st = check_launch(what)) return st;
+        }
+        return CRB_OK;
+    }
     hipLaunchKernelGGL(conv_split_filters_kernel<DGRAD>, dim3(ceil_div(total, 256u)), dim3(256), 0, s, Wt, Wf, C_IN, C_OUT, u32(C::NT), a.chunks,
                        u32(C::KG), total);
     if (int st = check_launch(what)) return st;
     hipLaunchKernelGGL((conv_split_kernel<C>), dim3(u32(tiles), 1, slices), dim3(C::NTH), 0, s, a);
     int st = check_launch(what);
-    if (st == CRB_OK && slices > 1) st = launch_splitk_reduce(part, Y, count, slices, ReduceEpi{bias, OH * OW, C_OUT, relu ? u32(EPI_RELU) : 0u}, s, what);
+    if (st == CRB_OK && slices > 1) st = launch_ordered_reduce(part, Y, count, slices, ReduceEpi{bias, OH * OW, C_OUT, relu ? u32(EPI_RELU) : 0u}, s, what);
     return st;
 }
 

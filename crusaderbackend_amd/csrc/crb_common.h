@@ -29,9 +29,20 @@ inline int scratch_get(size_t bytes, hipStream_t stream, const char *what, T **o
     *out = static_cast<T *>(p);
     return st;
 }
-// Whether scratch_get would serve such a request (taking that its hipMalloc succeeds): a kernel that wants scratch yields to one
-// that needs less where a scope or bound workspace is too small for it, or a capture forbids growth.
+// Whether scratch_get would serve such a request (taking that its hipMalloc succeeds); scratch_get without an error text, null if refused.
 bool scratch_available(size_t bytes, hipStream_t stream);
+void *scratch_try(size_t bytes, hipStream_t stream);
+// scratch_get for a call that can do without, more slowly: *out is null where the scratch cannot be had. Refused where not even the
+// instead() bytes could be had that the call would take on the fp32 kernel for it.
+template <class T, class F>
+inline int scratch_get_or_none(size_t bytes, F instead, hipStream_t stream, const char *what, T **out) {
+    *out = nullptr;
+    if (scratch_available(bytes, stream)) {
+        *out = static_cast<T *>(scratch_try(bytes, stream));
+        return CRB_OK;
+    }
+    return scratch_available(instead(), stream) ? CRB_OK : scratch_get(bytes, stream, what, out);
+}
 int scratch_bind(void *ptr, size_t bytes, hipStream_t stream);
 void arena_release();
 // While alive, every scratch_get of this thread is served from [ptr, ptr + bytes) or refused; nothing is allocated.

@@ -446,7 +446,7 @@ template <int F, int S, bool DG>
 static int run_conv_split_set(const ConvSplitPlan &p, const float *Wt, const float *X, float *Y, const float *bias, unsigned char *wf, u32 N, u32 C_IN,
                               u32 C_OUT, u32 H, u32 W, u32 OH, u32 OW, int pad_y, int pad_x, u32 relu, hipStream_t s, const char *what) {
     typedef ConvSplitSet<F, S> Set;
-    float *part = reinterpret_cast<float *>(wf + p.filter_bytes);
+    float *part = wf ? reinterpret_cast<float *>(wf + p.filter_bytes) : nullptr;
     switch (p.cfg) {
         case 0: return launch_conv_split<typename Set::C0, DG>(Wt, X, Y, bias, wf, N, C_IN, C_OUT, H, W, OH, OW, p.strips, p.slices, part, pad_y, pad_x, relu, s, what);
         case 1: return launch_conv_split<typename Set::C1, DG>(Wt, X, Y, bias, wf, N, C_IN, C_OUT, H, W, OH, OW, p.strips, p.slices, part, pad_y, pad_x, relu, s, what);
@@ -455,19 +455,21 @@ static int run_conv_split_set(const ConvSplitPlan &p, const float *Wt, const flo
         default: return launch_conv_split<typename Set::C3, DG>(Wt, X, Y, bias, wf, N, C_IN, C_OUT, H, W, OH, OW, p.strips, p.slices, part, pad_y, pad_x, relu, s, what);
     }
 }
+static size_t fwd_scratch_bytes(const crb_conv_geom *g, bool aligned, bool split);
+static size_t dgrad_scratch_bytes(const crb_conv_geom *g, bool aligned, bool split);
 static int run_conv_split_fwd(const ConvSplitPlan &p, const float *W, const float *X, float *Y, const float *bias, const crb_conv_geom *g, u32 relu,
-                              hipStream_t s, const char *what) {
+                              bool aligned, hipStream_t s, const char *what) {
     unsigned char *wf = nullptr;
-    if (int st = scratch_get(p.bytes, s, what, &wf)) return st;
+    if (int st = scratch_get_or_none(p.bytes, [&] { return fwd_scratch_bytes(g, aligned, false); }, s, what, &wf)) return st;
     const int py = int(g->pH), px = int(g->pW);
     if (g->sH == 2) return run_conv_split_set<3, 2, false>(p, W, X, Y, bias, wf, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, py, px, relu, s, what);
     if (g->FH == 5) return run_conv_split_set<5, 1, false>(p, W, X, Y, bias, wf, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, py, px, relu, s, what);
     return run_conv_split_set<3, 1, false>(p, W, X, Y, bias, wf, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, py, px, relu, s, what);
 }
-static int run_conv_split_dgrad(const ConvSplitPlan &p, const float *W, const float *dY, float *dX, const crb_conv_geom *g, hipStream_t s,
-                                const char *what) {
+static int run_conv_split_dgrad(const ConvSplitPlan &p, const float *W, const float *dY, float *dX, const crb_conv_geom *g, bool aligned,
+                                hipStream_t s, const char *what) {
     unsigned char *wf = nullptr;
-    if (int st = scratch_get(p.bytes, s, what, &wf)) return st;
+    if (int st = scratch_get_or_none(p.bytes, [&] { return dgrad_scratch_bytes(g, aligned, false); }, s, what, &wf)) return st;
     const int py = int(g->FH) - 1 - int(g->pH), px = int(g->FW) - 1 - int(g->pW);
     if (g->FH == 5) return run_conv_split_set<5, 1, true>(p, W, dY, dX, nullptr, wf, g->N, g->OC, g->IC, g->OH, g->OW, g->IH, g->IW, py, px, 0, s, what);
     return run_conv_split_set<3, 1, true>(p, W, dY, dX, nullptr, wf, g->N, g->OC, g->IC, g->OH, g->OW, g->IH, g->IW, py, px, 0, s, what);
@@ -1114,6 +1116,53 @@ static size_t wgrad_scratch_bytes(const crb_conv_geom *g, bool split) {
     return p.splits > 1 ? size_t(p.splits) * p.M * p.Ncols * sizeof(float) : 0;
 }
 
+// Scratch of crb_conv_fwd and crb_conv_dgrad; split: where the kernels on split operands may be taken.
+static size_t fwd_scratch_bytes(const crb_conv_geom *g, bool aligned, bool split) {
+    bool done = false;
+    if (pointwise_shape(g) && aligned) {
+        try_pointwise<false>(nullptr, nullptr, nullptr, nullptr, g->N, g->IC, g->OC, g->OH, g->OW, 0, nullptr, "", done, true);
+        if (done) return 0;
+    }
+    if (pointwise_shape(g)) return gemm_scratch_bytes(g->OC, g->IH * g->IW, g->IC, g->N);
+    if (split && !tiny2x2_shape(g))
+        if (const ConvSplitPlan p = conv_split_fwd_plan(g, aligned); p.cfg >= 0) return p.bytes;
+    if (tiny2x2_shape(g) && aligned) return gemm_scratch_bytes(g->N, g->OC * 4, g->IC * 4, 1, false);
+    if (aligned && (direct_shape(g, 1) || direct_shape(g, 2))) {
+        if (g->sH == 1)
+            try_direct<false, 1>(nullptr, nullptr, nullptr, nullptr, g->N, g->IC, g->OC, g->OH, g->OW, g->IH, 0, nullptr, "", done, true);
+        else
+            try_direct<false, 2>(nullptr, nullptr, nullptr, nullptr, g->N, g->IC, g->OC, g->OH, g->OW, g->IH, 0, nullptr, "", done, true);
+        if (done) return 0;
+    }
+    if (((tiled_s1_shape(g, 3) || tiled_s1_shape(g, 5) || tiled_s2_shape(g)) && tiled_pays(g->N, g->IC, g->OC, g->OH, g->OW, g->FH * g->FW)))
+        return 0;  // the tiled kernel
+    return nchw_scratch_bytes(g->OC, g->N * g->OH * g->OW, g->IC * g->FH * g->FW);
+}
+static size_t dgrad_scratch_bytes(const crb_conv_geom *g, bool aligned, bool split) {
+    bool done = false;
+    if (pointwise_shape(g) && aligned) {
+        try_pointwise<true>(nullptr, nullptr, nullptr, nullptr, g->N, g->OC, g->IC, g->OH, g->OW, 0, nullptr, "", done, true);
+        if (done) return 0;
+    }
+    if (pointwise_shape(g)) return gemm_scratch_bytes(g->IC, g->IH * g->IW, g->OC, g->N);
+    if (split && !tiny2x2_shape(g))
+        if (const ConvSplitPlan p = conv_split_dgrad_plan(g, aligned); p.cfg >= 0) return p.bytes;
+    if (tiny2x2_shape(g) && aligned) return gemm_scratch_bytes(g->N, g->IC * 4, g->OC * 4, 1, false);
+    if (aligned && (direct_shape(g, 1) || direct_shape(g, 2))) {
+        if (g->sH == 1)
+            try_direct<true, 1>(nullptr, nullptr, nullptr, nullptr, g->N, g->OC, g->IC, g->OH, g->OW, g->OH, 0, nullptr, "", done, true);
+        else
+            try_direct<true, 2>(nullptr, nullptr, nullptr, nullptr, g->N, g->OC, g->IC, g->OH, g->OW, g->OH, 0, nullptr, "", done, true);
+        if (done) return 0;
+    }
+    if (shortcut_shape(g) && aligned) return 0;
+    if ((tiled_s1_shape(g, 3) || tiled_s1_shape(g, 5)) && tiled_pays(g->N, g->OC, g->IC, g->IH, g->IW, g->FH * g->FW))
+        return 0;  // the tiled kernel
+    if (tiled_classes_pay(g)) return 0;                              // one tiled launch per residue class
+    if ((g->sH > 1 || g->sW > 1) && dgrad_classes_pay(g)) return 0;  // one launch per residue class, none of them cut
+    return nchw_scratch_bytes(g->IC, g->N * g->IH * g->IW, g->OC * g->FH * g->FW);
+}
+
 }  // namespace crb
 
 using namespace crb;
@@ -1138,8 +1187,8 @@ int crb_conv_fwd(const float *W, const float *X, float *Y, const float *bias_or_
     if (pointwise_shape(g))
         return gemm_nn_rowbias(W, X, Y, g->OC, g->IH * g->IW, g->IC, g->N, bias_or_null,
                                (flags & CRB_FLAG_RELU) ? u32(EPI_RELU) : 0u, s, "crb_conv_fwd");
-    if (const ConvSplitPlan p = conv_split_fwd_plan(g, aligned16(X) && aligned16(Y)); p.cfg >= 0 && !tiny2x2_shape(g) && scratch_available(p.bytes, s))
-        return run_conv_split_fwd(p, W, X, Y, bias_or_null, g, flags & CRB_FLAG_RELU, s, "crb_conv_fwd");
+    if (const ConvSplitPlan p = conv_split_fwd_plan(g, aligned16(X) && aligned16(Y)); p.cfg >= 0 && !tiny2x2_shape(g))
+        return run_conv_split_fwd(p, W, X, Y, bias_or_null, g, flags & CRB_FLAG_RELU, aligned16(X) && aligned16(Y), s, "crb_conv_fwd");
     if (tiny2x2_shape(g) && aligned16(X) && aligned16(Y))
         return conv2x2_fwd(W, X, Y, bias_or_null, g->N, g->IC, g->OC, (flags & CRB_FLAG_RELU) ? u32(EPI_RELU) : 0u, s, "crb_conv_fwd");
     if (aligned16(X) && aligned16(Y) && (direct_shape(g, 1) || direct_shape(g, 2))) {
@@ -1180,8 +1229,8 @@ int crb_conv_dgrad(const float *W, const float *dY, float *dX, const crb_conv_ge
     if (pointwise_shape(g))
         return gemm_tn_batched(W, dY, dX, g->IC, g->IH * g->IW, g->OC, g->N, hipStream_t(stream), "crb_conv_dgrad");
     if (const ConvSplitPlan p = conv_split_dgrad_plan(g, aligned16(dY) && aligned16(dX));
-        p.cfg >= 0 && !tiny2x2_shape(g) && scratch_available(p.bytes, hipStream_t(stream)))
-        return run_conv_split_dgrad(p, W, dY, dX, g, hipStream_t(stream), "crb_conv_dgrad");
+        p.cfg >= 0 && !tiny2x2_shape(g))
+        return run_conv_split_dgrad(p, W, dY, dX, g, aligned16(dY) && aligned16(dX), hipStream_t(stream), "crb_conv_dgrad");
     if (tiny2x2_shape(g) && aligned16(dY) && aligned16(dX))
         return conv2x2_dgrad(W, dY, dX, g->N, g->IC, g->OC, hipStream_t(stream), "crb_conv_dgrad");
     if (aligned16(dY) && aligned16(dX) && (direct_shape(g, 1) || direct_shape(g, 2))) {
@@ -1362,49 +1411,12 @@ int crb_conv_wgrad_noalloc(const float *dY, const float *X, float *dW, const crb
 
 size_t crb_conv_fwd_workspace_bytes(const crb_conv_geom *g, int operands_aligned16) {
     if (check_geom("crb_conv_fwd_workspace_bytes", g)) return 0;
-    bool done = false;
-    if (pointwise_shape(g) && operands_aligned16) {
-        try_pointwise<false>(nullptr, nullptr, nullptr, nullptr, g->N, g->IC, g->OC, g->OH, g->OW, 0, nullptr, "", done, true);
-        if (done) return 0;
-    }
-    if (pointwise_shape(g)) return gemm_scratch_bytes(g->OC, g->IH * g->IW, g->IC, g->N);
-    if (const ConvSplitPlan p = conv_split_fwd_plan(g, operands_aligned16 != 0); p.cfg >= 0 && !tiny2x2_shape(g)) return p.bytes;
-    if (tiny2x2_shape(g) && operands_aligned16) return gemm_scratch_bytes(g->N, g->OC * 4, g->IC * 4, 1, false);
-    if (operands_aligned16 && (direct_shape(g, 1) || direct_shape(g, 2))) {
-        if (g->sH == 1)
-            try_direct<false, 1>(nullptr, nullptr, nullptr, nullptr, g->N, g->IC, g->OC, g->OH, g->OW, g->IH, 0, nullptr, "", done, true);
-        else
-            try_direct<false, 2>(nullptr, nullptr, nullptr, nullptr, g->N, g->IC, g->OC, g->OH, g->OW, g->IH, 0, nullptr, "", done, true);
-        if (done) return 0;
-    }
-    if (((tiled_s1_shape(g, 3) || tiled_s1_shape(g, 5) || tiled_s2_shape(g)) && tiled_pays(g->N, g->IC, g->OC, g->OH, g->OW, g->FH * g->FW)))
-        return 0;  // the tiled kernel
-    return nchw_scratch_bytes(g->OC, g->N * g->OH * g->OW, g->IC * g->FH * g->FW);
+    return fwd_scratch_bytes(g, operands_aligned16 != 0, true);
 }
 
 size_t crb_conv_dgrad_workspace_bytes(const crb_conv_geom *g, int operands_aligned16) {
     if (check_geom("crb_conv_dgrad_workspace_bytes", g)) return 0;
-    bool done = false;
-    if (pointwise_shape(g) && operands_aligned16) {
-        try_pointwise<true>(nullptr, nullptr, nullptr, nullptr, g->N, g->OC, g->IC, g->OH, g->OW, 0, nullptr, "", done, true);
-        if (done) return 0;
-    }
-    if (pointwise_shape(g)) return gemm_scratch_bytes(g->IC, g->IH * g->IW, g->OC, g->N);
-    if (const ConvSplitPlan p = conv_split_dgrad_plan(g, operands_aligned16 != 0); p.cfg >= 0 && !tiny2x2_shape(g)) return p.bytes;
-    if (tiny2x2_shape(g) && operands_aligned16) return gemm_scratch_bytes(g->N, g->IC * 4, g->OC * 4, 1, false);
-    if (operands_aligned16 && (direct_shape(g, 1) || direct_shape(g, 2))) {
-        if (g->sH == 1)
-            try_direct<true, 1>(nullptr, nullptr, nullptr, nullptr, g->N, g->OC, g->IC, g->OH, g->OW, g->OH, 0, nullptr, "", done, true);
-        else
-            try_direct<true, 2>(nullptr, nullptr, nullptr, nullptr, g->N, g->OC, g->IC, g->OH, g->OW, g->OH, 0, nullptr, "", done, true);
-        if (done) return 0;
-    }
-    if (shortcut_shape(g) && operands_aligned16) return 0;
-    if ((tiled_s1_shape(g, 3) || tiled_s1_shape(g, 5)) && tiled_pays(g->N, g->OC, g->IC, g->IH, g->IW, g->FH * g->FW))
-        return 0;  // the tiled kernel
-    if (tiled_classes_pay(g)) return 0;                              // one tiled launch per residue class
-    if ((g->sH > 1 || g->sW > 1) && dgrad_classes_pay(g)) return 0;  // one launch per residue class, none of them cut
-    return nchw_scratch_bytes(g->IC, g->N * g->IH * g->IW, g->OC * g->FH * g->FW);
+    return dgrad_scratch_bytes(g, operands_aligned16 != 0, true);
 }
 
 int crb_conv_bwd(const float *W, const float *dY, const float *X, float *dX, float *dW, const crb_conv_geom *g, void *workspace,

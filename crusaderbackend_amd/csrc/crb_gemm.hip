@@ -111,6 +111,20 @@ static int run_tiles(const AOp &a, const BOp &b, const E &e, u32 M, u32 N, u32 K
     }
 }
 
+// Scratch bytes of the fp32 engine's slices (0: the contraction is not cut).
+static size_t engine_scratch_bytes(u32 M, u32 N, u32 K, u32 zdim) {
+    const GemmChoice c = choose_tiles(M, N, K, zdim, true);
+    SplitPlan sp;
+    switch (c.tile) {
+        case TILE_LARGE: sp = split_for<CfgLarge>(M, N, K, zdim, c.want_splits, true); break;
+        case TILE_SMALL_DEEP: sp = split_for<CfgSmallDeep>(M, N, K, zdim, c.want_splits, true); break;
+        case TILE_SMALL_DEEP8: sp = split_for<CfgSmallDeep8>(M, N, K, zdim, c.want_splits, true); break;
+        case TILE_SMALL_AHEAD: sp = split_for<CfgSmallAhead>(M, N, K, zdim, c.want_splits, true); break;
+        default: sp = split_for<CfgSmall>(M, N, K, zdim, c.want_splits, true); break;
+    }
+    return sp.splits > 1 ? size_t(sp.splits) * M * N * sizeof(float) : 0;
+}
+
 // ---- products of plain matrices on the split engine (igemm_split.h) -----------------------------------------------------------
 // Eight-wave workgroups, one to a CU, so the time goes by rounds of 256 tiles; a round costs its contraction times the tile's
 // rate plus what every launch pays. Measured (NN; us per round and k, us besides): 256 x 256 tiles 0.150 and 16 (4096^3 631 us,
@@ -160,23 +174,26 @@ static SplitChoice choose_split(u32 M, u32 N, u32 K, u32 zdim) {
 // ahead (fp32 / split, us: 700 x 600 x 100 7.8 / 10.8, 64 x 64 x 4096 8.6 / 10.4, 8 products of 16 x 528 x 41 5.5 / 6.1; above:
 // 528 x 2068 x 137 12.5 / 11.8, 768^3 19.4 / 15.6, 2000 x 2000 x 300 32.9 / 26.0).
 static bool split_pays(u32 M, u32 N, u32 K, u32 zdim) { return uint64_t(M) * N * K * zdim >= (uint64_t(1) << 28); }
-// ... and, where the contraction is cut, the slices' scratch can be had; the fp32 engine, which asks for less or refuses, otherwise.
-static bool takes_split(u32 M, u32 N, u32 K, u32 zdim, hipStream_t s) {
-    if (!split_pays(M, N, K, zdim)) return false;
-    const SplitChoice c = choose_split(M, N, K, zdim);
-    return c.splits == 1 || scratch_available(size_t(c.splits) * M * N * sizeof(float), s);
-}
 
 template <class Cfg, class AOp, class BOp, class E>
 static int run_split_cfg(const AOp &a, const BOp &b, const E &e, u32 M, u32 N, u32 K, u32 zdim, const SplitChoice &c, hipStream_t s,
                          const char *what) {
     if (c.splits == 1) return launch_split<Cfg>(a, b, e, M, N, K, zdim, 0, s, what);
     float *ws = nullptr;
-    if (int st = scratch_get(size_t(c.splits) * M * N * sizeof(float), s, what, &ws)) return st;
-    RowMajorEpi pe{ws, nullptr, N, M * N, 0u};
-    if (int st = launch_split<Cfg>(a, b, pe, M, N, K, c.splits, c.k_per_z, s, what)) return st;
-    const ReduceEpi re = e.row_bias ? ReduceEpi{e.row_bias, N, M, e.flags} : ReduceEpi{e.col_bias, 1, N, e.flags};
-    return launch_splitk_reduce(ws, e.C, M * N, c.splits, re, s, what);
+    if (int st = scratch_get_or_none(size_t(c.splits) * M * N * sizeof(float), [&] { return engine_scratch_bytes(M, N, K, zdim); }, s, what, &ws)) return st;
+    if (ws) {
+        RowMajorEpi pe{ws, nullptr, N, M * N, 0u};
+        if (int st = launch_split<Cfg>(a, b, pe, M, N, K, c.splits, c.k_per_z, s, what)) return st;
+        const ReduceEpi re = e.row_bias ? ReduceEpi{e.row_bias, N, M, e.flags} : ReduceEpi{e.col_bias, 1, N, e.flags};
+        return launch_ordered_reduce(ws, e.C, M * N, c.splits, re, s, what);
+    }
+    // no scratch to be had: one slice after the other, added to C in the order of the reduction (the same bits)
+    for (u32 z = 0; z < c.splits; ++z) {
+        RowMajorEpi pe{e.C, nullptr, N, 0u, z ? u32(EPI_ACCUM) : e.flags & u32(EPI_ACCUM)};
+        if (z + 1 == c.splits) pe.col_bias = e.col_bias, pe.row_bias = e.row_bias, pe.flags |= e.flags;
+        if (int st = launch_split<Cfg>(a, b, pe, M, N, K, 1, c.k_per_z, s, what, z)) return st;
+    }
+    return CRB_OK;
 }
 // C (M x N, dense rows) = A * B with the epilogue `e`. rowsum_done: whether e's row sums of A were formed along the way.
 template <class AOp, class BOp, class E>
@@ -206,16 +223,7 @@ size_t gemm_scratch_bytes(u32 M, u32 N, u32 K, u32 zdim, bool one_launch_form) {
             // (a K-concatenated batch whose entries are no multiple of 8 long stays on the fp32 engine, which the query cannot see)
         }
     }
-    const GemmChoice c = choose_tiles(M, N, K, zdim, true);
-    SplitPlan sp;
-    switch (c.tile) {
-        case TILE_LARGE: sp = split_for<CfgLarge>(M, N, K, zdim, c.want_splits, true); break;
-        case TILE_SMALL_DEEP: sp = split_for<CfgSmallDeep>(M, N, K, zdim, c.want_splits, true); break;
-        case TILE_SMALL_DEEP8: sp = split_for<CfgSmallDeep8>(M, N, K, zdim, c.want_splits, true); break;
-        case TILE_SMALL_AHEAD: sp = split_for<CfgSmallAhead>(M, N, K, zdim, c.want_splits, true); break;
-        default: sp = split_for<CfgSmall>(M, N, K, zdim, c.want_splits, true); break;
-    }
-    const size_t eng = sp.splits > 1 ? size_t(sp.splits) * M * N * sizeof(float) : 0;
+    const size_t eng = engine_scratch_bytes(M, N, K, zdim);
     return need > eng ? need : eng;
 }
 
@@ -263,7 +271,7 @@ static int gemm_nn(const float *A, const float *B, float *C, u32 M, u32 N, u32 K
         return launch_tiny_gemm(TinyGemmArgs{A, B, C, col_bias, row_bias, M, N, K, K, 1, N, 1, N, flags}, K, 0, 0, s, what);
     RowMajorEpi e{C, col_bias, N, M * N, flags};
     e.row_bias = row_bias;
-    if (takes_split(M, N, K, batch, s)) return run_split(SMatK<>{A, M, K, 0}, SMatR{B, N, N, K * N}, e, M, N, K, batch, s, what);
+    if (split_pays(M, N, K, batch)) return run_split(SMatK<>{A, M, K, 0}, SMatR{B, N, N, K * N}, e, M, N, K, batch, s, what);
     if (K % 4 == 0 && N % 4 == 0 && aligned16(A) && aligned16(B))
         return run_tiles(MatK<true>{A, M, K, 0}, MatR<true>{B, N, N, K * N}, e, M, N, K, batch, s, what);
     return run_tiles(MatK<false>{A, M, K, 0}, MatR<false>{B, N, N, K * N}, e, M, N, K, batch, s, what);
@@ -282,7 +290,7 @@ static int gemm_tn(const float *A, const float *B, float *C, u32 M, u32 N, u32 K
     RowMajorAccEpi ea;  // the dense layers' weight gradient
     static_cast<RowMajorEpi &>(ea) = e;
     ea.a_rowsum = a_rowsum;
-    if (takes_split(M, N, K, batch, s)) {
+    if (split_pays(M, N, K, batch)) {
         const SMatR a{A, M, M, 0}, b{B, N, N, K * N};
         if (flags & EPI_ACCUM) return run_split(a, b, ea, M, N, K, batch, s, what, rowsum_done);
         return run_split(a, b, e, M, N, K, batch, s, what);
@@ -300,7 +308,7 @@ static int gemm_nt(const float *A, const float *B, float *C, u32 M, u32 N, u32 K
     if (tiny_gemm_fits(M, N, K, 1, true))  // A (M x K) row-major, B stored N x K
         return launch_tiny_gemm(TinyGemmArgs{A, B, C, col_bias, nullptr, M, N, K, K, 1, 1, K, N, flags}, K, 0, 0, s, what);
     RowMajorEpi e{C, col_bias, N, 0, flags};
-    if (takes_split(M, N, K, 1, s)) return run_split(SMatK<>{A, M, K, 0}, SMatK<>{B, N, K, 0}, e, M, N, K, 1, s, what);
+    if (split_pays(M, N, K, 1)) return run_split(SMatK<>{A, M, K, 0}, SMatK<>{B, N, K, 0}, e, M, N, K, 1, s, what);
     if (K % 4 == 0 && aligned16(A) && aligned16(B)) return run_tiles(MatK<true>{A, M, K, 0}, MatK<true>{B, N, K, 0}, e, M, N, K, 1, s, what);
     return run_tiles(MatK<false>{A, M, K, 0}, MatK<false>{B, N, K, 0}, e, M, N, K, 1, s, what);
 }
@@ -413,7 +421,7 @@ int crb_sgemm_nta(const float *A, const float *B, float *C, uint32_t M, uint32_t
     hipStream_t s = hipStream_t(stream);
     if (tiny_gemm_fits(M, N, KK, 1))  // the batch concatenated along the contraction
         return launch_tiny_gemm(TinyGemmArgs{A, B, C, nullptr, nullptr, M, N, KK, K, 1, 1, K, N, EPI_ACCUM}, K, M * K, N * K, s, "crb_sgemm_nta");
-    if (K % 8 == 0 && takes_split(M, N, KK, 1, s)) {  // octets of the contraction stay inside a batch entry
+    if (K % 8 == 0 && split_pays(M, N, KK, 1)) {  // octets of the contraction stay inside a batch entry
         const SMatK<true> a{A, M, K, 0, M * K, FastDiv(K)}, b{B, N, K, 0, N * K, FastDiv(K)};
         return run_split(a, b, e, M, N, KK, 1, s, "crb_sgemm_nta");
     }

@@ -2,6 +2,7 @@
 // lazily grown device scratch arenas used for split-K partial sums.
 #include <cstdarg>
 #include <cstdio>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -121,6 +122,14 @@ int scratch_get(size_t bytes, hipStream_t stream, const char *what, void **out) 
     a.bytes = want;
     *out = p;
     return CRB_OK;
+}
+
+void *scratch_try(size_t bytes, hipStream_t stream) {
+    char before[sizeof(g_err)];
+    memcpy(before, g_err, sizeof(g_err));
+    void *p = nullptr;
+    if (scratch_get(bytes, stream, "", &p)) memcpy(g_err, before, sizeof(g_err));
+    return p;
 }
 
 int scratch_bind(void *ptr, size_t bytes, hipStream_t stream) {

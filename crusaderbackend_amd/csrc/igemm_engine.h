@@ -43,6 +43,7 @@ struct IgemmDims {
     u32 tiles_m, tiles_n;
     u32 k_per_z;  // K range handled per blockIdx.z when split_k != 0 (multiple of BK)
     u32 split_k;  // 0: blockIdx.z is a batch index; 1: blockIdx.z is a K-split index
+    u32 z0 = 0;   // (split engine) K-split index of blockIdx.z == 0
 };
 
 // PF_: how many K slabs ahead of the MFMAs the global loads run (1: the next slab's loads have one slab of MFMAs to
@@ -659,6 +660,45 @@ inline int launch_splitk_reduce(const float *partial, float *C, u32 count, u32 s
         hipLaunchKernelGGL(splitk_reduce_kernel<16>, dim3(ceil_div(count, 16)), dim3(256), 0, s, partial, C, count, splits, e, bdiv);
     else
         hipLaunchKernelGGL(splitk_reduce_kernel<8>, dim3(ceil_div(count, 8)), dim3(256), 0, s, partial, C, count, splits, e, bdiv);
+    return check_launch(what);
+}
+
+// C[i] (+)= sum over z of partial[z][i], left to right, then bias and ReLU: what launches of one slice after the other, each adding
+// to C, come to. For few slices of large results: a thread takes V neighbouring results, four slices requested at a time.
+template <int V>
+static __global__ void __launch_bounds__(256) ordered_reduce_kernel(const float *__restrict__ partial, float *__restrict__ C, u32 count, u32 splits,
+                                                                    ReduceEpi e, FastDiv bdiv) {
+    const u32 i = (blockIdx.x * 256 + threadIdx.x) * V;
+    if (i >= count) return;
+    typedef float vec __attribute__((ext_vector_type(V)));
+    const float *p = partial + i;
+    vec r = *reinterpret_cast<const vec *>(p);
+    if (e.flags & EPI_ACCUM) r = *reinterpret_cast<const vec *>(C + i) + r;
+    u32 z = 1;
+    for (; z + 3 < splits; z += 4) {
+        vec v[4];
+#pragma unroll
+        for (u32 q = 0; q < 4; ++q) v[q] = *reinterpret_cast<const vec *>(p + size_t(z + q) * count);
+#pragma unroll
+        for (u32 q = 0; q < 4; ++q) r += v[q];
+    }
+    for (; z < splits; ++z) r += *reinterpret_cast<const vec *>(p + size_t(z) * count);
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        float o = r[j];
+        if (e.bias) o += e.bias[bdiv.div(i + j) % e.bias_mod];
+        if (e.flags & EPI_RELU) o = o > 0.f ? o : 0.f;
+        r[j] = o;
+    }
+    *reinterpret_cast<vec *>(C + i) = r;
+}
+inline int launch_ordered_reduce(const float *partial, float *C, u32 count, u32 splits, ReduceEpi e, hipStream_t s, const char *what) {
+    const FastDiv bdiv(e.bias_div ? e.bias_div : 1);
+    if (!e.bias_mod) e.bias_mod = 1;
+    if (reduce_vec_ok(partial, count) && reinterpret_cast<uintptr_t>(C) % 16 == 0 && count >= 4u * 256u * 256u)
+        hipLaunchKernelGGL(ordered_reduce_kernel<4>, dim3(ceil_div(count, 1024u)), dim3(256), 0, s, partial, C, count, splits, e, bdiv);
+    else
+        hipLaunchKernelGGL(ordered_reduce_kernel<1>, dim3(ceil_div(count, 256u)), dim3(256), 0, s, partial, C, count, splits, e, bdiv);
     return check_launch(what);
 }
 

@@ -210,7 +210,7 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
 
     u32 tm, tn;
     swizzled_tile(blockIdx.x, d.tiles_m, d.tiles_n, tm, tn);
-    const u32 z = blockIdx.z;
+    const u32 z = blockIdx.z + d.z0;
     u32 kbeg = 0, kend = d.K;
     if (d.split_k) {
         kbeg = z * d.k_per_z;
@@ -219,7 +219,7 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
     } else {
         a.bind(z), b.bind(z);
     }
-    epi.bind(z);
+    epi.bind(blockIdx.z);
 
     const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) % (Cfg::WM * Cfg::WN), kgroup = (threadIdx.x >> 6) / (Cfg::WM * Cfg::WN);
     const int wave_m = wave / Cfg::WN, wave_n = wave % Cfg::WN;
@@ -562,11 +562,11 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
 
 template <class Cfg, class AOp, class BOp, class Epi>
 inline int launch_split(const AOp &a, const BOp &b, const Epi &epi, u32 M, u32 N, u32 K, u32 zdim, u32 k_per_z, hipStream_t stream,
-                        const char *what) {
+                        const char *what, u32 z0 = 0) {
     IgemmDims d;
     d.M = M, d.N = N, d.K = K;
     d.tiles_m = ceil_div(M, u32(Cfg::BM)), d.tiles_n = ceil_div(N, u32(Cfg::BN));
-    d.split_k = k_per_z != 0, d.k_per_z = k_per_z;
+    d.split_k = k_per_z != 0, d.k_per_z = k_per_z, d.z0 = z0;
     const uint64_t tiles = uint64_t(d.tiles_m) * d.tiles_n;
     if (tiles > 0x7fffffffull || zdim > 65535u) return fail(CRB_EINVAL_SHAPE, "%s: launch grid too large", what);
     hipLaunchKernelGGL((igemm_split_kernel<Cfg, AOp, BOp, Epi>), dim3(u32(tiles), 1, zdim), dim3(Cfg::NTH), 0, stream, a, b, epi, d);

@@ -368,9 +368,9 @@ struct RowMajorEpi {
     // A store that tests and reads nothing: the caller has checked the bounds and hands in the previous value (0 when the
     // form does not accumulate). Same order of additions as store().
     __device__ __forceinline__ void put(u32 row, const ColS &c, float v, float rowb, float old) const {
+        v += old;
         v += c.bias;
         v += rowb;
-        v += old;
         if (flags & EPI_RELU) v = v > 0.0f ? v : 0.0f;
         C[size_t(row) * ld + c.col] = v;
     }
@@ -382,12 +382,12 @@ struct RowMajorEpi {
     __device__ __forceinline__ void store(u32 row, const ColS &c, float v, float rowb, bool have_old = false, float old = 0.f) const {
         if (!c.ok) return;
         float *p = C + size_t(row) * ld + c.col;
-        v += c.bias;
-        v += rowb;
         if (have_old)
             v += old;
         else if (flags & EPI_ACCUM)
             v += *p;
+        v += c.bias;
+        v += rowb;
         if (flags & EPI_RELU) v = v > 0.0f ? v : 0.0f;
         *p = v;
     }

@@ -62,7 +62,9 @@ void crb_release_workspace(void);
  * of every entry point that takes no workspace argument of its own (the GEMM and dense-layer families, the general
  * convolution forward / data-gradient path, crb_conv_bias_grad, and the convolution entry points when their workspace
  * argument is NULL). While a block is bound, calls on that stream never allocate: a call that needs more than the block
- * holds returns CRB_EWORKSPACE. The *_workspace_bytes queries below tell what a call needs. workspace == NULL unbinds
+ * holds returns CRB_EWORKSPACE. The *_workspace_bytes queries below tell what a call needs. (Products, dense layers,
+ * crb_conv_fwd and crb_conv_dgrad on kernels that use scratch for speed only run without it all the same, more slowly: on too
+ * small a block, in a stream capture, or where the arena cannot grow. The result is the same, bit for bit.) workspace == NULL unbinds
  * (the library arena serves the stream again). The block must stay valid until the work queued on the stream that uses
  * it has finished; the library never frees it. No counterpart in the reference, whose operators never need scratch
  * (seblas/operations/cuGEMM.cu:1649-1714 launches one kernel per call). For callers that record the calls into a HIP
@@ -142,8 +144,9 @@ int crb_conv_fwd(const float *W, const float *X, float *Y, const float *bias_or_
  * W[oc,ic,fh,fw] * dY[n,oc,oh,ow]. Overwrite. */
 int crb_conv_dgrad(const float *W, const float *dY, float *dX, const crb_conv_geom *g, void *stream);
 
-/* Bytes of split scratch crb_conv_fwd / crb_conv_dgrad need for this geometry (0 for every shape with a kernel of its
- * own; the general implicit-GEMM path cuts short-and-wide contractions). operands_aligned16: whether the activation
+/* Bytes of split scratch crb_conv_fwd / crb_conv_dgrad need for this geometry: split filters (1.5 times the filters' bytes) and, where
+ * the contraction is cut, partial results, for 3x3 and 5x5 layers on split operands; partial results where the general
+ * implicit-GEMM path cuts short-and-wide contractions; 0 for the other shapes with a kernel of their own. operands_aligned16: whether the activation
  * tensors are 16-byte aligned (hipMalloc'd ones are); other alignments take the general path. Served from the block
  * bound with crb_bind_workspace, else from the library arena. */
 size_t crb_conv_fwd_workspace_bytes(const crb_conv_geom *g, int operands_aligned16);

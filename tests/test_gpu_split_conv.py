@@ -248,3 +248,81 @@ def test_the_gradient_that_allocates_nothing_has_the_same_bits(dev, shape):
         with pytest.raises(capi.CrbError) as ei:
             capi.conv_wgrad(dY, X, got[0], g, workspace=torch.empty(need // 8, device=dev))
         assert ei.value.status == capi.CRB_EWORKSPACE
+
+
+# One layer for each kernel configuration, with and without a cut contraction: (N, IC, H, W, OC, F, stride, pad), pass,
+# (configuration, slices)
+PLANS = [((94, 78, 6, 7, 38, 3, 1, 0), "dgrad", (0, 1)), ((2, 31, 18, 10, 498, 3, 1, 1), "dgrad", (0, 11)), ((21, 333, 12, 3, 80, 3, 1, 0), "dgrad", (1, 1)),
+         ((13, 206, 14, 3, 173, 3, 1, 0), "dgrad", (1, 4)), ((33, 129, 4, 5, 334, 3, 1, 0), "dgrad", (2, 11)), ((33, 129, 4, 14, 56, 3, 1, 0), "dgrad", (3, 1)),
+         ((95, 37, 15, 3, 123, 3, 1, 0), "dgrad", (3, 2)), ((4, 28, 50, 20, 50, 3, 1, 1), "dgrad", (4, 1)), ((4, 24, 54, 7, 314, 3, 1, 0), "dgrad", (4, 7)),
+         ((6, 35, 6, 38, 83, 3, 1, 2), "fwd", (0, 1)), ((2, 134, 10, 62, 27, 3, 1, 2), "fwd", (0, 3)), ((39, 72, 3, 34, 62, 3, 1, 0), "fwd", (1, 1)),
+         ((2, 139, 5, 58, 119, 3, 1, 0), "fwd", (1, 3)), ((15, 399, 5, 28, 30, 3, 1, 0), "fwd", (2, 13)), ((73, 59, 15, 5, 36, 3, 1, 0), "fwd", (3, 1)),
+         ((31, 402, 14, 3, 24, 3, 1, 1), "fwd", (3, 7)), ((3, 84, 35, 21, 30, 3, 1, 1), "fwd", (4, 1)), ((4, 116, 19, 40, 26, 3, 1, 1), "fwd", (4, 3)),
+         ((6, 40, 58, 20, 80, 3, 2, 1), "fwd", (0, 1)), ((21, 150, 5, 4, 147, 3, 2, 2), "fwd", (0, 4)), ((7, 66, 6, 104, 118, 3, 2, 0), "fwd", (1, 1)),
+         ((2, 496, 5, 15, 412, 3, 2, 0), "fwd", (1, 11)), ((10, 169, 53, 21, 25, 3, 2, 0), "fwd", (2, 6)), ((3, 29, 35, 29, 30, 5, 1, 0), "dgrad", (0, 1)),
+         ((3, 75, 4, 108, 42, 5, 1, 1), "dgrad", (0, 3)), ((42, 24, 3, 60, 35, 5, 1, 1), "dgrad", (1, 1)), ((15, 85, 5, 12, 197, 5, 1, 0), "dgrad", (1, 13)),
+         ((29, 171, 9, 5, 168, 5, 1, 0), "dgrad", (2, 6)), ((15, 138, 6, 37, 58, 5, 1, 0), "dgrad", (3, 1)), ((64, 18, 6, 8, 306, 5, 1, 0), "dgrad", (4, 15)),
+         ((2, 24, 8, 112, 30, 5, 1, 4), "fwd", (0, 1)), ((2, 38, 11, 3, 405, 5, 1, 3), "fwd", (0, 3)), ((38, 16, 5, 7, 235, 5, 1, 1), "fwd", (1, 1)),
+         ((43, 34, 16, 6, 57, 5, 1, 0), "fwd", (1, 3))]
+# layers whose fp32 kernel would not run in less scratch either
+REFUSED = {PLANS[i][0] for i in (3, 8, 10, 15, 16, 17, 20, 23, 26, 27, 28, 29, 30)}
+# output channels of a tile, K groups, taps the filters run ahead
+CONFIGURATIONS = ((64, 1, 4), (128, 1, 2), (128, 2, 2), (64, 4, 2), (32, 1, 4))
+
+
+def plan_bytes(plan, C_IN, C_OUT, F, results):
+    """Scratch of a plan: 3 KB of split filters per 32 output channels, 16 input channels and tap, in whole tiles and chunks."""
+    OCT, KG, ahead = CONFIGURATIONS[plan[0]]
+    filters = ((-(-C_OUT // OCT) * (OCT // 32)) * KG * -(-C_IN // (16 * KG)) * F * F + ahead) * 3072
+    return -(-filters // 256) * 256 + (4 * plan[1] * results if plan[1] > 1 else 0)
+
+
+@pytest.mark.parametrize("shape,which,plan", PLANS, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else v)
+def test_every_configuration(dev, shape, which, plan):
+    """Against the oracle, with operands that are not finite against float64, and with less scratch than it takes: the same bits."""
+    import torch
+    import torch.nn.functional as F_
+    from crusaderbackend_amd import capi
+
+    N, IC, H, W, OC, F, s, p = shape
+    g = capi.ConvGeom.make(N, IC, H, W, OC, F, F, s, s, p, p)
+    X, Wt, dY, b = normal(1, N, IC, H, W), he_normal(2, OC, IC, F, F), normal(3, N, OC, g.OH, g.OW), normal(4, OC)
+    fwd = which == "fwd"
+    need = capi.conv_fwd_workspace_bytes(g) if fwd else capi.conv_dgrad_workspace_bytes(g)
+    assert need == plan_bytes(plan, IC if fwd else OC, OC if fwd else IC, F, N * OC * g.OH * g.OW if fwd else N * IC * H * W)
+    K = (IC if fwd else OC) * F * F
+    Wd, bd = to_dev(Wt, dev), to_dev(b, dev)
+
+    def call(x, out, **kw):
+        if fwd:
+            capi.conv_fwd(Wd, x, out, bd, g, capi.CRB_FLAG_RELU, **kw)
+        else:
+            capi.conv_dgrad(Wd, x, out, g, **kw)
+
+    x = to_dev(X if fwd else dY, dev)
+    out = torch.empty(*((N, OC, g.OH, g.OW) if fwd else (N, IC, H, W)), device=dev)
+    call(x, out)
+    torch.cuda.synchronize()
+    ref = np.maximum(orc.conv(Wt, X, b, s, s, p, p), 0) if fwd else orc.convDerive(Wt, dY, (H, W), s, s, p, p)
+    assert_close(to_np(out), ref, K, f"{which} {shape}")
+
+    again, side, little = torch.empty_like(out), torch.cuda.Stream(device=dev), torch.empty(need // 4 - 64, device=dev)
+    torch.cuda.synchronize()
+    try:
+        capi.bind_workspace(little, stream=side)
+        call(x, again, stream=side)
+        side.synchronize()
+        assert torch.equal(out, again) and shape not in REFUSED
+    except capi.CrbError as e:
+        assert e.status == capi.CRB_EWORKSPACE and shape in REFUSED
+    finally:
+        capi.bind_workspace(None, stream=side)
+
+    big = x.clone()
+    big[0, 1, -1, -1], big[N - 1, 3, 0, 0] = float("inf"), -3.4e38
+    call(big, out)
+    torch.cuda.synchronize()
+    y = (F_.conv2d(big.cpu().double(), torch.from_numpy(Wt).double(), torch.from_numpy(b).double(), stride=s, padding=p).relu() if fwd else
+         F_.conv_transpose2d(big.cpu().double(), torch.from_numpy(Wt).double(), stride=s, padding=p)).numpy()
+    # (where the one large operand is, it is all of the sum; beside it K terms of order 1, each rounded once or twice)
+    np.testing.assert_allclose(to_np(out), np.where(np.abs(y) > 3.4028235e38, np.copysign(np.inf, y), y), rtol=K * 2.0**-23, atol=K * 2.0**-20, equal_nan=True)

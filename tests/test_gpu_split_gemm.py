@@ -203,3 +203,36 @@ def test_sums_of_one_product(dev, form, size):
     torch.cuda.synchronize()
     ulps = np.abs(to_np(C) - exact) / np.ldexp(1.0, np.floor(np.log2(exact)).astype(int) - 23)
     assert ulps.max() <= 1.5, (ulps.max(), np.sqrt((ulps**2).mean()))
+
+
+# contractions that only the split products cut: 3 slices of 256 x 256 tiles, 3 of 128 x 128, 3 of 64 x 64 tiles of four waves
+@pytest.mark.parametrize("size", [(3748, 1095, 1087), (389, 2305, 775), (3542, 135, 1044)], ids=lambda s: "x".join(map(str, s)))
+def test_products_that_no_scratch_can_be_had_for(dev, size):
+    """Recorded on a fresh stream, where nothing may be allocated: the bits of the eager call, for every form and epilogue."""
+    import torch
+    from crusaderbackend_amd import capi
+
+    M, N, K = size
+    assert capi.gemm_workspace_bytes(M, N, K, 1) > 0
+    A, At, B, Bt = (torch.randn(*s, device=dev) for s in ((M, K), (K, M), (K, N), (N, K)))
+    b, dB0, C0 = torch.randn(N, device=dev), torch.randn(M, device=dev), torch.randn(M, N, device=dev)
+
+    def calls(C, dB, s):
+        capi.sgemm_nn(A, B, C[0], M, N, K, stream=s)
+        capi.sgemm_tn(At, B, C[1], M, N, K, stream=s)
+        capi.sgemm_nta(A, Bt, C[2], M, N, K, stream=s)
+        capi.linear_fwd(A, Bt, b, C[3], M, K, N, capi.CRB_FLAG_RELU, stream=s)
+        capi.linear_wgrad(At, B, C[4], dB, K, N, M, stream=s)
+
+    want, dB = C0.repeat(5, 1, 1), dB0.clone()
+    calls(want, dB, torch.cuda.current_stream())
+    got, dBg = C0.repeat(5, 1, 1), dB0.clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream(device=dev)):
+        calls(got, dBg, torch.cuda.current_stream())
+    for _ in range(3):
+        got.copy_(C0.expand(5, M, N)), dBg.copy_(dB0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and torch.equal(dBg, dB)
