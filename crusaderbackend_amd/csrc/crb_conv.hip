@@ -13,7 +13,10 @@
 #include "gemm_internal.h"
 #include "operands.h"
 
+#include <cstring>
+#include <memory>
 #include <mutex>
+#include <new>
 
 namespace crb {
 
@@ -338,6 +341,30 @@ static int launch_tiled_any(const float *Wt, const float *X, float *Y, const flo
 // where a CU holds two of the first two's workgroups, 0.35 where all hold one, 0.34 and 0.19 for the others; on a few dozen CUs
 // (64 -> 64 @20 batch 8, 128 -> 128 @14 batch 8, 256 -> 256 @7 batch 4) 0.17 for the first two. A contraction may be cut into slices
 // on grids that leave CUs idle: one more launch, and the partial results written and read once.
+// Plans go by the geometry alone and take 1 to 10 us to form (every tile height against every strip), on calls that take 12 us and
+// up: a thread keeps those of the last geometries it saw, by value, one to a place.
+template <class Plan, class F>
+static Plan kept_plan(const crb_conv_geom *g, u32 kind, F make) {  // kind: 1 and up
+    struct Place {
+        crb_conv_geom g;
+        u32 kind;
+        Plan plan;
+    };
+    constexpr u32 kPlaces = 128;
+    static thread_local std::unique_ptr<Place[]> places;
+    if (!places) {
+        places.reset(new (std::nothrow) Place[kPlaces]());
+        if (!places) return make();
+    }
+    static_assert(sizeof(crb_conv_geom) == 13 * sizeof(u32), "thirteen numbers, nothing between them");
+    u32 v[13], h = kind;
+    memcpy(v, g, sizeof(v));
+    for (u32 x : v) h = (h ^ x) * 0x9e3779b1u, h ^= h >> 15;
+    Place &p = places[h % kPlaces];
+    if (p.kind != kind || memcmp(&p.g, g, sizeof(*g))) p.plan = make(), p.g = *g, p.kind = kind;
+    return p.plan;
+}
+
 struct ConvSplitPlan {
     int cfg = -1;
     u32 strips = 0, slices = 1;
@@ -415,7 +442,7 @@ static bool direct_shape(const crb_conv_geom *g, u32 stride) {
            g->IH == stride * g->OH && g->IW == stride * g->OW;
 }
 // The plan of a layer's forward pass / data gradient (cfg < 0: not taken): square filters, one stride, any padding up to F - 1.
-static ConvSplitPlan conv_split_fwd_plan(const crb_conv_geom *g, bool aligned) {
+static ConvSplitPlan make_conv_split_fwd_plan(const crb_conv_geom *g, bool aligned) {
     if (g->FH != g->FW || g->sH != g->sW || g->pH >= g->FH || g->pW >= g->FW) return ConvSplitPlan();
     bool direct = false;
     if (aligned && direct_shape(g, 1))
@@ -434,13 +461,19 @@ static ConvSplitPlan conv_split_fwd_plan(const crb_conv_geom *g, bool aligned) {
     if (direct && (g->N >= 8 || g->sH != 1 || g->IC * 9 < 512)) return ConvSplitPlan();
     return conv_split_plan(g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, g->FH, g->sH, direct, direct ? 30.f : 100.f);
 }
-static ConvSplitPlan conv_split_dgrad_plan(const crb_conv_geom *g, bool aligned) {
+static ConvSplitPlan make_conv_split_dgrad_plan(const crb_conv_geom *g, bool aligned) {
     if (g->FH != g->FW || g->sH != 1 || g->sW != 1 || g->pH >= g->FH || g->pW >= g->FW) return ConvSplitPlan();
     bool direct = false;
     if (aligned && direct_shape(g, 1))
         try_direct<true, 1>(nullptr, nullptr, nullptr, nullptr, g->N, g->OC, g->IC, g->OH, g->OW, g->OH, 0, nullptr, "", direct, true);
     if (direct) return ConvSplitPlan();  // (as the forward pass: the gradients enter the weights of the same training run)
     return conv_split_plan(g->N, g->OC, g->IC, g->OH, g->OW, g->IH, g->IW, g->FH, 1, false, 100.f);
+}
+static ConvSplitPlan conv_split_fwd_plan(const crb_conv_geom *g, bool aligned) {
+    return kept_plan<ConvSplitPlan>(g, 1 + aligned, [&] { return make_conv_split_fwd_plan(g, aligned); });
+}
+static ConvSplitPlan conv_split_dgrad_plan(const crb_conv_geom *g, bool aligned) {
+    return kept_plan<ConvSplitPlan>(g, 3 + aligned, [&] { return make_conv_split_dgrad_plan(g, aligned); });
 }
 template <int F, int S, bool DG>
 static int run_conv_split_set(const ConvSplitPlan &p, const float *Wt, const float *X, float *Y, const float *bias, unsigned char *wf, u32 N, u32 C_IN,
@@ -833,7 +866,7 @@ static SplitWgradChoice split_wgrad_choice_for(const crb_conv_geom *g, size_t mo
 }
 static size_t wgrad_scratch_bytes(const crb_conv_geom *g, bool split);
 // cfg < 0: not taken.
-static SplitWgradChoice split_wgrad_choice(const crb_conv_geom *g) {
+static SplitWgradChoice make_split_wgrad_choice(const crb_conv_geom *g) {
     const SplitWgradChoice none;
     if (g->FH != g->FW || g->sH != g->sW || g->pH >= g->FH || g->pW >= g->FW || g->IC < 16 || g->OC < 16 || tiny2x2_shape(g)) return none;
     WgradDirectPlan dp;
@@ -864,6 +897,9 @@ static SplitWgradChoice split_wgrad_choice(const crb_conv_geom *g) {
         else if (c.plan.workspace_bytes > kStaticScratchBytes && fp32 <= kStaticScratchBytes) c = choice(kStaticScratchBytes);
     }
     return c;
+}
+static SplitWgradChoice split_wgrad_choice(const crb_conv_geom *g) {
+    return kept_plan<SplitWgradChoice>(g, 1, [&] { return make_split_wgrad_choice(g); });
 }
 template <int F, int S>
 static int run_split_wgrad_set(const SplitWgradChoice &c, const float *dY, const float *X, float *dW, float *ws, const crb_conv_geom *g, hipStream_t s,
