@@ -142,7 +142,10 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
             for (int i = 0; i < C::NP; ++i) {
                 const u32 o = (threadIdx.x + i * C::NTH) / MAXPX;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) reg[i][j] = buffer_load(xrange, c0 + 8 * o + j < a.C_IN ? off[i] : kOutside, (c0 + j) * a.HW * 4u);
+                for (int j = 0; j < 8; ++j) {  // (channels past the last: kOutside, at an offset the range holds)
+                    const u32 ch = c0 + j < a.C_IN ? c0 + j : a.C_IN - 1;
+                    reg[i][j] = buffer_load(xrange, c0 + 8 * o + j < a.C_IN ? off[i] : kOutside, ch * a.HW * 4u);
+                }
             }
         } else {
 #pragma unroll

@@ -49,8 +49,9 @@ struct SplitWgradArgs {
     u32 m_ow, m_oh, m_prow, m_strip;  // SmallDiv multipliers of SW, OH, prow, strips
 };
 
-// floor(n / d) for n * d < 2^20 as one full-rate 24-bit multiplication and a shift, m = ceil(2^20 / d): decoding the positions of
-// every tile with 32-bit high multiplications (a quarter of the rate) cost as much as a third of a tile's MFMAs.
+// floor(n / d) for n * d < 2^20 and n / d < 4095 (the product stays under 2^32) as one full-rate 24-bit multiplication and a shift,
+// m = ceil(2^20 / d): decoding the positions of every tile with 32-bit high multiplications (a quarter of the rate) cost as much as
+// a third of a tile's MFMAs.
 __device__ __forceinline__ u32 small_div(u32 n, u32 m) { return __umul24(n, m) >> 20; }
 
 __device__ __forceinline__ bf16x8 read_transposed(const unsigned char *lds0, const unsigned char *lds1) {
@@ -138,12 +139,17 @@ __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a
         constexpr u32 XSTEP = C::NTH / MAXPX, DSTEP = C::NTH / PXT;  // octets between a thread's items
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
+            // (channels past the last: kOutside, at an offset the range holds)
 #pragma unroll
-            for (int i = 0; i < C::XNP; ++i)
-                xreg[i][j] = buffer_load(xr, !RAG || ic0 + 8 * (ox + XSTEP * i) + j < a.IC ? xoff : kOutside, (8 * XSTEP * i + j) * a.HW * 4u);
+            for (int i = 0; i < C::XNP; ++i) {
+                const u32 c = 8 * XSTEP * i + j, ch = !RAG || ic0 + c < a.IC ? c : a.IC - ic0 - 1;
+                xreg[i][j] = buffer_load(xr, !RAG || ic0 + 8 * ox + c < a.IC ? xoff : kOutside, ch * a.HW * 4u);
+            }
 #pragma unroll
-            for (int i = 0; i < C::DNP; ++i)
-                dreg[i][j] = buffer_load(dr, !RAG || oc0 + 8 * (od + DSTEP * i) + j < a.OC ? doff : kOutside, (8 * DSTEP * i + j) * a.OHW * 4u);
+            for (int i = 0; i < C::DNP; ++i) {
+                const u32 c = 8 * DSTEP * i + j, ch = !RAG || oc0 + c < a.OC ? c : a.OC - oc0 - 1;
+                dreg[i][j] = buffer_load(dr, !RAG || oc0 + 8 * od + c < a.OC ? doff : kOutside, ch * a.OHW * 4u);
+            }
         }
     };
     auto store_unit = [](unsigned char *dst, int part_stride, const float (&r)[8]) {
@@ -345,7 +351,9 @@ inline SplitWgradPlan split_wgrad_plan(u32 N, u32 IC, u32 OC, u32 H, u32 W, u32 
             p.strips = ns;
             break;
         }
-    // small_div's range, and the images a tile touches within 2 GiB (buffer loads)
+    // small_div's range (quotients are rows, images or strips of one tile, so at most its pixels or run and the 16 strips), and the
+    // images a tile touches within 2 GiB (buffer loads)
+    static_assert(C::PXT + 16 < 4095 && C::MAXPX + 16 < 4095, "quotients of small_div");
     const uint64_t sw = p.strips ? ceil_div(OW, p.strips) : 0, prow = C::S * (OH - 1) + C::F, run = C::MAXPX;
     const bool small = (C::PXT + sw) * sw < (1u << 20) && (OH + C::PXT) * uint64_t(OH) < (1u << 20) && (prow + run) * prow < (1u << 20);
     const uint64_t images = p.strips ? uint64_t(C::PXT) / (uint64_t(OH) * ceil_div(OW, p.strips)) + 3 : 0;

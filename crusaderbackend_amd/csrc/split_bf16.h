@@ -56,7 +56,8 @@ __device__ __forceinline__ void split8(const float *x, u32x4 (&part)[kSplit]) {
 
 // A float at `voffset + soffset` bytes behind a uniform base, by a buffer load: the address needs no vector arithmetic beyond
 // voffset, and an element that is to read as zero (halo, channels past the tensor) is named by kOutside, which the resource's
-// range check turns into 0. Ranges are under 2 GiB.
+// range check turns into 0. Ranges are under 2 GiB, and `soffset` lies inside the range also where `voffset` does not: whether the check
+// takes what is left behind `soffset` for a signed number or not is then all the same.
 constexpr u32 kOutside = 0x80000000u;
 typedef __amdgpu_buffer_rsrc_t BufferRange;
 __device__ __forceinline__ BufferRange buffer_range(const float *base, size_t floats) {

@@ -13,6 +13,8 @@ pytestmark = pytest.mark.gpu
 # a contraction cut into slices, every padding, 5x5 with its rows in separate workgroups, stride 2 with odd extents
 SHAPES = [(3, 64, 31, 33, 65, 3, 1, 1), (2, 33, 67, 61, 63, 3, 1, 1), (1, 47, 29, 131, 49, 3, 1, 1), (33, 96, 7, 5, 97, 3, 1, 1), (5, 129, 13, 14, 127, 3, 1, 0),
           (3, 80, 15, 17, 48, 3, 1, 2), (2, 300, 9, 11, 70, 3, 1, 1), (7, 31, 21, 19, 33, 5, 1, 2), (3, 40, 18, 23, 65, 5, 1, 0), (2, 36, 12, 50, 40, 5, 1, 4),
+          # one image, one channel in the last chunk and tile: channels past it lie behind the tensor's end
+          (1, 33, 67, 61, 65, 3, 1, 1), (1, 65, 61, 67, 129, 3, 2, 1), (1, 33, 37, 41, 65, 5, 1, 2),
           (4, 65, 33, 27, 97, 3, 2, 1), (3, 48, 30, 31, 66, 3, 2, 0), (70, 512, 4, 4, 96, 3, 1, 1), (64, 64, 32, 32, 64, 3, 1, 1), (9, 72, 20, 3, 80, 3, 1, 1),
           # under eight images on the width-specialised kernels' extents
           (1, 64, 32, 32, 64, 3, 1, 1), (2, 72, 16, 16, 128, 3, 1, 1), (3, 128, 8, 8, 80, 3, 1, 1), (7, 512, 4, 4, 512, 3, 1, 1)]
