@@ -9,12 +9,13 @@
 // [channel octet][position] units of 16 bytes, double-buffered. A tap is then a constant shift of a lane's position, whatever
 // the width, and a B fragment (32 pixels, 16 channels) is one 16-byte read at lane base + shift.
 // Filters are split by a kernel of their own into fragments in the order the waves consume them (conv_split_filters_kernel) and
-// go from L2 straight into registers, two taps ahead: a filter element is used once per workgroup tile, so LDS would only add
+// go from L2 straight into registers, two or four taps ahead: a filter element is used once per workgroup tile, so LDS would only add
 // a copy, and without them a barrier stands only every F*F taps.
 // KG wave groups take 16 channels each of every staged chunk and exchange their accumulators through LDS at the end.
 //
-// What bounds it: per tap a wave issues 6*TM*TN MFMAs (32 clocks each) against 3*TM KB of filters from L2 and 3*TN KB from LDS:
-// with 2 x 2 blocks per wave and two waves on a SIMD half of the vector memory path's and a quarter of LDS' time, so the MFMAs.
+// What bounds it: per tap a wave issues 6*TM*TN MFMAs (32 clocks each) against 3*TM KB of filters from L2 and 3*TN KB from LDS: with
+// the 1 x 2 blocks of every configuration and eight waves on a CU 768 clocks of MFMAs on each SIMD against 384 of the vector
+// memory path (64 bytes a clock) and 384 of LDS (128), so the MFMAs, between a first and a last phase that they do not fill.
 #pragma once
 #include "igemm_engine.h"
 #include "split_bf16.h"

@@ -333,7 +333,7 @@ static int launch_tiled_any(const float *Wt, const float *X, float *Y, const flo
 // Configurations <F, S, TM, TN, WM, WN, KG, MAXPX, AHEAD, BSET>: output channels x pixels of a workgroup tile and K groups.
 //   0: 64 x 128, four waves, two workgroups per CU      1: 128 x 64, four waves, two per CU
 //   2: 128 x 64 in two K groups, one per CU             3: 64 x 64 in four K groups, one per CU
-//   4: 32 x 256, four waves, two per CU
+//   4: 32 x 256, four waves, two per CU              (stride 2: 0 and 4 are 64 x 64 and 32 x 128 on two waves)
 // The choice is the smallest estimate: 6 us for the filters' launch and the workgroups' first and last phases, what splitting the
 // filters and reading the parts back takes (kFilterUs a million elements; by the difference of measured times and the rest of the
 // estimate, 18 layers of 4 to 53 million: 2.9 to 4.2 us for 3x3 filters, 4.2 to 5.2 for 5x5), plus rounds x steps (16 channels of one

@@ -154,14 +154,13 @@ def test_linear_relu_flag(dev):
     assert_close(to_np(Y), np.maximum(orc.linear(X, W, b), 0), IN, "linear+relu")
 
 
-# Shapes whose tile grid fills the chip in whole rounds and whose contraction is a multiple of 32 run on the kernel that
-# loads operand panels straight into LDS: 128 x 128 tiles (the first three), 64 x 64 tiles (the next three), the latter as
-# eight-wave workgroups when there is at most one per CU (the last two); ragged edge tiles included.
-DIRECT_TO_LDS = [(2048, 2048, 256), (2040, 2044, 288), (1024, 4096, 320), (512, 4096, 512), (508, 4092, 544), (32768, 64, 576),
+# Shapes whose tile grid fills the chip in whole rounds and whose contraction is a multiple of 32, from 2^28 multiply-adds: on split
+# operands, whole tiles and ragged edge tiles, one slab and a few.
+CHIP_FILLING = [(2048, 2048, 256), (2040, 2044, 288), (1024, 4096, 320), (512, 4096, 512), (508, 4092, 544), (32768, 64, 576),
                  (1000, 1020, 544), (768, 1024, 1024)]
 
 
-@pytest.mark.parametrize("M,N,K", DIRECT_TO_LDS)
+@pytest.mark.parametrize("M,N,K", CHIP_FILLING)
 def test_sgemm_forms_on_chip_filling_shapes(dev, M, N, K):
     run_nn(dev, M, N, K, 1, seed=71)
     run_nt(dev, M, N, K, seed=72)
@@ -217,9 +216,9 @@ def test_split_k_paths(dev, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(256, 2048, 2048), (512, 512, 4096), (128, 2048, 2048), (250, 1020, 2048), (128, 512, 8192)])
-def test_split_k_on_the_direct_to_lds_kernel(dev, M, N, K):
-    """Few tiles, contraction a multiple of 32: slices of K on the kernel that loads straight into LDS (128-wide and 64-wide tiles,
-    ragged edges), every form, and the dense-layer epilogues (bias, ReLU, accumulate with the bias gradient) behind the slice sum."""
+def test_split_k_of_larger_products(dev, M, N, K):
+    """Few tiles, contraction a multiple of 32: slices of K of products on split operands (128-wide and 64-wide tiles, ragged
+    edges), every form, and the dense-layer epilogues (bias, ReLU, accumulate with the bias gradient) behind the slice sum."""
     run_nn(dev, M, N, K, 1, seed=45)
     run_tn(dev, M, N, K, 1, seed=46)
     run_nt(dev, M, N, K, seed=47)

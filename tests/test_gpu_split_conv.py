@@ -8,6 +8,7 @@ from tests.util import assert_close, he_normal, normal, to_dev, to_np
 
 pytestmark = pytest.mark.gpu
 
+# Edges of the layers, whichever kernels their sizes choose (PLANS below: a layer for every configuration of the split ones).
 # (N, IC, H, W, OC, F, stride, pad): a last pixel tile of a few pixels, images narrower than a filter's reach and wider than a
 # strip (uneven strips, a strip of padding columns), several images per tile, channels one past / one short of 16, 32 and 64,
 # a contraction cut into slices, every padding, 5x5 with its rows in separate workgroups, stride 2 with odd extents
