@@ -2,7 +2,8 @@
 
 Each entry: launch duration from HIP events on the launch stream (average of back-to-back launches), nominal
 flops, algorithmic bytes (each operand read once, output written once), TFLOP/s, GB/s and the fraction of the
-roofline that bounds the shape (FP32 matrix peak above ~19.7 flop/B, HBM bandwidth below).
+roofline that bounds the shape (HBM bandwidth at few flops per byte; else the FP32 matrix peak, or for the calls that run on
+split operands what six bf16 products per fp32 one leave of the dense bf16 peak).
 """
 import hashlib
 import math
@@ -11,6 +12,7 @@ import os
 PEAK_TF = 157.3
 PEAK_GBS = 8000.0
 RIDGE = PEAK_TF * 1e3 / PEAK_GBS  # flop per byte
+PEAK_SPLIT_TF = 2500.0 / 6
 COLD_FOOTPRINT = 640e6  # bytes of distinct operands cycled through for the cold-cache figures
 
 
@@ -28,13 +30,32 @@ def csrc_hash():
     return h.hexdigest()[:16]
 
 
-def _entry(name, ms, flops, nbytes):
+def conv_on_split(capi, g, which):
+    """Whether a 3x3 or 5x5 layer's pass runs on split operands: forward and data gradient ask for room for the split filters;
+    the weight gradient where no width-specialised kernel (one with a sliced form) takes it, from 100 MFLOP (under 32 output
+    channels 250)."""
+    if g.FH != g.FW or g.FH not in (3, 5):
+        return False
+    if which in ("fwd", "dgrad"):
+        need = capi.conv_fwd_workspace_bytes(g) if which == "fwd" else capi.conv_dgrad_workspace_bytes(g)
+        return 6 * g.OC * g.IC * g.FH * g.FW <= need
+    mflop = 2e-6 * g.N * g.OC * g.OH * g.OW * g.IC * g.FH * g.FW
+    tiles = g.sH == 1 or (g.sH == 2 and g.FH == 3 and g.OC >= 64)
+    return which == "wgrad" and tiles and min(g.IC, g.OC) >= 16 and not capi.conv_bwd_slices(g) and mflop >= (250 if g.OC < 32 else 100)
+
+
+def product_on_split(M, N, K):
+    return M * N * K >= 1 << 28
+
+
+def _entry(name, ms, flops, nbytes, split=False):
     """`ms`: a time, or (smallest, mean) of the three averages of a row."""
     ms, ms_mean = ms if isinstance(ms, tuple) else (ms, ms)
     ai = flops / nbytes
     tf, gbs = flops / ms / 1e9, nbytes / ms / 1e6
-    bound = "mfma" if ai >= RIDGE else "hbm"
-    frac = tf / PEAK_TF if bound == "mfma" else gbs / PEAK_GBS
+    peak = PEAK_SPLIT_TF if split else PEAK_TF
+    bound = "mfma" if ai >= peak * 1e3 / PEAK_GBS else "hbm"
+    frac = tf / peak if bound == "mfma" else gbs / PEAK_GBS
     return {"name": name, "us": round(ms * 1e3, 2), "us_mean": round(ms_mean * 1e3, 2), "gflop": round(flops / 1e9, 3),
             "mbytes": round(nbytes / 1e6, 2), "ai": round(ai, 1), "tflops": round(tf, 2), "gbs": round(gbs, 1), "bound": bound,
             "frac": round(frac, 4)}
@@ -144,11 +165,11 @@ def _dense_rows(torch, capi, dev, settled):
                    ("sgemmNT 256x4096x4096", lambda: capi.sgemm_nt(X, W, Y, b, n, n)),
                    ("sgemm 256x4096x4096", lambda: capi.sgemm_nn(X, W, Y, b, n, n)),
                    ("sgemmTN 4096x4096x256", lambda: capi.sgemm_tn(X, X, dW, n, n, b))):
-        rows.append(_entry(nm, settled(fn, 20), fl, by))
+        rows.append(_entry(nm, settled(fn, 20), fl, by, product_on_split(b, n, n)))
     M, K, N = 32768, 576, 64
     A, B, C = rnd(M, K), rnd(K, N), torch.empty(M, N, device=dev)
     rows.append(_entry("sgemm tall-skinny 32768x64x576", settled(lambda: capi.sgemm_nn(A, B, C, M, N, K), 20),
-                       2.0 * M * N * K, 4.0 * (M * K + K * N + M * N)))
+                       2.0 * M * N * K, 4.0 * (M * K + K * N + M * N), product_on_split(M, N, K)))
     return rows
 
 
@@ -191,7 +212,7 @@ def compact(torch, capi, dev, event_time_ms, Layer):
     out = {}
     n = 1024
     A, B, C = (torch.rand(n, n, device=dev) * 2 - 1 for _ in range(3))
-    out["1_sgemm_1024^3"] = pick(_entry("", settled(lambda: capi.sgemm_nn(A, B, C, n, n, n), 20), 2.0 * n ** 3, 12.0 * n * n))
+    out["1_sgemm_1024^3"] = pick(_entry("", settled(lambda: capi.sgemm_nn(A, B, C, n, n, n), 20), 2.0 * n ** 3, 12.0 * n * n, product_on_split(n, n, n)))
     del A, B, C
     # config 3: every convolution and dense-layer call of one VGG-16 training step (fwd + dgrad + wgrad, bias fused), summed
     rows = []
@@ -245,7 +266,7 @@ def run(torch, capi, dev, event_time_ms, Layer):
     for n in (1024, 4096):
         A, B, C = rnd(n, n), rnd(n, n), torch.empty(n, n, device=dev)
         ms = settled(lambda: capi.sgemm_nn(A, B, C, n, n, n), 20 if n == 1024 else 10)
-        out["gemm"].append(_entry(f"sgemm {n}^3", ms, 2.0 * n ** 3, 12.0 * n * n))
+        out["gemm"].append(_entry(f"sgemm {n}^3", ms, 2.0 * n ** 3, 12.0 * n * n, product_on_split(n, n, n)))
 
     def conv_entries(key, specs, batch, bias):
         for i, (name, IC, H, OC, F, s, p) in enumerate(specs):
@@ -255,7 +276,7 @@ def run(torch, capi, dev, event_time_ms, Layer):
                 if pname in ("bwd", "bwd_sliced") and key != "resnet56":  # the one-call forms of both gradients: residual-network shapes
                     continue
                 reps = 30 if L.flops < 2e9 else 10
-                entries[pname] = _entry(f"{name}.{pname}", settled(fn, reps), fl, L.bytes[pname])
+                entries[pname] = _entry(f"{name}.{pname}", settled(fn, reps), fl, L.bytes[pname], conv_on_split(capi, L.g, pname))
                 out[key].append(entries[pname])
             # Bandwidth-bound shapes also get a cold-cache figure: the same call cycled over enough distinct buffer sets
             # (>= 640 MB in total, beyond L2 and the 256 MB memory-side cache) that no launch finds its operands cached.
