@@ -203,13 +203,13 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
         }
     };
 
-    v16f acc[TM][TN];
+    v16f acc[TM][TN], small[TM][TN];  // sums of the leading part products and of the others (split_bf16.h)
 #pragma unroll
     for (int mi = 0; mi < TM; ++mi)
 #pragma unroll
         for (int ni = 0; ni < TN; ++ni)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.0f;
+            for (int r = 0; r < 16; ++r) acc[mi][ni][r] = small[mi][ni][r] = 0.0f;
 
     bf16x8 fb[C::BSET][kSplit][TN];
     auto read_pixels = [&](int set, u32 shift) {
@@ -243,8 +243,10 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
 #pragma unroll
                 for (int mi = 0; mi < TM; ++mi)
 #pragma unroll
-                    for (int ni = 0; ni < TN; ++ni)
-                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[tap % NSET][kTermA[t]][mi], fb[tap % BS][kTermB[t]][ni], acc[mi][ni], 0, 0, 0);
+                    for (int ni = 0; ni < TN; ++ni) {
+                        v16f &sum = t + 1 < kTerms ? small[mi][ni] : acc[mi][ni];
+                        sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[tap % NSET][kTermA[t]][mi], fb[tap % BS][kTermB[t]][ni], sum, 0, 0, 0);
+                    }
 #pragma unroll
             for (int i = 0; i < TM * TN * kTerms; ++i) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -279,6 +281,7 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
     // Two channels of a tap per MFMA, 16 a step, the next step's operands requested ahead. Taps outside the image take no part
     // (an infinite filter element would make NaN of the zero read there): a lane's accumulators all belong to its pixel, so
     // it keeps the old ones. Ends early where every sum is a NaN.
+    add_small(acc, small);
     if (__builtin_expect(__any(int(scale_down(acc))), 0)) {
         struct Step {
             float w[8][TM], x[8][TN];

@@ -242,13 +242,22 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
     PB pb;
     pa.init(a, row0);
     pb.init(b, col0);
-    v16f acc[TM][TN];
+    // the five small part products have accumulators of their own on the 64 x 64 tiles (split_bf16.h)
+    constexpr bool kSmall = TM * TN <= 2;
+    constexpr int SM = kSmall ? TM : 1, SN = kSmall ? TN : 1;
+    v16f acc[TM][TN], small[SM][SN];
 #pragma unroll
     for (int mi = 0; mi < TM; ++mi)
 #pragma unroll
         for (int ni = 0; ni < TN; ++ni)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.0f;
+#pragma unroll
+    for (int mi = 0; mi < SM; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < SN; ++ni)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) small[mi][ni][r] = 0.0f;
 
     const u32 a_lane = (2 * kgroup + h) * PA::OCT + PA::slot(wave_m * Cfg::WTM + i32);
     const u32 b_lane = (2 * kgroup + h) * PB::OCT + PB::slot(wave_n * Cfg::WTN + i32) + PA::BYTES;
@@ -271,8 +280,10 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
 #pragma unroll
             for (int mi = 0; mi < TM; ++mi)
 #pragma unroll
-                for (int ni = 0; ni < TN; ++ni)
-                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[kTermA[t]][mi], f.b[kTermB[t]][ni], acc[mi][ni], 0, 0, 0);
+                for (int ni = 0; ni < TN; ++ni) {
+                    v16f &sum = kSmall && t + 1 < kTerms ? small[kSmall ? mi : 0][kSmall ? ni : 0] : acc[mi][ni];
+                    sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[kTermA[t]][mi], f.b[kTermB[t]][ni], sum, 0, 0, 0);
+                }
     };
     auto multiply = [&](const unsigned char *sm) {
 #pragma unroll
@@ -494,6 +505,7 @@ __global__ void __launch_bounds__(Cfg::NTH, Cfg::OCC) igemm_split_kernel(AOp a, 
             }
         }
     };
+    if constexpr (kSmall) add_small(acc, small);
     auto not_finite = [](const float *v, int n) {
         bool bad = false;
         for (int r = 0; r < n; ++r) bad |= !__builtin_isfinite(v[r]);

@@ -8,9 +8,12 @@
 // (mid*lo, lo*mid, lo*lo) are together at most 2^-24 of the product, the unit roundoff of one fp32 multiplication. All sums are
 // fp32, in the accumulators of the MFMA. Six sixteenths of the fp32 time per product remain: at the rates the pipes sustain on
 // this part (1.82 PFLOP/s bf16, 155 TFLOP/s fp32, dense random operands) 303 against 155 TFLOP/s of fp32 work.
-// Measured distance from float64 (2-norm, N(0,1) operands; fp32 MFMA / these products): K = 90 1.70e-7 / 0.97e-7, 257 2.87e-7 /
-// 1.20e-7, 777 4.98e-7 / 2.99e-7 - sixteen k's share one rounding of the sum, so the results are closer to the exact ones than those
-// of the fp32 pipe. (With the leading parts first 1.25e-7, 1.44e-7, 3.10e-7; forming all nine showed no difference to those.)
+// Measured distance from float64 (2-norm; fp32 MFMA / these products): N(0,1) products of K = 90 on 256-wide tiles 1.70e-7 / 0.97e-7,
+// 256 x 4096 x 4096 on 128-wide ones 5.75e-7 / 3.53e-7, 777 on 64-wide ones 4.98e-7 / 1.14e-7; layers behind a ReLU, forward, data
+// and weight gradient: 64 -> 64 @56 3.03e-7 / 1.04e-7, 4.28e-7 / 1.35e-7, 2.71e-7 / 3.43e-7, 256 -> 256 @14 5.85e-7 / 2.20e-7, 8.31e-7 /
+// 2.79e-7, 2.47e-7 / 2.17e-7. Sixteen k's share a rounding of the sum, or six where the parts share accumulators (tiles of 128 and 256,
+// weight gradients: their registers hold no second set). These six are not unbiased on the matrix pipe: 512 x 2048 x 4096 of U(0,1) is
+// 6.2e-7 off, all of it one-sided (fp32 3.2e-7).
 // An operand that is infinite, or beyond the range that is split (kSplitUp), has NaN among its parts, so it always shows
 // as NaN in the sum. Sums that are not finite are formed once more from the fp32 operands and are those of an fp32 contraction
 // (infinities keep their sign, large finite values stay finite). Convolutions: on the fp32 MFMA, straight from memory, by waves
@@ -68,6 +71,19 @@ __device__ __forceinline__ float buffer_load(BufferRange r, u32 voffset, u32 sof
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, int(voffset), int(soffset), 0));
 }
 
+// Where there are registers for it, the five part products behind the leading one have accumulators of their own, 2^-8 of the
+// others' size: the full sum is then rounded once per sixteen k instead of six times (forward 64 -> 64 @56 behind a ReLU 3.47e-7 ->
+// 1.04e-7 from float64; 32 registers, times unchanged: 81 passes of random layers 0.99 of what they were in the mean).
+template <class V, int TM, int TN>
+__device__ __forceinline__ void add_small(V (&acc)[TM][TN], const V (&small)[TM][TN]) {
+#pragma unroll
+    for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[mi][ni][r] += small[mi][ni][r];
+}
+
 // A lane's accumulators at their own scale; whether one of them is not finite.
 template <class V, int TM, int TN>
 __device__ __forceinline__ bool scale_down(V (&acc)[TM][TN]) {
@@ -82,8 +98,8 @@ __device__ __forceinline__ bool scale_down(V (&acc)[TM][TN]) {
 }
 
 // The products that are formed: (part of A, part of B), the smallest first: where one term is most of a sum, the roundings before
-// the last are then of its small parts (a sum of one product: off by 1.45 units in the last place at most, rms 0.39; the other way
-// round 3.38 and 0.60; one fp32 multiplication 0.5 and 0.29). kPartOrder: the parts in the order in which they are needed.
+// the last are then of its small parts (a sum of one product: off by 1.45 units in the last place at most, rms 0.39, or 0.95 and
+// 0.30 with accumulators of their own for the small ones; the other way round 3.38 and 0.60; one fp32 multiplication 0.5 and 0.29). kPartOrder: the parts in the order in which they are needed.
 constexpr int kTerms = 6;
 constexpr int kTermA[kTerms] = {2, 0, 1, 1, 0, 0};
 constexpr int kTermB[kTerms] = {0, 2, 1, 0, 1, 0};
