@@ -33,7 +33,7 @@ def csrc_hash():
 def conv_on_split(capi, g, which):
     """Whether a 3x3 or 5x5 layer's pass runs on split operands: forward and data gradient ask for room for the split filters;
     the weight gradient where no width-specialised kernel (one with a sliced form) takes it, from 100 MFLOP (under 32 output
-    channels 250)."""
+    channels 400, 3x3 only)."""
     if g.FH != g.FW or g.FH not in (3, 5):
         return False
     if which in ("fwd", "dgrad"):
@@ -41,7 +41,7 @@ def conv_on_split(capi, g, which):
         return 6 * g.OC * g.IC * g.FH * g.FW <= need
     mflop = 2e-6 * g.N * g.OC * g.OH * g.OW * g.IC * g.FH * g.FW
     tiles = g.sH == 1 or (g.sH == 2 and g.FH == 3 and g.OC >= 64)
-    return which == "wgrad" and tiles and min(g.IC, g.OC) >= 16 and not capi.conv_bwd_slices(g) and mflop >= (250 if g.OC < 32 else 100)
+    return which == "wgrad" and tiles and min(g.IC, g.OC) >= 16 and not capi.conv_bwd_slices(g) and (mflop >= 100 if g.OC >= 32 else mflop >= 400 and g.FH == 3)
 
 
 def product_on_split(M, N, K):

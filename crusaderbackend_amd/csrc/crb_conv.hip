@@ -830,7 +830,7 @@ constexpr size_t kStaticScratchBytes = CRB_NOALLOC_SCRATCH_BYTES;  // the buffer
 // ---- weight gradient on split bf16 operands (conv_split_wgrad.h) -----------------------------------------------------------------
 // Configurations <F, S, WM, WN, KG, MAXPX>: 32 x 32 channels and 128 pixels a tile, or 64 x 32 and 64 (wide images in fewer strips,
 // and 4 x 4 images, whose eight padded images do not fit the first's LDS); stride 2: 128 x 32 and 32. A tile of either of the first
-// two keeps a CU busy for 3.3 us (128 -> 128 @16 batch 128: 16 tiles a CU, 57 us); the slices, 37 KB or 74 KB per workgroup, are
+// two keeps a CU busy for 3.8 us (128 -> 128 @16 batch 128: 16 tiles a CU); the slices, 37 KB or 74 KB per workgroup, are
 // written and read once. The choice is the smaller sum.
 struct SplitWgradChoice {
     int cfg = -1;
@@ -856,7 +856,7 @@ static SplitWgradChoice split_wgrad_choice_for(const crb_conv_geom *g, size_t mo
         const SplitWgradPlan p = split_wgrad_plan<C>(g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, most);
         if (!p.strips || (p.splits > 1 && uint64_t(p.splits) * g->OC * g->IC * F * F > 0x7fffffffull)) return;
         const u32 rows = F / C::ROWS, rounds = ceil_div(p.pairs * p.splits * rows, 256u);
-        float us = 5.f + float(rounds * p.tiles_z) * 3.3f * C::NTW / 9.f;
+        float us = 5.f + float(rounds * p.tiles_z) * 3.8f * C::NTW / 9.f;
         if (p.splits > 1) us += 3.f + 2.f * float(p.workspace_bytes) / 5e6f;
         if (us < best_us) best_us = us, best.cfg = id, best.plan = p;
     };
@@ -874,11 +874,11 @@ static SplitWgradChoice make_split_wgrad_choice(const crb_conv_geom *g) {
     const bool direct = wgrad_direct(g, false, nullptr, nullptr, nullptr, nullptr, nullptr, dp, st);
     const float mflop = 2e-6f * g->N * g->OH * g->OW * g->IC * g->OC * g->FH * g->FW;
     if (direct) return none;  // (width-specialised layers: conv_split_fwd_plan)
-    // Against the fp32 kernels behind it on 70 random layers (16 to 512 channels, 5 to 64 wide, 100 MFLOP to 16 GFLOP): 0.91 to 4.5
-    // times as fast, geometric mean 1.6. The ones under 1 were those of under 32 output channels, which leave a part of every block
-    // idle, and 100 to 240 MFLOP (188 -> 28 @27x22 batch 2 22.0 -> 24.1 us, 97 -> 22 @33x31 batch 6 23.8 -> 24.4); from there on even
-    // 18 gain (370 -> 18 @6x11 batch 59, 467 MFLOP, 29.0 -> 24.4).
-    if (mflop < (g->OC < 32 ? 250.f : 100.f)) return none;
+    // Against the fp32 kernels behind it on 70 random layers that it takes (16 to 512 channels, 5 to 64 wide, 100 MFLOP to 16 GFLOP): 1.04
+    // to 3.8 times as fast, geometric mean 1.51. Left out are those of under 32 output channels, which leave a part of every block
+    // idle, with little work or 5x5 filters (188 -> 28 @27x22 batch 2, 113 MFLOP, 22.0 -> 24.1 us; 198 -> 21 5x5 @35x38 batch 3 38.0 ->
+    // 38.0 before the small products were summed by themselves); from 400 MFLOP on even 18 channels gain.
+    if (mflop < (g->OC < 32 ? 400.f : 100.f) || (g->OC < 32 && g->FH == 5)) return none;
     auto choice = [&](size_t most) {
         float us = 0.f;
         SplitWgradChoice c;

@@ -10,10 +10,10 @@
 // this part (1.82 PFLOP/s bf16, 155 TFLOP/s fp32, dense random operands) 303 against 155 TFLOP/s of fp32 work.
 // Measured distance from float64 (2-norm; fp32 MFMA / these products): N(0,1) products of K = 90 on 256-wide tiles 1.70e-7 / 0.97e-7,
 // 256 x 4096 x 4096 on 128-wide ones 5.75e-7 / 3.53e-7, 777 on 64-wide ones 4.98e-7 / 1.14e-7; layers behind a ReLU, forward, data
-// and weight gradient: 64 -> 64 @56 3.03e-7 / 1.04e-7, 4.28e-7 / 1.35e-7, 2.71e-7 / 3.43e-7, 256 -> 256 @14 5.85e-7 / 2.20e-7, 8.31e-7 /
-// 2.79e-7, 2.47e-7 / 2.17e-7. Sixteen k's share a rounding of the sum, or six where the parts share accumulators (tiles of 128 and 256,
-// weight gradients: their registers hold no second set). These six are not unbiased on the matrix pipe: 512 x 2048 x 4096 of U(0,1) is
-// 6.2e-7 off, all of it one-sided (fp32 3.2e-7).
+// and weight gradient: 64 -> 64 @56 3.03e-7 / 1.04e-7, 4.28e-7 / 1.35e-7, 2.71e-7 / 1.45e-7, 256 -> 256 @14 5.85e-7 / 2.20e-7, 8.31e-7 /
+// 2.79e-7, 2.47e-7 / 1.15e-7. Sixteen k's share a rounding of the sum (weight gradients: two), or six where the parts share
+// accumulators (products on tiles of 128 and 256, whose registers hold no second set). These six are not unbiased on the matrix
+// pipe: 512 x 2048 x 4096 of U(0,1) is 6.2e-7 off, all of it one-sided (fp32 3.2e-7).
 // An operand that is infinite, or beyond the range that is split (kSplitUp), has NaN among its parts, so it always shows
 // as NaN in the sum. Sums that are not finite are formed once more from the fp32 operands and are those of an fp32 contraction
 // (infinities keep their sign, large finite values stay finite). Convolutions: on the fp32 MFMA, straight from memory, by waves

@@ -335,7 +335,8 @@ def test_every_configuration(dev, shape, which, plan):
                          ids=lambda s: "x".join(map(str, s)))
 def test_a_sum_is_rounded_once_per_sixteen_terms(dev, shape):
     """Activations behind a ReLU, half of them 0. A rounding is at most half of 2^-23 of the sum so far, in the mean 0.29 of it; the
-    sums so far are 0.71 of the last one in the mean: sqrt(roundings) * 2^-25 at most, K groups and slices a few more."""
+    sums so far are 0.71 of the last one in the mean: sqrt(roundings) * 2^-25 at most, K groups and slices a few more. (The gradients
+    too are of one sign: their weight gradient is nowhere near the cancellation that would make its error larger than that.)"""
     import torch
     import torch.nn.functional as F_
     from crusaderbackend_amd import capi
@@ -352,6 +353,10 @@ def test_a_sum_is_rounded_once_per_sixteen_terms(dev, shape):
     if s == 1:
         capi.conv_dgrad(Wt.to(dev), dY.to(dev), dX, g)
         checks.append((dX, F_.conv_transpose2d(dY.double(), Wt.double(), stride=s, padding=p), OC * F * F))
+    # (weight gradients: two roundings per sixteen pixels of a sum that K groups and slices hold in at least eight parts)
+    dW = torch.zeros(OC, IC, F, F, device=dev)
+    capi.conv_wgrad(dY.to(dev), X.to(dev), dW, g)
+    checks.append((dW, torch.nn.grad.conv2d_weight(X.double(), Wt.shape, dY.double(), stride=s, padding=p), 2 * N * g.OH * g.OW / 8))
     torch.cuda.synchronize()
     for got, want, K in checks:
         assert (got.cpu().double() - want).norm() <= np.sqrt(K / 16 + 16) * 2.0**-25 * want.norm()

@@ -29,7 +29,7 @@ def test_layers_of_the_built_in_buffer_stay_in_it():
 
 
 def test_short_weight_gradients_of_few_output_channels_stay_on_fp32():
-    """Under 32 output channels and 250 MFLOP the fp32 slices (two per CU: twice as many) are the faster."""
+    """Under 32 output channels and 400 MFLOP the fp32 slices (two per CU: twice as many) are the faster."""
     for shape, slices in (((2, 188, 27, 22, 28, 3, 1, 1), 5), ((51, 113, 7, 7, 26, 3, 1, 1), 10)):
         N, IC, H, W, OC, F, s, p = shape
         assert queries(*shape)[2] == slices * OC * IC * F * F * 4
