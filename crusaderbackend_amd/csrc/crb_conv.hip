@@ -5,6 +5,7 @@
 #include "conv3x3_tiled_wgrad.h"
 #include "conv3x3_wgrad.h"
 #include "conv3x3_wgrad_image.h"
+#include "conv_few.h"
 #include "conv_split.h"
 #include "conv_split_wgrad.h"
 #include "conv1x1_s2.h"
@@ -441,6 +442,21 @@ static bool direct_shape(const crb_conv_geom *g, u32 stride) {
     return g->FH == 3 && g->FW == 3 && g->sH == stride && g->sW == stride && g->pH == 1 && g->pW == 1 &&
            g->IH == stride * g->OH && g->IW == stride * g->OW;
 }
+// Forward passes of width-specialised layers and 2 x 2 images under eight images (calls of inference: conv_split_fwd_plan) on few
+// pixels. By chunks of the whole grid, whose rate is 7.3 ns beyond one round, against 12 to 17 us of the split kernel on short
+// contractions, 20 to 26 on long ones: seven images of 64 -> 64 @32, 1792 chunks, 21.0 against 14.0 us, but 128 -> 128 @16 18.2 against
+// 19.9 and 256 -> 256 @8 16.5 against 23.0; five of 64 -> 64 @32, 1280, 16.5 against 14.0; four 13.1 against 17.4. From 64 channels on:
+// 32 -> 32 @16 5.1 against 5.7 us, but seven images of 16 -> 16 @32 7.2 against 4.9. (px_tiles == 0: not taken)
+static ConvFewPlan few_plan(const crb_conv_geom *g) {
+    ConvFewPlan none;
+    const bool shape = g->FH == 3 && g->FW == 3 && g->sH == 1 && g->sW == 1 && g->pH == 1 && g->pW == 1;
+    if (!shape || g->N >= 8 || g->IC < 64 || !conv_few_shape(g->N, g->IC, g->IH, g->IW)) return none;
+    const ConvFewPlan p = conv_few_plan(g->N, g->IC, g->OC, g->IH, g->IW);
+    return uint64_t(p.px_tiles) * p.oc_tiles * ceil_div(g->IC, u32(kFewCh)) <= 16 * g->IC ? p : none;
+}
+static size_t few_scratch_bytes(const ConvFewPlan &p, const crb_conv_geom *g) {
+    return p.slices > 1 ? size_t(p.slices) * g->N * g->OC * g->OH * g->OW * sizeof(float) : 0;
+}
 // The plan of a layer's forward pass / data gradient (cfg < 0: not taken): square filters, one stride, any padding up to F - 1.
 static ConvSplitPlan make_conv_split_fwd_plan(const crb_conv_geom *g, bool aligned) {
     if (g->FH != g->FW || g->sH != g->sW || g->pH >= g->FH || g->pW >= g->FW) return ConvSplitPlan();
@@ -455,9 +471,8 @@ static ConvSplitPlan make_conv_split_fwd_plan(const crb_conv_geom *g, bool align
     // start (its loss grows 5-fold over the first update) carries these into 2 to 5 % of the second step's input gradient, or
     // with the forward pass kept 0.06 to 0.3 %.
     // Under eight images, where calls are inference, that kernel puts one long contraction each on a few dozen CUs and takes as long
-    // for one image as for seven; the split kernel cuts the contraction. One / seven images, us: 64 -> 64 @32 41 -> 16 / 42 -> 13,
-    // 64 -> 128 @16 24 -> 17 / 24 -> 17, 128 -> 128 @16 43 -> 17 / 44 -> 19, 256 -> 256 @8 49 -> 19 / 50 -> 22, 256 -> 512 @4 26 -> 21 /
-    // 27 -> 25, 512 -> 512 @4 49 -> 23 / 49 -> 25. Under K = 512 or 30 MFLOP the filters' and the slices' launches eat the gain.
+    // for one image as for seven. What few_plan leaves of these runs here, the contraction cut (seven images: 64 -> 64 @32 42 -> 14 us).
+    // Under K = 512 or 30 MFLOP the filters' and the slices' launches eat the gain.
     if (direct && (g->N >= 8 || g->sH != 1 || g->IC * 9 < 512)) return ConvSplitPlan();
     return conv_split_plan(g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, g->FH, g->sH, direct, direct ? 30.f : 100.f);
 }
@@ -1160,6 +1175,7 @@ static size_t fwd_scratch_bytes(const crb_conv_geom *g, bool aligned, bool split
         if (done) return 0;
     }
     if (pointwise_shape(g)) return gemm_scratch_bytes(g->OC, g->IH * g->IW, g->IC, g->N);
+    if (const ConvFewPlan p = few_plan(g); split && p.px_tiles) return few_scratch_bytes(p, g);
     if (split && !tiny2x2_shape(g))
         if (const ConvSplitPlan p = conv_split_fwd_plan(g, aligned); p.cfg >= 0) return p.bytes;
     if (tiny2x2_shape(g) && aligned) return gemm_scratch_bytes(g->N, g->OC * 4, g->IC * 4, 1, false);
@@ -1223,6 +1239,14 @@ int crb_conv_fwd(const float *W, const float *X, float *Y, const float *bias_or_
     if (pointwise_shape(g))
         return gemm_nn_rowbias(W, X, Y, g->OC, g->IH * g->IW, g->IC, g->N, bias_or_null,
                                (flags & CRB_FLAG_RELU) ? u32(EPI_RELU) : 0u, s, "crb_conv_fwd");
+    if (const ConvFewPlan p = few_plan(g); p.px_tiles) {
+        float *part = nullptr;
+        if (const size_t need = few_scratch_bytes(p, g)) {
+            const bool aligned = aligned16(X) && aligned16(Y);
+            if (int st = scratch_get_or_none(need, [&] { return fwd_scratch_bytes(g, aligned, false); }, s, "crb_conv_fwd", &part)) return st;
+        }
+        return launch_conv_few(p, W, X, Y, bias_or_null, part, g->N, g->IC, g->OC, g->IH, g->IW, flags & CRB_FLAG_RELU, s, "crb_conv_fwd");
+    }
     if (const ConvSplitPlan p = conv_split_fwd_plan(g, aligned16(X) && aligned16(Y)); p.cfg >= 0 && !tiny2x2_shape(g))
         return run_conv_split_fwd(p, W, X, Y, bias_or_null, g, flags & CRB_FLAG_RELU, aligned16(X) && aligned16(Y), s, "crb_conv_fwd");
     if (tiny2x2_shape(g) && aligned16(X) && aligned16(Y))
