@@ -41,13 +41,16 @@ namespace crb {
 // KS_ = 2 (single-chunk configurations only): the contraction runs in two halves of the chunk's channels. The
 // first half's rows are requested first and multiplied (all pixel blocks) while the second half's are still arriving; the
 // second half then runs group by group with the stores in between, as with KS_ = 1.
+// SUB_ > 1 (double-buffered configurations): that many chunks are staged at a time and multiplied one after the other, in
+// the order of SUB_ = 1: small tiles, whose chunk is 18 MFMAs, wait less often for their loads and at barriers.
 template <int W_, int ROWS_, int CI_, int OCT_, int PBW_, int OBW_, bool DGRAD_, int OCC_, int NBUF_ = 2, int S_ = 1, int FS_ = 3, int PGS_ = 1,
-          int KS_ = 1>
+          int KS_ = 1, int SUB_ = 1>
 struct DirectCfg {
     static constexpr int W = W_, ROWS = ROWS_, CI = CI_, OCT = OCT_, PBW = PBW_, OBW = OBW_, OCC = OCC_, NBUF = NBUF_, S = S_;
     static constexpr int FS = FS_, NT = FS_ * FS_;  // filter size, taps
     static constexpr int PGS = PGS_, PGC = PBW_ / PGS_;  // pixel-block groups per wave, blocks per group
     static constexpr int KS = KS_;
+    static constexpr int SUB = SUB_, CIS = CI_ * SUB_;  // chunks, channels staged at a time
     static constexpr bool STREAM_OUT = PGS_ > 1 || FS_ == 1;  // non-temporal output stores (see store_out)
     static constexpr bool DGRAD = DGRAD_;
     // W = 4: the grid is a 4x4 image and a tile is ROWS / 4 whole images stacked, each staged with its own halo rows
@@ -83,8 +86,9 @@ struct DirectCfg {
     static constexpr int CIP = CI + 1;            // k index of (tap, channel) in a filter row is tap*CIP + channel: odd tap stride
     static constexpr int WSTR_MIN = NT * CIP;      // filter row stride == 2 mod 4: the 32 lanes of a half-wave (16 rows x 2 k) hit distinct banks
     static constexpr int WSTR = WSTR_MIN + ((2 - WSTR_MIN % 4) + 4) % 4;
-    static constexpr int X_SIZE = CI * XP;
-    static constexpr int W_SIZE = OCT * WSTR;
+    static constexpr int X_SIZE = CIS * XP;
+    static constexpr int W_SUB = OCT * WSTR;       // filter slice of a chunk
+    static constexpr int W_SIZE = SUB * W_SUB;
     static constexpr int SMEM_FLOATS = NBUF_ * (X_SIZE + W_SIZE);
     static_assert(W == 4 || W == 8 || W == 16 || W == 32, "grid width");
     static_assert(!MI || (S == 1 && FS == 3 && ROWS % 4 == 0), "stacked 4x4 images: 3x3 stride 1 only");
@@ -168,10 +172,11 @@ __device__ __forceinline__ void conv3x3_body(const DirectArgs &a, const u32 bid,
 
     // ---- staging helpers ----------------------------------------------------------------------------
     // input rows: CI planes x XR rows x SW/4 quads
-    constexpr int XQ = CI * XR * (SW / 4);
+    constexpr int CIS = Cfg::CIS;
+    constexpr int XQ = CIS * XR * (SW / 4);
     constexpr int XNP = (XQ + kThreads - 1) / kThreads;
     // filter slice: one (filter row j, chunk channel c) pair per item, 9 contiguous taps each
-    constexpr int WQ = OCT * CI;
+    constexpr int WQ = OCT * CIS;
     constexpr int WNP = (WQ + kThreads - 1) / kThreads;
     constexpr int NT = Cfg::NT;
     v4f xreg[XNP];
@@ -209,7 +214,7 @@ __device__ __forceinline__ void conv3x3_body(const DirectArgs &a, const u32 bid,
             const u32 e = t + i * kThreads;
             // forward: lanes run over chunk channels c (filter row j = e / CI): W[oc0 + j][c0 + c][0..8]
             // dgrad:   lanes run over filter rows j (gradient channel c = e / OCT): W[c0 + c][oc0 + j][0..8]
-            const u32 j = Cfg::DGRAD ? e % OCT : e / CI, c = Cfg::DGRAD ? e / OCT : e % CI;
+            const u32 j = Cfg::DGRAD ? e % OCT : e / CIS, c = Cfg::DGRAD ? e / OCT : e % CIS;
             const float *src = Cfg::DGRAD ? a.Wt + ((size_t(c0) + c) * a.C_OUT + oc0 + j) * NT
                                           : a.Wt + ((size_t(oc0) + j) * a.C_IN + c0 + c) * NT;
             // channels past the tensor's extent (ragged last chunk / last channel tile) are staged as zeros
@@ -260,10 +265,10 @@ __device__ __forceinline__ void conv3x3_body(const DirectArgs &a, const u32 bid,
         for (int i = 0; i < WNP; ++i) {
             const u32 e = t + i * kThreads;
             if (WQ % kThreads == 0 || e < WQ) {
-                const u32 j = Cfg::DGRAD ? e % OCT : e / CI, c = Cfg::DGRAD ? e / OCT : e % CI;
+                const u32 j = Cfg::DGRAD ? e % OCT : e / CIS, c = Cfg::DGRAD ? e / OCT : e % CIS;
 #pragma unroll
                 for (int tap = 0; tap < NT; ++tap)
-                    dW[j * WSTR + tap * Cfg::CIP + c] = (Cfg::KS == 2 && !wok[i]) ? 0.f : wreg[i * NT + tap];
+                    dW[c / CI * Cfg::W_SUB + j * WSTR + tap * Cfg::CIP + c % CI] = (Cfg::KS == 2 && !wok[i]) ? 0.f : wreg[i * NT + tap];
             }
         }
     };
@@ -273,8 +278,8 @@ __device__ __forceinline__ void conv3x3_body(const DirectArgs &a, const u32 bid,
     };
 
     // ---- zero the halo columns of both buffers once (never overwritten afterwards) ---------------------
-    for (u32 e = t; e < u32(NBUF) * CI * XR; e += kThreads) {
-        float *row = &sX[0][0] + (e / (CI * XR)) * Cfg::X_SIZE + ((e % (CI * XR)) / XR) * XP + (e % XR) * XS;
+    for (u32 e = t; e < u32(NBUF) * CIS * XR; e += kThreads) {
+        float *row = &sX[0][0] + (e / (CIS * XR)) * Cfg::X_SIZE + ((e % (CIS * XR)) / XR) * XP + (e % XR) * XS;
         row[3] = 0.f;
         row[SW + 4] = 0.f;
     }
@@ -425,17 +430,18 @@ __device__ __forceinline__ void conv3x3_body(const DirectArgs &a, const u32 bid,
     } else if constexpr (NBUF == 1) {
         compute(sX[0], sW[0], AllP0{}, AllPC{});
     } else {
-        const u32 nchunk = (a.C_IN + CI - 1) / CI;
+        const u32 nchunk = (a.C_IN + CIS - 1) / CIS;
         for (u32 ch = 0; ch < nchunk; ++ch) {
             const bool more = ch + 1 < nchunk;
-            if (more) fetch((ch + 1) * CI);
-            if (ch & 1) {
-                compute(sX[NBUF - 1], sW[NBUF - 1], AllP0{}, AllPC{});
-                if (more) commit(sX[0], sW[0]);
+            if (more) fetch((ch + 1) * CIS);
+            const float *cx = sX[ch & 1 ? NBUF - 1 : 0], *cw = sW[ch & 1 ? NBUF - 1 : 0];
+            if constexpr (Cfg::SUB == 1) {
+                compute(cx, cw, AllP0{}, AllPC{});
             } else {
-                compute(sX[0], sW[0], AllP0{}, AllPC{});
-                if (more) commit(sX[NBUF - 1], sW[NBUF - 1]);
+                const u32 left = a.C_IN - ch * CIS, subs = left < u32(CIS) ? (left + CI - 1) / CI : u32(Cfg::SUB);
+                for (u32 s = 0; s < subs; ++s) compute(cx + s * (CI * XP), cw + s * Cfg::W_SUB, AllP0{}, AllPC{});
             }
+            if (more) commit(sX[ch & 1 ? 0 : NBUF - 1], sW[ch & 1 ? 0 : NBUF - 1]);
             __syncthreads();
         }
     }

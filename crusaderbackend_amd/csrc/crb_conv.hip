@@ -193,6 +193,9 @@ static int try_direct(const float *Wt, const float *X, float *Y, const float *bi
         return probe ? int(CRB_OK) : launch_direct<DirectCfg<__VA_ARGS__>>(Wt, X, Y, bias, N, C_IN, C_OUT, gH, in_H, relu, s, what);
     // output-channel tile: the smallest of 16 / 32 / 64 that covers C_OUT, 64 beyond; chunks of 16 input channels at
     // stride 1 when C_IN > 8, chunks of 8 otherwise (stride 2 stages wider / more rows per chunk)
+    // Small batches: a wave's time is its chain of MFMAs, as many blocks as it holds after one another, whether the chip is full or not.
+    // On few workgroups tiles of one or two blocks a wave take their place. The contraction stays in the order of the larger tiles'
+    // chunks, two of them staged at a time (SUB) where a chunk is only a few MFMAs: every bit of the results is the same.
     if constexpr (S == 1) {
         if (gW == 32) {
             // forward: the contraction in two halves, the second half's rows still arriving while the first is multiplied
@@ -215,6 +218,9 @@ static int try_direct(const float *Wt, const float *X, float *Y, const float *bi
             if (C_IN <= 4) { CRB_TRY(32, 8, 4, 16, 4, 1, DG, 2, 1, 1, 3, 4) }
             if (C_OUT > 32 && C_OUT <= 48 && N * (gH / 8) < 512) { CRB_TRY(32, 4, 8, 48, 2, 3, DG, 2, 2, 1) }
             if (C_OUT > 32 && C_OUT <= 48) { CRB_TRY(32, 8, 8, 48, 4, 3, DG, 2, 2, 1) }
+            // (small tiles on few workgroups: above; 64 -> 64, batch 8 / 12 / 32: 41 -> 9.7 / 41 -> 14 / 43 -> 23 us, at batch 64 46 against 44)
+            if (C_OUT > 32 && N * (gH / 4) * ceil_div(C_OUT, 16u) <= 512) { CRB_TRY(32, 4, 8, 16, 2, 1, DG, 2, 2, 1, 3, 1, 1, 2) }
+            if (C_OUT > 32 && N * (gH / 4) * ceil_div(C_OUT, 32u) <= 640) { CRB_TRY(32, 4, 8, 32, 2, 2, DG, 2, 2, 1, 3, 1, 1, 2) }
             if (C_OUT > 32) { CRB_TRY(32, 8, 8, 64, 4, 4, DG, 2, 2, 1) }
             if (C_OUT > 16) { CRB_TRY(32, 8, 8, 32, 4, 2, DG, 2, 2, 1) }
             CRB_TRY(32, 8, 8, 16, 4, 1, DG, 2, 2, 1)
@@ -227,7 +233,11 @@ static int try_direct(const float *Wt, const float *X, float *Y, const float *bi
             if (!DG && C_IN > 32 && C_IN <= 48 && C_OUT <= 16) { CRB_TRY(16, 8, 48, 16, 2, 1, DG, 2, 1, 1, 3, 2) }
             if (C_IN > 8 && C_IN <= 12 && C_OUT > 32 && C_OUT <= 48) { CRB_TRY(16, 4, 12, 48, 1, 3, DG, 2, 1, 1) }
             if (one_chunk_w16(N, C_IN, C_OUT, gH)) { CRB_TRY(16, 8, 32, 16, 2, 1, DG, 2, 1, 1, 3, 2) }
+            // (128 -> 128, batch 8 / 12 / 32: 43 -> 11 / 43 -> 15 / 43 -> 25 us, at batch 64, 2048 workgroups, 45 against 46; 128 -> 64 14.5 -> 9.2 /
+            // 14.6 -> 9.4 / 15.0 -> 13.7, at batch 64, 1024, 24 against 26)
+            if (C_OUT > 64 && N * (gH / 4) * ceil_div(C_OUT, 16u) <= 1280) { CRB_TRY(16, 4, 8, 16, 1, 1, DG, 2, 2, 1, 3, 1, 1, 2) }
             if (C_OUT > 64) { CRB_TRY(16, 8, 8, 64, 2, 4, DG, 2, 2, 1) }
+            if (C_OUT > 16 && C_IN > 16 && N * (gH / 4) * ceil_div(C_OUT, 16u) <= 512) { CRB_TRY(16, 4, 16, 16, 1, 1, DG, 2, 2, 1, 3, 1, 1, 2) }
             if (C_OUT > 16 && C_IN > 8) { CRB_TRY(16, 4, 16, 32, 1, 2, DG, 2, 2, 1) }
             if (C_OUT > 16) { CRB_TRY(16, 4, 8, 32, 1, 2, DG, 2, 2, 1) }
             CRB_TRY(16, 8, 8, 16, 2, 1, DG, 2, 2, 1)
@@ -240,6 +250,11 @@ static int try_direct(const float *Wt, const float *X, float *Y, const float *bi
             if (!DG && C_IN > 32 && C_IN <= 48 && C_OUT <= 16) { CRB_TRY(8, 8, 48, 16, 1, 1, DG, 2, 1, 1) }  // (batch 64: 5.0 -> 4.6 us)
             // 64 output channels with chunks of 8: chunks of 16 would need more LDS than lets two workgroups share a CU, and a
             // SIMD with a single wave issues its MFMAs a third slower
+            // (256 -> 256, batch 8 / 12 / 32 / 64: 50 -> 19 / 50 -> 20 / 50 -> 29 / 52 -> 47 us, at batch 128 90 against 90; 256 -> 128 26 -> 16 at
+            // batch 8 to 32, at batch 64, 512 workgroups, 26.5 against 30.5)
+            if (C_OUT > 128 && C_IN > 8 && N * (gH / 8) * ceil_div(C_OUT, 16u) <= 512) { CRB_TRY(8, 8, 8, 16, 1, 1, DG, 2, 2, 1, 3, 1, 1, 2) }
+            if (C_OUT > 128 && C_IN > 8 && N * (gH / 8) * ceil_div(C_OUT, 32u) <= 512) { CRB_TRY(8, 8, 8, 32, 1, 2, DG, 2, 2, 1, 3, 1, 1, 2) }
+            if (C_OUT > 64 && C_IN > 16 && N * (gH / 8) * ceil_div(C_OUT, 16u) <= 256) { CRB_TRY(8, 8, 16, 16, 1, 1, DG, 2, 2, 1, 3, 1, 1, 2) }
             if (C_OUT > 128 && C_IN > 8) { CRB_TRY(8, 8, 8, 64, 1, 4, DG, 2, 2, 1) }
             if (C_OUT > 64 && C_IN > 8) { CRB_TRY(8, 8, 16, 32, 1, 2, DG, 2, 2, 1) }
             if (C_IN > 8) { CRB_TRY(8, 8, 16, 16, 1, 1, DG, 2, 2, 1) }
@@ -248,6 +263,8 @@ static int try_direct(const float *Wt, const float *X, float *Y, const float *bi
         } else if (gW == 4) {  // 4x4 images, four stacked per tile
             // at most 32 output channels per workgroup: 64 need 95-115 KB of LDS, one workgroup per CU and so one wave per
             // SIMD (512 -> 512 at batch 128: forward 105.9 -> 96.9 us, data gradient 100.5 -> 91.3 us with 32)
+            // (512 -> 512, batch 8 to 32: 50 -> 32 us, batch 64, 512 workgroups, 50 -> 48, at batch 128 85 against 92; two chunks at a time 44)
+            if (C_OUT > 16 && C_IN > 8 && ceil_div(N, 4u) * ceil_div(C_OUT, 16u) <= 512) { CRB_TRY(4, 16, 16, 16, 1, 1, DG, 2, 2, 1) }
             if (C_OUT > 16 && C_IN > 8) { CRB_TRY(4, 16, 16, 32, 1, 2, DG, 2, 2, 1) }
             if (C_IN > 8) { CRB_TRY(4, 16, 16, 16, 1, 1, DG, 2, 2, 1) }
             CRB_TRY(4, 16, 8, 16, 1, 1, DG, 2, 2, 1)
