@@ -5,7 +5,9 @@ Network: 3x3 pad-1 convolutions 64,64,M,128,128,M,256x3,M,512x3,M,512x3,M with b
 at every M, then FC 512->512 + ReLU -> 10, softmax, cross-entropy; momentum update with L2 weight decay on the weights.
 The order of calls is the reference's Sequential (seann/containers/Sequential.cu:43-47 forward, :79-85 backward with
 xGrads then paramGrads per operand from last to first, :93-97 update): every operand's input gradient is computed,
-the first convolution's included. ReLU is a separate pass, as in the reference (no fused epilogue is used here).
+the first convolution's included. Two things take fewer passes than the reference's operators, with the same bits: a ReLU is
+applied by the layer that feeds it (its mask is where its output is positive), and all parameters are updated by one launch
+(batch 128: 44 launches, 0.24 ms, less).
 
 All device buffers are torch tensors; torch performs no arithmetic. `params()` copies the learnable state to numpy so
 a CPU replica can be run on identical values.
@@ -49,7 +51,7 @@ class Vgg16Step:
                 st = {"g": g, "IC": C, "OC": OC, "H": H,
                       "W": dev_randn(OC, C, 3, 3, std=math.sqrt(2.0 / (C * 9))), "b": dev_randn(OC, std=math.sqrt(2.0 / OC)),
                       "dW": zeros(OC, C, 3, 3), "dB": zeros(OC), "mW": zeros(OC, C, 3, 3), "mB": zeros(OC),
-                      "z": zeros(batch, OC, H, H), "dz": zeros(batch, OC, H, H),
+                      "dz": zeros(batch, OC, H, H),
                       "out": zeros(batch, OC, H, H), "dout": zeros(batch, OC, H, H),
                       "ws": torch.empty(max(nbytes // 4, 1), dtype=torch.float32, device=dev) if nbytes else None}
                 self.learn += [(st, "W", "dW", "mW", True), (st, "b", "dB", "mB", False)]
@@ -62,7 +64,7 @@ class Vgg16Step:
             st = {"IN": IN, "OUT": OUT, "relu": relu,
                   "W": dev_randn(OUT, IN, std=math.sqrt(2.0 / IN)), "b": dev_randn(OUT, std=math.sqrt(2.0 / IN)),
                   "dW": zeros(OUT, IN), "dB": zeros(OUT), "mW": zeros(OUT, IN), "mB": zeros(OUT),
-                  "z": zeros(batch, OUT), "dz": zeros(batch, OUT), "out": zeros(batch, OUT), "dout": zeros(batch, OUT)}
+                  "dz": zeros(batch, OUT), "out": zeros(batch, OUT), "dout": zeros(batch, OUT)}
             self.learn += [(st, "W", "dW", "mW", True), (st, "b", "dB", "mB", False)]
             self.fc.append(st)
             IN = OUT
@@ -70,6 +72,8 @@ class Vgg16Step:
         self.loss = zeros(1)
         n = capi.cross_entropy_scratch_floats(batch * classes)
         self.loss_scratch = zeros(max(n, 1))
+        self._update_key = None
+        self._lay_update_table()
         self.flops = self._flops()
 
     def _flops(self):
@@ -87,18 +91,13 @@ class Vgg16Step:
         cur = self.x
         for kind, st in self.stages:
             if kind == "conv":
-                c.conv_fwd(st["W"], cur, st["z"], st["b"], st["g"])
-                c.relu_fwd(st["z"], st["out"], st["z"].numel())
+                c.conv_fwd(st["W"], cur, st["out"], st["b"], st["g"], c.CRB_FLAG_RELU)
             else:
                 c.maxpool_fwd(cur, st["out"], st["rec"], B * st["C"], st["IH"], st["IH"], 2, 2, 2, 2)
             cur = st["out"]
         for st in self.fc:
-            c.linear_fwd(cur, st["W"], st["b"], st["z"], B, st["IN"], st["OUT"])
-            if st["relu"]:
-                c.relu_fwd(st["z"], st["out"], st["z"].numel())
-                cur = st["out"]
-            else:
-                cur = st["z"]
+            c.linear_fwd(cur, st["W"], st["b"], st["out"], B, st["IN"], st["OUT"], c.CRB_FLAG_RELU if st["relu"] else 0)
+            cur = st["out"]
         c.softmax(cur, self.probs, B, self.classes)
         c.cross_entropy_loss(self.probs, self.labels, self.loss_scratch, self.loss, B * self.classes)
 
@@ -111,7 +110,7 @@ class Vgg16Step:
             st = self.fc[i]
             src = self.fc[i - 1] if i > 0 else self.stages[-1][1]
             if st["relu"]:
-                c.relu_bwd(st["z"], st["dout"], st["dz"], st["z"].numel())
+                c.relu_bwd(st["out"], st["dout"], st["dz"], st["out"].numel())
             c.linear_dgrad(st["dz"], st["W"], src["dout"], B, st["IN"], st["OUT"])
             c.linear_wgrad(st["dz"], src["out"], st["dW"], st["dB"], B, st["IN"], st["OUT"])
         for i in range(len(self.stages) - 1, -1, -1):
@@ -121,15 +120,25 @@ class Vgg16Step:
             if kind == "pool":
                 c.maxpool_bwd(src_dout, st["dout"], st["rec"], B * st["C"], st["IH"], st["IH"], 2, 2, 2, 2)
             else:
-                c.relu_bwd(st["z"], st["dout"], st["dz"], st["z"].numel())
+                c.relu_bwd(st["out"], st["dout"], st["dz"], st["out"].numel())
                 c.conv_dgrad(st["W"], st["dz"], src_dout, st["g"])
                 c.conv_wgrad(st["dz"], src_out, st["dW"], st["g"], workspace=st["ws"])
                 c.conv_bias_grad(st["dz"], st["dB"], B, st["OC"], st["H"] * st["H"])
 
-    def update(self):
+    def _lay_update_table(self):
+        # long tensors in pieces, so that they spread over the chip; laid anew where a tensor or a rate was replaced
+        key = [(st[p].data_ptr(), st[g].data_ptr(), st[m].data_ptr()) for st, p, g, m, _ in self.learn] + [self.lr, self.beta, self.l2]
+        if key == self._update_key:
+            return
+        entries = []
         for st, p, g, m, is_weight in self.learn:
-            self.capi.momentum_apply(st[p], st[g], st[m], st[p].numel(), self.lr, self.beta,
-                                     1.0 - self.l2 if is_weight else 1.0)
+            for x, dx, mx in zip(*(st[k].view(-1).split(1 << 18) for k in (p, g, m))):
+                entries.append((x, dx, mx, self.lr, self.beta, 1.0 - self.l2 if is_weight else 1.0))
+        self._update_table, self._update_key = self.capi.momentum_table(self.torch, self.dev, entries), key
+
+    def update(self):
+        self._lay_update_table()
+        self.capi.momentum_apply_multi(*self._update_table)
 
     def step(self):
         self.forward()
