@@ -22,7 +22,7 @@
 
 namespace crb {
 
-template <int F_, int S_, int TM_, int TN_, int WM_, int WN_, int KG_, int MAXPX_, int AHEAD_ = 2, int BSET_ = 2>
+template <int F_, int S_, int TM_, int TN_, int WM_, int WN_, int KG_, int MAXPX_, int AHEAD_ = 2, int BSET_ = 2, int NBUF_ = 2>
 struct ConvSplitCfg {
     static constexpr int F = F_, S = S_, TM = TM_, TN = TN_, WM = WM_, WN = WN_, KG = KG_, MAXPX = MAXPX_;
     static constexpr int NT = F * F, CI = 16 * KG, KO = CI / 8, NTH = 64 * WM * WN * KG;
@@ -32,6 +32,9 @@ struct ConvSplitCfg {
     static_assert(KO * MAXPX % NTH == 0, "whole staging items per thread");
     static constexpr int AHEAD = AHEAD_;  // taps the filter fragments run ahead
     static constexpr int BSET = BSET_;    // 2: pixel fragments are read a tap ahead
+    // 1: the run has one place in LDS and the next chunk takes it between two barriers. The run of a strided 5x5 tile is large, its
+    // 25 taps per chunk many; two or three workgroups then share a CU, which two places would leave to one (96 KB).
+    static constexpr int NBUF = NBUF_;
 };
 
 struct ConvSplitArgs {
@@ -89,7 +92,7 @@ __global__ void __launch_bounds__(256) conv_split_filters_kernel(const float *__
 template <class C, bool PLAIN = false>
 __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) {
     constexpr int TM = C::TM, TN = C::TN, KG = C::KG, NT = C::NT, F = C::F, S = C::S, MAXPX = C::MAXPX, NSET = C::AHEAD + 1;
-    __shared__ __attribute__((aligned(16))) unsigned char smem[2 * C::STAGE];
+    __shared__ __attribute__((aligned(16))) unsigned char smem[C::NBUF * C::STAGE];
     // an XCD gets a contiguous run of tiles, the output-channel tiles of a pixel tile behind one another: they share X in its L2
     const u32 ntile = a.px_tiles * a.oc_tiles, q8 = ntile / kXcds, r8 = ntile % kXcds, xcd = blockIdx.x % kXcds;
     const u32 tile = xcd * q8 + (xcd < r8 ? xcd : r8) + blockIdx.x / kXcds;
@@ -225,7 +228,7 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
     commit(smem);
     lds_barrier();
     u32 buf = 0;
-    for (u32 chunk = chunk0; chunk < chunk1; ++chunk, buf = C::STAGE - buf) {
+    for (u32 chunk = chunk0; chunk < chunk1; ++chunk, buf = (C::NBUF - 1) * C::STAGE - buf) {
         if (chunk + 1 < chunk1) fetch(chunk + 1);
         if (C::BSET == 2) read_pixels(0, buf);
         // The scheduler is fenced tap by tap: left alone it sinks the requests made for later taps to where they are used.
@@ -237,7 +240,7 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
             if (BS == 1) read_pixels(0, buf + (tap / F * a.pitch + tap % F) * 16);
             else if (tap + 1 < NT) read_pixels((tap + 1) % BS, buf + ((tap + 1) / F * a.pitch + (tap + 1) % F) * 16);
             // the next chunk: split and stored in the shadow of the last taps' MFMAs (once more behind the last chunk, for nobody)
-            if (tap == (NT > 1 ? NT - 2 : 0)) commit(smem + (C::STAGE - buf));
+            if (C::NBUF == 2 && tap == (NT > 1 ? NT - 2 : 0)) commit(smem + (C::STAGE - buf));
 #pragma unroll
             for (int t = 0; t < kTerms; ++t)
 #pragma unroll
@@ -252,7 +255,7 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                if (tap == (NT > 1 ? NT - 2 : 0)) {
+                if (C::NBUF == 2 && tap == (NT > 1 ? NT - 2 : 0)) {
                     __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
                     __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
                 }
@@ -275,6 +278,10 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
                     for (int mi = 0; mi < TM; ++mi) fa[s][p][mi] = tmp[s][p][mi];
         }
         lds_barrier();
+        if constexpr (C::NBUF == 1) {
+            if (chunk + 1 < chunk1) commit(smem);
+            lds_barrier();
+        }
     }
 
     // ---- sums that are not finite: this wave's blocks once more, on the fp32 MFMA from the fp32 operands (split_bf16.h) ------
@@ -404,7 +411,7 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
     } else {
         // the K groups exchange their accumulators, BR blocks of every wave at a time; each sums (in group order) and stores a share
         constexpr int NB = TM * TN, BR = NB < KG ? NB : KG, NR = BR * 16 / KG;
-        static_assert(NB % BR == 0 && NR % 4 == 0 && BR * 4096 * C::WM * C::WN * KG <= 2 * C::STAGE, "exchange space");
+        static_assert(NB % BR == 0 && NR % 4 == 0 && BR * 4096 * C::WM * C::WN * KG <= C::NBUF * C::STAGE, "exchange space");
         float *x = reinterpret_cast<float *>(smem);
 #pragma unroll
         for (int q = 0; q < NB / BR; ++q) {

@@ -25,7 +25,9 @@ namespace crb {
 template <int F_, int S_, int WM_, int WN_, int KG_, int MAXPX_>
 struct SplitWgradCfg {
     static constexpr int F = F_, S = S_, WM = WM_, WN = WN_, KG = KG_, MAXPX = MAXPX_;
-    static constexpr int ROWS = F <= 3 ? F : 1, NTW = ROWS * F;  // filter rows, taps of a workgroup (5x5: one row, blockIdx.y)
+    // filter rows, taps of a workgroup. 5x5: one row, blockIdx.y; of X it then stages only the rows that its filter row meets, one for
+    // each row of dY
+    static constexpr int ROWS = F <= 3 ? F : 1, NTW = ROWS * F;
     static constexpr int NTH = 64 * WM * WN * KG, PXT = 16 * KG, OCT = 32 * WM, ICT = 32 * WN;
     static constexpr int XO = ICT / 8, DO = OCT / 8;             // channel octets
     // 64 bytes behind each octet: the four octets a transposing read touches then start 64 bytes apart in a 256-byte bank row
@@ -124,10 +126,10 @@ __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a
         const BufferRange dr = buffer_range(a.dY + (size_t(f.img) * a.OC + oc0) * a.OHW, (left * a.OC - oc0) * a.OHW);
         const u32 ox = threadIdx.x / MAXPX, od = threadIdx.x / PXT, k = threadIdx.x % PXT;  // first items' octets
         u32 dv, y, x, dimg, strip;
-        const u32 rr = S * f.y + xpr;
+        const u32 rr = (C::ROWS == 1 ? 1 : S) * f.y + xpr;
         dv = small_div(rr, a.m_prow);
         image(f, dv, dimg, strip);
-        const int iy = int(rr - dv * a.prow) - a.pad_y, ix = int(xpc + S * strip * a.SW) - a.pad_x;
+        const int iy = (C::ROWS == 1 ? S * int(rr - dv * a.prow) + fh0 : int(rr - dv * a.prow)) - a.pad_y, ix = int(xpc + S * strip * a.SW) - a.pad_x;
         // (positions behind the run are read too where they exist; no pixel names them)
         const bool xin = dimg < u32(left) && u32(iy) < a.H && u32(ix) < a.W;
         const u32 xbytes = ((dimg * a.IC + 8 * ox) * a.HW + u32(iy) * a.W + u32(ix)) * 4u, xoff = xin ? xbytes : kOutside;
@@ -184,7 +186,7 @@ __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a
             u32 k = kpos + 4 * i, dv, y, x;
             k = f.p + k < a.npix ? k : 0;  // (dY is zero there)
             pixel(f, k, dv, y, x);
-            xs[i] = ((dv * a.prow + S * (y - f.y) + fh0) * a.pitch + S * x) * 16 + x_lane;
+            xs[i] = ((dv * a.prow + (C::ROWS == 1 ? 1 : S) * (y - f.y)) * a.pitch + S * x) * 16 + x_lane;
         }
     };
     auto main_loop = [&](auto ragged_c) {
@@ -351,19 +353,27 @@ struct SplitWgradPlan {
     u32 strips = 0, pairs = 0, splits = 0, tiles = 0, tiles_z = 0;
     size_t workspace_bytes = 0;
 };
+// Padded rows of an image, positions of the longest run a tile touches.
+template <class C>
+inline u32 split_wgrad_prow(u32 OH) { return C::ROWS == 1 ? OH : C::S * (OH - 1) + C::F; }
+template <class C>
+inline u32 split_wgrad_window(u32 OH, u32 SW) {
+    const u32 pitch = C::S * (SW - 1) + C::F;
+    return C::ROWS == 1 ? conv_split_window(C::PXT, OH, SW, 1, 1) / SW * pitch : conv_split_window(C::PXT, OH, SW, C::F, C::S);
+}
 // most: bytes the slices may take
 template <class C>
 inline SplitWgradPlan split_wgrad_plan(u32 N, u32 IC, u32 OC, u32 H, u32 W, u32 OH, u32 OW, size_t most) {
     SplitWgradPlan p;
     for (u32 ns = ceil_div(OW, 64u); ns <= OW && ns <= 16; ++ns)
-        if (conv_split_window(C::PXT, OH, ceil_div(OW, ns), C::F, C::S) <= u32(C::MAXPX)) {
+        if (split_wgrad_window<C>(OH, ceil_div(OW, ns)) <= u32(C::MAXPX)) {
             p.strips = ns;
             break;
         }
     // small_div's range (quotients are rows, images or strips of one tile, so at most its pixels or run and the 16 strips), and the
     // images a tile touches within 2 GiB (buffer loads)
     static_assert(C::PXT + 16 < 4095 && C::MAXPX + 16 < 4095, "quotients of small_div");
-    const uint64_t sw = p.strips ? ceil_div(OW, p.strips) : 0, prow = C::S * (OH - 1) + C::F, run = C::MAXPX;
+    const uint64_t sw = p.strips ? ceil_div(OW, p.strips) : 0, prow = split_wgrad_prow<C>(OH), run = C::MAXPX;
     const bool small = (C::PXT + sw) * sw < (1u << 20) && (OH + C::PXT) * uint64_t(OH) < (1u << 20) && (prow + run) * prow < (1u << 20);
     const uint64_t images = p.strips ? uint64_t(C::PXT) / (uint64_t(OH) * ceil_div(OW, p.strips)) + 3 : 0;
     if (!p.strips || !small || images * IC * H * W * 4 > 0x7fffffffull || images * OC * OH * OW * 4 > 0x7fffffffull) {
@@ -390,7 +400,7 @@ inline int launch_split_wgrad(const SplitWgradPlan &p, const float *dY, const fl
     a.dY = dY, a.X = X, a.out = p.splits > 1 ? ws : dW;
     a.images = N, a.IC = IC, a.OC = OC, a.H = H, a.W = W, a.HW = H * W, a.OHW = OH * OW, a.OW = OW;
     a.strips = p.strips, a.SW = ceil_div(OW, p.strips), a.npix = N * p.strips * OH * a.SW;
-    a.prow = C::S * (OH - 1) + C::F, a.pitch = C::S * (a.SW - 1) + C::F;
+    a.prow = split_wgrad_prow<C>(OH), a.pitch = C::S * (a.SW - 1) + C::F;
     a.pad_y = pad_y, a.pad_x = pad_x;
     a.ic_tiles = ceil_div(IC, u32(C::ICT)), a.splits = p.splits, a.tiles = p.tiles, a.tiles_z = p.tiles_z;
     a.ohw.init(OH * a.SW), a.ow.init(a.SW), a.pitch_d.init(a.pitch), a.strip_d.init(p.strips);

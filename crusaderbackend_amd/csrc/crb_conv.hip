@@ -397,6 +397,17 @@ struct ConvSplitSet {
     typedef ConvSplitCfg<F, S, 1, 2, 2, 1, 4, 192, 2, 1> C3;
     typedef ConvSplitCfg<F, S, 1, 2, 1, S == 2 ? 2 : 4, 1, 384, 4, 2> C4;
 };
+// 5x5 stride 2: 128, 96 and 64 channels x 64 pixels on four, three and two waves, the run in one place (up to 512 positions, 48 KB).
+// Against the engine's gathers, forward (us): 30 -> 75 @61x47 batch 24 77.7 -> 35.8, 32 -> 64 @56 batch 32 81 -> 36, 128 -> 200 @31 batch 4 44 ->
+// 30; 24 random layers 0.98 to 3.1 times as fast, half of them under the line of conv_split_plan and unchanged.
+template <>
+struct ConvSplitSet<5, 2> {
+    typedef ConvSplitCfg<5, 2, 1, 2, 4, 1, 1, 512, 2, 1, 1> C0;
+    typedef ConvSplitCfg<5, 2, 1, 2, 3, 1, 1, 480, 2, 1, 1> C1;
+    typedef ConvSplitCfg<5, 2, 1, 2, 2, 1, 1, 512, 2, 1, 1> C2;
+    typedef C0 C3;
+    typedef C0 C4;
+};
 template <int F, int S>
 static ConvSplitPlan conv_split_plan_for(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 W, u32 OH, u32 OW, float &best_us) {
     typedef ConvSplitSet<F, S> Set;
@@ -427,6 +438,12 @@ static ConvSplitPlan conv_split_plan_for(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 
             }
         }
     };
+    if constexpr (F == 5 && S == 2) {
+        consider(0, typename Set::C0(), 0.64f, 2);
+        consider(1, typename Set::C1(), 0.5f, 2);
+        consider(2, typename Set::C2(), 0.32f, 2);
+        return best;
+    }
     consider(0, typename Set::C0(), S == 2 ? 0.32f : 0.64f, 2);
     consider(1, typename Set::C1(), 0.64f, 2);
     consider(2, typename Set::C2(), 0.68f, 1);  // (per step of 32 channels)
@@ -445,6 +462,7 @@ static ConvSplitPlan conv_split_plan(u32 N, u32 C_IN, u32 C_OUT, u32 H, u32 W, u
     if (F == 3 && S == 1) p = conv_split_plan_for<3, 1>(N, C_IN, C_OUT, H, W, OH, OW, us);
     if (F == 5 && S == 1) p = conv_split_plan_for<5, 1>(N, C_IN, C_OUT, H, W, OH, OW, us);
     if (F == 3 && S == 2) p = conv_split_plan_for<3, 2>(N, C_IN, C_OUT, H, W, OH, OW, us);
+    if (F == 5 && S == 2) p = conv_split_plan_for<5, 2>(N, C_IN, C_OUT, H, W, OH, OW, us);
     // against the fp32 kernels: the tiled one's throughput or, on few workgroups, the length of a workgroup's contraction; the
     // engine's throughput or, where a few images meet wide filters, the reading of these. There the filters' split does not pay
     // (fp32 / split, us: 1088 -> 1096 5x5 @4 batch 3 122 / 192, 1122 -> 1874 5x5 @5 batch 4 213 / 348, 1648 -> 2000 @10 batch 1 110 /
@@ -527,6 +545,8 @@ static int run_conv_split_fwd(const ConvSplitPlan &p, const float *W, const floa
     unsigned char *wf = nullptr;
     if (int st = scratch_get_or_none(p.bytes, [&] { return fwd_scratch_bytes(g, aligned, false); }, s, what, &wf)) return st;
     const int py = int(g->pH), px = int(g->pW);
+    if (g->sH == 2 && g->FH == 5)
+        return run_conv_split_set<5, 2, false>(p, W, X, Y, bias, wf, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, py, px, relu, s, what);
     if (g->sH == 2) return run_conv_split_set<3, 2, false>(p, W, X, Y, bias, wf, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, py, px, relu, s, what);
     if (g->FH == 5) return run_conv_split_set<5, 1, false>(p, W, X, Y, bias, wf, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, py, px, relu, s, what);
     return run_conv_split_set<3, 1, false>(p, W, X, Y, bias, wf, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, py, px, relu, s, what);
@@ -878,6 +898,13 @@ struct SplitWgradSet<3, 2> {
     typedef SplitWgradCfg<3, 2, 4, 1, 2, 256> C0;
     typedef C0 C1;
 };
+// (24 random layers of 5x5 stride 2 against the engine: 1.0 to 1.7 times as fast; 30 -> 75 @61x47 batch 24 63 -> 50 us, 32 -> 217 @54 batch 18
+// 110 -> 67. A tile is bound by its loads, 192 dword requests for 60 MFMAs a wave: each of the five filter rows stages anew.)
+template <>
+struct SplitWgradSet<5, 2> {
+    typedef SplitWgradCfg<5, 2, 2, 1, 4, 256> C0;
+    typedef C0 C1;
+};
 template <int F, int S>
 static SplitWgradChoice split_wgrad_choice_for(const crb_conv_geom *g, size_t most, float &best_us) {
     typedef SplitWgradSet<F, S> Set;
@@ -918,6 +945,7 @@ static SplitWgradChoice make_split_wgrad_choice(const crb_conv_geom *g) {
         if (g->FH == 5 && g->sH == 1) c = split_wgrad_choice_for<5, 1>(g, most, us);
         // (the stride-2 tile is 128 output channels wide: 32 -> 32 @56 batch 32 28 -> 31 us, 64 -> 128 @56 64 -> 51)
         if (g->FH == 3 && g->sH == 2 && g->OC >= 64) c = split_wgrad_choice_for<3, 2>(g, most, us);
+        if (g->FH == 5 && g->sH == 2) c = split_wgrad_choice_for<5, 2>(g, most, us);
         return c;
     };
     SplitWgradChoice c = choice(SIZE_MAX);
@@ -943,6 +971,7 @@ static int run_split_wgrad_set(const SplitWgradChoice &c, const float *dY, const
 }
 static int run_split_wgrad(const SplitWgradChoice &c, const float *dY, const float *X, float *dW, float *ws, const crb_conv_geom *g, hipStream_t s,
                            const char *what) {
+    if (g->sH == 2 && g->FH == 5) return run_split_wgrad_set<5, 2>(c, dY, X, dW, ws, g, s, what);
     if (g->sH == 2) return run_split_wgrad_set<3, 2>(c, dY, X, dW, ws, g, s, what);
     if (g->FH == 5) return run_split_wgrad_set<5, 1>(c, dY, X, dW, ws, g, s, what);
     return run_split_wgrad_set<3, 1>(c, dY, X, dW, ws, g, s, what);
