@@ -1,4 +1,4 @@
-// Convolution forward (stride S) and, at stride 1, data gradient on split bf16 operands (split_bf16.h), any image extent and any
+// Convolution forward (stride S) and data gradient (stride 1; stride 2 by residue classes, below) on split bf16 operands (split_bf16.h), any image extent and any
 // padding: Y[n][oc][y][x] = sum over (ic, fh, fw) of W[oc][ic][fh][fw] * X[n][ic][S*y + fh - pad][S*x + fw - pad]; the data
 // gradient is the same with dY as X, the filters' channel roles swapped and their taps mirrored.
 //
@@ -22,10 +22,10 @@
 
 namespace crb {
 
-template <int F_, int S_, int TM_, int TN_, int WM_, int WN_, int KG_, int MAXPX_, int AHEAD_ = 2, int BSET_ = 2, int NBUF_ = 2>
-struct ConvSplitCfg {
-    static constexpr int F = F_, S = S_, TM = TM_, TN = TN_, WM = WM_, WN = WN_, KG = KG_, MAXPX = MAXPX_;
-    static constexpr int NT = F * F, CI = 16 * KG, KO = CI / 8, NTH = 64 * WM * WN * KG;
+template <int FH_, int FW_, int S_, int TM_, int TN_, int WM_, int WN_, int KG_, int MAXPX_, int AHEAD_ = 2, int BSET_ = 2, int NBUF_ = 2>
+struct ConvSplitRect {
+    static constexpr int FH = FH_, FW = FW_, S = S_, TM = TM_, TN = TN_, WM = WM_, WN = WN_, KG = KG_, MAXPX = MAXPX_;
+    static constexpr int NT = FH * FW, CI = 16 * KG, KO = CI / 8, NTH = 64 * WM * WN * KG;
     static constexpr int OCT = 32 * TM * WM, PXT = 32 * TN * WN;
     static constexpr int PART = KO * MAXPX * 16, STAGE = kSplit * PART;  // bytes
     static constexpr int NP = KO * MAXPX / NTH;
@@ -37,11 +37,17 @@ struct ConvSplitCfg {
     static constexpr int NBUF = NBUF_;
 };
 
+template <int F_, int S_, int TM_, int TN_, int WM_, int WN_, int KG_, int MAXPX_, int AHEAD_ = 2, int BSET_ = 2, int NBUF_ = 2>
+struct ConvSplitCfg : ConvSplitRect<F_, F_, S_, TM_, TN_, WM_, WN_, KG_, MAXPX_, AHEAD_, BSET_, NBUF_> {
+    static constexpr int F = F_;
+};
+
 struct ConvSplitArgs {
     const float *X;
     const unsigned char *Wf;  // split filters
-    const float *Wt;          // the filters: element (output channel, input channel, tap) at oc * w_oc + ic * w_ic + tap (mirrored: NT-1-tap)
-    u32 w_oc, w_ic, mirrored;
+    const float *Wt;          // the filters: element (output channel, input channel, tap (i, j)) at oc * w_oc + ic * w_ic + tap0 + i * tap_i + j * tap_j
+    u32 w_oc, w_ic;
+    int tap0, tap_i, tap_j;
     float *Y;
     const float *bias;
     u32 C_IN, C_OUT, chunks;
@@ -56,6 +62,8 @@ struct ConvSplitArgs {
     size_t zstride;
     u32 z0, add;     // (PLAIN) the slice that blockIdx.z == 0 takes, and whether it adds to Y
     FastDiv ohw, ow, pitch_d, prow_d, strip_d;  // pixels of a strip, its width, ...
+    u32 osy, osx, oy0, ox0, out_w;  // (SCATTER) pixel (y, x) of the grid is (osy*y + oy0, osx*x + ox0) of a result `out_w` wide, OHW its pixels
+    __device__ __forceinline__ u32 w_tap(u32 tap, u32 fw) const { return u32(tap0 + int(tap / fw) * tap_i + int(tap % fw) * tap_j); }
 };
 
 // Filters -> fragments: [output block of 32][K group][chunk][tap][part] of 1 KB (lane l: output channel l % 32 of the block,
@@ -89,13 +97,13 @@ __global__ void __launch_bounds__(256) conv_split_filters_kernel(const float *__
 
 // PLAIN: for calls that no scratch can be had for. The filters are split as they are read, a lane's eight channels of a tap from eight
 // places, and slices of the contraction are launched one after the other, each adding to Y: the same bits, several times the time.
-template <class C, bool PLAIN = false>
-__global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) {
-    constexpr int TM = C::TM, TN = C::TN, KG = C::KG, NT = C::NT, F = C::F, S = C::S, MAXPX = C::MAXPX, NSET = C::AHEAD + 1;
-    __shared__ __attribute__((aligned(16))) unsigned char smem[C::NBUF * C::STAGE];
+// The work of workgroup `bid` of `px_tiles * oc_tiles`, slice `slice` of the launch; `smem`: C::NBUF * C::STAGE bytes.
+template <class C, bool PLAIN, bool SCATTER>
+__device__ __forceinline__ void conv_split_body(const ConvSplitArgs &a, const u32 bid, const u32 slice, unsigned char *smem) {
+    constexpr int TM = C::TM, TN = C::TN, KG = C::KG, NT = C::NT, FH = C::FH, FW = C::FW, S = C::S, MAXPX = C::MAXPX, NSET = C::AHEAD + 1;
     // an XCD gets a contiguous run of tiles, the output-channel tiles of a pixel tile behind one another: they share X in its L2
-    const u32 ntile = a.px_tiles * a.oc_tiles, q8 = ntile / kXcds, r8 = ntile % kXcds, xcd = blockIdx.x % kXcds;
-    const u32 tile = xcd * q8 + (xcd < r8 ? xcd : r8) + blockIdx.x / kXcds;
+    const u32 ntile = a.px_tiles * a.oc_tiles, q8 = ntile / kXcds, r8 = ntile % kXcds, xcd = bid % kXcds;
+    const u32 tile = xcd * q8 + (xcd < r8 ? xcd : r8) + bid / kXcds;
     const u32 pt = tile / a.oc_tiles, ot = tile % a.oc_tiles;
 
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = wv % (C::WM * C::WN), kgroup = wv / (C::WM * C::WN);
@@ -108,7 +116,7 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
     y0 = a.ow.div(r0);
     a.ohw.divmod(p1, n1, r1);
     y1 = a.ow.div(r1);
-    const u32 R0 = n0 * a.prow + S * y0, wpx = (n1 * a.prow + S * y1 + F - R0) * a.pitch;
+    const u32 R0 = n0 * a.prow + S * y0, wpx = (n1 * a.prow + S * y1 + FH - R0) * a.pitch;
     u32 b_lane[TN];  // LDS byte of the pixel's first tap, this lane's channel half
 #pragma unroll
     for (int ni = 0; ni < TN; ++ni) {
@@ -138,7 +146,7 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
     }
     float reg[C::NP][8];
     const bool ragged = a.C_IN % C::CI != 0;
-    const u32 chunk0 = (blockIdx.z + (PLAIN ? a.z0 : 0u)) * a.chunks_z, chunk1 = chunk0 + a.chunks_z < a.chunks ? chunk0 + a.chunks_z : a.chunks;
+    const u32 chunk0 = (slice + (PLAIN ? a.z0 : 0u)) * a.chunks_z, chunk1 = chunk0 + a.chunks_z < a.chunks ? chunk0 + a.chunks_z : a.chunks;
     auto fetch = [&](u32 chunk) {
         const u32 c0 = chunk * C::CI;
         if (ragged && chunk + 1 == a.chunks) {
@@ -187,7 +195,7 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const bool ok = oc < a.C_OUT && ic0 + j < a.C_IN;
-                    const float v = a.Wt[ok ? size_t(oc) * a.w_oc + size_t(ic0 + j) * a.w_ic + (a.mirrored ? NT - 1 - tap : tap) : 0];
+                    const float v = a.Wt[ok ? size_t(oc) * a.w_oc + size_t(ic0 + j) * a.w_ic + a.w_tap(tap, FW) : 0];
                     w[j] = ok ? v : 0.f;
                 }
                 u32x4 part[kSplit];
@@ -237,8 +245,8 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
             __builtin_amdgcn_sched_barrier(0);
             load_filters((tap + C::AHEAD) % NSET);  // (behind the last step: padding at the end of the filter buffer)
             constexpr int BS = C::BSET;
-            if (BS == 1) read_pixels(0, buf + (tap / F * a.pitch + tap % F) * 16);
-            else if (tap + 1 < NT) read_pixels((tap + 1) % BS, buf + ((tap + 1) / F * a.pitch + (tap + 1) % F) * 16);
+            if (BS == 1) read_pixels(0, buf + (tap / FW * a.pitch + tap % FW) * 16);
+            else if (tap + 1 < NT) read_pixels((tap + 1) % BS, buf + ((tap + 1) / FW * a.pitch + (tap + 1) % FW) * 16);
             // the next chunk: split and stored in the shadow of the last taps' MFMAs (once more behind the last chunk, for nobody)
             if (C::NBUF == 2 && tap == (NT > 1 ? NT - 2 : 0)) commit(smem + (C::STAGE - buf));
 #pragma unroll
@@ -316,7 +324,7 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
             const u32 tap = s % NT, c0 = (chunk0 + s / NT) * C::CI + 16 * kgroup;
 #pragma unroll
             for (int ni = 0; ni < TN; ++ni) {
-                const int iy = py[ni] + int(tap / F), ix = px[ni] + int(tap % F);
+                const int iy = py[ni] + int(tap / FW), ix = px[ni] + int(tap % FW);
                 f.in[ni] = u32(iy) < a.H && u32(ix) < a.W;
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
@@ -329,7 +337,7 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const u32 ic = c0 + 2 * j + h;
-                    const float w = wrow[mi][ic < a.C_IN ? size_t(ic) * a.w_ic + (a.mirrored ? NT - 1 - tap : tap) : 0];
+                    const float w = wrow[mi][ic < a.C_IN ? size_t(ic) * a.w_ic + a.w_tap(tap, FW) : 0];
                     f.w[j][mi] = ic < a.C_IN ? w : 0.f;
                 }
         };
@@ -385,7 +393,8 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
         a.strip_d.divmod(v, img, strip);
         xx += strip * a.SW;
         if (p >= a.npix || xx >= a.OW) return;
-        float *y = a.Y + blockIdx.z * a.zstride + size_t(img) * a.C_OUT * a.OHW + yy * a.OW + xx;
+        const u32 at = SCATTER ? (a.osy * yy + a.oy0) * a.out_w + a.osx * xx + a.ox0 : yy * a.OW + xx;
+        float *y = a.Y + slice * a.zstride + size_t(img) * a.C_OUT * a.OHW + at;
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
             const u32 oc = oc0 + 8 * (r / 4) + (r % 4);
@@ -435,10 +444,16 @@ __global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) 
     }
 }
 
+template <class C, bool PLAIN = false>
+__global__ void __launch_bounds__(C::NTH, 2) conv_split_kernel(ConvSplitArgs a) {
+    __shared__ __attribute__((aligned(16))) unsigned char smem[C::NBUF * C::STAGE];
+    conv_split_body<C, PLAIN, false>(a, blockIdx.x, blockIdx.z, smem);
+}
+
 // Positions of the longest run of padded rows that a tile of PXT consecutive pixels touches. Tiles start at multiples of PXT, so
 // their places inside an image repeat; where that takes long, the bound for any start.
-inline u32 conv_split_window(u32 pxt, u32 OH, u32 OW, u32 F, u32 S) {
-    const u32 ohw = OH * OW, prow = S * (OH - 1) + F, pitch = S * (OW - 1) + F;
+inline u32 conv_split_window(u32 pxt, u32 OH, u32 OW, u32 F, u32 FW, u32 S) {  // F: rows of the filter
+    const u32 ohw = OH * OW, prow = S * (OH - 1) + F, pitch = S * (OW - 1) + FW;
     u32 g = pxt, r = ohw;
     while (r) {
         const u32 t = g % r;
@@ -463,7 +478,7 @@ inline u32 conv_split_window(u32 pxt, u32 OH, u32 OW, u32 F, u32 S) {
 template <class C>
 inline u32 conv_split_strips(u32 OH, u32 OW) {
     for (u32 ns = ceil_div(OW, 64u); ns <= OW && ns <= 16; ++ns)
-        if (conv_split_window(C::PXT, OH, ceil_div(OW, ns), C::F, C::S) <= u32(C::MAXPX)) return ns;
+        if (conv_split_window(C::PXT, OH, ceil_div(OW, ns), C::FH, C::FW, C::S) <= u32(C::MAXPX)) return ns;
     return 0;
 }
 
@@ -473,6 +488,23 @@ inline size_t conv_split_filter_bytes(u32 C_IN, u32 C_OUT) {
     return (blocks * C::KG * chunks * C::NT + C::AHEAD) * kSplit * 1024;
 }
 
+// What does not depend on where the filters and the result lie. (OH, OW): pixel grid, (H, W): extent of X.
+template <class C>
+inline ConvSplitArgs conv_split_args(const float *Wt, const float *X, float *Y, const float *bias, unsigned char *Wf, u32 N, u32 C_IN, u32 C_OUT, u32 H,
+                                     u32 W, u32 OH, u32 OW, u32 strips, u32 slices, int pad_y, int pad_x) {
+    ConvSplitArgs a = {};
+    a.Wt = Wt, a.X = X, a.Wf = Wf, a.Y = Y, a.bias = bias;
+    a.C_IN = C_IN, a.C_OUT = C_OUT, a.chunks = ceil_div(C_IN, u32(C::CI));
+    a.strips = strips, a.SW = ceil_div(OW, strips);
+    a.images = N, a.H = H, a.W = W, a.HW = H * W, a.OHW = OH * OW, a.OW = OW, a.npix = N * strips * OH * a.SW;
+    a.prow = C::S * (OH - 1) + C::FH, a.pitch = C::S * (a.SW - 1) + C::FW;
+    a.pad_y = pad_y, a.pad_x = pad_x;
+    a.px_tiles = ceil_div(a.npix, u32(C::PXT)), a.oc_tiles = ceil_div(C_OUT, u32(C::OCT));
+    a.chunks_z = ceil_div(a.chunks, slices);
+    a.ohw.init(OH * a.SW), a.ow.init(a.SW), a.pitch_d.init(a.pitch), a.prow_d.init(a.prow), a.strip_d.init(strips);
+    return a;
+}
+
 // Wf: conv_split_filter_bytes of scratch, or null (PLAIN). (OH, OW): extent of the result, (H, W): of X; window origin (-pad_y, -pad_x); strips:
 // conv_split_strips. slices > 1: the contraction is cut; partial results go to `part` (slices x the result) and are summed in
 // fixed order by one more launch, which applies bias and ReLU.
@@ -480,18 +512,13 @@ template <class C, bool DGRAD>
 inline int launch_conv_split(const float *Wt, const float *X, float *Y, const float *bias, unsigned char *Wf, u32 N, u32 C_IN, u32 C_OUT, u32 H,
                              u32 W, u32 OH, u32 OW, u32 strips, u32 slices, float *part, int pad_y, int pad_x, u32 relu, hipStream_t s,
                              const char *what) {
-    ConvSplitArgs a;
-    a.Wt = Wt, a.w_oc = DGRAD ? C::NT : C_IN * C::NT, a.w_ic = DGRAD ? C_OUT * C::NT : C::NT, a.mirrored = DGRAD;
-    a.X = X, a.Wf = Wf, a.Y = slices > 1 ? part : Y, a.bias = slices > 1 ? nullptr : bias;
-    a.C_IN = C_IN, a.C_OUT = C_OUT, a.chunks = ceil_div(C_IN, u32(C::CI));
-    a.strips = strips, a.SW = ceil_div(OW, strips);
-    a.images = N, a.H = H, a.W = W, a.HW = H * W, a.OHW = OH * OW, a.OW = OW, a.npix = N * strips * OH * a.SW;
-    a.prow = C::S * (OH - 1) + C::F, a.pitch = C::S * (a.SW - 1) + C::F;
-    a.pad_y = pad_y, a.pad_x = pad_x;
-    a.px_tiles = ceil_div(a.npix, u32(C::PXT)), a.oc_tiles = ceil_div(C_OUT, u32(C::OCT)), a.relu = slices > 1 ? 0 : relu;
+    ConvSplitArgs a = conv_split_args<C>(Wt, X, Y, bias, Wf, N, C_IN, C_OUT, H, W, OH, OW, strips, slices, pad_y, pad_x);
+    a.w_oc = DGRAD ? C::NT : C_IN * C::NT, a.w_ic = DGRAD ? C_OUT * C::NT : C::NT;
+    a.tap0 = DGRAD ? C::NT - 1 : 0, a.tap_i = DGRAD ? -C::FW : C::FW, a.tap_j = DGRAD ? -1 : 1;
+    a.relu = relu;
+    if (slices > 1) a.Y = part, a.bias = nullptr, a.relu = 0;
     const u32 count = N * C_OUT * OH * OW;
-    a.chunks_z = ceil_div(a.chunks, slices), a.zstride = count;
-    a.ohw.init(OH * a.SW), a.ow.init(a.SW), a.pitch_d.init(a.pitch), a.prow_d.init(a.prow), a.strip_d.init(strips);
+    a.zstride = count;
     const uint64_t tiles = uint64_t(a.px_tiles) * a.oc_tiles;
     if (tiles > 0x7fffffffull) return fail(CRB_EINVAL_SHAPE, "%s: launch grid too large", what);
     const u32 total = a.oc_tiles * (C::OCT / 32) * C::KG * a.chunks * C::NT * 64;
@@ -512,6 +539,137 @@ inline int launch_conv_split(const float *Wt, const float *X, float *Y, const fl
     int st = check_launch(what);
     if (st == CRB_OK && slices > 1) st = launch_ordered_reduce(part, Y, count, slices, ReduceEpi{bias, OH * OW, C_OUT, relu ? u32(EPI_RELU) : 0u}, s, what);
     return st;
+}
+
+// ---- data gradient at stride 2: the four residue classes of input pixels -----------------------------------------------------------
+// dX(2y + py, 2x + px) only receives the taps fh = (py + pad) mod 2, + 2, ...: each class is a correlation of dY at stride 1 with 1 to 3 x 1
+// to 3 taps. One launch runs all four, the larger tap grids first; a workgroup belongs to one. R: taps of the largest grid on a side.
+template <int R_, int WM, int WN, int MAXPX>
+struct ConvSplitClassCfg {
+    static constexpr int R = R_;
+    typedef ConvSplitRect<R, R, 1, 1, 2, WM, WN, 1, MAXPX, 2, 2> C0;
+    typedef ConvSplitRect<R, R - 1, 1, 1, 2, WM, WN, 1, MAXPX, 2, 2> C1;
+    typedef ConvSplitRect<R - 1, R, 1, 1, 2, WM, WN, 1, MAXPX, 2, 2> C2;
+    typedef ConvSplitRect<R - 1, R - 1, 1, 1, 2, WM, WN, 1, MAXPX, 2, 2> C3;
+};
+struct ConvSplitClassArgs {
+    ConvSplitArgs c[4];
+    u32 first[4];  // workgroups of a class begin here
+};
+template <class Set, bool PLAIN>
+__global__ void __launch_bounds__(Set::C0::NTH, 2) conv_split_class_kernel(ConvSplitClassArgs a) {
+    __shared__ __attribute__((aligned(16))) unsigned char smem[2 * Set::C0::STAGE];
+    const u32 b = blockIdx.x;
+    if (b < a.first[1]) conv_split_body<typename Set::C0, PLAIN, true>(a.c[0], b, 0, smem);
+    else if (b < a.first[2]) conv_split_body<typename Set::C1, PLAIN, true>(a.c[1], b - a.first[1], 0, smem);
+    else if (b < a.first[3]) conv_split_body<typename Set::C2, PLAIN, true>(a.c[2], b - a.first[2], 0, smem);
+    else conv_split_body<typename Set::C3, PLAIN, true>(a.c[3], b - a.first[3], 0, smem);
+}
+// Fragments of the four classes' filters behind one another, each as conv_split_filters_kernel lays them. (C_IN: channels of dY)
+struct ConvSplitClassFilters {
+    u32 first[4], nt[4], fw[4];  // first 1 KB step of a class, its taps, taps in a row
+    int tap0[4], tap_i, tap_j;
+    u32 c_in, c_out, nt_all, chunks, total;
+};
+static __global__ void __launch_bounds__(256) conv_split_class_filters_kernel(const float *__restrict__ W, unsigned char *__restrict__ Wf,
+                                                                              ConvSplitClassFilters a) {
+    const u32 t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= a.total) return;
+    const u32 lane = t & 63, frag = t >> 6, k = frag < a.first[1] ? 0 : (frag < a.first[2] ? 1 : (frag < a.first[3] ? 2 : 3));
+    const u32 f = frag - a.first[k], tap = f % a.nt[k], rest = f / a.nt[k], ch = rest % a.chunks, ob = rest / a.chunks;
+    const u32 oc = ob * 32 + (lane & 31), ic0 = ch * 16 + 8 * (lane >> 5);
+    const u32 w_tap = u32(a.tap0[k] + int(tap / a.fw[k]) * a.tap_i + int(tap % a.fw[k]) * a.tap_j);
+    float w[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const bool ok = oc < a.c_out && ic0 + j < a.c_in;
+        const float v = W[ok ? (size_t(ic0 + j) * a.c_out + oc) * a.nt_all + w_tap : 0];
+        w[j] = ok ? v : 0.f;
+    }
+    u32x4 part[kSplit];
+    split8(w, part);
+    unsigned char *dst = Wf + size_t(frag) * (kSplit * 1024) + lane * 16;
+#pragma unroll
+    for (int p = 0; p < kSplit; ++p) *reinterpret_cast<u32x4 *>(dst + p * 1024) = part[p];
+}
+
+// Class k: its taps begin at (fh0, fw0) and are nfh x nfw, its pixels at (py, px) and CH x CW.
+struct ConvSplitClass {
+    u32 nfh, nfw, fh0, fw0, py, px, CH, CW;
+};
+inline ConvSplitClass conv_split_class(u32 k, u32 R, u32 IH, u32 IW, u32 pH, u32 pW) {
+    ConvSplitClass c;
+    c.nfh = R - k / 2, c.nfw = R - k % 2, c.fh0 = k / 2, c.fw0 = k % 2;  // (of an odd filter's taps, one more begin at 0)
+    c.py = (c.fh0 + pH) & 1, c.px = (c.fw0 + pW) & 1;
+    c.CH = IH > c.py ? ceil_div(IH - c.py, 2u) : 0, c.CW = IW > c.px ? ceil_div(IW - c.px, 2u) : 0;
+    return c;
+}
+// Column strips of the four classes; false: a class does not fit the LDS.
+template <class Set>
+inline bool conv_split_class_strips(u32 IH, u32 IW, u32 pH, u32 pW, u32 (&strips)[4]) {
+    for (u32 k = 0; k < 4; ++k) {
+        const ConvSplitClass c = conv_split_class(k, Set::R, IH, IW, pH, pW);
+        strips[k] = 1;
+        if (!c.CH || !c.CW) continue;
+        strips[k] = k == 0   ? conv_split_strips<typename Set::C0>(c.CH, c.CW)
+                    : k == 1 ? conv_split_strips<typename Set::C1>(c.CH, c.CW)
+                    : k == 2 ? conv_split_strips<typename Set::C2>(c.CH, c.CW)
+                             : conv_split_strips<typename Set::C3>(c.CH, c.CW);
+        if (!strips[k]) return false;
+    }
+    return true;
+}
+template <class Set>
+inline size_t conv_split_class_filter_bytes(u32 C_IN, u32 C_OUT) {
+    typedef typename Set::C0 C;
+    const size_t blocks = ceil_div(C_OUT, u32(C::OCT)) * (C::OCT / 32), chunks = ceil_div(C_IN, 16u), taps = (2 * Set::R - 1) * (2 * Set::R - 1);
+    return (blocks * chunks * taps + C::AHEAD) * kSplit * 1024;
+}
+// F = 2R - 1. Wf: conv_split_class_filter_bytes of scratch, or null (PLAIN).
+template <class Set>
+inline int launch_conv_split_classes(const float *Wt, const float *dY, float *dX, unsigned char *Wf, u32 N, u32 IC, u32 OC, u32 IH, u32 IW, u32 OH, u32 OW,
+                                     const u32 (&strips)[4], u32 pH, u32 pW, hipStream_t s, const char *what) {
+    typedef typename Set::C0 C;
+    constexpr u32 F = 2 * Set::R - 1;
+    ConvSplitClassArgs a = {};
+    ConvSplitClassFilters f = {};
+    f.c_in = OC, f.c_out = IC, f.nt_all = F * F, f.chunks = ceil_div(OC, 16u), f.tap_i = -2 * int(F), f.tap_j = -2;
+    const u32 blocks = ceil_div(IC, u32(C::OCT)) * (C::OCT / 32);
+    u32 steps = 0;
+    uint64_t tiles = 0;
+    for (u32 k = 0; k < 4; ++k) {
+        const ConvSplitClass g = conv_split_class(k, Set::R, IH, IW, pH, pW);
+        a.first[k] = u32(tiles);
+        f.first[k] = steps, f.nt[k] = g.nfh * g.nfw, f.fw[k] = g.nfw;
+        f.tap0[k] = int((g.fh0 + 2 * (g.nfh - 1)) * F + g.fw0 + 2 * (g.nfw - 1));  // (the last tap meets the window's first row and column)
+        const u32 first = steps;
+        steps += blocks * f.chunks * f.nt[k];
+        if (!g.CH || !g.CW) continue;
+        // tap i of pixel y reads row y + (py + pH) / 2 - i of dY
+        const int pad_y = int(g.nfh) - 1 - int((g.py + pH) / 2), pad_x = int(g.nfw) - 1 - int((g.px + pW) / 2);
+        auto fill = [&](auto cfg) {
+            ConvSplitArgs &c = a.c[k];
+            c = conv_split_args<decltype(cfg)>(Wt, dY, dX, nullptr, Wf ? Wf + size_t(first) * (kSplit * 1024) : nullptr, N, OC, IC, OH, OW, g.CH, g.CW,
+                                               strips[k], 1, pad_y, pad_x);
+            c.w_oc = F * F, c.w_ic = IC * F * F, c.tap0 = f.tap0[k], c.tap_i = f.tap_i, c.tap_j = f.tap_j;
+            c.OHW = IH * IW, c.out_w = IW, c.osy = c.osx = 2, c.oy0 = g.py, c.ox0 = g.px;
+            tiles += uint64_t(c.px_tiles) * c.oc_tiles;
+        };
+        if (k == 0) fill(typename Set::C0());
+        if (k == 1) fill(typename Set::C1());
+        if (k == 2) fill(typename Set::C2());
+        if (k == 3) fill(typename Set::C3());
+    }
+    if (tiles > 0x7fffffffull) return fail(CRB_EINVAL_SHAPE, "%s: launch grid too large", what);
+    if (!Wf) {
+        hipLaunchKernelGGL((conv_split_class_kernel<Set, true>), dim3(u32(tiles)), dim3(C::NTH), 0, s, a);
+        return check_launch(what);
+    }
+    f.total = steps * 64;
+    hipLaunchKernelGGL(conv_split_class_filters_kernel, dim3(ceil_div(f.total, 256u)), dim3(256), 0, s, Wt, Wf, f);
+    if (int st = check_launch(what)) return st;
+    hipLaunchKernelGGL((conv_split_class_kernel<Set, false>), dim3(u32(tiles)), dim3(C::NTH), 0, s, a);
+    return check_launch(what);
 }
 
 }  // namespace crb

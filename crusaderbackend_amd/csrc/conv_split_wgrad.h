@@ -359,7 +359,7 @@ inline u32 split_wgrad_prow(u32 OH) { return C::ROWS == 1 ? OH : C::S * (OH - 1)
 template <class C>
 inline u32 split_wgrad_window(u32 OH, u32 SW) {
     const u32 pitch = C::S * (SW - 1) + C::F;
-    return C::ROWS == 1 ? conv_split_window(C::PXT, OH, SW, 1, 1) / SW * pitch : conv_split_window(C::PXT, OH, SW, C::F, C::S);
+    return C::ROWS == 1 ? conv_split_window(C::PXT, OH, SW, 1, 1, 1) / SW * pitch : conv_split_window(C::PXT, OH, SW, C::F, C::F, C::S);
 }
 // most: bytes the slices may take
 template <class C>

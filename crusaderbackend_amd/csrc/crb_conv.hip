@@ -525,6 +525,83 @@ static ConvSplitPlan conv_split_fwd_plan(const crb_conv_geom *g, bool aligned) {
 static ConvSplitPlan conv_split_dgrad_plan(const crb_conv_geom *g, bool aligned) {
     return kept_plan<ConvSplitPlan>(g, 3 + aligned, [&] { return make_conv_split_dgrad_plan(g, aligned); });
 }
+// Data gradient at stride 2, 3x3 and 5x5 (conv_split.h: residue classes). 0: 64 channels x 128 pixels, 1: 32 x 256, 2: 128 x 64. A step
+// (16 channels of one tap) as in the forward pass; 7 us for the filters' launch and a workgroup's first and last phases. Against the fp32
+// class kernels (us): 30 <- 75 5x5 @61x47 batch 24 52 -> 32, 64 <- 128 3x3 @56 batch 16 53 -> 29, 219 <- 132 @16x19 batch 43 68 -> 32,
+// 256 <- 256 @14 batch 8 43 -> 34; 32 random layers that it takes 1.26 to 2.6 times as fast, distance from float64 a third.
+struct ConvSplitClassPlan {
+    int cfg = -1;
+    u32 strips[4] = {1, 1, 1, 1};
+    size_t bytes = 0;  // split filters
+};
+static bool tiled_classes_pay(const crb_conv_geom *g, bool *together);
+template <int R>
+struct ConvSplitClassSets {
+    typedef ConvSplitClassCfg<R, 2, 2, 256> S0;
+    typedef ConvSplitClassCfg<R, 1, 4, 384> S1;
+    typedef ConvSplitClassCfg<R, 4, 1, 256> S2;
+};
+template <int R>
+static ConvSplitClassPlan conv_split_class_plan_for(const crb_conv_geom *g, float &best_us) {
+    ConvSplitClassPlan best;
+    best_us = 3e38f;
+    const float wide = (R == 3 ? 4.8e-6f : 3.4e-6f) * g->IC * g->OC * g->FH * g->FW;
+    auto consider = [&](int id, auto set, float rate) {
+        typedef decltype(set) Set;
+        typedef typename Set::C0 C;
+        ConvSplitClassPlan p;
+        if (!conv_split_class_strips<Set>(g->IH, g->IW, g->pH, g->pW, p.strips)) return;
+        const u32 chunks = ceil_div(g->OC, 16u);
+        float steps = 0.f;
+        for (u32 k = 0; k < 4; ++k) {
+            const ConvSplitClass c = conv_split_class(k, R, g->IH, g->IW, g->pH, g->pW);
+            if (!c.CH || !c.CW) continue;
+            const u32 SW = ceil_div(c.CW, p.strips[k]);
+            // the images a tile touches lie within 2 GiB (buffer loads)
+            if ((uint64_t(C::PXT) / (uint64_t(c.CH) * SW) + 3) * g->OC * g->OH * g->OW * 4 > 0x7fffffffull) return;
+            steps += float(ceil_div(g->N * p.strips[k] * c.CH * SW, u32(C::PXT))) * ceil_div(g->IC, u32(C::OCT)) * c.nfh * c.nfw * chunks;
+        }
+        const float us = 7.f + wide + std::max(0.35f * R * R * chunks, steps * rate / 512.f);
+        if (us < best_us) best_us = us, best = p, best.cfg = id, best.bytes = conv_split_class_filter_bytes<Set>(g->OC, g->IC);
+    };
+    typedef ConvSplitClassSets<R> Sets;
+    consider(0, typename Sets::S0(), 0.64f);
+    consider(1, typename Sets::S1(), 0.66f);
+    consider(2, typename Sets::S2(), 0.64f);
+    return best;
+}
+static ConvSplitClassPlan make_conv_split_class_plan(const crb_conv_geom *g, bool aligned) {
+    ConvSplitClassPlan p;
+    if (g->FH != g->FW || g->sH != 2 || g->sW != 2 || g->pH >= g->FH || g->pW >= g->FW || g->OC < 16 || g->IC < 24) return p;
+    const float mflop = 2e-6f * g->N * g->OH * g->OW * g->IC * g->OC * g->FH * g->FW;
+    if (mflop < 100.f || uint64_t(g->IC) * g->OC * g->FH * g->FW * (2 * kSplit) > (256u << 20)) return p;
+    bool direct = false;
+    if (aligned && direct_shape(g, 2))
+        try_direct<true, 2>(nullptr, nullptr, nullptr, nullptr, g->N, g->OC, g->IC, g->OH, g->OW, g->OH, 0, nullptr, "", direct, true);
+    // (the engine's one gather, which cuts its contraction, stands behind the layers that neither class kernel takes: on those nothing is
+    // gained, 114 <- 182 5x5 @7 batch 14 39.7 / 39.3 us, and long contractions are closer to float64 cut)
+    if (direct || (!tiled_classes_pay(g, nullptr) && !dgrad_classes_pay(g))) return p;
+    float us = 3e38f;
+    if (g->FH == 3) p = conv_split_class_plan_for<2>(g, us);
+    if (g->FH == 5) p = conv_split_class_plan_for<3>(g, us);
+    // the fp32 kernels' throughput or, on few workgroups, the length of a contraction over the largest class's taps
+    const float k = float(g->OC * ((g->FH + 1) / 2) * ((g->FH + 1) / 2));
+    if (us > std::max(5.f + mflop / 38.f, 8.f + 0.033f * k)) p.cfg = -1;
+    return p;
+}
+static ConvSplitClassPlan conv_split_class_plan(const crb_conv_geom *g, bool aligned) {
+    return kept_plan<ConvSplitClassPlan>(g, 5 + aligned, [&] { return make_conv_split_class_plan(g, aligned); });
+}
+template <int R>
+static int run_conv_split_classes_set(const ConvSplitClassPlan &p, const float *W, const float *dY, float *dX, unsigned char *wf, const crb_conv_geom *g,
+                                      hipStream_t s, const char *what) {
+    typedef ConvSplitClassSets<R> Sets;
+    if (p.cfg == 0)
+        return launch_conv_split_classes<typename Sets::S0>(W, dY, dX, wf, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, p.strips, g->pH, g->pW, s, what);
+    if (p.cfg == 1)
+        return launch_conv_split_classes<typename Sets::S1>(W, dY, dX, wf, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, p.strips, g->pH, g->pW, s, what);
+    return launch_conv_split_classes<typename Sets::S2>(W, dY, dX, wf, g->N, g->IC, g->OC, g->IH, g->IW, g->OH, g->OW, p.strips, g->pH, g->pW, s, what);
+}
 template <int F, int S, bool DG>
 static int run_conv_split_set(const ConvSplitPlan &p, const float *Wt, const float *X, float *Y, const float *bias, unsigned char *wf, u32 N, u32 C_IN,
                               u32 C_OUT, u32 H, u32 W, u32 OH, u32 OW, int pad_y, int pad_x, u32 relu, hipStream_t s, const char *what) {
@@ -558,6 +635,13 @@ static int run_conv_split_dgrad(const ConvSplitPlan &p, const float *W, const fl
     const int py = int(g->FH) - 1 - int(g->pH), px = int(g->FW) - 1 - int(g->pW);
     if (g->FH == 5) return run_conv_split_set<5, 1, true>(p, W, dY, dX, nullptr, wf, g->N, g->OC, g->IC, g->OH, g->OW, g->IH, g->IW, py, px, 0, s, what);
     return run_conv_split_set<3, 1, true>(p, W, dY, dX, nullptr, wf, g->N, g->OC, g->IC, g->OH, g->OW, g->IH, g->IW, py, px, 0, s, what);
+}
+
+static int run_conv_split_classes(const ConvSplitClassPlan &p, const float *W, const float *dY, float *dX, const crb_conv_geom *g, bool aligned,
+                                  hipStream_t s, const char *what) {
+    unsigned char *wf = nullptr;
+    if (int st = scratch_get_or_none(p.bytes, [&] { return dgrad_scratch_bytes(g, aligned, false); }, s, what, &wf)) return st;
+    return g->FH == 3 ? run_conv_split_classes_set<2>(p, W, dY, dX, wf, g, s, what) : run_conv_split_classes_set<3>(p, W, dY, dX, wf, g, s, what);
 }
 
 // Direct kernel configurations for 1x1 / stride 1 / no padding layers <W, ROWS, CI, OCT, PBW, OBW, DGRAD, OCC, NBUF, S, FS=1>.
@@ -1301,6 +1385,8 @@ static size_t dgrad_scratch_bytes(const crb_conv_geom *g, bool aligned, bool spl
     if (pointwise_shape(g)) return gemm_scratch_bytes(g->IC, g->IH * g->IW, g->OC, g->N);
     if (split && !tiny2x2_shape(g))
         if (const ConvSplitPlan p = conv_split_dgrad_plan(g, aligned); p.cfg >= 0) return p.bytes;
+    if (split)
+        if (const ConvSplitClassPlan p = conv_split_class_plan(g, aligned); p.cfg >= 0) return p.bytes;
     if (tiny2x2_shape(g) && aligned) return gemm_scratch_bytes(g->N, g->IC * 4, g->OC * 4, 1, false);
     if (aligned && (direct_shape(g, 1) || direct_shape(g, 2))) {
         if (g->sH == 1)
@@ -1393,6 +1479,8 @@ int crb_conv_dgrad(const float *W, const float *dY, float *dX, const crb_conv_ge
     if (const ConvSplitPlan p = conv_split_dgrad_plan(g, aligned16(dY) && aligned16(dX));
         p.cfg >= 0 && !tiny2x2_shape(g))
         return run_conv_split_dgrad(p, W, dY, dX, g, aligned16(dY) && aligned16(dX), hipStream_t(stream), "crb_conv_dgrad");
+    if (const ConvSplitClassPlan p = conv_split_class_plan(g, aligned16(dY) && aligned16(dX)); p.cfg >= 0)
+        return run_conv_split_classes(p, W, dY, dX, g, aligned16(dY) && aligned16(dX), hipStream_t(stream), "crb_conv_dgrad");
     if (tiny2x2_shape(g) && aligned16(dY) && aligned16(dX))
         return conv2x2_dgrad(W, dY, dX, g->N, g->IC, g->OC, hipStream_t(stream), "crb_conv_dgrad");
     if (aligned16(dY) && aligned16(dX) && (direct_shape(g, 1) || direct_shape(g, 2))) {

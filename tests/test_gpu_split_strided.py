@@ -1,5 +1,6 @@
 """Strided layers on split bf16 operands where tiles, strips, chunks and filter rows end: 5x5 stride 2 forward and weight gradient
-(csrc/conv_split.h with one place for the run, csrc/conv_split_wgrad.h by filter rows)."""
+(csrc/conv_split.h with one place for the run, csrc/conv_split_wgrad.h by filter rows), 3x3 and 5x5 data gradient at stride 2 by residue
+classes (csrc/conv_split.h)."""
 import numpy as np
 import pytest
 
@@ -11,7 +12,9 @@ pytestmark = pytest.mark.gpu
 # (N, IC, H, W, OC, F, stride, pad): odd and even extents, every padding, channels that fill no chunk or block, one image row, many
 # strips, tiles that cross images, a cut contraction
 SHAPES = [(24, 30, 61, 47, 75, 5, 2, 2), (3, 31, 41, 39, 133, 5, 2, 1), (40, 50, 13, 12, 70, 5, 2, 4), (2, 90, 5, 151, 97, 5, 2, 0), (9, 233, 11, 13, 150, 5, 2, 2),
-          (64, 40, 9, 9, 100, 5, 2, 3), (5, 17, 64, 65, 193, 5, 2, 2), (33, 65, 15, 8, 65, 5, 2, 2)]
+          (64, 40, 9, 9, 100, 5, 2, 3), (5, 17, 64, 65, 193, 5, 2, 2), (33, 65, 15, 8, 65, 5, 2, 2),
+          (16, 64, 57, 55, 128, 3, 2, 1), (6, 200, 30, 28, 77, 3, 2, 1), (50, 33, 9, 8, 250, 3, 2, 0), (3, 130, 41, 96, 65, 3, 2, 2), (29, 28, 3, 50, 130, 5, 2, 3),
+          (90, 300, 7, 7, 90, 3, 2, 1), (200, 24, 2, 31, 120, 3, 2, 1)]
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
@@ -53,7 +56,7 @@ def test_strided_layers(dev, shape):
             capi.bind_workspace(None, stream=side)
 
 
-@pytest.mark.parametrize("shape", [SHAPES[1], SHAPES[4]], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("shape", [SHAPES[1], SHAPES[4], SHAPES[9], SHAPES[11]], ids=lambda s: "x".join(map(str, s)))
 def test_strided_layers_with_infinities(dev, shape):
     """Infinite operands and ones that round to infinity in 16 bits give what sums in fp32 give."""
     import torch
