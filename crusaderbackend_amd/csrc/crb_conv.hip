@@ -651,10 +651,28 @@ template <bool DG>
 static int try_pointwise(const float *Wt, const float *X, float *Y, const float *bias, u32 N, u32 C_IN, u32 C_OUT, u32 gH, u32 gW,
                          u32 relu, hipStream_t s, const char *what, bool &done, bool probe = false) {
     done = true;
+#define CRB_TRY(...)                                                                                          \
+    if (direct_fits<DirectCfg<__VA_ARGS__>>(C_IN, gH, gW))                                                     \
+        return probe ? int(CRB_OK) : launch_direct<DirectCfg<__VA_ARGS__>>(Wt, X, Y, bias, N, C_IN, C_OUT, gH, gH, relu, s, what);
+    // Small batches: tiles of 16 channels and four rows (an image @8), as many workgroups as there are; the batched products cut their
+    // contraction for want of tiles and add the slices in a second launch, and the streaming kernel has too few waves. Batch 8 / 16 / 32 (us):
+    // 204 -> 48 @32 10.5 -> 7.8 / 11.8 -> 9.7 / 15.1 -> 12.4, at batch 64, 1536 workgroups, 16 against 21; 288 -> 48 @16 12.5 -> 6.2 / 12.5 -> 6.3 /
+    // 9.8 -> 7.8; 330 -> 48 @8 17.0 -> 6.6 / 17.0 -> 6.7 / 16.9 -> 6.8; data gradients 48 -> 24 @32 5.3 -> 4.0, 48 -> 150 @8 5.5 -> 4.0. 70 random
+    // layers 1.19 (forward) and 1.28 times as fast in the mean. Not for one image, which is one small product (328 -> 206 @24x8 5.8 against
+    // 6.8), and not where the streaming kernel has a single block of channels (337 -> 11 @24x32 batch 46 13.1 against 16.3).
+    const bool stream = pw_stream_fits(N, DG ? C_IN : C_OUT, gH * gW);
+    if (N > 1 && C_IN <= 384 && !(stream && C_OUT <= 16)) {
+        const u32 wgs = N * ceil_div(gH, gW == 8 ? 8u : 4u) * ceil_div(C_OUT, 16u);
+        if (gW == 32 && wgs <= 1024) { CRB_TRY(32, 4, 16, 16, 2, 1, DG, 2, 2, 1, 1) }
+        if (gW == 16 && wgs <= 512 && C_IN >= 192) { CRB_TRY(16, 4, 48, 16, 1, 1, DG, 3, 2, 1, 1) }
+        if (gW == 16 && wgs <= 512) { CRB_TRY(16, 4, 16, 16, 1, 1, DG, 3, 2, 1, 1) }
+        if (gW == 8 && wgs <= 256 && C_IN >= 192) { CRB_TRY(8, 8, 48, 16, 1, 1, DG, 2, 2, 1, 1) }
+        if (gW == 8 && wgs <= 256) { CRB_TRY(8, 8, 16, 16, 1, 1, DG, 2, 2, 1, 1) }
+    }
     // large layers whose short side (forward: the output channels; data gradient: the contraction) fits one wave: the
     // activations go from global memory straight into the MFMAs (204 -> 48 @ 32x32, batch 64: forward 20.2 -> 17.0 us,
     // data gradient 23.0 -> 17.6 us)
-    if (pw_stream_fits(N, DG ? C_IN : C_OUT, gH * gW))
+    if (stream)
         return probe ? int(CRB_OK) : launch_pw_stream(DG, Wt, X, Y, bias, N, DG ? C_OUT : C_IN, DG ? C_IN : C_OUT, gH * gW, relu, s, what);
     if ((gW != 32 && gW != 16 && gW != 8) || gH % 8 != 0) {  // every configuration below tiles rows by 8 or 4
         done = false;
@@ -665,9 +683,6 @@ static int try_pointwise(const float *Wt, const float *X, float *Y, const float 
         const u32 nt = ceil_div(C_OUT, oct);
         return nt * oct * 3 <= C_OUT * 4 + 3 * 15 && tiles * nt >= 192;  // <= 25 % padding (one ragged 16-block allowed)
     };
-#define CRB_TRY(...)                                                                                          \
-    if (direct_fits<DirectCfg<__VA_ARGS__>>(C_IN, gH, gW))                                                     \
-        return probe ? int(CRB_OK) : launch_direct<DirectCfg<__VA_ARGS__>>(Wt, X, Y, bias, N, C_IN, C_OUT, gH, gH, relu, s, what);
     // long contractions with few workgroups: half-height tiles, so two workgroups share a CU and one multiplies while
     // the other waits for its next channel chunk
     const bool half = C_IN > 64 && tiles * ceil_div(C_OUT, 48u) < 512;
