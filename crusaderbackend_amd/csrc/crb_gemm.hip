@@ -173,7 +173,18 @@ static SplitChoice choose_split(u32 M, u32 N, u32 K, u32 zdim) {
 // Under 2^28 multiply-adds a call is mostly what every launch pays, and the fp32 engine's shorter prologue and smaller code are
 // ahead (fp32 / split, us: 700 x 600 x 100 7.8 / 10.8, 64 x 64 x 4096 8.6 / 10.4, 8 products of 16 x 528 x 41 5.5 / 6.1; above:
 // 528 x 2068 x 137 12.5 / 11.8, 768^3 19.4 / 15.6, 2000 x 2000 x 300 32.9 / 26.0).
+// The line lies lower for single products. Rows that are no multiple of 16 bytes long (`ragged`) the engine loads one element at
+// a time; there it is behind from 3 * 2^24 on (270 x 1277 x 150 13.6 / 9.5, 531 x 1268 x 111 9.7 / 6.6, 1215 x 337 x 281 16.5 /
+// 10.5, 223 x 1067 x 971 21.6 / 15.2; against it only 60 x 2270 x 685 13.4 / 14.0 and 180 x 672 x 817 12.2 / 13.2), but for
+// contractions under two slabs (768 x 1625 x 42 7.3 / 8.1, 2385 x 1236 x 55 10.2 / 12.1). On whole rows it is behind from 2^27
+// on (384 x 1920 x 256 9.5 / 9.0, 576 x 320 x 1216 15.9 / 13.4; below 1152 x 64 x 1216 10.6 / 11.7; short 2048 x 1856 x 64 10.8 /
+// 11.5). Of 90 random products of 2^24 to 2^28 the mean goes to 0.94 of its time, and the distance from float64 of those that move
+// to a third (2.2e-7 to 0.7e-7). The row lengths decide and not the addresses, so the bits do not depend on where a matrix lies.
 static bool split_pays(u32 M, u32 N, u32 K, u32 zdim) { return uint64_t(M) * N * K * zdim >= (uint64_t(1) << 28); }
+static bool split_pays_sooner(u32 M, u32 N, u32 K, u32 zdim, bool ragged) {
+    const uint64_t macs = uint64_t(M) * N * K;
+    return split_pays(M, N, K, zdim) || (zdim == 1 && (ragged ? macs >= (uint64_t(3) << 24) && K >= 64 : macs >= (uint64_t(1) << 27) && K >= 128));
+}
 
 template <class Cfg, class AOp, class BOp, class E>
 static int run_split_cfg(const AOp &a, const BOp &b, const E &e, u32 M, u32 N, u32 K, u32 zdim, const SplitChoice &c, hipStream_t s,
@@ -216,7 +227,7 @@ size_t gemm_scratch_bytes(u32 M, u32 N, u32 K, u32 zdim, bool one_launch_form) {
     size_t need = 0;
     if (one_launch_form) {
         if (tiny_gemm_fits(M, N, K, zdim)) return 0;  // one launch, no partial results
-        if (split_pays(M, N, K, zdim)) {
+        if (split_pays_sooner(M, N, K, zdim, true)) {  // (rows: the query does not know the form)
             const SplitChoice c = choose_split(M, N, K, zdim);
             need = c.splits > 1 ? size_t(c.splits) * M * N * sizeof(float) : 0;
             if (zdim != 1) return need;
@@ -271,7 +282,7 @@ static int gemm_nn(const float *A, const float *B, float *C, u32 M, u32 N, u32 K
         return launch_tiny_gemm(TinyGemmArgs{A, B, C, col_bias, row_bias, M, N, K, K, 1, N, 1, N, flags}, K, 0, 0, s, what);
     RowMajorEpi e{C, col_bias, N, M * N, flags};
     e.row_bias = row_bias;
-    if (split_pays(M, N, K, batch)) return run_split(SMatK<>{A, M, K, 0}, SMatR{B, N, N, K * N}, e, M, N, K, batch, s, what);
+    if (split_pays_sooner(M, N, K, batch, K % 4 || N % 4)) return run_split(SMatK<>{A, M, K, 0}, SMatR{B, N, N, K * N}, e, M, N, K, batch, s, what);
     if (K % 4 == 0 && N % 4 == 0 && aligned16(A) && aligned16(B))
         return run_tiles(MatK<true>{A, M, K, 0}, MatR<true>{B, N, N, K * N}, e, M, N, K, batch, s, what);
     return run_tiles(MatK<false>{A, M, K, 0}, MatR<false>{B, N, N, K * N}, e, M, N, K, batch, s, what);
@@ -290,7 +301,7 @@ static int gemm_tn(const float *A, const float *B, float *C, u32 M, u32 N, u32 K
     RowMajorAccEpi ea;  // the dense layers' weight gradient
     static_cast<RowMajorEpi &>(ea) = e;
     ea.a_rowsum = a_rowsum;
-    if (split_pays(M, N, K, batch)) {
+    if (split_pays_sooner(M, N, K, batch, M % 4 || N % 4)) {
         const SMatR a{A, M, M, 0}, b{B, N, N, K * N};
         if (flags & EPI_ACCUM) return run_split(a, b, ea, M, N, K, batch, s, what, rowsum_done);
         return run_split(a, b, e, M, N, K, batch, s, what);
@@ -308,7 +319,7 @@ static int gemm_nt(const float *A, const float *B, float *C, u32 M, u32 N, u32 K
     if (tiny_gemm_fits(M, N, K, 1, true))  // A (M x K) row-major, B stored N x K
         return launch_tiny_gemm(TinyGemmArgs{A, B, C, col_bias, nullptr, M, N, K, K, 1, 1, K, N, flags}, K, 0, 0, s, what);
     RowMajorEpi e{C, col_bias, N, 0, flags};
-    if (split_pays(M, N, K, 1)) return run_split(SMatK<>{A, M, K, 0}, SMatK<>{B, N, K, 0}, e, M, N, K, 1, s, what);
+    if (split_pays_sooner(M, N, K, 1, K % 4)) return run_split(SMatK<>{A, M, K, 0}, SMatK<>{B, N, K, 0}, e, M, N, K, 1, s, what);
     if (K % 4 == 0 && aligned16(A) && aligned16(B)) return run_tiles(MatK<true>{A, M, K, 0}, MatK<true>{B, N, K, 0}, e, M, N, K, 1, s, what);
     return run_tiles(MatK<false>{A, M, K, 0}, MatK<false>{B, N, K, 0}, e, M, N, K, 1, s, what);
 }
