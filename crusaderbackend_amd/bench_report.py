@@ -45,7 +45,8 @@ def conv_on_split(capi, g, which):
 
 
 def product_on_split(M, N, K):
-    return M * N * K >= 1 << 28
+    """Whether a product on whole rows (multiples of four floats, as all here) runs on split operands."""
+    return M * N * K >= 1 << 28 or (M * N * K >= 1 << 27 and 192 <= K < 512)
 
 
 def _entry(name, ms, flops, nbytes, split=False):

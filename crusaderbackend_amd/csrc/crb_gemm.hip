@@ -174,16 +174,20 @@ static SplitChoice choose_split(u32 M, u32 N, u32 K, u32 zdim) {
 // ahead (fp32 / split, us: 700 x 600 x 100 7.8 / 10.8, 64 x 64 x 4096 8.6 / 10.4, 8 products of 16 x 528 x 41 5.5 / 6.1; above:
 // 528 x 2068 x 137 12.5 / 11.8, 768^3 19.4 / 15.6, 2000 x 2000 x 300 32.9 / 26.0).
 // The line lies lower for single products. Rows that are no multiple of 16 bytes long (`ragged`) the engine loads one element at
-// a time; there it is behind from 3 * 2^24 on (270 x 1277 x 150 13.6 / 9.5, 531 x 1268 x 111 9.7 / 6.6, 1215 x 337 x 281 16.5 /
-// 10.5, 223 x 1067 x 971 21.6 / 15.2; against it only 60 x 2270 x 685 13.4 / 14.0 and 180 x 672 x 817 12.2 / 13.2), but for
-// contractions under two slabs (768 x 1625 x 42 7.3 / 8.1, 2385 x 1236 x 55 10.2 / 12.1). On whole rows it is behind from 2^27
-// on (384 x 1920 x 256 9.5 / 9.0, 576 x 320 x 1216 15.9 / 13.4; below 1152 x 64 x 1216 10.6 / 11.7; short 2048 x 1856 x 64 10.8 /
-// 11.5). Of 90 random products of 2^24 to 2^28 the mean goes to 0.94 of its time, and the distance from float64 of those that move
-// to a third (2.2e-7 to 0.7e-7). The row lengths decide and not the addresses, so the bits do not depend on where a matrix lies.
+// a time; there it is behind from 3 * 2^24 on if the contraction is under 512 long and so is not cut (270 x 1277 x 150 13.6 / 9.5,
+// 531 x 1268 x 111 9.7 / 6.6, 1215 x 337 x 281 16.5 / 10.5, 513 x 513 x 257 14.0 / 9.3; against it under two slabs, 768 x 1625 x 42
+// 7.3 / 8.1, 2385 x 1236 x 55 10.2 / 12.1), and from 2^27 on if it is (223 x 1067 x 971 21.6 / 15.2, 33 x 2047 x 2047 17.9 / 11.9,
+// 511 x 513 x 511 16.7 / 12.6; below 180 x 672 x 817 12.2 / 13.2, 63 x 63 x 16383 14.9 / 16.8, 256 x 1001 x 513 TN added 12.8 / 14.9).
+// On whole rows it is behind from 2^27 on for contractions that fill a few slabs and are not cut (1024 x 512 x 256 11.0 / 8.0, 128 x
+// 4096 x 256 10.9 / 7.9, 640 x 640 x 384 13.2 / 9.7; 2048 x 1856 x 64 10.8 / 11.5, 512 x 2048 x 128 6.2 / 6.4, 128 x 2048 x 512
+// 8.9 / 11.1, 128 x 128 x 8192 10.2 / 13.0). The distance from float64 of those that move goes to a third (2.2e-7 to 0.7e-7). The
+// row lengths decide and not the addresses, so the bits do not depend on where a matrix lies.
 static bool split_pays(u32 M, u32 N, u32 K, u32 zdim) { return uint64_t(M) * N * K * zdim >= (uint64_t(1) << 28); }
 static bool split_pays_sooner(u32 M, u32 N, u32 K, u32 zdim, bool ragged) {
     const uint64_t macs = uint64_t(M) * N * K;
-    return split_pays(M, N, K, zdim) || (zdim == 1 && (ragged ? macs >= (uint64_t(3) << 24) && K >= 64 : macs >= (uint64_t(1) << 27) && K >= 128));
+    if (split_pays(M, N, K, zdim) || zdim != 1) return split_pays(M, N, K, zdim);
+    if (K >= 512) return ragged && macs >= (uint64_t(1) << 27);
+    return ragged ? K >= 64 && macs >= (uint64_t(3) << 24) : K >= 192 && macs >= (uint64_t(1) << 27);
 }
 
 template <class Cfg, class AOp, class BOp, class E>

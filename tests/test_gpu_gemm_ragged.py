@@ -1,12 +1,13 @@
 """Products on either side of the lines from which split operands take them (csrc/crb_gemm.hip, split_pays_sooner): rows that are
-no multiple of 16 bytes long from 3 * 2^24 multiply-adds, whole rows from 2^27."""
+no multiple of 16 bytes long from 3 * 2^24 multiply-adds, 2^27 where the contraction is cut; whole rows from 2^27 where it is not."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 # (M, N, K)
-SIZES = [(270, 1277, 150), (271, 1277, 145), (1201, 875, 64), (1201, 890, 63), (1216, 864, 128), (1024, 1024, 128), (1028, 1024, 127), (59, 719, 1961), (33, 2047, 997)]
+SIZES = [(270, 1277, 150), (271, 1277, 145), (1201, 875, 64), (1201, 890, 63), (768, 912, 192), (768, 916, 191), (512, 513, 511), (513, 513, 512),
+         (129, 2031, 513), (33, 2047, 1987)]
 
 
 @pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
