@@ -7,7 +7,10 @@
 // v_mfma_f32_16x16x4_f32 (wave64, lane l): A value = A[i = l%16][k = l/16], B value = B[k = l/16][j = l%16], accumulator
 // register r = C[4*(l/16) + r][l%16]. When both operands are contiguous along k, a lane loads 16 bytes — the k values
 // 16 s + 4 (l/16) + t, t = 0..3 — and feeds them to four MFMAs in turn (A and B agree on the order, which is all the
-// contraction needs).
+// contraction needs). That load asks for no more than the element's alignment: rows of any length at any address take it, and
+// up to three k past the last quad are one MFMA more. Element by element a lane's 64 loads of a row share a line with three
+// other lanes only, sixteen lines an instruction (NT, K no multiple of 4, us: 255 x 257 x 2047 38.1 -> 16.4, 63 x 1025 x 2047
+// 37.9 -> 17.2, 30 x 510 x 4090 44.2 -> 16.1, 126 x 510 x 1022 12.9 -> 5.9, 62 x 1022 x 1022 12.9 -> 6.1).
 #pragma once
 #include "igemm_engine.h"
 
@@ -55,20 +58,22 @@ __global__ void __launch_bounds__(256) tiny_gemm_kernel(TinyGemmArgs a) {
     v4f acc = {0.f, 0.f, 0.f, 0.f};
     float asum = 0.f;  // this lane's share of row li's sum of A
     if constexpr (KVEC) {
-        // both operands contiguous along k, K % 4 == 0, 16-byte aligned rows
+        // both operands contiguous along k; a batch entry's contraction a multiple of 4
+        typedef float v4fu __attribute__((ext_vector_type(4), aligned(4)));
+        const u32 kq = ke & ~3u;
         const float *pa = a.A + size_t(row0 + li) * a.a_rs;
         const float *pb = a.B + size_t(col0 + li) * a.b_cs;
         constexpr int U = 4;  // 16-k groups requested together
-        for (u32 k = kb; k < ke; k += 16 * U) {
+        for (u32 k = kb; k < kq; k += 16 * U) {
             v4f va[U], vb[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const u32 kk = k + 16 * u + 4 * g;
-                const bool in = kk < ke;  // ke, kk and the batch length are multiples of 4: a quad is inside or outside as a whole
+                const bool in = kk < kq;  // kq, kk and a batch entry's length are multiples of 4: a quad is inside or outside as a whole
                 u32 nd, kr;
                 a.kb_len.divmod(kk, nd, kr);
-                va[u] = (in && row_ok) ? *reinterpret_cast<const v4f *>(pa + size_t(nd) * a.a_bs + kr) : v4f{0.f, 0.f, 0.f, 0.f};
-                vb[u] = (in && col_ok) ? *reinterpret_cast<const v4f *>(pb + size_t(nd) * a.b_bs + kr) : v4f{0.f, 0.f, 0.f, 0.f};
+                va[u] = (in && row_ok) ? v4f(*reinterpret_cast<const v4fu *>(pa + size_t(nd) * a.a_bs + kr)) : v4f{0.f, 0.f, 0.f, 0.f};
+                vb[u] = (in && col_ok) ? v4f(*reinterpret_cast<const v4fu *>(pb + size_t(nd) * a.b_bs + kr)) : v4f{0.f, 0.f, 0.f, 0.f};
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
@@ -78,6 +83,12 @@ __global__ void __launch_bounds__(256) tiny_gemm_kernel(TinyGemmArgs a) {
                 acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va[u].z, vb[u].z, acc, 0, 0, 0);
                 acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va[u].w, vb[u].w, acc, 0, 0, 0);
             }
+        }
+        if (kq < ke && kb <= kq) {  // K % 4 more (no batch then), in the wave that holds them
+            const bool in = kq + g < ke;
+            const float va = (in && row_ok) ? pa[kq + g] : 0.f, vb = (in && col_ok) ? pb[kq + g] : 0.f;
+            asum += va;
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va, vb, acc, 0, 0, 0);
         }
     } else {
         const float *pa = a.A + size_t(row0 + li) * a.a_rs;
@@ -144,8 +155,7 @@ inline int launch_tiny_gemm(TinyGemmArgs a, u32 kb_len, u32 a_bs, u32 b_bs, hipS
     a.tiles_n = ceil_div(a.N, 16u);
     a.k_per_wave = ceil_div(ceil_div(a.K, 4u), 16u) * 16u;
     const u32 blocks = ceil_div(a.M, 16u) * a.tiles_n;
-    const bool kvec = a.a_ks == 1 && a.b_ks == 1 && kb_len % 4 == 0 && a_bs % 4 == 0 && b_bs % 4 == 0 && a.a_rs % 4 == 0 && a.b_cs % 4 == 0 &&
-                      (reinterpret_cast<uintptr_t>(a.A) & 15u) == 0 && (reinterpret_cast<uintptr_t>(a.B) & 15u) == 0;
+    const bool kvec = a.a_ks == 1 && a.b_ks == 1 && (kb_len == a.K || (kb_len % 4 == 0 && a_bs % 4 == 0 && b_bs % 4 == 0));
     if (kvec)
         hipLaunchKernelGGL(tiny_gemm_kernel<true>, dim3(blocks), dim3(256), 0, s, a);
     else

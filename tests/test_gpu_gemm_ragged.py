@@ -61,3 +61,45 @@ def test_dense_layers_around_the_lines(dev, batch, IN, OUT):
         assert e.status == capi.CRB_EWORKSPACE
     finally:
         capi.bind_workspace(None, stream=side)
+
+
+# K one past / one short of a quad, of a wave's share and of the group of loads; blocks of 16 that are not full
+@pytest.mark.parametrize("size", [(1, 1, 1), (17, 33, 3), (16, 16, 5), (5, 70, 66), (33, 31, 255), (20, 18, 257), (130, 125, 1021), (30, 510, 4090)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_small_products_on_ragged_contractions(dev, size):
+    """Both operands contiguous along a contraction that is no multiple of four, at any address: the same bits."""
+    import torch
+    from crusaderbackend_amd import capi
+
+    M, N, K = size
+
+    def at(t, off):
+        buf = torch.full((t.numel() + 8,), float("nan"), device=dev)
+        buf[off:off + t.numel()] = t.flatten()
+        return buf[off:off + t.numel()].view(t.shape)
+
+    A, B, bias, C0 = torch.randn(M, K, device=dev), torch.randn(N, K, device=dev), torch.randn(N, device=dev), torch.randn(M, N, device=dev)
+    first = None
+    for oa, ob in ((0, 0), (1, 0), (3, 2)):
+        Y, C = torch.empty(M, N, device=dev), C0.clone()
+        capi.linear_fwd(at(A, oa), at(B, ob), bias, Y, M, K, N, capi.CRB_FLAG_RELU)
+        capi.sgemm_nta(at(A, oa), at(B, ob), C, M, N, K, 1)
+        first = first or (Y, C)
+        assert torch.equal(Y, first[0]) and torch.equal(C, first[1])
+    p = A.cpu().double() @ B.cpu().double().t()
+    for got, ref in ((first[0], (p + bias.cpu().double()).relu()), (first[1], p + C0.cpu().double())):
+        assert (got.cpu().double() - ref).norm() <= 2 * np.sqrt(K + 2) * 2.0**-25 * (p.norm() + ref.norm())
+
+
+@pytest.mark.parametrize("K", [3, 8, 30])
+def test_small_products_over_a_batch(dev, K):
+    """Entries that end inside a quad, and whole ones at an odd address."""
+    import torch
+    from crusaderbackend_amd import capi
+
+    M, N, batch = 19, 33, 7
+    A, B = (torch.randn(batch * r * K + 1, device=dev)[1:].view(batch, r, K) for r in (M, N))
+    C = torch.zeros(M, N, device=dev)
+    capi.sgemm_nta(A, B, C, M, N, K, batch)
+    ref = sum(a.double() @ b.double().t() for a, b in zip(A.cpu(), B.cpu()))
+    assert (C.cpu().double() - ref).norm() <= 2 * np.sqrt(K * batch) * 2.0**-25 * ref.norm()
