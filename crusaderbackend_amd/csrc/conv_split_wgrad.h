@@ -63,9 +63,119 @@ __device__ __forceinline__ bf16x8 read_transposed(const unsigned char *lds0, con
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
+// Sums that are not finite are formed again on the fp32 MFMA from the fp32 operands (split_bf16.h). x: the block in dW's order.
+// The waves take the 32 x 32 channels of one tap in turn, over all pixels of the slice: two per MFMA, eight a step, the next
+// step's operands requested ahead. Where the tap of a pixel lies outside the image both operands are zero (an infinite
+// gradient would make NaN of the zero read there). Ends early where every sum is a NaN.
+// p0, p1: the slice's pixels, as pixel_of counts them: whether tap (fh, fw) of one lies inside the image, and if so which image, and where in a
+// plane of dY and of X.
+template <class C, class PixelOf>
+__device__ __forceinline__ void split_wgrad_again(float *x, const float *dY, const float *X, u32 IC, u32 OC, u32 HW, u32 OHW, u32 oc0, u32 ic0, int fh0, u32 p0,
+                                                  u32 p1, PixelOf pixel_of) {
+    constexpr int F = C::F, KG = C::KG, NTW = C::NTW, NW = C::WM * C::WN;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int unit = wv; unit < NW * NTW; unit += NW * KG) {
+        const int tap = unit % NTW, um = unit / NTW / C::WN, un = unit / NTW % C::WN, i32 = lane & 31, h = lane >> 5;
+        float *const res = x + ((um * 32 + 4 * h) * C::ICT + un * 32 + i32) * NTW + tap;  // register r: row 8 * (r / 4) + r % 4
+        bool again = false;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) again |= !__builtin_isfinite(res[(8 * (r / 4) + r % 4) * C::ICT * NTW]);
+        if (!__any(int(again))) continue;
+        struct Step {
+            float d[4], x[4];
+        };
+        const u32 oc = oc0 + um * 32 + i32, ic = ic0 + un * 32 + i32;
+        const float *drow = dY + size_t(oc < OC ? oc : OC - 1) * OHW, *xrow = X + size_t(ic < IC ? ic : IC - 1) * HW;
+        auto fetch_step = [&](u32 start, Step &f) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const u32 p = start + 2 * q + h;
+                u32 img, dpix, xpix;  // image, place in a plane of dY and of X
+                const bool in = pixel_of(p, fh0 + tap / F, tap % F, img, dpix, xpix);
+                const float d = drow[in ? size_t(img) * OC * OHW + dpix : 0];
+                const float e = xrow[in ? size_t(img) * IC * HW + xpix : 0];
+                f.d[q] = in && oc < OC ? d : 0.f, f.x[q] = in && ic < IC ? e : 0.f;
+            }
+        };
+        v16f sum;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum[r] = 0.0f;
+        Step next;
+        fetch_step(p0, next);
+#pragma unroll 1
+        for (u32 p = p0; p < p1; p += 8) {
+            const Step now = next;
+            fetch_step(p + 8, next);  // (behind the slice's last pixel: for nobody)
+            u32 numbers = 0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(now.d[q], now.x[q], sum, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) numbers |= __builtin_isnan(sum[r]) ? 0u : 1u;
+            if (!__any(int(numbers))) break;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) res[(8 * (r / 4) + r % 4) * C::ICT * NTW] = sum[r];
+    }
+    lds_barrier();
+}
+
+// The end of a workgroup: sums over its K groups and out with the block.
+template <class C, class PixelOf>
+__device__ __forceinline__ void split_wgrad_finish(v16f (&acc)[C::NTW], unsigned char *smem, const float *dY, const float *X, float *dst0, u32 splits, u32 IC,
+                                                   u32 OC, u32 HW, u32 OHW, u32 z, u32 oc0, u32 ic0, int fh0, u32 p0, u32 p1, PixelOf pixel_of) {
+    constexpr int F = C::F, KG = C::KG, NTW = C::NTW;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = wv % (C::WM * C::WN), kgroup = wv / (C::WM * C::WN);
+    const int wm = wave / C::WN, wn = wave % C::WN;
+    // ---- sum the K groups (each its share of the registers), bring the block into dW's order, store whole rows of it ---------
+    constexpr int NW = C::WM * C::WN, NR = 16 / KG;
+    float own[NTW][NR];
+    float *x = reinterpret_cast<float *>(smem);
+#pragma unroll
+    for (int q = 0; q < NTW / C::RT; ++q) {
+        if (q) lds_barrier();
+#pragma unroll
+        for (int t = 0; t < C::RT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) x[((kgroup * NW + wave) * C::RT + t) * 1024 + r * 64 + lane] = acc[q * C::RT + t][r];
+        lds_barrier();
+#pragma unroll
+        for (int t = 0; t < C::RT; ++t)
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                float v = x[(wave * C::RT + t) * 1024 + (kgroup * NR + i) * 64 + lane];
+#pragma unroll
+                for (int g = 1; g < KG; ++g) v += x[((g * NW + wave) * C::RT + t) * 1024 + (kgroup * NR + i) * 64 + lane];
+                own[q * C::RT + t][i] = v * kSplitDown;
+            }
+    }
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+        const int r = kgroup * NR + i, row = wm * 32 + 8 * (r / 4) + 4 * (lane >> 5) + r % 4;
+#pragma unroll
+        for (int t = 0; t < NTW; ++t) x[(row * C::ICT + wn * 32 + (lane & 31)) * NTW + t] = own[t][i];
+    }
+    bool bad = false;
+#pragma unroll
+    for (int t = 0; t < NTW; ++t)
+#pragma unroll
+        for (int i = 0; i < NR; ++i) bad |= !__builtin_isfinite(own[t][i]);
+    if (__builtin_expect(__syncthreads_or(bad), 0)) split_wgrad_again<C>(x, dY, X, IC, OC, HW, OHW, oc0, ic0, fh0, p0, p1, pixel_of);
+    constexpr u32 ROW = C::ICT * NTW;
+    const u32 nic = IC - ic0 < u32(C::ICT) ? IC - ic0 : u32(C::ICT);
+    float *out = dst0 + (splits > 1 ? size_t(z) * OC * IC * (F * F) : 0);
+    for (u32 e = threadIdx.x; e < u32(C::OCT) * ROW; e += C::NTH) {
+        const u32 oc = e / ROW, rest = e % ROW, ic = rest / NTW, t = rest % NTW;
+        if (oc0 + oc < OC && ic < nic) {
+            float *dst = out + ((size_t(oc0 + oc) * IC + ic0 + ic) * (F * F) + fh0 * F + t);
+            if (splits > 1) *dst = x[e]; else *dst += x[e];
+        }
+    }
+}
+
 template <class C>
 __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a) {
-    constexpr int F = C::F, S = C::S, KG = C::KG, NTW = C::NTW, MAXPX = C::MAXPX, PXT = C::PXT;
+    constexpr int F = C::F, S = C::S, NTW = C::NTW, MAXPX = C::MAXPX, PXT = C::PXT;
     __shared__ __attribute__((aligned(256))) unsigned char smem[C::LDS];
     // slice z of all channel blocks has ids equal mod `splits`: with a multiple of 8 of them they share an XCD's L2
     const u32 z = blockIdx.x % a.splits, pair = blockIdx.x / a.splits, ot = pair / a.ic_tiles, it = pair % a.ic_tiles;
@@ -249,104 +359,17 @@ __global__ void __launch_bounds__(C::NTH, 2) split_wgrad_kernel(SplitWgradArgs a
     };
     if (a.IC - ic0 < u32(C::ICT) || a.OC - oc0 < u32(C::OCT)) main_loop(std::true_type()); else main_loop(std::false_type());
 
-    // ---- sum the K groups (each its share of the registers), bring the block into dW's order, store whole rows of it ---------
-    constexpr int NW = C::WM * C::WN, NR = 16 / KG;
-    float own[NTW][NR];
-    float *x = reinterpret_cast<float *>(smem);
-#pragma unroll
-    for (int q = 0; q < NTW / C::RT; ++q) {
-        if (q) lds_barrier();
-#pragma unroll
-        for (int t = 0; t < C::RT; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) x[((kgroup * NW + wave) * C::RT + t) * 1024 + r * 64 + lane] = acc[q * C::RT + t][r];
-        lds_barrier();
-#pragma unroll
-        for (int t = 0; t < C::RT; ++t)
-#pragma unroll
-            for (int i = 0; i < NR; ++i) {
-                float v = x[(wave * C::RT + t) * 1024 + (kgroup * NR + i) * 64 + lane];
-#pragma unroll
-                for (int g = 1; g < KG; ++g) v += x[((g * NW + wave) * C::RT + t) * 1024 + (kgroup * NR + i) * 64 + lane];
-                own[q * C::RT + t][i] = v * kSplitDown;
-            }
-    }
-    lds_barrier();
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
-        const int r = kgroup * NR + i, row = wm * 32 + 8 * (r / 4) + 4 * (lane >> 5) + r % 4;
-#pragma unroll
-        for (int t = 0; t < NTW; ++t) x[(row * C::ICT + wn * 32 + (lane & 31)) * NTW + t] = own[t][i];
-    }
-    bool bad = false;
-#pragma unroll
-    for (int t = 0; t < NTW; ++t)
-#pragma unroll
-        for (int i = 0; i < NR; ++i) bad |= !__builtin_isfinite(own[t][i]);
-    // ---- sums that are not finite: formed again on the fp32 MFMA from the fp32 operands (split_bf16.h) ------------------------
-    // The waves take the 32 x 32 channels of one tap in turn, over all pixels of the slice: two per MFMA, eight a step, the next
-    // step's operands requested ahead. Where the tap of a pixel lies outside the image both operands are zero (an infinite
-    // gradient would make NaN of the zero read there). Ends early where every sum is a NaN.
-    if (__builtin_expect(__syncthreads_or(bad), 0)) {
-        for (int unit = wv; unit < NW * NTW; unit += NW * KG) {
-            const int tap = unit % NTW, um = unit / NTW / C::WN, un = unit / NTW % C::WN, i32 = lane & 31, h = lane >> 5;
-            float *const res = x + ((um * 32 + 4 * h) * C::ICT + un * 32 + i32) * NTW + tap;  // register r: row 8 * (r / 4) + r % 4
-            bool again = false;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) again |= !__builtin_isfinite(res[(8 * (r / 4) + r % 4) * C::ICT * NTW]);
-            if (!__any(int(again))) continue;
-            struct Step {
-                float d[4], x[4];
-            };
-            const u32 oc = oc0 + um * 32 + i32, ic = ic0 + un * 32 + i32;
-            const float *drow = a.dY + size_t(oc < a.OC ? oc : a.OC - 1) * a.OHW, *xrow = a.X + size_t(ic < a.IC ? ic : a.IC - 1) * a.HW;
-            auto fetch_step = [&](u32 p0, Step &f) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const u32 p = p0 + 2 * q + h;
-                    u32 v, rem, py, px, img, strip;
-                    a.ohw.divmod(p < a.npix ? p : a.npix - 1, v, rem);
-                    a.ow.divmod(rem, py, px);
-                    a.strip_d.divmod(v, img, strip);
-                    px += strip * a.SW;
-                    const int iy = int(S * py) + fh0 + tap / F - a.pad_y, ix = int(S * px) + tap % F - a.pad_x;
-                    const bool in = p < a.npix && px < a.OW && u32(iy) < a.H && u32(ix) < a.W;
-                    const float d = drow[in ? size_t(img) * a.OC * a.OHW + py * a.OW + px : 0];
-                    const float e = xrow[in ? size_t(img) * a.IC * a.HW + u32(iy) * a.W + u32(ix) : 0];
-                    f.d[q] = in && oc < a.OC ? d : 0.f, f.x[q] = in && ic < a.IC ? e : 0.f;
-                }
-            };
-            v16f sum;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) sum[r] = 0.0f;
-            Step next;
-            fetch_step(t0 * PXT, next);
-#pragma unroll 1
-            for (u32 p = t0 * PXT; p < t1 * PXT; p += 8) {
-                const Step now = next;
-                fetch_step(p + 8, next);  // (behind the slice's last pixel: for nobody)
-                u32 numbers = 0;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(now.d[q], now.x[q], sum, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < 16; ++r) numbers |= __builtin_isnan(sum[r]) ? 0u : 1u;
-                if (!__any(int(numbers))) break;
-            }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) res[(8 * (r / 4) + r % 4) * C::ICT * NTW] = sum[r];
-        }
-        lds_barrier();
-    }
-    constexpr u32 ROW = C::ICT * NTW;
-    const u32 nic = a.IC - ic0 < u32(C::ICT) ? a.IC - ic0 : u32(C::ICT);
-    float *out = a.out + (a.splits > 1 ? size_t(z) * a.OC * a.IC * (F * F) : 0);
-    for (u32 e = threadIdx.x; e < u32(C::OCT) * ROW; e += C::NTH) {
-        const u32 oc = e / ROW, rest = e % ROW, ic = rest / NTW, t = rest % NTW;
-        if (oc0 + oc < a.OC && ic < nic) {
-            float *dst = out + ((size_t(oc0 + oc) * a.IC + ic0 + ic) * (F * F) + fh0 * F + t);
-            if (a.splits > 1) *dst = x[e]; else *dst += x[e];
-        }
-    }
+    split_wgrad_finish<C>(acc, smem, a.dY, a.X, a.out, a.splits, a.IC, a.OC, a.HW, a.OHW, z, oc0, ic0, fh0, t0 * PXT, t1 * PXT,
+                          [&](u32 p, int fh, int fw, u32 &img, u32 &dpix, u32 &xpix) {
+                              u32 v, rem, py, px, strip;
+                              a.ohw.divmod(p < a.npix ? p : a.npix - 1, v, rem);
+                              a.ow.divmod(rem, py, px);
+                              a.strip_d.divmod(v, img, strip);
+                              px += strip * a.SW;
+                              const int iy = int(S * py) + fh - a.pad_y, ix = int(S * px) + fw - a.pad_x;
+                              dpix = py * a.OW + px, xpix = u32(iy) * a.W + u32(ix);
+                              return p < a.npix && px < a.OW && u32(iy) < a.H && u32(ix) < a.W;
+                          });
 }
 
 struct SplitWgradPlan {
