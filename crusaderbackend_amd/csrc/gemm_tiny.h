@@ -1,7 +1,7 @@
 // Small dense products in ONE launch: C (M x N) = A * B with a result of at most a few hundred thousand elements and a
 // contraction too short to be worth a split over workgroups plus a second reduction launch (the dense layers of the CIFAR
-// networks: 128 x 512 x 512, 128 x 10 x 512 and their gradients). A workgroup owns one 16 x 16 block of C; its four waves
-// each take a quarter of the contraction, fed straight from global memory (the operands are L2-resident at these sizes,
+// networks: 128 x 512 x 512, 128 x 10 x 512 and their gradients). A workgroup owns one 16 x 16 block of C; its four (long contractions:
+// eight, sixteen) waves each take their share of the contraction, fed straight from global memory (the operands are L2-resident at these sizes,
 // so there is no LDS staging), and their accumulators are summed through LDS in wave order: bit-reproducible.
 //
 // v_mfma_f32_16x16x4_f32 (wave64, lane l): A value = A[i = l%16][k = l/16], B value = B[k = l/16][j = l%16], accumulator
@@ -13,6 +13,8 @@
 // 37.9 -> 17.2, 30 x 510 x 4090 44.2 -> 16.1, 126 x 510 x 1022 12.9 -> 5.9, 62 x 1022 x 1022 12.9 -> 6.1).
 #pragma once
 #include "igemm_engine.h"
+
+#include <type_traits>
 
 namespace crb {
 
@@ -36,80 +38,159 @@ struct TinyGemmArgs {
     float *a_rowsum = nullptr;
 };
 
-template <bool KVEC>
-__global__ void __launch_bounds__(256) tiny_gemm_kernel(TinyGemmArgs a) {
-    __shared__ __attribute__((aligned(16))) float red[4 * 256];
-    __shared__ float rsum[256];
-    const u32 t = threadIdx.x, lane = t & 63, wave = t >> 6;
+// Register t of lane group g (of four) <-> register g of lane group t.
+__device__ __forceinline__ v4f exchange_groups(v4f v) {
+    typedef u32 u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 r = __builtin_bit_cast(u32x4, v);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const auto p = __builtin_amdgcn_permlane32_swap(r[t], r[t + 2], false, false);
+        r[t] = p[0], r[t + 2] = p[1];
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t += 2) {
+        const auto p = __builtin_amdgcn_permlane16_swap(r[t], r[t + 1], false, false);
+        r[t] = p[0], r[t + 1] = p[1];
+    }
+    return __builtin_bit_cast(v4f, r);
+}
+
+// BATCH: a K-concatenated batch of more than one entry. Without one, whole groups of sixteen k are loaded from addresses that are a lane's
+// constant offset behind a uniform one and need no vector arithmetic (a division by the entry's length, a 64-bit product and the tests of
+// row, column and k for every load were most of the kernel's instructions). Us, before / after: NN 128 x 512 x 512 6.6 / 4.0, 256 x 256 x 1024 11.2 /
+// 5.8, TN 128 x 512 x 512 5.4 / 3.3, 128 x 128 x 2048 15.1 / 7.1, NT 128 x 512 x 512 4.5 / 4.0, 256 x 256 x 1024 6.7 / 5.7; the same bits. What bounds
+// it now is a launch (3 us of these) and the reading of every block's rows from L2.
+template <bool KVEC, bool BATCH, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) tiny_gemm_kernel(TinyGemmArgs a) {
+    __shared__ __attribute__((aligned(16))) float red[WAVES * 256];
+    __shared__ float rsum[WAVES * 64];
+    const u32 t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const u32 li = lane & 15, g = lane >> 4;
     const u32 row0 = (blockIdx.x / a.tiles_n) * 16, col0 = (blockIdx.x % a.tiles_n) * 16;
     const u32 kb = wave * a.k_per_wave;
     const u32 ke = kb + a.k_per_wave < a.K ? kb + a.k_per_wave : a.K;
-    const bool row_ok = row0 + li < a.M, col_ok = col0 + li < a.N;
     // What the epilogue adds to the element this thread finishes (row t / 16, column t % 16) is requested now: loaded at
     // the end, bias and previous value would each cost a memory round trip of their own.
-    const u32 er = t >> 4, ec = t & 15;
+    const u32 er = t >> 4 & 15, ec = t & 15;
     const u32 erow = row0 + er, ecol = col0 + ec;
-    const bool e_ok = erow < a.M && ecol < a.N;
+    const bool e_ok = t < 256 && erow < a.M && ecol < a.N;
     float *ep = a.C + size_t(e_ok ? erow : 0) * a.ldc + (e_ok ? ecol : 0);
     const float e_cb = (a.col_bias && e_ok) ? a.col_bias[ecol] : 0.f;
     const float e_rb = (a.row_bias && e_ok) ? a.row_bias[erow] : 0.f;
     const float e_old = ((a.flags & EPI_ACCUM) && e_ok) ? *ep : 0.f;
     v4f acc = {0.f, 0.f, 0.f, 0.f};
     float asum = 0.f;  // this lane's share of row li's sum of A
+    // (rows and columns past the last are read from the last one: nothing is stored of them)
+    const float *pa = a.A + size_t(row0 + li < a.M ? row0 + li : a.M - 1) * a.a_rs;
+    const float *pb = a.B + size_t(col0 + li < a.N ? col0 + li : a.N - 1) * a.b_cs;
+    u32 k = kb;
+    // `whole(n)`: the next n groups of sixteen k, all inside; requested together
+    auto groups = [&](auto whole) {
+        for (; k + 64 <= ke; k += 64) whole(std::integral_constant<int, 4>());
+        const u32 left = k < ke ? (ke - k) / 16 : 0;
+        if (left == 3) whole(std::integral_constant<int, 3>());
+        else if (left == 2) whole(std::integral_constant<int, 2>());
+        else if (left == 1) whole(std::integral_constant<int, 1>());
+        k += 16 * left;
+    };
+    typedef float v4fu __attribute__((ext_vector_type(4), aligned(4)));
     if constexpr (KVEC) {
         // both operands contiguous along k; a batch entry's contraction a multiple of 4
-        typedef float v4fu __attribute__((ext_vector_type(4), aligned(4)));
         const u32 kq = ke & ~3u;
-        const float *pa = a.A + size_t(row0 + li) * a.a_rs;
-        const float *pb = a.B + size_t(col0 + li) * a.b_cs;
-        constexpr int U = 4;  // 16-k groups requested together
-        for (u32 k = kb; k < kq; k += 16 * U) {
+        auto add = [&](const v4f &va, const v4f &vb) {
+            asum += (va.x + va.y) + (va.z + va.w);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va.x, vb.x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va.y, vb.y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va.z, vb.z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va.w, vb.w, acc, 0, 0, 0);
+        };
+        if constexpr (!BATCH) {
+            const float *qa = pa + 4 * g, *qb = pb + 4 * g;
+            groups([&](auto n_c) {
+                constexpr int n = decltype(n_c)::value;
+                v4f va[n], vb[n];
+#pragma unroll
+                for (int u = 0; u < n; ++u) va[u] = *reinterpret_cast<const v4fu *>(qa + k + 16 * u), vb[u] = *reinterpret_cast<const v4fu *>(qb + k + 16 * u);
+#pragma unroll
+                for (int u = 0; u < n; ++u) add(va[u], vb[u]);
+            });
+        }
+        constexpr int U = BATCH ? 4 : 1;  // 16-k groups requested together (without a batch: what is left of the last one)
+        for (; k < kq; k += 16 * U) {
             v4f va[U], vb[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const u32 kk = k + 16 * u + 4 * g;
                 const bool in = kk < kq;  // kq, kk and a batch entry's length are multiples of 4: a quad is inside or outside as a whole
-                u32 nd, kr;
-                a.kb_len.divmod(kk, nd, kr);
-                va[u] = (in && row_ok) ? v4f(*reinterpret_cast<const v4fu *>(pa + size_t(nd) * a.a_bs + kr)) : v4f{0.f, 0.f, 0.f, 0.f};
-                vb[u] = (in && col_ok) ? v4f(*reinterpret_cast<const v4fu *>(pb + size_t(nd) * a.b_bs + kr)) : v4f{0.f, 0.f, 0.f, 0.f};
+                u32 nd = 0, kr = in ? kk : 0;
+                if constexpr (BATCH) a.kb_len.divmod(kr, nd, kr);
+                va[u] = *reinterpret_cast<const v4fu *>(pa + size_t(nd) * a.a_bs + kr), vb[u] = *reinterpret_cast<const v4fu *>(pb + size_t(nd) * a.b_bs + kr);
+                if (!in) va[u] = vb[u] = v4f{0.f, 0.f, 0.f, 0.f};
             }
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                asum += (va[u].x + va[u].y) + (va[u].z + va[u].w);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va[u].x, vb[u].x, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va[u].y, vb[u].y, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va[u].z, vb[u].z, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va[u].w, vb[u].w, acc, 0, 0, 0);
-            }
+            for (int u = 0; u < U; ++u) add(va[u], vb[u]);
         }
         if (kq < ke && kb <= kq) {  // K % 4 more (no batch then), in the wave that holds them
             const bool in = kq + g < ke;
-            const float va = (in && row_ok) ? pa[kq + g] : 0.f, vb = (in && col_ok) ? pb[kq + g] : 0.f;
+            const float va = in ? pa[kq + g] : 0.f, vb = in ? pb[kq + g] : 0.f;
             asum += va;
             acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va, vb, acc, 0, 0, 0);
         }
     } else {
-        const float *pa = a.A + size_t(row0 + li) * a.a_rs;
-        const float *pb = a.B + size_t(col0 + li) * a.b_cs;
-        constexpr int U = 16;  // MFMA steps requested together
-        for (u32 k = kb; k < ke; k += 4 * U) {
+        auto add = [&](float va, float vb) {
+            asum += va;
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va, vb, acc, 0, 0, 0);
+        };
+        if constexpr (!BATCH) {
+            const u32 la = u32(pa - a.A) + g * a.a_ks, lb = u32(pb - a.B) + g * a.b_ks;
+            const float *qa = pa + 4 * g;
+            auto fetch_b = [&](auto n_c, float *vb) {
+#pragma unroll
+                for (int u = 0; u < 4 * decltype(n_c)::value; ++u) vb[u] = (a.B + size_t(k + 4 * u) * a.b_ks)[lb];
+            };
+            if (a.a_ks == 1) {
+                // A contiguous along k: a lane loads four k and the lane groups exchange them (register t of group g, k = 4 g + t, becomes register
+                // g of group t), so that the sum's order is the same
+                groups([&](auto n_c) {
+                    constexpr int n = decltype(n_c)::value;
+                    v4f va[n];
+                    float vb[4 * n];
+#pragma unroll
+                    for (int u = 0; u < n; ++u) va[u] = *reinterpret_cast<const v4fu *>(qa + k + 16 * u);
+                    fetch_b(n_c, vb);
+#pragma unroll
+                    for (int u = 0; u < n; ++u) {
+                        const v4f q = exchange_groups(va[u]);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) add(q[i], vb[4 * u + i]);
+                    }
+                });
+            } else {
+                groups([&](auto n_c) {
+                    constexpr int n = decltype(n_c)::value;
+                    float va[4 * n], vb[4 * n];
+#pragma unroll
+                    for (int u = 0; u < 4 * n; ++u) va[u] = (a.A + size_t(k + 4 * u) * a.a_ks)[la];
+                    fetch_b(n_c, vb);
+#pragma unroll
+                    for (int u = 0; u < 4 * n; ++u) add(va[u], vb[u]);
+                });
+            }
+        }
+        constexpr int U = BATCH ? 16 : 4;  // MFMA steps requested together (without a batch: what is left of the last group)
+        for (; k < ke; k += 4 * U) {
             float va[U], vb[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const u32 kk = k + 4 * u + g;
                 const bool in = kk < ke;
-                u32 nd, kr;
-                a.kb_len.divmod(kk, nd, kr);
-                va[u] = (in && row_ok) ? pa[size_t(nd) * a.a_bs + size_t(kr) * a.a_ks] : 0.f;
-                vb[u] = (in && col_ok) ? pb[size_t(nd) * a.b_bs + size_t(kr) * a.b_ks] : 0.f;
+                u32 nd = 0, kr = in ? kk : 0;
+                if constexpr (BATCH) a.kb_len.divmod(kr, nd, kr);
+                va[u] = pa[size_t(nd) * a.a_bs + size_t(kr) * a.a_ks], vb[u] = pb[size_t(nd) * a.b_bs + size_t(kr) * a.b_ks];
+                if (!in) va[u] = vb[u] = 0.f;
             }
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                asum += va[u];
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va[u], vb[u], acc, 0, 0, 0);
-            }
+            for (int u = 0; u < U; ++u) add(va[u], vb[u]);
         }
     }
     *reinterpret_cast<v4f *>(red + wave * 256 + lane * 4) = acc;
@@ -119,7 +200,7 @@ __global__ void __launch_bounds__(256) tiny_gemm_kernel(TinyGemmArgs a) {
     if (do_rowsum && t < 16 && row0 + t < a.M) {
         float v = 0.f;
 #pragma unroll
-        for (int q = 0; q < 16; ++q) v += rsum[q * 16 + t];  // wave q / 4, k lane group q % 4
+        for (int q = 0; q < 4 * WAVES; ++q) v += rsum[q * 16 + t];  // wave q / 4, k lane group q % 4
         a.a_rowsum[row0 + t] += v;
     }
     // thread t finishes element (row t / 16, column t % 16): register row % 4 of lane (row / 4) * 16 + column
@@ -127,7 +208,7 @@ __global__ void __launch_bounds__(256) tiny_gemm_kernel(TinyGemmArgs a) {
     const u32 e = ((er >> 2) * 16 + ec) * 4 + (er & 3);
     float v = red[e];
 #pragma unroll
-    for (int w = 1; w < 4; ++w) v += red[w * 256 + e];
+    for (int w = 1; w < WAVES; ++w) v += red[w * 256 + e];
     if (a.col_bias) v += e_cb;
     if (a.row_bias) v += e_rb;
     if (a.flags & EPI_ACCUM) v += e_old;
@@ -135,7 +216,7 @@ __global__ void __launch_bounds__(256) tiny_gemm_kernel(TinyGemmArgs a) {
     *ep = v;
 }
 
-// Whether the one-launch form takes a product: a small result, a contraction short enough that a quarter of it per wave is
+// Whether the one-launch form takes a product ahead of all others: a small result, a contraction short enough that a quarter of it per wave is
 // a few dozen MFMA steps, and enough 16 x 16 blocks (or little enough work) that the chip is not left idle for long.
 // K: the whole contraction (batch * K for the K-concatenated accumulate-NT form); batch: independent products (must be 1).
 // kfast: both operands are contiguous along k (the NT forms: 16-byte loads). Every block re-reads its operand rows from L2,
@@ -149,17 +230,40 @@ inline bool tiny_gemm_fits(u32 M, u32 N, u32 K, u32 batch, bool kfast = false) {
     return blocks >= 64u || uint64_t(M) * N * K <= (1u << 22);
 }
 
+// Products that would go to the fp32 engine: where that has too few tiles for the chip or cuts the contraction, a workgroup for every 16 x 16 block is
+// ahead as long as the chip takes the blocks in two rounds of eight on a CU and they re-read no more than this of their operands (us, engine / here:
+// 128 x 96 x 352 11.3 / 3.7, 41 x 315 x 818 12.0 / 4.2, 2304 x 144 x 224 11.0 / 5.9, 1088 x 256 x 64 4.7 / 3.4, 60 x 3268 x 526 12.5 / 11.7; beyond,
+// 1958 x 802 x 18, 6273 blocks, 6.5 / 9.9, 1984 x 64 x 960 10.8 / 11.1). 73 random products 0.59 of the time in the mean, none slower.
+inline bool tiny_gemm_beats_engine(u32 M, u32 N, u32 K, u32 batch) {
+    const uint64_t blocks = uint64_t(ceil_div(M, 16u)) * ceil_div(N, 16u);
+    return batch == 1 && K <= 2048u && blocks <= 2048u && blocks * K <= 442368u;
+}
+
+// Waves of a workgroup, which share its contraction. More of them keep the chains of a long one short, in time (us, 4 / 8 / 16 waves: NT 11 x 2012 x
+// 3053 15.1 / 10.5 / 10.8, 13 x 107 x 2127 7.5 / 6.8 / 7.0) and in roundings (TN 112 x 112 x 1200 3.2 / 2.3 / 1.8e-7 from float64, the engine, which
+// cuts it, 2.2e-7; 502 x 15 x 614 2.3e-7 on either).
+inline u32 tiny_gemm_waves(u32 K) { return K <= 640u ? 4u : (K <= 1024u ? 8u : 16u); }
+
 // kb_len: length of one batch entry's contraction (a.K for a plain product); a.K = the whole contraction.
 inline int launch_tiny_gemm(TinyGemmArgs a, u32 kb_len, u32 a_bs, u32 b_bs, hipStream_t s, const char *what) {
     a.kb_len = FastDiv(kb_len), a.a_bs = a_bs, a.b_bs = b_bs;
     a.tiles_n = ceil_div(a.N, 16u);
-    a.k_per_wave = ceil_div(ceil_div(a.K, 4u), 16u) * 16u;
-    const u32 blocks = ceil_div(a.M, 16u) * a.tiles_n;
+    const u32 blocks = ceil_div(a.M, 16u) * a.tiles_n, waves = tiny_gemm_waves(a.K);
+    a.k_per_wave = ceil_div(ceil_div(a.K, waves), 16u) * 16u;
     const bool kvec = a.a_ks == 1 && a.b_ks == 1 && (kb_len == a.K || (kb_len % 4 == 0 && a_bs % 4 == 0 && b_bs % 4 == 0));
-    if (kvec)
-        hipLaunchKernelGGL(tiny_gemm_kernel<true>, dim3(blocks), dim3(256), 0, s, a);
-    else
-        hipLaunchKernelGGL(tiny_gemm_kernel<false>, dim3(blocks), dim3(256), 0, s, a);
+    auto launch = [&](auto w_c) {
+        constexpr int W = decltype(w_c)::value;
+        if (kb_len != a.K) {
+            if (kvec) hipLaunchKernelGGL((tiny_gemm_kernel<true, true, W>), dim3(blocks), dim3(64 * W), 0, s, a);
+            else hipLaunchKernelGGL((tiny_gemm_kernel<false, true, W>), dim3(blocks), dim3(64 * W), 0, s, a);
+        } else {
+            if (kvec) hipLaunchKernelGGL((tiny_gemm_kernel<true, false, W>), dim3(blocks), dim3(64 * W), 0, s, a);
+            else hipLaunchKernelGGL((tiny_gemm_kernel<false, false, W>), dim3(blocks), dim3(64 * W), 0, s, a);
+        }
+    };
+    if (waves == 4) launch(std::integral_constant<int, 4>());
+    else if (waves == 8) launch(std::integral_constant<int, 8>());
+    else launch(std::integral_constant<int, 16>());
     return check_launch(what);
 }
 
