@@ -1,14 +1,17 @@
-"""ctypes binding of the C ABI declared in include/crusader_hip.h.
+"""Python binding of the C ABI declared in include/crusader_hip.h.
 
-This module is plumbing for tests and the benchmark: it loads the in-tree
-``lib/libcrusader_hip.so`` and passes raw device pointers (``tensor.data_ptr()``) and sizes
-straight through. There is no CPU fallback: if the shared library is missing, loading raises.
+It loads the in-tree ``lib/libcrusader_hip.so`` and passes raw device pointers (``tensor.data_ptr()``) and sizes straight
+through: the launching calls by way of ``lib/_crb_calls.so`` (csrc/crb_calls.cpp), size queries, the few calls on host
+tables and prepared ones by ctypes. There is no CPU fallback: if either library is missing, loading raises.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libcrusader_hip.so")
+CALLS_PATH = os.path.join(_HERE, "lib", "_crb_calls.so")
 
 CRB_OK = 0
 CRB_EINVAL_SHAPE = -1
@@ -96,18 +99,34 @@ SIGNATURES = {
 _lib = None
 
 
+class _Unloaded:
+    """Stands in for the native calls until the first of them is made."""
+
+    def __getattr__(self, name):
+        load()
+        return getattr(_calls, name)
+
+
+# The launching entry points, which take tensors, None, ConvGeom, numbers and a stream as they are (csrc/crb_calls.cpp).
+_calls = _Unloaded()
+
+
 def load():
     """Load the HIP library (once) and attach signatures. Raises OSError if it has not been built."""
-    global _lib
+    global _lib, _calls
     if _lib is None:
-        if not os.path.exists(LIB_PATH):
+        if not (os.path.exists(LIB_PATH) and os.path.exists(CALLS_PATH)):
             raise OSError(f"{LIB_PATH} not found: build it with `make -C crusaderbackend_amd/csrc`")
         lib = ctypes.CDLL(LIB_PATH)
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
-        _lib = lib
+        loader = importlib.machinery.ExtensionFileLoader("_crb_calls", CALLS_PATH)
+        calls = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_crb_calls", CALLS_PATH, loader=loader))
+        loader.exec_module(calls)
+        calls.bind(ConvGeom, ctypes.ArgumentError)
+        _lib, _calls = lib, calls
     return _lib
 
 
@@ -179,19 +198,36 @@ class _Recorder:
         return passthrough
 
 
+class _Converted:
+    """Stands in for the native calls while `frozen` records: the same arguments, converted for the library's ctypes functions."""
+
+    def __init__(self, lib):
+        self._lib = lib
+
+    def __getattr__(self, name):
+        fn = getattr(self._lib, name)
+
+        def call(*args):
+            return fn(*(ctypes.byref(a) if isinstance(a, ConvGeom) else a.data_ptr() if hasattr(a, "data_ptr") else a.cuda_stream if hasattr(a, "cuda_stream") else a
+                        for a in args))
+
+        return call
+
+
 def frozen(fn):
     """Runs `fn` (any composition of the wrappers below) once and returns a zero-argument callable that re-issues the
     same entry points with the same already-converted arguments. For timing loops over short kernels, like `prepared`,
     without spelling the C argument list out. Every tensor `fn` touches must outlive the callable; host-side decisions
     `fn` makes (workspace sizes, branches) are frozen with it."""
-    global _lib
+    global _lib, _calls
     real = load()
+    native = _calls
     rec = _Recorder(real)
-    _lib = rec
+    _lib, _calls = rec, _Converted(rec)
     try:
         fn()
     finally:
-        _lib = real
+        _lib, _calls = real, native
     calls = tuple(rec.calls)
     if not calls:  # `fn` does not go through the wrappers (already prepared calls): nothing to freeze
         return fn
@@ -214,39 +250,39 @@ def frozen(fn):
 
 # Thin helpers over torch CUDA tensors (device memory + streams only; no torch math).
 def sgemm_nn(A, B, C, M, N, K, batch=1, stream=None):
-    check(load().crb_sgemm_nn(_p(A), _p(B), _p(C), M, N, K, batch, _stream(stream)))
+    check(_calls.crb_sgemm_nn(A, B, C, M, N, K, batch, stream))
 
 
 def sgemm_tn(A, B, C, M, N, K, batch=1, stream=None):
-    check(load().crb_sgemm_tn(_p(A), _p(B), _p(C), M, N, K, batch, _stream(stream)))
+    check(_calls.crb_sgemm_tn(A, B, C, M, N, K, batch, stream))
 
 
 def sgemm_nt(A, B, C, M, N, K, stream=None):
-    check(load().crb_sgemm_nt(_p(A), _p(B), _p(C), M, N, K, _stream(stream)))
+    check(_calls.crb_sgemm_nt(A, B, C, M, N, K, stream))
 
 
 def sgemm_nta(A, B, C, M, N, K, batch=1, stream=None):
-    check(load().crb_sgemm_nta(_p(A), _p(B), _p(C), M, N, K, batch, _stream(stream)))
+    check(_calls.crb_sgemm_nta(A, B, C, M, N, K, batch, stream))
 
 
 def linear_fwd(X, W, bias, Y, batch, IN, OUT, flags=0, stream=None):
-    check(load().crb_linear_fwd(_p(X), _p(W), _p(bias), _p(Y), batch, IN, OUT, flags, _stream(stream)))
+    check(_calls.crb_linear_fwd(X, W, bias, Y, batch, IN, OUT, flags, stream))
 
 
 def linear_dgrad(dY, W, dX, batch, IN, OUT, stream=None):
-    check(load().crb_linear_dgrad(_p(dY), _p(W), _p(dX), batch, IN, OUT, _stream(stream)))
+    check(_calls.crb_linear_dgrad(dY, W, dX, batch, IN, OUT, stream))
 
 
 def linear_wgrad(dY, X, dW, dB, batch, IN, OUT, stream=None):
-    check(load().crb_linear_wgrad(_p(dY), _p(X), _p(dW), _p(dB), batch, IN, OUT, _stream(stream)))
+    check(_calls.crb_linear_wgrad(dY, X, dW, dB, batch, IN, OUT, stream))
 
 
 def conv_fwd(W, X, Y, bias, geom, flags=0, stream=None):
-    check(load().crb_conv_fwd(_p(W), _p(X), _p(Y), _p(bias), ctypes.byref(geom), flags, _stream(stream)))
+    check(_calls.crb_conv_fwd(W, X, Y, bias, geom, flags, stream))
 
 
 def conv_dgrad(W, dY, dX, geom, stream=None):
-    check(load().crb_conv_dgrad(_p(W), _p(dY), _p(dX), ctypes.byref(geom), _stream(stream)))
+    check(_calls.crb_conv_dgrad(W, dY, dX, geom, stream))
 
 
 def conv_wgrad_workspace_bytes(geom):
@@ -254,13 +290,13 @@ def conv_wgrad_workspace_bytes(geom):
 
 
 def conv_wgrad(dY, X, dW, geom, workspace=None, stream=None):
-    nbytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    check(load().crb_conv_wgrad(_p(dY), _p(X), _p(dW), ctypes.byref(geom), _p(workspace), nbytes, _stream(stream)))
+    nbytes = 0 if workspace is None else workspace.nbytes
+    check(_calls.crb_conv_wgrad(dY, X, dW, geom, workspace, nbytes, stream))
 
 
 def conv_wgrad_noalloc(dY, X, dW, geom, stream=None):
     """conv_wgrad on the library's built-in scratch buffer: the call allocates nothing."""
-    check(load().crb_conv_wgrad_noalloc(_p(dY), _p(X), _p(dW), ctypes.byref(geom), _stream(stream)))
+    check(_calls.crb_conv_wgrad_noalloc(dY, X, dW, geom, stream))
 
 
 NOALLOC_SCRATCH_BYTES = 8 << 20  # CRB_NOALLOC_SCRATCH_BYTES
@@ -268,7 +304,7 @@ NOALLOC_SCRATCH_BYTES = 8 << 20  # CRB_NOALLOC_SCRATCH_BYTES
 
 def bind_workspace(workspace, stream=None):
     """Bind `workspace` (a torch tensor, or None to unbind) as the split scratch of calls on `stream`."""
-    nbytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
+    nbytes = 0 if workspace is None else workspace.nbytes
     check(load().crb_bind_workspace(_p(workspace), nbytes, _stream(stream)))
 
 
@@ -290,8 +326,8 @@ def conv_bias_grad_workspace_bytes(N, C, HW):
 
 def conv_bwd(W, dY, X, dX, dW, geom, workspace=None, stream=None):
     """Data gradient and weight gradient of one layer in one call (one launch for the residual-network layer shapes)."""
-    nbytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    check(load().crb_conv_bwd(_p(W), _p(dY), _p(X), _p(dX), _p(dW), ctypes.byref(geom), _p(workspace), nbytes, _stream(stream)))
+    nbytes = 0 if workspace is None else workspace.nbytes
+    check(_calls.crb_conv_bwd(W, dY, X, dX, dW, geom, workspace, nbytes, stream))
 
 
 def conv_bwd_slices(geom):
@@ -300,8 +336,8 @@ def conv_bwd_slices(geom):
 
 def conv_bwd_sliced(W, dY, X, dX, geom, workspace, stream=None):
     """dX now; the weight gradient stays as conv_bwd_slices(geom) partial sums in `workspace` until sum_slices_multi."""
-    nbytes = workspace.numel() * workspace.element_size()
-    check(load().crb_conv_bwd_sliced(_p(W), _p(dY), _p(X), _p(dX), ctypes.byref(geom), _p(workspace), nbytes, _stream(stream)))
+    nbytes = workspace.nbytes
+    check(_calls.crb_conv_bwd_sliced(W, dY, X, dX, geom, workspace, nbytes, stream))
 
 
 class SliceSumItem(ctypes.Structure):
@@ -323,51 +359,51 @@ def sum_slices_multi(table, stream=None):
 
 
 def conv_bias(Y, bias, N, C, HW, stream=None):
-    check(load().crb_conv_bias(_p(Y), _p(bias), N, C, HW, _stream(stream)))
+    check(_calls.crb_conv_bias(Y, bias, N, C, HW, stream))
 
 
 def conv_bias_grad(dY, dB, N, C, HW, stream=None):
-    check(load().crb_conv_bias_grad(_p(dY), _p(dB), N, C, HW, _stream(stream)))
+    check(_calls.crb_conv_bias_grad(dY, dB, N, C, HW, stream))
 
 
 def tensor_add_inplace(a, b, count, stream=None):
-    check(load().crb_tensor_add_inplace(_p(a), _p(b), count, _stream(stream)))
+    check(_calls.crb_tensor_add_inplace(a, b, count, stream))
 
 
 def tensor_fill(a, value, count, stream=None):
-    check(load().crb_tensor_fill(_p(a), value, count, _stream(stream)))
+    check(_calls.crb_tensor_fill(a, value, count, stream))
 
 
 def tensor_sub_inplace(a, b, count, stream=None):
-    check(load().crb_tensor_sub_inplace(_p(a), _p(b), count, _stream(stream)))
+    check(_calls.crb_tensor_sub_inplace(a, b, count, stream))
 
 
 def tensor_scale_inplace(a, factor, count, stream=None):
-    check(load().crb_tensor_scale_inplace(_p(a), factor, count, _stream(stream)))
+    check(_calls.crb_tensor_scale_inplace(a, factor, count, stream))
 
 
 def relu_fwd(X, Y, count, stream=None):
-    check(load().crb_relu_fwd(_p(X), _p(Y), count, _stream(stream)))
+    check(_calls.crb_relu_fwd(X, Y, count, stream))
 
 
 def relu_bwd(X, dY, dX, count, stream=None):
-    check(load().crb_relu_bwd(_p(X), _p(dY), _p(dX), count, _stream(stream)))
+    check(_calls.crb_relu_bwd(X, dY, dX, count, stream))
 
 
 def maxpool_fwd(X, Y, record, planes, IH, IW, sH, sW, rH, rW, stream=None):
-    check(load().crb_maxpool_fwd(_p(X), _p(Y), _p(record), planes, IH, IW, sH, sW, rH, rW, _stream(stream)))
+    check(_calls.crb_maxpool_fwd(X, Y, record, planes, IH, IW, sH, sW, rH, rW, stream))
 
 
 def maxpool_bwd(dX, dY, record, planes, IH, IW, sH, sW, rH, rW, stream=None):
-    check(load().crb_maxpool_bwd(_p(dX), _p(dY), _p(record), planes, IH, IW, sH, sW, rH, rW, _stream(stream)))
+    check(_calls.crb_maxpool_bwd(dX, dY, record, planes, IH, IW, sH, sW, rH, rW, stream))
 
 
 def softmax(A, out, rows, step, stream=None):
-    check(load().crb_softmax(_p(A), _p(out), rows, step, _stream(stream)))
+    check(_calls.crb_softmax(A, out, rows, step, stream))
 
 
 def cross_entropy_grad(Y, labels, dY, count, stream=None):
-    check(load().crb_cross_entropy_grad(_p(Y), _p(labels), _p(dY), count, _stream(stream)))
+    check(_calls.crb_cross_entropy_grad(Y, labels, dY, count, stream))
 
 
 def cross_entropy_scratch_floats(count):
@@ -377,31 +413,31 @@ def cross_entropy_scratch_floats(count):
 def cross_entropy_loss(Y, labels, scratch, loss_out, count, stream=None):
     """`loss_out`: one-element device tensor; `scratch`: device tensor of cross_entropy_scratch_floats(count) floats or None."""
     n = 0 if scratch is None else scratch.numel()
-    check(load().crb_cross_entropy_loss(_p(Y), _p(labels), _p(scratch), n, _p(loss_out), count, _stream(stream)))
+    check(_calls.crb_cross_entropy_loss(Y, labels, scratch, n, loss_out, count, stream))
 
 
 def momentum_apply(X, G, M, count, lr, beta, decay=1.0, stream=None):
-    check(load().crb_momentum_apply(_p(X), _p(G), _p(M), count, lr, beta, decay, _stream(stream)))
+    check(_calls.crb_momentum_apply(X, G, M, count, lr, beta, decay, stream))
 
 
 def batchnorm_fwd(X, beta, gamma, mean, var, Y, xHat, N, F, stream=None):
-    check(load().crb_batchnorm_fwd(_p(X), _p(beta), _p(gamma), _p(mean), _p(var), _p(Y), _p(xHat), N, F, _stream(stream)))
+    check(_calls.crb_batchnorm_fwd(X, beta, gamma, mean, var, Y, xHat, N, F, stream))
 
 
 def batchnorm_bwd(dY, gamma, X, dX, N, F, dGamma=None, dBeta=None, stream=None):
-    check(load().crb_batchnorm_bwd(_p(dY), _p(gamma), _p(X), _p(dX), _p(dGamma), _p(dBeta), N, F, _stream(stream)))
+    check(_calls.crb_batchnorm_bwd(dY, gamma, X, dX, dGamma, dBeta, N, F, stream))
 
 
 def batchnorm_param_grads(dY, xHat, dGamma, dBeta, N, F, stream=None):
-    check(load().crb_batchnorm_param_grads(_p(dY), _p(xHat), _p(dGamma), _p(dBeta), N, F, _stream(stream)))
+    check(_calls.crb_batchnorm_param_grads(dY, xHat, dGamma, dBeta, N, F, stream))
 
 
 def tensor_copy(dst, src, count, stream=None):
-    check(load().crb_tensor_copy(_p(dst), _p(src), count, _stream(stream)))
+    check(_calls.crb_tensor_copy(dst, src, count, stream))
 
 
 def tensor_add_clear(a, b, count, stream=None):
-    check(load().crb_tensor_add_clear(_p(a), _p(b), count, _stream(stream)))
+    check(_calls.crb_tensor_add_clear(a, b, count, stream))
 
 
 class MomentumItem(ctypes.Structure):
@@ -422,19 +458,19 @@ def momentum_table(torch, dev, entries):
 
 
 def momentum_apply_multi(table, n_items, max_count, stream=None):
-    check(load().crb_momentum_apply_multi(_p(table), n_items, max_count, _stream(stream)))
+    check(_calls.crb_momentum_apply_multi(table, n_items, max_count, stream))
 
 
 def tensor_add(dst, a, b, count, stream=None):
-    check(load().crb_tensor_add(_p(dst), _p(a), _p(b), count, _stream(stream)))
+    check(_calls.crb_tensor_add(dst, a, b, count, stream))
 
 
 def tensor_add_clear_copy(dst, a, b, count, stream=None):
-    check(load().crb_tensor_add_clear_copy(_p(dst), _p(a), _p(b), count, _stream(stream)))
+    check(_calls.crb_tensor_add_clear_copy(dst, a, b, count, stream))
 
 
 def tensor_copy2(dst1, dst2, src, count, stream=None):
-    check(load().crb_tensor_copy2(_p(dst1), _p(dst2), _p(src), count, _stream(stream)))
+    check(_calls.crb_tensor_copy2(dst1, dst2, src, count, stream))
 
 
 NORM_NONE, NORM_UNIFORM, NORM_DISTRIBUTION = 0, 1, 2
@@ -456,22 +492,20 @@ def image_aug_table(torch, dev, entries):
 
 
 def images_from_bytes(src, dst, images, channels, H, W, norm=NORM_NONE, p0=0.0, p1=1.0, aug=None, stream=None):
-    check(load().crb_images_from_bytes(_p(src), _p(dst), images, channels, H, W, norm, p0, p1, _p(aug), _stream(stream)))
+    check(_calls.crb_images_from_bytes(src, dst, images, channels, H, W, norm, p0, p1, aug, stream))
 
 
 def batchnorm_relu_fwd(X, beta, gamma, mean, var, reluOut, N, F, Y=None, xHat=None, addend=None, stream=None):
-    check(load().crb_batchnorm_relu_fwd(_p(X), _p(beta), _p(gamma), _p(mean), _p(var), _p(Y), _p(xHat), _p(addend), _p(reluOut), N, F,
-                                        _stream(stream)))
+    check(_calls.crb_batchnorm_relu_fwd(X, beta, gamma, mean, var, Y, xHat, addend, reluOut, N, F, stream))
 
 
 def batchnorm_relu_bwd(dY, reluOut, gamma, X, dX, N, F, dGamma=None, dBeta=None, dY2=None, dYmasked=None, stream=None):
-    check(load().crb_batchnorm_relu_bwd(_p(dY), _p(dY2), _p(reluOut), _p(gamma), _p(X), _p(dX), _p(dGamma), _p(dBeta), _p(dYmasked), N, F,
-                                        _stream(stream)))
+    check(_calls.crb_batchnorm_relu_bwd(dY, dY2, reluOut, gamma, X, dX, dGamma, dBeta, dYmasked, N, F, stream))
 
 
 def tensor_add_relu(dst, a, b, count, stream=None):
-    check(load().crb_tensor_add_relu(_p(dst), _p(a), _p(b), count, _stream(stream)))
+    check(_calls.crb_tensor_add_relu(dst, a, b, count, stream))
 
 
 def tensor_relu_grad_copy2(dst1, dst2, relu_out, dY, count, dY2=None, stream=None):
-    check(load().crb_tensor_relu_grad_copy2(_p(dst1), _p(dst2), _p(relu_out), _p(dY), _p(dY2), count, _stream(stream)))
+    check(_calls.crb_tensor_relu_grad_copy2(dst1, dst2, relu_out, dY, dY2, count, stream))

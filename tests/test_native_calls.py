@@ -1,0 +1,57 @@
+"""The launching entry points as Python callables (csrc/crb_calls.cpp): the same calls as by ctypes, refused where those are (no GPU is touched)."""
+import ctypes
+import re
+
+import pytest
+
+from crusaderbackend_amd import capi
+
+
+def test_every_launching_wrapper_has_its_call():
+    lib = capi.load()
+    text = open(capi.__file__).read()
+    names = set(re.findall(r"_calls\.(crb_\w+)\(", text))
+    assert len(names) >= 40
+    for n in names:
+        assert callable(getattr(capi._calls, n)) and capi.SIGNATURES[n][0] is ctypes.c_int and hasattr(lib, n)
+
+
+def test_arguments_reach_the_library():
+    """Refused by the library before any device work, with the text that says which argument it saw."""
+    g = capi.ConvGeom.make(2, 3, 8, 9, 4, 3, 3, 1, 1, 1, 1)
+    for call in (lambda: capi.sgemm_nn(None, None, None, 1, 1, 1), lambda: capi.conv_fwd(None, None, None, None, g), lambda: capi.linear_wgrad(None, None, None, None, 2, 3, 4),
+                 lambda: capi.momentum_apply(None, None, None, 4, 0.1, 0.9), lambda: capi.images_from_bytes(None, None, 1, 3, 4, 4)):
+        with pytest.raises(capi.CrbError) as e:
+            call()
+        assert e.value.status == capi.CRB_ENULL
+
+    class Tensor:
+        def data_ptr(self):
+            return 4096
+
+    t = Tensor()
+    with pytest.raises(capi.CrbError) as e:
+        capi.sgemm_nn(t, t, t, 1, 0, 1)
+    assert e.value.status == capi.CRB_EINVAL_SHAPE
+    g.OW = 5
+    with pytest.raises(capi.CrbError) as e:
+        capi.conv_fwd(t, t, t, None, g)
+    assert e.value.status == capi.CRB_EINVAL_SHAPE
+
+
+def test_arguments_of_the_wrong_kind_are_refused():
+    g = capi.ConvGeom.make(2, 3, 8, 9, 4, 3, 3, 1, 1, 1, 1)
+    for call in (lambda: capi.sgemm_nn(None, None, None, 1.0, 1, 1), lambda: capi.sgemm_nn(None, None, None, None, 1, 1), lambda: capi.conv_dgrad(None, None, None, (2, 3)),
+                 lambda: capi.conv_dgrad(None, None, None, None), lambda: capi.momentum_apply(None, None, None, 4, "0.1", 0.9)):
+        with pytest.raises((ctypes.ArgumentError, TypeError)):
+            call()
+    for call in (lambda: capi.sgemm_nn(4096, None, None, 1, 1, 1), lambda: capi.conv_fwd(b"x", None, None, None, g), lambda: capi.relu_fwd(None, None, 4, stream=7)):
+        with pytest.raises(AttributeError):
+            call()
+
+
+def test_frozen_wrappers_are_recorded():
+    call = capi.frozen(lambda: pytest.raises(capi.CrbError, capi.sgemm_nt, None, None, None, 1, 1, 1))
+    with pytest.raises(capi.CrbError):
+        call()
+    assert not isinstance(capi._calls, capi._Converted)
