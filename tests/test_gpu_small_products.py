@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 # the last K of four and of eight waves, the most K, blocks and blocks * K that are taken and one more of each
 SHAPES = [(1, 1, 1), (17, 15, 3), (1, 33, 64), (33, 1, 100), (16, 16, 16), (31, 65, 63), (128, 10, 512), (65, 200, 333), (100, 300, 640), (100, 300, 641), (50, 90, 1024),
           (50, 90, 1025), (12, 40, 2048), (128, 96, 352), (502, 15, 614), (41, 315, 818), (2304, 144, 16), (512, 1024, 18), (513, 1024, 18), (3, 272, 2049), (432, 256, 1024),
-          (448, 256, 1025)]
+          (448, 256, 1025), (512, 512, 1024), (640, 256, 1024), (368, 784, 896)]
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
