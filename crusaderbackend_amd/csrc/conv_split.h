@@ -72,10 +72,18 @@ struct ConvSplitArgs {
 // channels 8 * (l / 32) + 0..7 of the group's 16), zero beyond the channel counts. A thread takes one channel octet of one
 // output channel and tap: eight loads in flight, and enough threads to cover the chip (all taps per thread: 147 K filter
 // elements took 14 us, a chain of 72 loads on 8 workgroups).
-template <bool DGRAD>
+// SUM: the first workgroups sum a weight gradient's slices (of the call's other gradient): one launch for two that the chip is not filled by.
+template <bool DGRAD, bool SUM = false>
 __global__ void __launch_bounds__(256) conv_split_filters_kernel(const float *__restrict__ W, unsigned char *__restrict__ Wf, u32 C_IN, u32 C_OUT,
-                                                                 u32 NT, u32 chunks, u32 KG, u32 total) {
-    const u32 t = blockIdx.x * 256 + threadIdx.x;
+                                                                 u32 NT, u32 chunks, u32 KG, u32 total, PendingSum sum) {
+    if constexpr (SUM) {
+        __shared__ __attribute__((aligned(16))) float red[kPendingSumFloats];
+        if (blockIdx.x < sum.blocks) {
+            pending_sum_block(sum, blockIdx.x, red);
+            return;
+        }
+    }
+    const u32 t = (blockIdx.x - (SUM ? sum.blocks : 0)) * 256 + threadIdx.x;
     if (t >= total) return;
     const u32 lane = t & 63, frag = t >> 6;  // fragments in memory order
     const u32 tap = frag % NT, rest = frag / NT;
@@ -579,7 +587,7 @@ inline ConvSplitArgs conv_split_args(const float *Wt, const float *X, float *Y, 
 template <class C, bool DGRAD>
 inline int launch_conv_split(const float *Wt, const float *X, float *Y, const float *bias, unsigned char *Wf, u32 N, u32 C_IN, u32 C_OUT, u32 H,
                              u32 W, u32 OH, u32 OW, u32 strips, u32 slices, float *part, int pad_y, int pad_x, u32 relu, hipStream_t s,
-                             const char *what) {
+                             const char *what, const PendingSum *sum) {
     ConvSplitArgs a = conv_split_args<C>(Wt, X, Y, bias, Wf, N, C_IN, C_OUT, H, W, OH, OW, strips, slices, pad_y, pad_x);
     a.w_oc = DGRAD ? C::NT : C_IN * C::NT, a.w_ic = DGRAD ? C_OUT * C::NT : C::NT;
     a.tap0 = DGRAD ? C::NT - 1 : 0, a.tap_i = DGRAD ? -C::FW : C::FW, a.tap_j = DGRAD ? -1 : 1;
@@ -600,8 +608,12 @@ inline int launch_conv_split(const float *Wt, const float *X, float *Y, const fl
         }
         return CRB_OK;
     }
-    hipLaunchKernelGGL(conv_split_filters_kernel<DGRAD>, dim3(ceil_div(total, 256u)), dim3(256), 0, s, Wt, Wf, C_IN, C_OUT, u32(C::NT), a.chunks,
-                       u32(C::KG), total);
+    if (DGRAD && sum)
+        hipLaunchKernelGGL((conv_split_filters_kernel<DGRAD, DGRAD>), dim3(sum->blocks + ceil_div(total, 256u)), dim3(256), 0, s, Wt, Wf, C_IN, C_OUT, u32(C::NT),
+                           a.chunks, u32(C::KG), total, *sum);
+    else
+        hipLaunchKernelGGL(conv_split_filters_kernel<DGRAD>, dim3(ceil_div(total, 256u)), dim3(256), 0, s, Wt, Wf, C_IN, C_OUT, u32(C::NT), a.chunks,
+                           u32(C::KG), total, PendingSum());
     if (int st = check_launch(what)) return st;
     hipLaunchKernelGGL((conv_split_kernel<C>), dim3(u32(tiles), 1, slices), dim3(C::NTH), 0, s, a);
     int st = check_launch(what);
@@ -639,9 +651,17 @@ struct ConvSplitClassFilters {
     int tap0[4], tap_i, tap_j;
     u32 c_in, c_out, nt_all, chunks, total;
 };
+template <bool SUM>
 static __global__ void __launch_bounds__(256) conv_split_class_filters_kernel(const float *__restrict__ W, unsigned char *__restrict__ Wf,
-                                                                              ConvSplitClassFilters a) {
-    const u32 t = blockIdx.x * 256 + threadIdx.x;
+                                                                              ConvSplitClassFilters a, PendingSum sum) {
+    if constexpr (SUM) {
+        __shared__ __attribute__((aligned(16))) float red[kPendingSumFloats];
+        if (blockIdx.x < sum.blocks) {
+            pending_sum_block(sum, blockIdx.x, red);
+            return;
+        }
+    }
+    const u32 t = (blockIdx.x - (SUM ? sum.blocks : 0)) * 256 + threadIdx.x;
     if (t >= a.total) return;
     const u32 lane = t & 63, frag = t >> 6, k = frag < a.first[1] ? 0 : (frag < a.first[2] ? 1 : (frag < a.first[3] ? 2 : 3));
     const u32 f = frag - a.first[k], tap = f % a.nt[k], rest = f / a.nt[k], ch = rest % a.chunks, ob = rest / a.chunks;
@@ -696,7 +716,7 @@ inline size_t conv_split_class_filter_bytes(u32 C_IN, u32 C_OUT) {
 // F = 2R - 1. Wf: conv_split_class_filter_bytes of scratch, or null (PLAIN).
 template <class Set>
 inline int launch_conv_split_classes(const float *Wt, const float *dY, float *dX, unsigned char *Wf, u32 N, u32 IC, u32 OC, u32 IH, u32 IW, u32 OH, u32 OW,
-                                     const u32 (&strips)[4], u32 pH, u32 pW, hipStream_t s, const char *what) {
+                                     const u32 (&strips)[4], u32 pH, u32 pW, hipStream_t s, const char *what, const PendingSum *sum) {
     typedef typename Set::C0 C;
     constexpr u32 F = 2 * Set::R - 1;
     ConvSplitClassArgs a = {};
@@ -734,7 +754,10 @@ inline int launch_conv_split_classes(const float *Wt, const float *dY, float *dX
         return check_launch(what);
     }
     f.total = steps * 64;
-    hipLaunchKernelGGL(conv_split_class_filters_kernel, dim3(ceil_div(f.total, 256u)), dim3(256), 0, s, Wt, Wf, f);
+    if (sum)
+        hipLaunchKernelGGL(conv_split_class_filters_kernel<true>, dim3(sum->blocks + ceil_div(f.total, 256u)), dim3(256), 0, s, Wt, Wf, f, *sum);
+    else
+        hipLaunchKernelGGL(conv_split_class_filters_kernel<false>, dim3(ceil_div(f.total, 256u)), dim3(256), 0, s, Wt, Wf, f, PendingSum());
     if (int st = check_launch(what)) return st;
     hipLaunchKernelGGL((conv_split_class_kernel<Set, false>), dim3(u32(tiles)), dim3(C::NTH), 0, s, a);
     return check_launch(what);

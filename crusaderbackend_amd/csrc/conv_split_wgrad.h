@@ -416,9 +416,10 @@ inline SplitWgradPlan split_wgrad_plan(u32 N, u32 IC, u32 OC, u32 H, u32 W, u32 
     return p;
 }
 
+// later: null, or where the slices' sum is left for another launch.
 template <class C>
 inline int launch_split_wgrad(const SplitWgradPlan &p, const float *dY, const float *X, float *dW, float *ws, u32 N, u32 IC, u32 OC, u32 H, u32 W,
-                              u32 OH, u32 OW, int pad_y, int pad_x, hipStream_t s, const char *what) {
+                              u32 OH, u32 OW, int pad_y, int pad_x, hipStream_t s, const char *what, PendingSum *later) {
     SplitWgradArgs a;
     a.dY = dY, a.X = X, a.out = p.splits > 1 ? ws : dW;
     a.images = N, a.IC = IC, a.OC = OC, a.H = H, a.W = W, a.HW = H * W, a.OHW = OH * OW, a.OW = OW;
@@ -432,6 +433,7 @@ inline int launch_split_wgrad(const SplitWgradPlan &p, const float *dY, const fl
     if (uint64_t(p.pairs) * p.splits > 0x7fffffffull) return fail(CRB_EINVAL_SHAPE, "%s: launch grid too large", what);
     hipLaunchKernelGGL((split_wgrad_kernel<C>), dim3(p.pairs * p.splits, C::F / C::ROWS), dim3(C::NTH), 0, s, a);
     if (int st = check_launch(what)) return st;
+    if (p.splits > 1 && later) return *later = pending_sum(ws, dW, OC * IC * C::F * C::F, p.splits), CRB_OK;
     if (p.splits > 1) return launch_splitk_reduce(ws, dW, OC * IC * C::F * C::F, p.splits, ReduceEpi{nullptr, 1, 1, EPI_ACCUM}, s, what);
     return CRB_OK;
 }

@@ -287,7 +287,7 @@ inline SplitWgradPlan rows_wgrad_plan(u32 N, u32 IC, u32 OC, u32 H, u32 W, size_
 }
 
 inline int launch_rows_wgrad(const SplitWgradPlan &p, const float *dY, const float *X, float *dW, float *ws, u32 N, u32 IC, u32 OC, u32 H, u32 W, hipStream_t s,
-                             const char *what) {
+                             const char *what, PendingSum *later) {
     RowsWgradArgs a;
     a.dY = dY, a.X = X, a.out = p.splits > 1 ? ws : dW;
     a.images = N, a.IC = IC, a.OC = OC, a.H = H, a.W = W, a.HW = H * W;
@@ -301,6 +301,7 @@ inline int launch_rows_wgrad(const SplitWgradPlan &p, const float *dY, const flo
     else if (at % 8 == 0) hipLaunchKernelGGL((rows_wgrad_kernel<2>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((rows_wgrad_kernel<1>), grid, block, 0, s, a);
     if (int st = check_launch(what)) return st;
+    if (p.splits > 1 && later) return *later = pending_sum(ws, dW, OC * IC * 9, p.splits), CRB_OK;
     if (p.splits > 1) return launch_splitk_reduce(ws, dW, OC * IC * 9, p.splits, ReduceEpi{nullptr, 1, 1, EPI_ACCUM}, s, what);
     return CRB_OK;
 }

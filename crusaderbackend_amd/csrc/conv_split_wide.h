@@ -32,10 +32,17 @@ struct ConvWideCfg {
 
 // Filters -> fragments: [output block of 32][chunk of 32][tap][half of the block][part] of 1 KB (lane l: output channel l % 16 of the half,
 // channels 8 * (l / 16) + 0..7 of the chunk), zero beyond the channel counts.
-template <bool DGRAD>
+template <bool DGRAD, bool SUM = false>
 __global__ void __launch_bounds__(256) conv_wide_filters_kernel(const float *__restrict__ W, unsigned char *__restrict__ Wf, u32 C_IN, u32 C_OUT,
-                                                                u32 NT, u32 chunks, u32 total) {
-    const u32 t = blockIdx.x * 256 + threadIdx.x;
+                                                                u32 NT, u32 chunks, u32 total, PendingSum sum) {
+    if constexpr (SUM) {
+        __shared__ __attribute__((aligned(16))) float red[kPendingSumFloats];
+        if (blockIdx.x < sum.blocks) {
+            pending_sum_block(sum, blockIdx.x, red);
+            return;
+        }
+    }
+    const u32 t = (blockIdx.x - (SUM ? sum.blocks : 0)) * 256 + threadIdx.x;
     if (t >= total) return;
     const u32 lane = t & 63, frag = t >> 6, half = frag & 1, step = frag >> 1;  // fragments in memory order
     const u32 tap = step % NT, rest = step / NT, ch = rest % chunks, ob = rest / chunks;
@@ -360,7 +367,7 @@ inline size_t conv_wide_filter_bytes(u32 C_IN, u32 C_OUT) {  // (a tap more: fil
 template <class C, bool DGRAD>
 inline int launch_conv_wide(const float *Wt, const float *X, float *Y, const float *bias, unsigned char *Wf, u32 N, u32 C_IN, u32 C_OUT, u32 H,
                             u32 W, u32 OH, u32 OW, u32 strips, u32 slices, float *part, int pad_y, int pad_x, u32 relu, hipStream_t s,
-                            const char *what) {
+                            const char *what, const PendingSum *sum) {
     ConvSplitArgs a = conv_split_args<C>(Wt, X, Y, bias, Wf, N, C_IN, C_OUT, H, W, OH, OW, strips, slices, pad_y, pad_x);
     a.w_oc = DGRAD ? C::NT : C_IN * C::NT, a.w_ic = DGRAD ? C_OUT * C::NT : C::NT;
     a.tap0 = DGRAD ? C::NT - 1 : 0, a.tap_i = DGRAD ? -C::FW : C::FW, a.tap_j = DGRAD ? -1 : 1;
@@ -381,7 +388,11 @@ inline int launch_conv_wide(const float *Wt, const float *X, float *Y, const flo
         return CRB_OK;
     }
     const u32 total = a.oc_tiles * C::WM * a.chunks * C::NT * 128;
-    hipLaunchKernelGGL(conv_wide_filters_kernel<DGRAD>, dim3(ceil_div(total, 256u)), dim3(256), 0, s, Wt, Wf, C_IN, C_OUT, u32(C::NT), a.chunks, total);
+    if (DGRAD && sum)
+        hipLaunchKernelGGL((conv_wide_filters_kernel<DGRAD, DGRAD>), dim3(sum->blocks + ceil_div(total, 256u)), dim3(256), 0, s, Wt, Wf, C_IN, C_OUT, u32(C::NT),
+                           a.chunks, total, *sum);
+    else
+        hipLaunchKernelGGL(conv_wide_filters_kernel<DGRAD>, dim3(ceil_div(total, 256u)), dim3(256), 0, s, Wt, Wf, C_IN, C_OUT, u32(C::NT), a.chunks, total, PendingSum());
     if (int st = check_launch(what)) return st;
     hipLaunchKernelGGL((conv_wide_kernel<C>), dim3(u32(tiles), 1, slices), dim3(C::NTH), 0, s, a);
     int st = check_launch(what);

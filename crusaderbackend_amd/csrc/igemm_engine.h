@@ -534,13 +534,13 @@ struct ReduceEpi {
     u32 flags;  // EPI_ACCUM | EPI_RELU
 };
 
+// `red`: 256 floats of LDS; `block`: which group of OUTS results this workgroup sums.
 template <int OUTS>
-static __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float *__restrict__ partial, float *__restrict__ C, u32 count,
-                                                                   u32 splits, ReduceEpi e, FastDiv bdiv) {
+__device__ __forceinline__ void reduce_block(const float *__restrict__ partial, float *__restrict__ C, u32 count, u32 splits, const ReduceEpi &e,
+                                             const FastDiv &bdiv, u32 block, float *red) {
     constexpr u32 ZL = 256 / OUTS;
-    __shared__ float red[ZL][OUTS];
     const u32 o = threadIdx.x % OUTS, g = threadIdx.x / OUTS;
-    const u32 i = blockIdx.x * OUTS + o;
+    const u32 i = block * OUTS + o;
     float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
     if (i < count) {
         const float *p = partial + i;
@@ -553,17 +553,24 @@ static __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float *
         }
         for (; zz < splits; zz += ZL) s0 += p[size_t(zz) * count];
     }
-    red[g][o] = (s0 + s1) + (s2 + s3);
+    red[g * OUTS + o] = (s0 + s1) + (s2 + s3);
     __syncthreads();
     if (g == 0 && i < count) {
-        float r = red[0][o];
+        float r = red[o];
 #pragma unroll
-        for (u32 k = 1; k < ZL; ++k) r += red[k][o];
+        for (u32 k = 1; k < ZL; ++k) r += red[k * OUTS + o];
         if (e.bias) r += e.bias[bdiv.div(i) % e.bias_mod];
         if (e.flags & EPI_ACCUM) r += C[i];
         if (e.flags & EPI_RELU) r = r > 0.f ? r : 0.f;
         C[i] = r;
     }
+}
+
+template <int OUTS>
+static __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float *__restrict__ partial, float *__restrict__ C, u32 count,
+                                                                   u32 splits, ReduceEpi e, FastDiv bdiv) {
+    __shared__ float red[256];
+    reduce_block<OUTS>(partial, C, count, splits, e, bdiv, blockIdx.x, red);
 }
 
 // Same reduction with 16-byte loads: OL lanes cover 4 * OL consecutive results of one slice (a full 128-byte line
@@ -661,6 +668,34 @@ inline int launch_splitk_reduce(const float *partial, float *C, u32 count, u32 s
     else
         hipLaunchKernelGGL(splitk_reduce_kernel<8>, dim3(ceil_div(count, 8)), dim3(256), 0, s, partial, C, count, splits, e, bdiv);
     return check_launch(what);
+}
+
+// The accumulating reduction of launch_splitk_reduce as a part of another launch: its first `blocks` workgroups of 256 threads.
+struct PendingSum {
+    const float *partial = nullptr;
+    float *C = nullptr;
+    u32 count = 0, splits = 0, lanes = 0, blocks = 0;  // lanes: of reduce_vec_block, or 1000 + results of reduce_block
+};
+inline PendingSum pending_sum(const float *partial, float *C, u32 count, u32 splits) {
+    PendingSum p;
+    p.partial = partial, p.C = C, p.count = count, p.splits = splits;
+    if (reduce_vec_ok(partial, count)) p.lanes = reduce_vec_ol(count, splits), p.blocks = ceil_div(count, 4 * p.lanes);
+    else p.lanes = 1000 + (count >= 32u * 512u ? 32 : count >= 16u * 256u ? 16 : 8), p.blocks = ceil_div(count, p.lanes - 1000);
+    return p;
+}
+constexpr int kPendingSumFloats = (256 / 8) * (4 * 8 + 4);  // LDS; the other forms take less
+__device__ __forceinline__ void pending_sum_block(const PendingSum &p, u32 block, float *red) {
+    const ReduceEpi e{nullptr, 1, 1, EPI_ACCUM};
+    const FastDiv one;
+    switch (p.lanes) {
+        case 8: reduce_vec_block<8>(p.partial, p.C, p.count, p.splits, e, one, block, red); break;
+        case 16: reduce_vec_block<16>(p.partial, p.C, p.count, p.splits, e, one, block, red); break;
+        case 32: reduce_vec_block<32>(p.partial, p.C, p.count, p.splits, e, one, block, red); break;
+        case 64: reduce_vec_block<64>(p.partial, p.C, p.count, p.splits, e, one, block, red); break;
+        case 1032: reduce_block<32>(p.partial, p.C, p.count, p.splits, e, one, block, red); break;
+        case 1016: reduce_block<16>(p.partial, p.C, p.count, p.splits, e, one, block, red); break;
+        default: reduce_block<8>(p.partial, p.C, p.count, p.splits, e, one, block, red); break;
+    }
 }
 
 // C[i] (+)= sum over z of partial[z][i], left to right, then bias and ReLU: what launches of one slice after the other, each adding

@@ -1,0 +1,47 @@
+"""crb_conv_bwd where both gradients run on split operands: the slices' sum rides on the launch that splits the filters. The bits of the two calls."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# (N, IC, H, W, OC, F, stride, pad): sums of whole quads and not, of each number of lanes, filters in steps of 16 and 32 channels, K groups, residue classes
+SHAPES = [(32, 64, 28, 28, 64, 3, 1, 1), (40, 64, 44, 40, 64, 3, 1, 1), (12, 64, 24, 24, 96, 3, 1, 1), (9, 41, 31, 33, 65, 3, 1, 1), (4, 256, 14, 14, 256, 3, 1, 1),
+          (24, 30, 61, 47, 75, 5, 2, 2), (16, 64, 28, 28, 128, 3, 2, 1), (7, 64, 21, 19, 48, 5, 1, 2), (8, 33, 20, 22, 33, 3, 1, 0)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_the_two_calls(dev, shape):
+    import torch
+    from crusaderbackend_amd import capi
+
+    N, IC, H, W, OC, F, s, p = shape
+    g = capi.ConvGeom.make(N, IC, H, W, OC, F, F, s, s, p, p)
+    X, Wt, dY, dW0 = (torch.randn(*a, device=dev) for a in ((N, IC, H, W), (OC, IC, F, F), (N, OC, g.OH, g.OW), (OC, IC, F, F)))
+    need = capi.conv_wgrad_workspace_bytes(g)
+    dX, dW = torch.empty_like(X), dW0.clone()
+    capi.conv_dgrad(Wt, dY, dX, g)
+    capi.conv_wgrad(dY, X, dW, g, workspace=torch.empty(need // 4 + 4, device=dev))
+    torch.cuda.synchronize()
+
+    def check(stream=None, workspace=None):
+        a, b = torch.full_like(dX, 7.0), dW0.clone()
+        torch.cuda.synchronize()
+        capi.conv_bwd(Wt, dY, X, a, b, g, workspace=workspace, stream=stream)
+        torch.cuda.synchronize()
+        assert torch.equal(a, dX) and torch.equal(b, dW)
+
+    ws = torch.empty(need // 4 + 4, device=dev)
+    check(workspace=ws)
+    check()
+    side, shared = torch.cuda.Stream(device=dev), torch.empty((need + capi.conv_dgrad_workspace_bytes(g)) // 4 + 64, device=dev)
+    try:
+        capi.bind_workspace(shared, stream=side)  # split filters and slices in one place
+        check(side, shared)
+        capi.bind_workspace(shared[:64], stream=side)  # no room for split filters
+        try:
+            check(side, ws)
+        except capi.CrbError as e:
+            assert e.status == capi.CRB_EWORKSPACE
+            with pytest.raises(capi.CrbError):  # where the data gradient alone is refused too
+                capi.conv_dgrad(Wt, dY, dX, g, stream=side)
+    finally:
+        capi.bind_workspace(None, stream=side)
