@@ -55,6 +55,28 @@ __device__ __forceinline__ v4f exchange_groups(v4f v) {
     return __builtin_bit_cast(v4f, r);
 }
 
+// A lane's place in a K-concatenated batch: offsets of its element of A and of B, which go on by addition (behind the batch's end they are not used).
+struct BatchWalk {
+    u32 kr, oa, ob;
+    __device__ __forceinline__ BatchWalk(const TinyGemmArgs &a, const float *pa, const float *pb, u32 kk) {
+        u32 nd;
+        a.kb_len.divmod(kk, nd, kr);
+        oa = u32(pa - a.A) + nd * a.a_bs + kr * a.a_ks, ob = u32(pb - a.B) + nd * a.b_bs + kr * a.b_ks;
+    }
+    __device__ __forceinline__ void step(const TinyGemmArgs &a, u32 n) {
+        const u32 len = a.kb_len.d;
+        kr += n, oa += n * a.a_ks, ob += n * a.b_ks;
+        if (len >= n) {  // at most one entry on
+            const bool over = kr >= len;
+            kr -= over ? len : 0u, oa += over ? a.a_bs - len * a.a_ks : 0u, ob += over ? a.b_bs - len * a.b_ks : 0u;
+        } else {
+            u32 nd;
+            a.kb_len.divmod(kr, nd, kr);
+            oa += nd * (a.a_bs - len * a.a_ks), ob += nd * (a.b_bs - len * a.b_ks);
+        }
+    }
+};
+
 // BATCH: a K-concatenated batch of more than one entry. Without one, whole groups of sixteen k are loaded from addresses that are a lane's
 // constant offset behind a uniform one and need no vector arithmetic (a division by the entry's length, a 64-bit product and the tests of
 // row, column and k for every load were most of the kernel's instructions). Us, before / after: NN 128 x 512 x 512 6.6 / 4.0, 256 x 256 x 1024 11.2 /
@@ -116,15 +138,19 @@ __global__ void __launch_bounds__(64 * WAVES) tiny_gemm_kernel(TinyGemmArgs a) {
             });
         }
         constexpr int U = BATCH ? 4 : 1;  // 16-k groups requested together (without a batch: what is left of the last one)
+        BatchWalk at(a, pa, pb, k + 4 * g);
         for (; k < kq; k += 16 * U) {
             v4f va[U], vb[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const u32 kk = k + 16 * u + 4 * g;
                 const bool in = kk < kq;  // kq, kk and a batch entry's length are multiples of 4: a quad is inside or outside as a whole
-                u32 nd = 0, kr = in ? kk : 0;
-                if constexpr (BATCH) a.kb_len.divmod(kr, nd, kr);
-                va[u] = *reinterpret_cast<const v4fu *>(pa + size_t(nd) * a.a_bs + kr), vb[u] = *reinterpret_cast<const v4fu *>(pb + size_t(nd) * a.b_bs + kr);
+                if constexpr (BATCH) {
+                    va[u] = *reinterpret_cast<const v4fu *>(a.A + (in ? at.oa : 0)), vb[u] = *reinterpret_cast<const v4fu *>(a.B + (in ? at.ob : 0));
+                    at.step(a, 16);
+                } else {
+                    va[u] = *reinterpret_cast<const v4fu *>(pa + (in ? kk : 0)), vb[u] = *reinterpret_cast<const v4fu *>(pb + (in ? kk : 0));
+                }
                 if (!in) va[u] = vb[u] = v4f{0.f, 0.f, 0.f, 0.f};
             }
 #pragma unroll
@@ -178,15 +204,19 @@ __global__ void __launch_bounds__(64 * WAVES) tiny_gemm_kernel(TinyGemmArgs a) {
             }
         }
         constexpr int U = BATCH ? 16 : 4;  // MFMA steps requested together (without a batch: what is left of the last group)
+        BatchWalk at(a, pa, pb, k + g);
         for (; k < ke; k += 4 * U) {
             float va[U], vb[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const u32 kk = k + 4 * u + g;
                 const bool in = kk < ke;
-                u32 nd = 0, kr = in ? kk : 0;
-                if constexpr (BATCH) a.kb_len.divmod(kr, nd, kr);
-                va[u] = pa[size_t(nd) * a.a_bs + size_t(kr) * a.a_ks], vb[u] = pb[size_t(nd) * a.b_bs + size_t(kr) * a.b_ks];
+                if constexpr (BATCH) {
+                    va[u] = a.A[in ? at.oa : 0], vb[u] = a.B[in ? at.ob : 0];
+                    at.step(a, 4);
+                } else {
+                    va[u] = pa[size_t(in ? kk : 0) * a.a_ks], vb[u] = pb[size_t(in ? kk : 0) * a.b_ks];
+                }
                 if (!in) va[u] = vb[u] = 0.f;
             }
 #pragma unroll
@@ -245,26 +275,25 @@ inline bool tiny_gemm_beats_engine(u32 M, u32 N, u32 K, u32 batch, u32 most) {
 // Waves of a workgroup, which share its contraction. More of them keep the chains of a long one short, in time (us, 4 / 8 / 16 waves: NT 11 x 2012 x
 // 3053 15.1 / 10.5 / 10.8, 13 x 107 x 2127 7.5 / 6.8 / 7.0) and in roundings (TN 112 x 112 x 1200 3.2 / 2.3 / 1.8e-7 from float64, the engine, which
 // cuts it, 2.2e-7; 502 x 15 x 614 2.3e-7 on either).
-inline u32 tiny_gemm_waves(u32 K) { return K <= 640u ? 4u : (K <= 1024u ? 8u : 16u); }
+// A batch stays on four, whose loads are more arithmetic than a chain (NTA 82 x 14 x 10 * 225 on sixteen: a 1x1 layer's three passes 35.6 -> 41.4).
+inline u32 tiny_gemm_waves(u32 K, bool batch) { return batch || K <= 640u ? 4u : (K <= 1024u ? 8u : 16u); }
 
 // kb_len: length of one batch entry's contraction (a.K for a plain product); a.K = the whole contraction.
 inline int launch_tiny_gemm(TinyGemmArgs a, u32 kb_len, u32 a_bs, u32 b_bs, hipStream_t s, const char *what) {
     a.kb_len = FastDiv(kb_len), a.a_bs = a_bs, a.b_bs = b_bs;
     a.tiles_n = ceil_div(a.N, 16u);
-    const u32 blocks = ceil_div(a.M, 16u) * a.tiles_n, waves = tiny_gemm_waves(a.K);
+    const u32 blocks = ceil_div(a.M, 16u) * a.tiles_n, waves = tiny_gemm_waves(a.K, kb_len != a.K);
     a.k_per_wave = ceil_div(ceil_div(a.K, waves), 16u) * 16u;
     const bool kvec = a.a_ks == 1 && a.b_ks == 1 && (kb_len == a.K || (kb_len % 4 == 0 && a_bs % 4 == 0 && b_bs % 4 == 0));
     auto launch = [&](auto w_c) {
         constexpr int W = decltype(w_c)::value;
-        if (kb_len != a.K) {
-            if (kvec) hipLaunchKernelGGL((tiny_gemm_kernel<true, true, W>), dim3(blocks), dim3(64 * W), 0, s, a);
-            else hipLaunchKernelGGL((tiny_gemm_kernel<false, true, W>), dim3(blocks), dim3(64 * W), 0, s, a);
-        } else {
-            if (kvec) hipLaunchKernelGGL((tiny_gemm_kernel<true, false, W>), dim3(blocks), dim3(64 * W), 0, s, a);
-            else hipLaunchKernelGGL((tiny_gemm_kernel<false, false, W>), dim3(blocks), dim3(64 * W), 0, s, a);
-        }
+        if (kvec) hipLaunchKernelGGL((tiny_gemm_kernel<true, false, W>), dim3(blocks), dim3(64 * W), 0, s, a);
+        else hipLaunchKernelGGL((tiny_gemm_kernel<false, false, W>), dim3(blocks), dim3(64 * W), 0, s, a);
     };
-    if (waves == 4) launch(std::integral_constant<int, 4>());
+    if (kb_len != a.K) {
+        if (kvec) hipLaunchKernelGGL((tiny_gemm_kernel<true, true, 4>), dim3(blocks), dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((tiny_gemm_kernel<false, true, 4>), dim3(blocks), dim3(256), 0, s, a);
+    } else if (waves == 4) launch(std::integral_constant<int, 4>());
     else if (waves == 8) launch(std::integral_constant<int, 8>());
     else launch(std::integral_constant<int, 16>());
     return check_launch(what);
