@@ -182,8 +182,10 @@ int crb_conv_bias(float *Y, const float *bias, uint32_t N, uint32_t C, uint32_t 
  * calls Conv2D::xGrads / Conv2D::paramGrads make back to back (seann/operands/seblas/Conv2D.cu:18-29: convDerive, then
  * convError): the two are independent, and for the 3x3 layer shapes of CIFAR residual networks (stride 1, and the 16 -> 32
  * stride-2 transition) and the growth-12 layers of dense networks (48 -> 12) they run as one launch that shares the chip;
- * other shapes run the two calls one after the other. Results are identical to the separate calls.
- * dX must not overlap X or dY. */
+ * layers of other shapes whose gradients both run on split operands take the weight gradient first, its slices (in `workspace`, if
+ * given) summed by the launch that splits the data gradient's filters; the rest run the two calls one after the other. Results are
+ * identical to the separate calls. dX must not overlap X or dY; for the shapes of one launch dW must not overlap W, dY or dX
+ * (elsewhere such a dW takes the two calls in their order). */
 int crb_conv_bwd(const float *W, const float *dY, const float *X, float *dX, float *dW, const crb_conv_geom *g, void *workspace,
                  size_t workspace_bytes, void *stream);
 

@@ -45,3 +45,37 @@ def test_the_two_calls(dev, shape):
                 capi.conv_dgrad(Wt, dY, dX, g, stream=side)
     finally:
         capi.bind_workspace(None, stream=side)
+
+
+@pytest.mark.parametrize("over,off", [("W", 0), ("W", 4), ("dY", 0), ("dY", 1), ("dX", 8), ("workspace", 0)])
+@pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[5]], ids=lambda s: "x".join(map(str, s)))
+def test_weight_gradient_on_top_of_an_operand(dev, shape, over, off):
+    """dW on the filters, on dY or on dX, and the filters on the workspace: what the two calls in their order leave there."""
+    import torch
+    from crusaderbackend_amd import capi
+
+    N, IC, H, W, OC, F, s, p = shape
+    g = capi.ConvGeom.make(N, IC, H, W, OC, F, F, s, s, p, p)
+    n_w = OC * IC * F * F
+    flat = {"X": N * IC * H * W, "W": n_w, "dY": N * OC * g.OH * g.OW, "dX": N * IC * H * W, "workspace": capi.conv_wgrad_workspace_bytes(g) // 4}
+    start = {k: torch.randn(n + 16, device=dev) for k, n in flat.items()}
+    start["dW"] = torch.randn(n_w, device=dev)
+
+    def result(fn):
+        t = {k: v.clone() for k, v in start.items()}
+        if over == "workspace":
+            t["W"] = t["workspace"][:n_w]
+            t["W"].copy_(start["W"][:n_w])
+        else:
+            t["dW"] = t[over][off : off + n_w]
+        torch.cuda.synchronize()
+        fn(t)
+        torch.cuda.synchronize()
+        return [t[k] for k in ("dX", "dW", "dY")]
+
+    def two(t):
+        capi.conv_dgrad(t["W"], t["dY"], t["dX"], g)
+        capi.conv_wgrad(t["dY"], t["X"], t["dW"], g, workspace=t["workspace"])
+
+    for a, b in zip(result(two), result(lambda t: capi.conv_bwd(t["W"], t["dY"], t["X"], t["dX"], t["dW"], g, workspace=t["workspace"]))):
+        assert torch.equal(a, b)
