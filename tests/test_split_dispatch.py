@@ -107,3 +107,11 @@ def test_strided_wide_filters_on_few_channels():
         N, IC, H, W, OC, F, s, p = shape
         assert queries(*shape)[0] == slices * N * OC * ((H + 2 * p - F) // 2 + 1) * ((W + 2 * p - F) // 2 + 1) * 4, shape
     assert queries(28, 146, 9, 6, 28, 5, 2, 4)[0] == (10 * 2 * 25 + 2) * 3072 + 28 * 28 * 7 * 5 * 4 * 10
+
+
+def test_tilings_of_the_weight_gradient_beside_the_rows_kernel():
+    """What a tile of the transposing kernel is charged against the rows kernel does not move the choice between its own two tilings, where the
+    rows kernel is not for the layer: ten slices, not twenty-one of 64-wide blocks, three instead of seven, one instead of three."""
+    for shape, slices in (((45, 96, 37, 8, 256, 3, 1, 1), 10), ((36, 96, 19, 32, 256, 3, 1, 1), 10), ((10, 64, 50, 32, 376, 3, 1, 1), 10), ((7, 469, 12, 8, 261, 3, 1, 1), 0),
+                          ((83, 64, 44, 33, 64, 3, 1, 1), 61), ((55, 355, 7, 7, 189, 3, 1, 1), 3), ((22, 32, 50, 50, 192, 3, 1, 2), 39), ((64, 64, 15, 15, 320, 3, 1, 2), 12)):
+        assert queries(*shape)[2] == slices * shape[1] * shape[4] * 36, shape
