@@ -115,3 +115,12 @@ def test_tilings_of_the_weight_gradient_beside_the_rows_kernel():
     for shape, slices in (((45, 96, 37, 8, 256, 3, 1, 1), 10), ((36, 96, 19, 32, 256, 3, 1, 1), 10), ((10, 64, 50, 32, 376, 3, 1, 1), 10), ((7, 469, 12, 8, 261, 3, 1, 1), 0),
                           ((83, 64, 44, 33, 64, 3, 1, 1), 61), ((55, 355, 7, 7, 189, 3, 1, 1), 3), ((22, 32, 50, 50, 192, 3, 1, 2), 39), ((64, 64, 15, 15, 320, 3, 1, 2), 12)):
         assert queries(*shape)[2] == slices * shape[1] * shape[4] * 36, shape
+
+
+def test_rows_weight_gradients_stay_in_the_scratch_of_the_kernel_before():
+    """What the transposing kernel takes without slices, or with no more of them than the built-in buffer holds, the rows kernel takes so too:
+    crb_conv_wgrad_noalloc and calls without scratch are refused nothing."""
+    for N, IC, H, W, OC in ((4, 199, 10, 10, 316), (5, 206, 9, 10, 87), (1, 85, 21, 22, 281), (5, 452, 10, 10, 40)):
+        assert queries(N, IC, H, W, OC, 3, 1, 1)[2] == 0, (N, IC, H, W, OC)
+    for N, IC, H, W, OC in ((51, 481, 18, 18, 32), (59, 128, 29, 30, 57), (4, 315, 60, 56, 32), (14, 255, 11, 14, 160), (27, 158, 10, 10, 155), (13, 64, 56, 56, 64)):
+        assert 0 < queries(N, IC, H, W, OC, 3, 1, 1)[2] <= 8 << 20, (N, IC, H, W, OC)
