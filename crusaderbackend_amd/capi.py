@@ -111,6 +111,20 @@ class _Unloaded:
 _calls = _Unloaded()
 
 
+def _number(kind, value):
+    """What ctypes makes of `value` as its type `kind`: anything with __index__, for c_float __float__ (numpy scalars, tensors of one element), a ctypes
+    number of that type, or what stands for it by _as_parameter_."""
+    of = getattr(ctypes, kind)
+    if isinstance(value, of):
+        return value.value
+    try:
+        return of(value).value
+    except Exception as e:
+        if hasattr(value, "_as_parameter_"):
+            return _number(kind, value._as_parameter_)
+        raise ctypes.ArgumentError(f"{type(value).__name__} is no {kind}: {e}") from None
+
+
 def load():
     """Load the HIP library (once) and attach signatures. Raises OSError if it has not been built."""
     global _lib, _calls
@@ -125,7 +139,7 @@ def load():
         loader = importlib.machinery.ExtensionFileLoader("_crb_calls", CALLS_PATH)
         calls = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_crb_calls", CALLS_PATH, loader=loader))
         loader.exec_module(calls)
-        calls.bind(ConvGeom, ctypes.ArgumentError)
+        calls.bind(ConvGeom, ctypes.ArgumentError, _number)
         _lib, _calls = lib, calls
     return _lib
 

@@ -12,18 +12,31 @@
 
 namespace {
 
-PyObject *geom_type, *argument_error, *s_data_ptr, *s_cuda_stream;  // ConvGeom, ctypes.ArgumentError; interned names
+PyObject *geom_type, *argument_error, *number_of, *s_data_ptr, *s_cuda_stream;  // ConvGeom, ctypes.ArgumentError, capi._number; interned names
 
 bool wrong(const char *what) {
     PyErr_SetString(argument_error ? argument_error : PyExc_TypeError, what);
     return false;
 }
 
+// What ctypes takes for a number of type `kind` and is no int or float of Python's: numpy scalars, tensors of one element, numbers of ctypes itself.
+bool converted(PyObject *o, const char *kind, PyObject *&out) {
+    if (!number_of) return wrong("a number is required");
+    out = PyObject_CallFunction(number_of, "sO", kind, o);
+    return out != nullptr;
+}
+
 template <class T>
-bool from_int(PyObject *o, T &out) {  // (as ctypes: no overflow check)
-    if (!PyLong_Check(o)) return wrong("an integer is required");
-    out = T(PyLong_AsUnsignedLongLongMask(o));
-    return true;
+bool from_int(PyObject *o, const char *kind, T &out) {  // (as ctypes: no overflow check)
+    PyObject *n = nullptr;
+    if (!PyLong_Check(o)) {
+        if (!converted(o, kind, n)) return false;
+        o = n;
+    }
+    const bool is = PyLong_Check(o);
+    if (is) out = T(PyLong_AsUnsignedLongLongMask(o));
+    Py_XDECREF(n);
+    return is || wrong("an integer is required");
 }
 
 // A device address: None, or what `name` of the object says (a method of tensors, an attribute of streams).
@@ -32,6 +45,7 @@ bool address(PyObject *o, PyObject *name, bool method, void *&out) {
     if (o == Py_None) return true;
     PyObject *v = method ? PyObject_CallMethodNoArgs(o, name) : PyObject_GetAttr(o, name);
     if (!v) return false;
+    if (v == Py_None) return Py_DECREF(v), true;
     out = PyLong_AsVoidPtr(v);
     Py_DECREF(v);
     return !(out == nullptr && PyErr_Occurred());
@@ -42,25 +56,30 @@ struct Arg;
 template <>
 struct Arg<uint32_t> {
     uint32_t v;
-    bool get(PyObject *o, bool) { return from_int(o, v); }
+    bool get(PyObject *o, bool) { return from_int(o, "c_uint32", v); }
 };
 template <>
 struct Arg<int> {
     int v;
-    bool get(PyObject *o, bool) { return from_int(o, v); }
+    bool get(PyObject *o, bool) { return from_int(o, "c_int", v); }
 };
 template <>
 struct Arg<size_t> {
     size_t v;
-    bool get(PyObject *o, bool) { return from_int(o, v); }
+    bool get(PyObject *o, bool) { return from_int(o, "c_size_t", v); }
 };
 template <>
 struct Arg<float> {
     float v;
     bool get(PyObject *o, bool) {
-        if (!PyFloat_Check(o) && !PyLong_Check(o)) return wrong("a number is required");
+        PyObject *n = nullptr;
+        if (!PyFloat_Check(o) && !PyLong_Check(o)) {
+            if (!converted(o, "c_float", n)) return false;
+            o = n;
+        }
         const double d = PyFloat_AsDouble(o);
         v = float(d);
+        Py_XDECREF(n);
         return !(d == -1.0 && PyErr_Occurred());
     }
 };
@@ -82,7 +101,7 @@ struct Arg<const crb_conv_geom *> {
         if (!geom_type || !PyObject_TypeCheck(o, reinterpret_cast<PyTypeObject *>(geom_type))) return wrong("a ConvGeom is required");
         Py_buffer b;
         if (PyObject_GetBuffer(o, &b, PyBUF_SIMPLE)) return false;
-        const bool fits = b.len == Py_ssize_t(sizeof(copy));
+        const bool fits = b.len >= Py_ssize_t(sizeof(copy));  // (a derived structure may have more fields)
         if (fits) copy = *static_cast<const crb_conv_geom *>(b.buf);
         PyBuffer_Release(&b);
         v = &copy;
@@ -110,13 +129,14 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
     return call(fn, args, n);
 }
 
-PyObject *bind(PyObject *, PyObject *args) {  // (ConvGeom, the error that ctypes raises)
-    PyObject *g, *e;
-    if (!PyArg_ParseTuple(args, "OO", &g, &e)) return nullptr;
+PyObject *bind(PyObject *, PyObject *args) {  // (ConvGeom, the error that ctypes raises, what makes a Python number of any that ctypes takes)
+    PyObject *g, *e, *n;
+    if (!PyArg_ParseTuple(args, "OOO", &g, &e, &n)) return nullptr;
     if (!PyType_Check(g)) return wrong("a type is required"), nullptr;
-    Py_INCREF(g), Py_INCREF(e);
+    Py_INCREF(g), Py_INCREF(e), Py_INCREF(n);
     Py_XSETREF(geom_type, g);
     Py_XSETREF(argument_error, e);
+    Py_XSETREF(number_of, n);
     Py_RETURN_NONE;
 }
 

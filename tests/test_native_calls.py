@@ -1,4 +1,4 @@
-"""The launching entry points as Python callables (csrc/crb_calls.cpp): the same calls as by ctypes, refused where those are (no GPU is touched)."""
+"""The launching entry points as Python callables (csrc/crb_calls.cpp): the same calls as by ctypes, taken and refused where those are (no GPU is touched)."""
 import ctypes
 import re
 
@@ -48,6 +48,48 @@ def test_arguments_of_the_wrong_kind_are_refused():
     for call in (lambda: capi.sgemm_nn(4096, None, None, 1, 1, 1), lambda: capi.conv_fwd(b"x", None, None, None, g), lambda: capi.relu_fwd(None, None, 4, stream=7)):
         with pytest.raises(AttributeError):
             call()
+
+
+def test_numbers_that_ctypes_takes_are_taken():
+    """Sizes and factors that are numpy scalars, tensors of one element, ctypes numbers or stand for one: the status is that of the plain number."""
+    import numpy as np
+    import torch
+
+    class Tensor:
+        def data_ptr(self):
+            return 4096
+
+    class Stands:
+        def __init__(self, v):
+            self._as_parameter_ = v
+
+    class Geom(capi.ConvGeom):
+        _fields_ = [("more", ctypes.c_uint32)]
+
+    t = Tensor()
+    kinds = (np.int64, np.uint32, np.int8, torch.tensor, ctypes.c_uint32, Stands, lambda v: np.array(v)[()], lambda v: Stands(np.int64(v)), int)
+    for kind in kinds:
+        for zero in (4, 5, 6):  # M, N, K: the one that is zero is refused as zero
+            dims = [kind(0 if i == zero else 3) for i in (4, 5, 6)]
+            with pytest.raises(capi.CrbError) as e:
+                capi.sgemm_nn(t, t, t, *dims)
+            assert e.value.status == capi.CRB_EINVAL_SHAPE and "zero dimension" in str(e.value)
+        with pytest.raises(capi.CrbError) as e:
+            capi.sgemm_nn(None, t, t, kind(1), kind(1), kind(1))
+        assert e.value.status == capi.CRB_ENULL
+    for kind in (np.float32, np.float64, np.int64, torch.tensor, ctypes.c_float, Stands, int):
+        v = kind(2)
+        assert capi._number("c_float", v) == 2.0
+        with pytest.raises(capi.CrbError) as e:
+            capi.momentum_apply(None, None, None, np.uint32(4), v, v)
+        assert e.value.status == capi.CRB_ENULL
+    g = Geom(*[getattr(capi.ConvGeom.make(2, 3, 8, 9, 4, 3, 3, 1, 1, 1, 1), n) for n, _ in capi.ConvGeom._fields_], 7)
+    with pytest.raises(capi.CrbError) as e:
+        capi.conv_dgrad(None, t, t, g)
+    assert e.value.status == capi.CRB_ENULL
+    for bad in (np.float32(3), 3.0, "3", None, (3,), ctypes.c_float(3), Stands("3"), torch.tensor([3, 3])):
+        with pytest.raises(ctypes.ArgumentError):
+            capi.sgemm_nn(t, t, t, bad, 0, 1)
 
 
 def test_frozen_wrappers_are_recorded():
