@@ -96,6 +96,8 @@ SIGNATURES = {
                                              _ptr, _ptr]),
 }
 
+_NUMBERS = (_u32, ctypes.c_int, ctypes.c_size_t, ctypes.c_float)
+
 _lib = None
 
 
@@ -220,10 +222,15 @@ class _Converted:
 
     def __getattr__(self, name):
         fn = getattr(self._lib, name)
+        types = SIGNATURES[name][1]
+
+        def convert(a, kind, last):
+            if kind is _ptr:  # (the last argument is the stream)
+                return _stream(a) if last else _p(a)
+            return a if kind in _NUMBERS else ctypes.byref(a)
 
         def call(*args):
-            return fn(*(ctypes.byref(a) if isinstance(a, ConvGeom) else a.data_ptr() if hasattr(a, "data_ptr") else a.cuda_stream if hasattr(a, "cuda_stream") else a
-                        for a in args))
+            return fn(*(convert(a, t, i + 1 == len(types)) for i, (a, t) in enumerate(zip(args, types))))
 
         return call
 

@@ -97,3 +97,18 @@ def test_frozen_wrappers_are_recorded():
     with pytest.raises(capi.CrbError):
         call()
     assert not isinstance(capi._calls, capi._Converted)
+
+
+def test_frozen_wrappers_keep_numbers_that_have_an_address():
+    """A factor or a size that is a tensor of one element is that number in a frozen call too, not its address."""
+    import torch
+
+    lib = capi.load()
+    rec = capi._Recorder(lib)
+    calls = capi._Converted(rec)
+    assert calls.crb_momentum_apply(None, None, None, torch.tensor(4), torch.tensor(0.25), 0.5, torch.tensor(1.0), None) == capi.CRB_ENULL
+    assert [float(a) for a in rec.calls[0][1][3:7]] == [4, 0.25, 0.5, 1.0]
+    call = capi.frozen(lambda: pytest.raises(capi.CrbError, capi.tensor_fill, None, torch.tensor(2.0), torch.tensor(3)))
+    with pytest.raises(capi.CrbError) as e:
+        call()
+    assert e.value.status == capi.CRB_ENULL
