@@ -1,17 +1,19 @@
 """Python binding of the C ABI declared in include/crusader_hip.h.
 
 It loads the in-tree ``lib/libcrusader_hip.so`` and passes raw device pointers (``tensor.data_ptr()``) and sizes straight
-through: the launching calls by way of ``lib/_crb_calls.so`` (csrc/crb_calls.cpp), size queries, the few calls on host
-tables and prepared ones by ctypes. There is no CPU fallback: if either library is missing, loading raises.
+through: the launching calls by way of the module ``lib/_crb_calls`` (csrc/crb_calls.cpp, built for one interpreter), size
+queries, the few calls on host tables and prepared ones by ctypes. Without that module every call goes by ctypes, a few
+microseconds slower. There is no CPU fallback: if the library is missing, loading raises.
 """
 import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libcrusader_hip.so")
-CALLS_PATH = os.path.join(_HERE, "lib", "_crb_calls.so")
+CALLS_PATH = os.path.join(_HERE, "lib", "_crb_calls" + importlib.machinery.EXTENSION_SUFFIXES[0])
 
 CRB_OK = 0
 CRB_EINVAL_SHAPE = -1
@@ -131,17 +133,22 @@ def load():
     """Load the HIP library (once) and attach signatures. Raises OSError if it has not been built."""
     global _lib, _calls
     if _lib is None:
-        if not (os.path.exists(LIB_PATH) and os.path.exists(CALLS_PATH)):
+        if not os.path.exists(LIB_PATH):
             raise OSError(f"{LIB_PATH} not found: build it with `make -C crusaderbackend_amd/csrc`")
         lib = ctypes.CDLL(LIB_PATH)
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
-        loader = importlib.machinery.ExtensionFileLoader("_crb_calls", CALLS_PATH)
-        calls = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_crb_calls", CALLS_PATH, loader=loader))
-        loader.exec_module(calls)
-        calls.bind(ConvGeom, ctypes.ArgumentError, _number)
+        if os.path.exists(CALLS_PATH):
+            loader = importlib.machinery.ExtensionFileLoader("_crb_calls", CALLS_PATH)
+            calls = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_crb_calls", CALLS_PATH, loader=loader))
+            loader.exec_module(calls)
+            calls.bind(ConvGeom, ctypes.ArgumentError, _number)
+        else:
+            warnings.warn(f"{CALLS_PATH} not found (`make -C crusaderbackend_amd/csrc PYTHON=...` builds it where that interpreter's headers are): every "
+                          "call goes by ctypes, 2 to 3 us slower", RuntimeWarning, stacklevel=2)
+            calls = _Converted(lib)
         _lib, _calls = lib, calls
     return _lib
 
@@ -215,7 +222,8 @@ class _Recorder:
 
 
 class _Converted:
-    """Stands in for the native calls while `frozen` records: the same arguments, converted for the library's ctypes functions."""
+    """Stands in for the native calls, while `frozen` records or where they are not built: the same arguments, converted for the library's
+    ctypes functions."""
 
     def __init__(self, lib):
         self._lib = lib

@@ -1,6 +1,10 @@
 """The launching entry points as Python callables (csrc/crb_calls.cpp): the same calls as by ctypes, taken and refused where those are (no GPU is touched)."""
 import ctypes
+import importlib.util
+import os
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -112,3 +116,31 @@ def test_frozen_wrappers_keep_numbers_that_have_an_address():
     with pytest.raises(capi.CrbError) as e:
         call()
     assert e.value.status == capi.CRB_ENULL
+
+
+def test_the_library_is_built_and_loaded_without_python_headers(tmp_path):
+    """The C library's build needs no Python; where the module of native calls is not built, or for another interpreter, calls go by ctypes."""
+    csrc = os.path.join(os.path.dirname(capi.__file__), "csrc")
+
+    def recipes(python):
+        out = subprocess.run(["make", "-n", "-B", "-C", csrc, "PYTHON=" + python], capture_output=True, text=True, check=True).stdout
+        return "libcrusader_hip.so" in out, "_crb_calls" in out
+
+    assert recipes(str(tmp_path / "python3")) == (True, False)
+    assert recipes(sys.executable)[0] and os.path.basename(capi.CALLS_PATH).startswith("_crb_calls.")
+
+    spec = importlib.util.spec_from_file_location("capi_by_ctypes", capi.__file__)
+    other = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(other)
+    other.CALLS_PATH = str(tmp_path / "_crb_calls.so")
+    with pytest.warns(RuntimeWarning, match="ctypes"):
+        other.load()
+    g = other.ConvGeom.make(2, 3, 8, 9, 4, 3, 3, 1, 1, 1, 1)
+    for call in (lambda: other.sgemm_nn(None, None, None, 1, 1, 1), lambda: other.conv_fwd(None, None, None, None, g), lambda: other.tensor_fill(None, 0.5, 4)):
+        for c in (call, other.frozen(lambda: pytest.raises(other.CrbError, call))):
+            with pytest.raises(other.CrbError) as e:
+                c()
+            assert e.value.status == other.CRB_ENULL
+    other.LIB_PATH, other._lib = str(tmp_path / "libcrusader_hip.so"), None
+    with pytest.raises(OSError, match="libcrusader_hip.so"):
+        other.load()
