@@ -18,9 +18,9 @@
 namespace crb {
 
 // WM x WN waves of 32 channels x 64 pixels each.
-template <int F_, int S_, int WM_, int WN_, int MAXPX_>
+template <int WM_, int WN_, int MAXPX_>
 struct ConvWideCfg {
-    static constexpr int F = F_, FH = F_, FW = F_, S = S_, WM = WM_, WN = WN_, MAXPX = MAXPX_;
+    static constexpr int F = 3, FH = F, FW = F, S = 1, WM = WM_, WN = WN_, MAXPX = MAXPX_;
     static constexpr int NT = F * F, CI = 32, KG = 1, KO = CI / 8, NTH = 64 * WM * WN;
     static constexpr int OCT = 32 * WM, PXT = 64 * WN;
     static constexpr int PART = KO * MAXPX * 16, STAGE = kSplit * PART;  // bytes

@@ -683,7 +683,7 @@ inline PendingSum pending_sum(const float *partial, float *C, u32 count, u32 spl
     else p.lanes = 1000 + (count >= 32u * 512u ? 32 : count >= 16u * 256u ? 16 : 8), p.blocks = ceil_div(count, p.lanes - 1000);
     return p;
 }
-constexpr int kPendingSumFloats = (256 / 8) * (4 * 8 + 4);  // LDS; the other forms take less
+constexpr int kPendingSumFloats = kReduceVecLds;  // (reduce_block takes 256)
 __device__ __forceinline__ void pending_sum_block(const PendingSum &p, u32 block, float *red) {
     const ReduceEpi e{nullptr, 1, 1, EPI_ACCUM};
     const FastDiv one;
