@@ -261,15 +261,25 @@ inline bool tiny_gemm_fits(u32 M, u32 N, u32 K, u32 batch, bool kfast = false) {
 }
 
 // Products that would go to the fp32 engine: where that has too few tiles for the chip or cuts the contraction, a workgroup for every 16 x 16 block is
-// ahead as long as the chip takes the blocks in two rounds of eight on a CU and they re-read no more than `most` k of their operands (us, engine / here:
+// ahead as long as the chip takes the blocks in two rounds of eight on a CU and they re-read no more than `blocks_k` k of their operands (us, engine / here:
 // 128 x 96 x 352 11.3 / 3.7, 41 x 315 x 818 12.0 / 4.2, 2304 x 144 x 224 11.0 / 5.9, 1088 x 256 x 64 4.7 / 3.4, 60 x 3268 x 526 12.5 / 11.7; beyond,
-// 1958 x 802 x 18, 6273 blocks, 6.5 / 9.9). 73 random products 0.59 of the time in the mean, none slower.
-// `most` goes by the form: 2^20 for NN, which the engine is slowest at (368 x 784 x 896 19.2 / 13.8, 3136 x 80 x 608 17.2 / 10.0), 5 * 2^17 for NT (117 x 951 x
+// 1958 x 802 x 18, 6273 blocks, 6.5 / 9.9).
+// `blocks_k` goes by the form: 2^20 for NN, which the engine is slowest at (368 x 784 x 896 19.2 / 13.8, 3136 x 80 x 608 17.2 / 10.0), 5 * 2^17 for NT (117 x 951 x
 // 1284 15.6 / 9.0; beyond 64 x 3584 x 896 14.0 / 15.1), 27 * 2^14 for TN (beyond 1984 x 64 x 960 10.8 / 11.1, 1064 x 124 x 1640 16.2 / 20.1).
-constexpr u32 kTinyMostNN = 1u << 20, kTinyMostNT = 5u << 17, kTinyMostTN = 27u << 14;
-inline bool tiny_gemm_beats_engine(u32 M, u32 N, u32 K, u32 batch, u32 most) {
-    const uint64_t blocks = uint64_t(ceil_div(M, 16u)) * ceil_div(N, 16u);
-    return batch == 1 && K <= 2048u && blocks <= 2048u && blocks * K <= most;
+// Blocks go to the XCDs in turn, so each of these reads all rows of A that its columns meet and, unless a row of blocks is a multiple of eight, all columns
+// of B: a number of floats from beyond the L2s that is held to `far`. Sixteen waves (more than 1024 terms) hide less of it, two workgroups on a CU instead of eight, and
+// are held to `far_long`. Beyond, 103 x 3732 x 640 16.5 / 24.5, 64 x 2240 x 1536 14.9 / 22.2, NT 1104 x 64 x 2016 11.4 / 17.2, TN 1536 x 64 x 1152 10.9 / 13.2. NT rows that
+// are no whole quads, which the engine loads a float at a time, gain in all cases. Of 24000 random products of up to 2048 blocks and terms, 2^14 to 2^20 block rows (0.63 / 0.69 / 0.83
+// of the engine's time in the mean, NN / TN / NT), 22 are slower by more than a twentieth, by 1.23 at most; of 9000 of all sizes none.
+struct TinyLines {
+    u32 blocks_k, far, far_long;
+};
+constexpr TinyLines kTinyNN{1u << 20, 10000000, 8000000}, kTinyTN{27u << 14, 10000000, 6000000}, kTinyNT{5u << 17, ~0u, 8000000}, kTinyNTRagged{5u << 17, ~0u, ~0u};
+inline bool tiny_gemm_beats_engine(u32 M, u32 N, u32 K, u32 batch, const TinyLines &most) {
+    const uint64_t tm = ceil_div(M, 16u), tn = ceil_div(N, 16u), blocks = tm * tn;
+    if (batch != 1 || K > 2048u || blocks > 2048u || blocks * K > most.blocks_k) return false;
+    const uint64_t far = K * (M * (tn < kXcds ? tn : kXcds) + N * (tn % kXcds == 0 ? 1 : tm < kXcds ? tm : kXcds));
+    return far <= (K > 1024u ? most.far_long : most.far);
 }
 
 // Waves of a workgroup, which share its contraction. More of them keep the chains of a long one short, in time (us, 4 / 8 / 16 waves: NT 11 x 2012 x

@@ -2,6 +2,8 @@
 import numpy as np
 import pytest
 
+from tests.util import launched
+
 pytestmark = pytest.mark.gpu
 
 # (M, N, K): blocks that end early, single rows and columns, contractions of one to four groups a wave with 0 to 15 k behind them, waves without work,
@@ -53,3 +55,20 @@ def test_dense_layers(dev, batch, IN, OUT):
     ref = (x @ w.t() + b.cpu().double()).relu(), d @ w, dW0.cpu().double() + d.t() @ x, dB0.cpu().double() + d.sum(0)
     for g, r, K in zip((Y, dX, dW, dB), ref, (IN, OUT, batch, batch)):
         assert (g.cpu().double() - r).norm() <= 2 * np.sqrt(K + 2) * 2.0**-25 * r.norm()
+
+
+# (form, M, N, K), taken from the engine or left to it: few rows of many columns, of which every XCD reads all, and the same where eight blocks or a multiple
+# make a row of C; contractions of more than 1024 terms, shared by sixteen waves; few columns of many rows
+LINES = [("nn", 103, 3732, 640, False), ("nn", 64, 2240, 1536, False), ("nn", 64, 1600, 1024, True), ("nn", 64, 2048, 1536, True), ("nn", 726, 188, 1812, False),
+         ("nn", 368, 784, 896, True), ("nt", 1104, 64, 2016, False), ("nt", 118, 770, 1446, True), ("nt", 64, 1024, 1284, True), ("tn", 1536, 64, 1152, False), ("tn", 1536, 64, 704, True),
+         ("tn", 45, 1373, 1608, False)]
+
+
+@pytest.mark.parametrize("form,M,N,K,taken", LINES, ids=lambda v: str(v))
+def test_products_taken_from_the_engine(dev, form, M, N, K, taken):
+    import torch
+    from crusaderbackend_amd import capi
+
+    A, B, C = (torch.zeros(n, device=dev) for n in (M * K, N * K, M * N))
+    names = [name for name, _ in launched(dev, lambda s: getattr(capi, "sgemm_" + form)(A, B, C, M, N, K, stream=s))]
+    assert any("tiny_gemm_kernel" in n for n in names) == taken, names

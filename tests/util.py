@@ -65,3 +65,45 @@ def to_dev(a, dev):
 
 def to_np(t):
     return t.detach().cpu().numpy()
+
+
+def launched(dev, fn):
+    """The kernels that `fn(stream)` launches, as (name, workgroups): recorded into a graph that is read and never run. Scratch that the call grows has to
+    be there: make the call on the same stream once before."""
+    import ctypes
+
+    import torch
+
+    class Params(ctypes.Structure):  # hipKernelNodeParams
+        _fields_ = [("block", ctypes.c_uint32 * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint32 * 3), ("params", ctypes.c_void_p),
+                    ("shared", ctypes.c_uint32)]
+
+    with open("/proc/self/maps") as maps:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    hip.hipKernelNameRefByPtr.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+
+    def ok(status):
+        assert status == 0, f"HIP status {status}"
+
+    stream = torch.cuda.Stream(device=dev)
+    fn(stream)
+    torch.cuda.synchronize()
+    at, graph = ctypes.c_void_p(stream.cuda_stream), ctypes.c_void_p()
+    ok(hip.hipStreamBeginCapture(at, 1))  # (this thread's calls)
+    try:
+        fn(stream)
+    finally:
+        ok(hip.hipStreamEndCapture(at, ctypes.byref(graph)))
+    n = ctypes.c_size_t()
+    ok(hip.hipGraphGetNodes(graph, None, ctypes.byref(n)))
+    nodes, found = (ctypes.c_void_p * n.value)(), []
+    ok(hip.hipGraphGetNodes(graph, nodes, ctypes.byref(n)))
+    for node in nodes:
+        kind, p = ctypes.c_int(), Params()
+        ok(hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)))
+        if kind.value == 0:  # (hipGraphNodeTypeKernel)
+            ok(hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)))
+            found.append((hip.hipKernelNameRefByPtr(p.func, at).decode(), p.grid[0] * p.grid[1] * p.grid[2]))
+    ok(hip.hipGraphDestroy(graph))
+    return found
