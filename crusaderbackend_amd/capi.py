@@ -319,7 +319,7 @@ def conv_wgrad_workspace_bytes(geom):
 
 
 def conv_wgrad(dY, X, dW, geom, workspace=None, stream=None):
-    nbytes = 0 if workspace is None else workspace.nbytes
+    nbytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
     check(_calls.crb_conv_wgrad(dY, X, dW, geom, workspace, nbytes, stream))
 
 
@@ -333,7 +333,7 @@ NOALLOC_SCRATCH_BYTES = 8 << 20  # CRB_NOALLOC_SCRATCH_BYTES
 
 def bind_workspace(workspace, stream=None):
     """Bind `workspace` (a torch tensor, or None to unbind) as the split scratch of calls on `stream`."""
-    nbytes = 0 if workspace is None else workspace.nbytes
+    nbytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
     check(load().crb_bind_workspace(_p(workspace), nbytes, _stream(stream)))
 
 
@@ -355,7 +355,7 @@ def conv_bias_grad_workspace_bytes(N, C, HW):
 
 def conv_bwd(W, dY, X, dX, dW, geom, workspace=None, stream=None):
     """Data gradient and weight gradient of one layer in one call (one launch for the residual-network layer shapes)."""
-    nbytes = 0 if workspace is None else workspace.nbytes
+    nbytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
     check(_calls.crb_conv_bwd(W, dY, X, dX, dW, geom, workspace, nbytes, stream))
 
 
@@ -365,7 +365,7 @@ def conv_bwd_slices(geom):
 
 def conv_bwd_sliced(W, dY, X, dX, geom, workspace, stream=None):
     """dX now; the weight gradient stays as conv_bwd_slices(geom) partial sums in `workspace` until sum_slices_multi."""
-    nbytes = workspace.nbytes
+    nbytes = workspace.numel() * workspace.element_size()
     check(_calls.crb_conv_bwd_sliced(W, dY, X, dX, geom, workspace, nbytes, stream))
 
 

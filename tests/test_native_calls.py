@@ -96,6 +96,27 @@ def test_numbers_that_ctypes_takes_are_taken():
             capi.sgemm_nn(t, t, t, bad, 0, 1)
 
 
+def test_workspaces_need_no_more_than_a_size_and_an_address():
+    """What has data_ptr, numel and element_size is a workspace; nothing else is asked of it."""
+
+    class Workspace:
+        def data_ptr(self):
+            return 4096
+
+        def numel(self):
+            return 1 << 20
+
+        def element_size(self):
+            return 4
+
+    ws, g = Workspace(), capi.ConvGeom.make(2, 3, 8, 9, 4, 3, 3, 1, 1, 1, 1)
+    for call in (lambda: capi.conv_wgrad(None, ws, ws, g, workspace=ws), lambda: capi.conv_bwd(None, ws, ws, ws, ws, g, workspace=ws),
+                 lambda: capi.conv_bwd_sliced(None, ws, ws, ws, g, ws)):
+        with pytest.raises(capi.CrbError) as e:
+            call()
+        assert e.value.status == capi.CRB_ENULL
+
+
 def test_frozen_wrappers_are_recorded():
     call = capi.frozen(lambda: pytest.raises(capi.CrbError, capi.sgemm_nt, None, None, None, 1, 1, 1))
     with pytest.raises(capi.CrbError):
