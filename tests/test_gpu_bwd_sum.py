@@ -1,15 +1,26 @@
 """crb_conv_bwd where both gradients run on split operands: the slices' sum rides on the launch that splits the filters. The bits of the two calls."""
 import pytest
 
+from tests.util import launched
+
 pytestmark = pytest.mark.gpu
 
-# (N, IC, H, W, OC, F, stride, pad): sums of whole quads and not, of each number of lanes, filters in steps of 16 and 32 channels, K groups, residue classes
+# (N, IC, H, W, OC, F, stride, pad), how the slices are summed (rows of 16 bytes by 8 to 64 lanes, or as many single results from 1000 on): each way, filters in
+# steps of 16 and 32 channels, K groups, residue classes
 SHAPES = [(32, 64, 28, 28, 64, 3, 1, 1), (40, 64, 44, 40, 64, 3, 1, 1), (12, 64, 24, 24, 96, 3, 1, 1), (9, 41, 31, 33, 65, 3, 1, 1), (4, 256, 14, 14, 256, 3, 1, 1),
-          (24, 30, 61, 47, 75, 5, 2, 2), (16, 64, 28, 28, 128, 3, 2, 1), (7, 64, 21, 19, 48, 5, 1, 2), (8, 33, 20, 22, 33, 3, 1, 0)]
+          (24, 30, 61, 47, 75, 5, 2, 2), (16, 64, 28, 28, 128, 3, 2, 1), (7, 64, 21, 19, 48, 5, 1, 2), (31, 24, 35, 24, 46, 3, 1, 1), (38, 26, 6, 20, 47, 3, 1, 1),
+          (77, 25, 30, 55, 18, 3, 1, 1)]
+LANES = [16, 16, 32, 1032, 64, 1032, 32, 32, 8, 1016, 1008]
 
 
-@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
-def test_the_two_calls(dev, shape):
+def lanes(slices, count):
+    if count % 4 == 0:
+        return 8 if slices >= 64 else 16 if slices >= 32 else 32 if slices >= 16 or count < 1 << 17 else 64
+    return 1032 if count >= 1 << 14 else 1016 if count >= 1 << 12 else 1008
+
+
+@pytest.mark.parametrize("shape,way", zip(SHAPES, LANES), ids=lambda s: "x".join(map(str, s)) if isinstance(s, tuple) else str(s))
+def test_the_two_calls(dev, shape, way):
     import torch
     from crusaderbackend_amd import capi
 
@@ -32,17 +43,28 @@ def test_the_two_calls(dev, shape):
     ws = torch.empty(need // 4 + 4, device=dev)
     check(workspace=ws)
     check()
+    assert lanes(need // (4 * dW.numel()), dW.numel()) == way
+    a, b = torch.empty_like(dX), torch.empty_like(dW)
+    kernels = [k for k, _ in launched(dev, lambda stream: capi.conv_bwd(Wt, dY, X, a, b, g, workspace=ws, stream=stream))]
+    assert not any("splitk_reduce" in k for k in kernels), kernels
+    assert any("filters_kernelILb1ELb1E" in k or "class_filters_kernelILb1E" in k for k in kernels), kernels
     side, shared = torch.cuda.Stream(device=dev), torch.empty((need + capi.conv_dgrad_workspace_bytes(g)) // 4 + 64, device=dev)
     try:
         capi.bind_workspace(shared, stream=side)  # split filters and slices in one place
         check(side, shared)
         capi.bind_workspace(shared[:64], stream=side)  # no room for split filters
         try:
-            check(side, ws)
+            capi.conv_dgrad(Wt, dY, a, g, stream=side)
+            alone = capi.CRB_OK
         except capi.CrbError as e:
-            assert e.status == capi.CRB_EWORKSPACE
-            with pytest.raises(capi.CrbError):  # where the data gradient alone is refused too
-                capi.conv_dgrad(Wt, dY, dX, g, stream=side)
+            alone = e.status
+        if alone == capi.CRB_OK:
+            check(side, ws)
+        else:  # the data gradient is refused alone, and so is the pair
+            assert alone == capi.CRB_EWORKSPACE
+            with pytest.raises(capi.CrbError) as e:
+                check(side, ws)
+            assert e.value.status == alone
     finally:
         capi.bind_workspace(None, stream=side)
 

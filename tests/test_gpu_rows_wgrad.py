@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 from oracle import seblas_oracle as orc
-from tests.util import assert_close, normal, to_dev, to_np
+from tests.util import assert_close, launched, normal, to_dev, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -41,6 +41,9 @@ def test_rows_weight_gradient_edges(dev, shape):
     torch.cuda.synchronize()
     assert_close(to_np(dW), orc.convError(dY, X, dW0, 1, 1, 1, 1), N * H * W, f"weight gradient {shape}")
     assert torch.equal(dW, again)
+    words = 4 if W % 4 == 0 and off % 4 == 0 else 2 if off % 2 == 0 else 1
+    kernels = [k for k, _ in launched(dev, lambda stream: capi.conv_wgrad(dYd, Xd, again, g, stream=stream))]
+    assert any(f"rows_wgrad_kernelILi{words}E" in k for k in kernels), kernels
 
 
 @pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[2], SHAPES[3], SHAPES[9]], ids=lambda s: "x".join(map(str, s)))
