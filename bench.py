@@ -129,8 +129,8 @@ class Layer:
         self.capi.conv_dgrad(W, dY, dX, self.g)
         self.capi.conv_wgrad(dY, X, dW, self.g, workspace=self.ws)
 
-    # The per-call timing loops issue prepared calls (arguments converted once): through the plain ctypes wrappers a loop
-    # is bound by 3.5-4.5 us of argument conversion per call, more than the small layers' kernels take.
+    # The per-call timing loops issue prepared calls (arguments converted once): by ctypes, which the plain
+    # wrappers take where the native calls are not built, conversion costs 3.5-4.5 us per call, more than the small layers' kernels take.
     def _prepare(self):
         c, ws = self.capi, self.ws
         nbytes = 0 if ws is None else ws.numel() * ws.element_size()

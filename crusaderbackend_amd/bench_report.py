@@ -67,8 +67,8 @@ VGG16_CONVS = [(3, 32, 64), (64, 32, 64), (64, 16, 128), (128, 16, 128), (128, 8
 
 
 def _settled(torch, capi, event_time_ms, fn, reps):
-    """One row's time: the call is frozen (argument conversion done once: a plain wrapper call costs the host 3.5-4.5 us,
-    more than the shortest kernels take), repeated until the timed region is at least a millisecond, three such averages.
+    """One row's time: the call is frozen (argument conversion done once: by ctypes a plain wrapper call costs the host
+    3.5-4.5 us, more than the shortest kernels take), repeated until the timed region is at least a millisecond, three such averages.
     Returns (smallest, mean). Rows follow tensor allocation and host work during which the device clock drops, and its
     ramp back up takes tens of milliseconds (a dense layer timed right after its tensors were made read 13 % longer than
     the same call timed a little later), so a row first runs untimed for about 20 ms."""

@@ -80,8 +80,8 @@ struct BatchWalk {
 // BATCH: a K-concatenated batch of more than one entry. Without one, whole groups of sixteen k are loaded from addresses that are a lane's
 // constant offset behind a uniform one and need no vector arithmetic (a division by the entry's length, a 64-bit product and the tests of
 // row, column and k for every load were most of the kernel's instructions). Us, before / after: NN 128 x 512 x 512 6.6 / 4.0, 256 x 256 x 1024 11.2 /
-// 5.8, TN 128 x 512 x 512 5.4 / 3.3, 128 x 128 x 2048 15.1 / 7.1, NT 128 x 512 x 512 4.5 / 4.0, 256 x 256 x 1024 6.7 / 5.7; the same bits. What bounds
-// it now is a launch (3 us of these) and the reading of every block's rows from L2.
+// 5.8, TN 128 x 512 x 512 5.4 / 3.3, 128 x 128 x 2048 15.1 / 7.1, NT 128 x 512 x 512 4.5 / 4.0, 256 x 256 x 1024 6.7 / 5.7; up to 640 terms the same bits (beyond
+// them the contraction is cut over more waves: tiny_gemm_waves). What bounds it now is a launch (3 us of these) and the reading of every block's rows from L2.
 template <bool KVEC, bool BATCH, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES) tiny_gemm_kernel(TinyGemmArgs a) {
     __shared__ __attribute__((aligned(16))) float red[WAVES * 256];
@@ -284,7 +284,9 @@ inline bool tiny_gemm_beats_engine(u32 M, u32 N, u32 K, u32 batch, const TinyLin
 
 // Waves of a workgroup, which share its contraction. More of them keep the chains of a long one short, in time (us, 4 / 8 / 16 waves: NT 11 x 2012 x
 // 3053 15.1 / 10.5 / 10.8, 13 x 107 x 2127 7.5 / 6.8 / 7.0) and in roundings (TN 112 x 112 x 1200 3.2 / 2.3 / 1.8e-7 from float64, the engine, which
-// cuts it, 2.2e-7; 502 x 15 x 614 2.3e-7 on either).
+// cuts it, 2.2e-7; 502 x 15 x 614 2.3e-7 on either). Up to 640 terms four stay: these products were here before there were others, the bits of a VGG-16 head among
+// them, and eight from 257 on would bring little: 6000 random products 0.99 of the time in the mean, 110 slower by more than a twentieth, by 1.23 at most, nearly all of
+// these under 480 terms (480 to 640: 0.98).
 // A batch stays on four, whose loads are more arithmetic than a chain (NTA 82 x 14 x 10 * 225 on sixteen: a 1x1 layer's three passes 35.6 -> 41.4).
 inline u32 tiny_gemm_waves(u32 K, bool batch) { return batch || K <= 640u ? 4u : (K <= 1024u ? 8u : 16u); }
 
